@@ -73,6 +73,9 @@ struct Options {
   int64_t rank_stagger_bytes = 0;
   int64_t rank_stride_align = 16384;  // rank regions start on multiples of this (read when an arena is created)
   int64_t alloc_align = 16384;        // so do symmetric allocations at least this large
+  int64_t cached_arena_bytes = 192ll << 20;   // see cache_policy
+  int64_t cached_output_bytes = 64ll << 20;
+  int64_t cached_gradient_bytes = 128ll << 20;
 };
 Options g_opt;
 std::mutex g_opt_mu;
@@ -97,6 +100,9 @@ int64_t* option_slot(const char* name) {
   if (!strcmp(name, "store_blocks_per_cu")) return &g_opt.store_blocks_per_cu;
   if (!strcmp(name, "store_resident_cap")) return &g_opt.store_resident_cap;
   if (!strcmp(name, "publish_resident_cap")) return &g_opt.publish_resident_cap;
+  if (!strcmp(name, "cached_arena_bytes")) return &g_opt.cached_arena_bytes;
+  if (!strcmp(name, "cached_output_bytes")) return &g_opt.cached_output_bytes;
+  if (!strcmp(name, "cached_gradient_bytes")) return &g_opt.cached_gradient_bytes;
   return nullptr;
 }
 
@@ -128,7 +134,7 @@ struct odc_arena {
   bool dry_run = false;
   std::map<uint64_t, uint64_t> live;  // offset -> size (rounded)
   std::map<uint64_t, uint64_t> free_; // offset -> size, coalesced
-  uint64_t in_use = 0;
+  std::atomic<uint64_t> in_use{0};  // changed under mu, read by launches without it
   uint64_t high_water = 0;
   std::mutex mu;
 };
@@ -206,6 +212,36 @@ uint32_t grid_for(const odc_arena* a, int64_t blocks_per_cu, uint32_t n_tiles, b
   const uint64_t g = (uint64_t)a->n_cu * (uint64_t)blocks_per_cu;
   return (uint32_t)std::min<uint64_t>(g, n_tiles);
 }
+
+// What a launch leaves in the caches. Nontemporal accesses stream fastest when nothing will be
+// found again (a decoder layer's 2.2 GB: +15 % over plain ones), but they also pass by what IS in
+// the 256 MB last-level cache and leave nothing there for the kernel that comes next. Measured as
+// pairs, in us (16 Mi elements at W = 8, 24 sets of buffers in turn so that nothing else stays
+// cached / 3 sets), nontemporal -> plain on the stream named:
+//   * the gradient, written by the backward just before: fill + accumulate 35.7 -> 33.3 / 35.5 -> 32.9,
+//     fill + store 28.8 -> 24.3 / 28.7 -> 23.8 (nine items), 64 Mi elements 126.8 -> 115.7. Without
+//     the fill 64 Mi elements lose 1.5 %, beyond that nothing is left of the gradient when it is
+//     read, so the line is 128 MiB of gradient.
+//   * the gathers' output, read by the forward or backward just after: gather + read 20.3 -> 18.7 /
+//     19.2 -> 17.5, still 64.7 -> 62.3 at 64 Mi elements, but the gather alone is then 42.1 -> 45.8
+//     (22.1 -> 19.1 at 32 Mi): the line is 64 MiB of output.
+//   * shards and accumulations come back only in the next microbatch, so what counts is whether ALL
+//     symmetric memory in use stays in the cache from one to the next: with 72 MB of it (4 Mi
+//     elements, 3 sets) fill + accumulate 12.7 -> 10.8 and accumulate alone 8.9 -> 7.9, with 144 MB
+//     accumulate alone 14.6 -> 12.4 and gather alone 7.0 -> 6.2; with 600 MB (24 sets) fill +
+//     accumulate 12.8 -> 13.1 and gather + read 7.4 -> 8.0. The line is 192 MiB of the 256.
+// A store does not read the accumulation and keeps it nontemporal (level at best when plain); so does
+// the converting gather with its output unless the arena fits: what the reader gains there (nine
+// items: nothing) the gather loses (17.9 -> 19.8).
+CachePolicy cache_policy(const odc_arena* a, const Options& opt, uint64_t read_bytes, int64_t read_line,
+                         uint64_t written_bytes, int64_t written_line) {
+  const bool arena_fits = a->in_use.load(std::memory_order_relaxed) * a->world <= (uint64_t)opt.cached_arena_bytes;
+  CachePolicy p;
+  p.read = read_line < 0 ? arena_fits : read_bytes <= (uint64_t)read_line;
+  p.written = written_line < 0 ? arena_fits : written_bytes <= (uint64_t)written_line;
+  return p;
+}
+constexpr int64_t kSymmetric = -1;  // a line: the stream lies in symmetric memory
 
 // One-workgroup-per-tile launches are dealt out by the hardware dispatcher, which keeps as many
 // workgroups resident as fit. Fewer resident workgroups (a smaller window of memory in flight)
@@ -536,6 +572,9 @@ int odc_gather(odc_arena* a, const odc_gather_item* items, uint32_t n_items, uin
     if (n < 0) return n;
     if (n == 0) continue;
     bool ragged = false;
+    uint64_t shard_bytes = 0;
+    for (uint32_t k = 0; k < L.tt.n_items; ++k) shard_bytes += L.item[k].seg_bytes;
+    L.policy = cache_policy(a, opt, 0, kSymmetric, shard_bytes * a->world, opt.cached_output_bytes);
     for (uint32_t k = 0; k < L.tt.n_items; ++k)
       ragged |= (((uintptr_t)L.item[k].dst | L.item[k].src_off | L.item[k].seg_bytes) & 15u) != 0;
     const uint32_t grid = grid_for(a, opt.gather_blocks_per_cu, L.tt.n_tiles, ragged);
@@ -583,6 +622,7 @@ int odc_gather_cast(odc_arena* a, const odc_gather_cast_item* items, uint32_t n_
         });
     if (n < 0) return n;
     if (n == 0) continue;
+    L.policy = cache_policy(a, opt, 0, kSymmetric, 0, kSymmetric);
     const uint32_t grid = grid_for(a, opt.gather_blocks_per_cu, L.tt.n_tiles);
     const uint32_t lds = lds_claim_for(a, opt.cast_resident_cap, grid, L.tt.n_tiles);
     if (int rc = launch_tiles(a, L, grid, [&] {
@@ -629,6 +669,7 @@ int odc_convert(odc_arena* a, const odc_convert_item* items, uint32_t n_items, i
         });
     if (n < 0) return n;
     if (n == 0) continue;
+    L.policy = cache_policy(a, opt, 0, kSymmetric, 0, kSymmetric);
     const uint32_t grid = grid_for(a, opt.gather_blocks_per_cu, L.tt.n_tiles);
     const uint32_t lds = lds_claim_for(a, opt.cast_resident_cap, grid, L.tt.n_tiles);
     if (int rc = launch_tiles(a, L, grid, [&] {
@@ -765,6 +806,9 @@ int scatter_launch(odc_arena* a, const odc_accum_item* items, uint32_t n_items, 
       ragged |= (L.item[k].acc_off & 127u) != 0 || ((L.item[k].seg_elems * ab) & 127u) != 0 ||
                 ((L.item[k].seg_elems * gb) & 127u) != 0 || ((uintptr_t)L.item[k].grad & 127u) != 0 ||
                 L.item[k].grad_elems != L.item[k].seg_elems * a->world;
+    uint64_t grad_elems = 0;
+    for (uint32_t k = 0; k < L.tt.n_items; ++k) grad_elems += L.item[k].grad_elems;
+    L.policy = cache_policy(a, opt, grad_elems * gb, opt.cached_gradient_bytes, 0, kSymmetric);
     int64_t blocks_per_cu = store ? opt.store_blocks_per_cu : opt.accum_blocks_per_cu;
     if (blocks_per_cu < 0)
       blocks_per_cu = L.tt.n_tiles < (uint64_t)opt.accum_persistent_below_tiles * segments ? 1 : 0;

@@ -19,9 +19,10 @@
 // are read with scalar loads, so a call needs no device-side work list, no host->device copy and
 // no allocation; longer item lists are split over several launches.
 //
-// Each wavefront issues its 2 or 4 independent 128-bit nontemporal loads per stream before the
-// first store: on this part the nontemporal hint on both loads and stores is worth ~15 % over
-// plain accesses for these single-touch streams. Deeper unrolling or prefetching the next tile
+// Each wavefront issues its 2 or 4 independent 128-bit loads per stream before the first store.
+// Streams larger than the 256 MB last-level cache are nontemporal on both sides (worth ~15 % over
+// plain accesses there); what fits the cache and was just produced, or is about to be consumed, is
+// left in it (cache_policy in odc_host.cpp). Deeper unrolling or prefetching the next tile
 // measured slower: the memory system prefers a small window to more requests in flight.
 // Workgroup i runs on XCD i % 8; binding XCDs to address classes (256 B .. 64 KiB granules)
 // changed nothing measurable and giving every XCD one contiguous eighth of the tiles costs the
@@ -69,15 +70,28 @@ template <class V> struct Unaligned;
 template <> struct Unaligned<u32x4> { typedef u32x4_u type; };
 template <> struct Unaligned<u32x2> { typedef u32x2_u type; };
 
-template <class V>
-__device__ __forceinline__ V load_stream(const uint8_t* p) {  // nontemporal, any alignment
-  return __builtin_nontemporal_load(reinterpret_cast<const typename Unaligned<V>::type*>(p));
+// kCached: a plain access, which leaves its line in the caches; otherwise nontemporal. Which one a
+// stream of a launch takes is the host's choice (cache_policy in odc_host.cpp).
+template <bool kCached, class V>
+__device__ __forceinline__ V load_any(const uint8_t* p) {  // any alignment
+  const auto* q = reinterpret_cast<const typename Unaligned<V>::type*>(p);
+  if constexpr (kCached) return *q; else return __builtin_nontemporal_load(q);
+}
+
+template <bool kCached, class V>
+__device__ __forceinline__ V load_vec(const V* p) {  // aligned
+  if constexpr (kCached) return *p; else return __builtin_nontemporal_load(p);
+}
+
+template <bool kCached, class V>
+__device__ __forceinline__ void store_vec(V* p, V v) {  // aligned
+  if constexpr (kCached) *p = v; else __builtin_nontemporal_store(v, p);
 }
 
 // ---- gather -------------------------------------------------------------------------------
 // Everything of a tile that is not a run of kTileVecs whole vectors: the last partial run, the
 // head and the tail. Kept out of line so that the streaming loop stays tight.
-template <int T, int U>
+template <bool kSrcCached, bool kDstCached, int T, int U>
 __device__ __attribute__((noinline)) void gather_edges(uint8_t* d, const uint8_t* s, uint32_t chunk, SegShape g) {
   // Every load of the tile is issued before its first store (a lone resident workgroup would
   // otherwise pay one memory round trip per step).
@@ -93,19 +107,19 @@ __device__ __attribute__((noinline)) void gather_edges(uint8_t* d, const uint8_t
   uint8_t head_byte = 0, tail_byte = 0;
 #pragma unroll
   for (int u = 0; u < U; ++u)
-    if (u * T + tid < left) v[u] = load_stream<u32x4>(sb + (size_t)(u * T + tid) * 16);
+    if (u * T + tid < left) v[u] = load_any<kSrcCached, u32x4>(sb + (size_t)(u * T + tid) * 16);
   if (do_head) head_byte = s[tid];
   if (do_tail) tail_byte = s[tail_at];
 #pragma unroll
   for (int u = 0; u < U; ++u)
-    if (u * T + tid < left) __builtin_nontemporal_store(v[u], db + u * T + tid);
+    if (u * T + tid < left) store_vec<kDstCached>(db + u * T + tid, v[u]);
   if (do_head) d[tid] = head_byte;
   if (do_tail) d[tail_at] = tail_byte;
 }
 
 // T threads do a tile in U steps of T vectors (T * U = kTileVecs, so the geometry is that of every
 // other kernel); the copies stream best from 512-thread workgroups, of which 4 fit a CU.
-template <int T, int U>
+template <bool kSrcCached, bool kDstCached, int T, int U>
 __global__ __launch_bounds__(T) void gather_kernel(const GatherLaunch launch) {
   static_assert(T * U == (int)kTileVecs, "one tile per workgroup step");
   const uint32_t tid = threadIdx.x;
@@ -128,7 +142,7 @@ __global__ __launch_bounds__(T) void gather_kernel(const GatherLaunch launch) {
       u32x4* db = reinterpret_cast<u32x4*>(d + g.head) + w.v0 + tid;
       u32x4 v[U];
 #pragma unroll
-      for (int u = 0; u < U; ++u) v[u] = load_stream<u32x4>(sb + (size_t)u * T * 16);
+      for (int u = 0; u < U; ++u) v[u] = load_any<kSrcCached, u32x4>(sb + (size_t)u * T * 16);
       // a whole tile that also owns its segment's head or tail (the first and last tile of a
       // ragged segment) reads those bytes with the same round trip as its vectors
       const bool do_head = w.head && tid < g.head;
@@ -138,11 +152,11 @@ __global__ __launch_bounds__(T) void gather_kernel(const GatherLaunch launch) {
       if (do_head) head_byte = s[tid];
       if (do_tail) tail_byte = s[tail_at];
 #pragma unroll
-      for (int u = 0; u < U; ++u) __builtin_nontemporal_store(v[u], db + u * T);
+      for (int u = 0; u < U; ++u) store_vec<kDstCached>(db + u * T, v[u]);
       if (do_head) d[tid] = head_byte;
       if (do_tail) d[tail_at] = tail_byte;
     } else if (has_edges(w)) {
-      gather_edges<T, U>(d, s, c.chunk, g);
+      gather_edges<kSrcCached, kDstCached, T, U>(d, s, c.chunk, g);
     }
   }
 }
@@ -277,7 +291,7 @@ template <> struct Quad<f16_tag> {
 // gradient's end may cut is read as elements by the lane that owns it. Nine items of 3 640
 // elements per rank (W = 8, one partial tile each) take 3.8 us instead of 5.4, with gradients that end inside
 // the last rank's segment 4.0 instead of 4.8 (13 889 elements per rank).
-template <class G, class A, bool kStore, int T, int U>
+template <class G, class A, bool kStore, bool kGradCached, bool kAccCached, int T, int U>
 __device__ __attribute__((noinline)) void accum_edges(uint8_t* acc, const uint8_t* grad, uint64_t g_seg,
                                                       uint64_t grad_elems, uint32_t chunk, SegShape g,
                                                       bool body) {
@@ -311,9 +325,9 @@ __device__ __attribute__((noinline)) void accum_edges(uint8_t* acc, const uint8_
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const uint32_t q = u * T + tid;
-    if (q < left && q < whole_quads) graw[u] = load_stream<gvec_t>(grad + (g0 + (uint64_t)q * 4) * kGB);
+    if (q < left && q < whole_quads) graw[u] = load_any<kGradCached, gvec_t>(grad + (g0 + (uint64_t)q * 4) * kGB);
     if constexpr (!kStore) {
-      if (q < left) araw[u] = __builtin_nontemporal_load(ap + q);
+      if (q < left) araw[u] = load_vec<kAccCached>(ap + q);
     }
   }
   if (has_cut) {
@@ -343,7 +357,7 @@ __device__ __attribute__((noinline)) void accum_edges(uint8_t* acc, const uint8_
       if constexpr (!kStore) Quad<A>::widen(araw[u], af);
 #pragma unroll
       for (int k = 0; k < 4; ++k) af[k] = af[k] + gf[k];
-      __builtin_nontemporal_store(Quad<A>::narrow(af), ap + q);
+      store_vec<kAccCached>(ap + q, Quad<A>::narrow(af));
     }
   }
   // (raw zero widens to +0 in every type)
@@ -351,7 +365,7 @@ __device__ __attribute__((noinline)) void accum_edges(uint8_t* acc, const uint8_
   if (do_tail) as[tail_at] = Codec<A>::narrow(Codec<A>::widen(tail_araw) + Codec<G>::widen(tail_graw));
 }
 
-template <class G, class A, bool kStore, int T, int U>
+template <class G, class A, bool kStore, bool kGradCached, bool kAccCached, int T, int U>
 __global__ __launch_bounds__(T) void accum_kernel(const AccumLaunch launch) {
   static_assert(T * U == (int)kTileVecs, "one tile per workgroup step");
   typedef typename Quad<G>::vec_t gvec_t;
@@ -381,10 +395,10 @@ __global__ __launch_bounds__(T) void accum_kernel(const AccumLaunch launch) {
       gvec_t graw[U];
       avec_t araw[U];
 #pragma unroll
-      for (int u = 0; u < U; ++u) graw[u] = load_stream<gvec_t>(gb + (size_t)u * T * sizeof(gvec_t));
+      for (int u = 0; u < U; ++u) graw[u] = load_any<kGradCached, gvec_t>(gb + (size_t)u * T * sizeof(gvec_t));
       if constexpr (!kStore) {
 #pragma unroll
-        for (int u = 0; u < U; ++u) araw[u] = __builtin_nontemporal_load(ap + u * T);
+        for (int u = 0; u < U; ++u) araw[u] = load_vec<kAccCached>(ap + u * T);
       }
 #pragma unroll
       for (int u = 0; u < U; ++u) {
@@ -393,11 +407,11 @@ __global__ __launch_bounds__(T) void accum_kernel(const AccumLaunch launch) {
         if constexpr (!kStore) Quad<A>::widen(araw[u], af);
 #pragma unroll
         for (int k = 0; k < 4; ++k) af[k] = af[k] + gf[k];
-        __builtin_nontemporal_store(Quad<A>::narrow(af), ap + u * T);
+        store_vec<kAccCached>(ap + u * T, Quad<A>::narrow(af));
       }
     }
     if (!whole ? (w.nv != 0 || w.head || w.tail) : (w.head || w.tail))
-      accum_edges<G, A, kStore, T, U>(acc, it.grad, g_seg, it.grad_elems, c.chunk, g, !whole);
+      accum_edges<G, A, kStore, kGradCached, kAccCached, T, U>(acc, it.grad, g_seg, it.grad_elems, c.chunk, g, !whole);
   }
 }
 
@@ -407,7 +421,7 @@ __global__ __launch_bounds__(T) void accum_kernel(const AccumLaunch launch) {
 // segment's size: the converted segments lie back to back), or, with stride = the distance
 // between rank regions and dst inside rank 0's region, the conversion of every rank's shard into
 // a second symmetric buffer.
-template <class S, class D, int T, int U>
+template <class S, class D, bool kCached, int T, int U>
 __device__ __attribute__((noinline)) void cast_edges(uint8_t* d, const uint8_t* s, uint32_t chunk, SegShape g) {
   typedef typename Quad<S>::vec_t svec_t;
   typedef typename Quad<D>::vec_t dvec_t;
@@ -431,7 +445,7 @@ __device__ __attribute__((noinline)) void cast_edges(uint8_t* d, const uint8_t* 
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const uint32_t q = u * T + tid;
-    if (q < left) raw[u] = load_stream<svec_t>(sb + (size_t)q * sizeof(svec_t));
+    if (q < left) raw[u] = load_any<kCached, svec_t>(sb + (size_t)q * sizeof(svec_t));
   }
   if (do_head) head_raw = ss[tid];
   if (do_tail) tail_raw = ss[tail_at];
@@ -441,14 +455,14 @@ __device__ __attribute__((noinline)) void cast_edges(uint8_t* d, const uint8_t* 
     if (q < left) {
       float f[4];
       Quad<S>::widen(raw[u], f);
-      __builtin_nontemporal_store(Quad<D>::narrow(f), dp + q);
+      store_vec<kCached>(dp + q, Quad<D>::narrow(f));
     }
   }
   if (do_head) ds[tid] = Codec<D>::narrow(Codec<S>::widen(head_raw));
   if (do_tail) ds[tail_at] = Codec<D>::narrow(Codec<S>::widen(tail_raw));
 }
 
-template <class S, class D, int T, int U>
+template <class S, class D, bool kCached, int T, int U>
 __global__ __launch_bounds__(T) void cast_gather_kernel(const CastGatherLaunch launch) {
   static_assert(T * U == (int)kTileVecs, "one tile per workgroup step");
   typedef typename Quad<S>::vec_t svec_t;
@@ -475,7 +489,7 @@ __global__ __launch_bounds__(T) void cast_gather_kernel(const CastGatherLaunch l
       dvec_t* dp = reinterpret_cast<dvec_t*>(d + e0 * kDB) + tid;
       svec_t raw[U];
 #pragma unroll
-      for (int u = 0; u < U; ++u) raw[u] = load_stream<svec_t>(sb + (size_t)u * T * sizeof(svec_t));
+      for (int u = 0; u < U; ++u) raw[u] = load_any<kCached, svec_t>(sb + (size_t)u * T * sizeof(svec_t));
       // the head and the tail of the segment, when this whole tile owns them, in the same round trip
       typedef typename Codec<S>::raw_t sraw_t;
       typedef typename Codec<D>::raw_t draw_t;
@@ -491,12 +505,12 @@ __global__ __launch_bounds__(T) void cast_gather_kernel(const CastGatherLaunch l
       for (int u = 0; u < U; ++u) {
         float f[4];
         Quad<S>::widen(raw[u], f);
-        __builtin_nontemporal_store(Quad<D>::narrow(f), dp + u * T);
+        store_vec<kCached>(dp + u * T, Quad<D>::narrow(f));
       }
       if (do_head) ds[tid] = Codec<D>::narrow(Codec<S>::widen(head_raw));
       if (do_tail) ds[tail_at] = Codec<D>::narrow(Codec<S>::widen(tail_raw));
     } else if (has_edges(w)) {
-      cast_edges<S, D, T, U>(d, s, c.chunk, g);
+      cast_edges<S, D, kCached, T, U>(d, s, c.chunk, g);
     }
   }
 }
@@ -624,6 +638,7 @@ __global__ __launch_bounds__(kThreads) void publish_kernel(const PublishLaunch l
 // ------------------------------------------------------------------------------------------------
 // dtype dispatch
 // ------------------------------------------------------------------------------------------------
+typedef void (*gather_fn)(const GatherLaunch);
 typedef void (*accum_fn)(const AccumLaunch);
 typedef void (*cast_gather_fn)(const CastGatherLaunch);
 typedef void (*publish_fn)(const PublishLaunch);
@@ -639,17 +654,42 @@ typedef void (*publish_fn)(const PublishLaunch);
   X(ODC_DTYPE_F32, f32_tag, ODC_DTYPE_F16, f16_tag)     \
   X(ODC_DTYPE_F32, f32_tag, ODC_DTYPE_F32, f32_tag)
 
-accum_fn pick_accum(int g, int a, bool store) {  // (gradient dtype, accumulation dtype)
-#define X(E1, T1, E2, T2) \
-  if (g == E1 && a == E2)                                                            \
-    return store ? accum_kernel<T1, T2, true, kStoreThreads, kStoreUnroll> : accum_kernel<T1, T2, false, kThreads, kUnroll>;
+// (gradient dtype, accumulation dtype). The store form never reads the accumulation and keeps it
+// nontemporal; the read-modify-write keeps it cached only together with the gradient.
+template <class G, class A>
+accum_fn pick_accum_policy(bool store, CachePolicy policy) {
+  if (store)
+    return policy.read ? accum_kernel<G, A, true, true, false, kStoreThreads, kStoreUnroll>
+                       : accum_kernel<G, A, true, false, false, kStoreThreads, kStoreUnroll>;
+  if (policy.read && policy.written) return accum_kernel<G, A, false, true, true, kThreads, kUnroll>;
+  return policy.read ? accum_kernel<G, A, false, true, false, kThreads, kUnroll>
+                     : accum_kernel<G, A, false, false, false, kThreads, kUnroll>;
+}
+
+accum_fn pick_accum(int g, int a, bool store, CachePolicy policy) {
+#define X(E1, T1, E2, T2) if (g == E1 && a == E2) return pick_accum_policy<T1, T2>(store, policy);
   ODC_FOR_EACH_DTYPE_PAIR(X)
 #undef X
   return nullptr;
 }
 
-cast_gather_fn pick_cast_gather(int s, int d) {  // (shard dtype, output dtype)
-#define X(E1, T1, E2, T2) if (s == E1 && d == E2) return cast_gather_kernel<T1, T2, kCopyThreads, kCopyUnroll>;
+gather_fn pick_gather(CachePolicy policy) {
+  if (policy.read)
+    return policy.written ? gather_kernel<true, true, kCopyThreads, kCopyUnroll>
+                          : gather_kernel<true, false, kCopyThreads, kCopyUnroll>;
+  return policy.written ? gather_kernel<false, true, kCopyThreads, kCopyUnroll>
+                        : gather_kernel<false, false, kCopyThreads, kCopyUnroll>;
+}
+
+// Shards and output of the converting gather are cached together or not at all.
+template <class S, class D>
+cast_gather_fn pick_cast_gather_policy(CachePolicy policy) {
+  return policy.read ? cast_gather_kernel<S, D, true, kCopyThreads, kCopyUnroll>
+                     : cast_gather_kernel<S, D, false, kCopyThreads, kCopyUnroll>;
+}
+
+cast_gather_fn pick_cast_gather(int s, int d, CachePolicy policy) {  // (shard dtype, output dtype)
+#define X(E1, T1, E2, T2) if (s == E1 && d == E2) return pick_cast_gather_policy<T1, T2>(policy);
   ODC_FOR_EACH_DTYPE_PAIR(X)
 #undef X
   return nullptr;
@@ -712,20 +752,20 @@ bool is_out_of_memory(int code) { return code == (int)hipErrorOutOfMemory; }
 
 const char* error_string(int code) { return hipGetErrorString(static_cast<hipError_t>(code)); }
 
-bool has_accum(int g, int a) { return pick_accum(g, a, false) != nullptr; }
-bool has_cast_gather(int s, int d) { return pick_cast_gather(s, d) != nullptr; }
+bool has_accum(int g, int a) { return pick_accum(g, a, false, {}) != nullptr; }
+bool has_cast_gather(int s, int d) { return pick_cast_gather(s, d, {}) != nullptr; }
 bool has_publish(int a, int o) { return pick_publish(a, o) != nullptr; }
 
 int launch_gather(const GatherLaunch& L, uint32_t grid, uint32_t lds_bytes, void* stream) {
-  return launch(gather_kernel<kCopyThreads, kCopyUnroll>, L, grid, kCopyThreads, lds_bytes, stream);
+  return launch(pick_gather(L.policy), L, grid, kCopyThreads, lds_bytes, stream);
 }
 
 int launch_cast_gather(int s, int d, const CastGatherLaunch& L, uint32_t grid, uint32_t lds_bytes, void* stream) {
-  return launch(pick_cast_gather(s, d), L, grid, kCopyThreads, lds_bytes, stream);
+  return launch(pick_cast_gather(s, d, L.policy), L, grid, kCopyThreads, lds_bytes, stream);
 }
 
 int launch_accum(int g, int a, bool store, const AccumLaunch& L, uint32_t grid, uint32_t lds_bytes, void* stream) {
-  return launch(pick_accum(g, a, store), L, grid, store ? kStoreThreads : kThreads, lds_bytes, stream);
+  return launch(pick_accum(g, a, store, L.policy), L, grid, store ? kStoreThreads : kThreads, lds_bytes, stream);
 }
 
 int launch_clear(const ClearLaunch& L, uint32_t grid, void* stream) {

@@ -19,6 +19,14 @@ namespace odc_launch {
 using odc_tiles::kMaxItems;
 using odc_tiles::TileTable;
 
+// Whether a launch leaves what it reads / what it writes in the caches (plain accesses) or streams
+// past them (nontemporal ones). For the accumulate "read" is the gradient and "written" the
+// accumulation, read and written; for the gathers they are the shards and the output.
+struct CachePolicy {
+  bool read = false;
+  bool written = false;
+};
+
 // One record per item, read with scalar loads by the workgroup that works on the item.
 struct GatherDesc {
   uint8_t* dst;
@@ -29,6 +37,7 @@ struct GatherLaunch {
   TileTable tt;
   const uint8_t* base;  // arena base (rank 0 region)
   uint64_t rank_stride;
+  CachePolicy policy;  // picks the kernel
   GatherDesc item[kMaxItems];
 };
 
@@ -42,6 +51,7 @@ struct CastGatherLaunch {
   TileTable tt;
   const uint8_t* base;
   uint64_t rank_stride;
+  CachePolicy policy;  // picks the kernel
   CastGatherDesc item[kMaxItems];
 };
 
@@ -55,6 +65,7 @@ struct AccumLaunch {
   TileTable tt;
   uint8_t* base;
   uint64_t rank_stride;
+  CachePolicy policy;  // picks the kernel
   AccumDesc item[kMaxItems];
 };
 
