@@ -8,8 +8,11 @@ hard when it has not been built): there is no Python or CPU fallback behind any 
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 import subprocess
+import sysconfig
 import threading
 from pathlib import Path
 
@@ -22,6 +25,9 @@ LIB_PATH = Path(os.environ["ODC_HIP_LIBRARY"]) if os.environ.get("ODC_HIP_LIBRAR
 HOST_SOURCES = [CSRC_DIR / "odc_host.cpp"]
 DEVICE_SOURCES = [CSRC_DIR / "odc_kernels.hip"]
 SOURCES = HOST_SOURCES + DEVICE_SOURCES
+# the host path of the service calls: a CPython extension against torch's headers (plain C++, no HIP)
+TORCH_BINDING_PATH = CSRC_DIR / "odc_torch.so"
+TORCH_BINDING_SOURCE = CSRC_DIR / "odc_torch.cpp"
 # measurement-only companion: bare streaming kernels that bench.py times as the practical ceiling
 CEILING_LIB_PATH = CSRC_DIR / "libodc_ceiling.so"
 CEILING_SOURCES = [CSRC_DIR / "ceiling_kernels.hip"]
@@ -187,6 +193,53 @@ def build_ceiling_library(verbose: bool = False) -> Path:
     """Compile libodc_ceiling.so (bench.py's bare streaming kernels) in-tree for gfx950."""
     _run_hipcc(hipcc_command(CEILING_LIB_PATH, CEILING_SOURCES), verbose)
     return CEILING_LIB_PATH
+
+
+def build_torch_binding(verbose: bool = False) -> Path:
+    """Compile odc_torch.so in-tree: host code only, against the torch that is importable here."""
+    import torch
+
+    root = Path(torch.__file__).resolve().parent
+    cmd = [
+        os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
+        f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+        f"-I{INCLUDE_DIR}", f"-I{root / 'include'}", f"-I{root / 'include' / 'torch' / 'csrc' / 'api' / 'include'}",
+        f"-I{sysconfig.get_paths()['include']}", str(TORCH_BINDING_SOURCE), "-o", str(TORCH_BINDING_PATH),
+        f"-L{root / 'lib'}", "-ltorch_python", "-ltorch_cpu", "-lc10",
+    ]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if verbose or proc.returncode != 0:
+        print(" ".join(cmd))
+        print(proc.stdout)
+        print(proc.stderr)
+    if proc.returncode != 0:
+        raise RuntimeError(f"building {TORCH_BINDING_PATH.name} failed with exit code {proc.returncode}")
+    return TORCH_BINDING_PATH
+
+
+_torch_binding = None
+
+
+def load_torch_binding():
+    """The extension module of odc_torch.cpp, bound to the entry points of the library ``load()``
+    returns; built on first use when missing. There is no Python path behind it."""
+    global _torch_binding
+    lib = load()
+    with _lib_lock:
+        if _torch_binding is None:
+            if not TORCH_BINDING_PATH.exists():
+                build_torch_binding()
+            loader = importlib.machinery.ExtensionFileLoader("odc_torch", str(TORCH_BINDING_PATH))
+            spec = importlib.util.spec_from_file_location("odc_torch", TORCH_BINDING_PATH, loader=loader)
+            module = importlib.util.module_from_spec(spec)
+            loader.exec_module(module)
+            entry_points = []
+            for name in ("odc_gather", "odc_gather_cast", "odc_scatter_accumulate", "odc_scatter_store", "odc_clear",
+                         "odc_publish", "odc_arena_locate", "odc_last_error"):
+                entry_points += [name, ctypes.cast(getattr(lib, name), ctypes.c_void_p).value]
+            module.bind(*entry_points)
+            _torch_binding = module
+    return _torch_binding
 
 
 def load_ceiling() -> ctypes.CDLL:

@@ -21,27 +21,21 @@ from odc_amd.primitives.utils import (
     BufferSplitter,
     SymmBufferRegistry,
     comm_stream_section,
-    get_rank,
     get_world,
     group_size,
     native_dtype,
+    plain_launch_stream,
     stream_from_handle,
 )
 
 logger = logging.getLogger(__name__)
 
-
-class _GatherPlan:
-    """The cached part of one gather call: its item array with everything but the output
-    pointers filled in."""
-
-    __slots__ = ("items", "n", "cast", "src_code", "dst_code", "out_numels")
+_host_path = _native.load_torch_binding()
 
 
 class GatherService:
     def __init__(self):
         self.buffer_splitter = BufferSplitter()
-        self._plans = threading.local()  # per host thread: plan key -> _GatherPlan
         self._lock = threading.Lock()
         self._conversion = None  # (stream handle, event) of the latest convert_symm_buffer
         self._met_conversion = frozenset()  # streams ordered after it (replaced, never mutated)
@@ -64,88 +58,22 @@ class GatherService:
         world = get_world()  # raises when there is no arena (no GPU, or init_nvshmem not called)
         if not len(input_tensors):
             return
-        src_dtype = input_tensors[0].dtype
-        pointers, numels = [], []
-        for inp in input_tensors:
-            assert inp.is_cuda and inp.is_contiguous(), "shards are contiguous GPU tensors"
-            assert inp.dtype == src_dtype, "one launch takes one dtype pair"
-            pointers.append(inp.data_ptr())
-            numels.append(inp.numel())
-        # where a shard lies in the arena follows from its address alone, so the symmetric
-        # offsets of a list of shards are looked up once per list of addresses (and host thread)
-        cache = getattr(self._plans, "offsets", None)
-        if cache is None:
-            cache = self._plans.offsets = {}
-        key = (world.serial, tuple(pointers), tuple(numels))
-        known = cache.get(key)
-        if known is None:
-            registry = SymmBufferRegistry.get_instance()
-            keep = [k for k, n in enumerate(numels) if n]
-            known = cache[key] = (
-                keep if len(keep) != len(numels) else None,
-                [registry.symmetric_offset_of(input_tensors[k]) for k in keep],
-                [numels[k] for k in keep],
-            )
-        keep, offsets, kept_numels = known
-        if keep is not None:  # empty shards have empty outputs and take no part in the launch
-            for k, n in enumerate(numels):
-                assert n or not output_tensors[k].numel(), f"output {k} is not empty but its shard is"
-            output_tensors = [output_tensors[k] for k in keep]
-            if not output_tensors:
-                return
-        self._gather(output_tensors, offsets, kept_numels, src_dtype, pg)
+        self._launch(_host_path.gather, world, pg, output_tensors, input_tensors)
 
-    def _gather(self, outs, src_offsets, shard_numels, src_dtype, pg) -> None:
-        """One launch (per 64 items): ``outs[k].view(W, -1)[r]`` = the ``shard_numels[k]`` elements
-        of ``src_dtype`` at symmetric byte offset ``src_offsets[k]`` of rank r. The item array is
-        built once per (offsets, sizes, dtypes) and host thread; later calls only rewrite the
-        output pointers."""
-        world = get_world()
-        W = group_size(pg)
-        assert W == world.world_size, f"group size {W} != arena world size {world.world_size}"
-        dst_dtype = outs[0].dtype
-        cache = getattr(self._plans, "cache", None)
-        if cache is None:
-            cache = self._plans.cache = {}
-        plan_key = (world.serial, tuple(src_offsets), tuple(shard_numels), src_dtype, dst_dtype)
-        plan = cache.get(plan_key)
-        if plan is None:
-            plan = cache[plan_key] = _GatherPlan()
-            plan.n = len(outs)
-            plan.cast = src_dtype != dst_dtype
-            plan.items = ((_native.GatherCastItem if plan.cast else _native.GatherItem) * plan.n)()
-            plan.out_numels = [W * n for n in shard_numels]
-            es = src_dtype.itemsize
-            for item, offset, n in zip(plan.items, src_offsets, shard_numels):
-                item.src_offset = offset
-                if plan.cast:
-                    item.shard_elems = n
-                else:
-                    item.shard_bytes = n * es
-            # shards kept in one dtype (fp32 master copies), full parameter wanted in another
-            # (bf16): converted on the way instead of gathered and then cast
-            # (odc/fsdp/fsdp1.py:199-223, odc/fsdp/fsdp2.py:341-343)
-            plan.src_code = native_dtype(src_dtype) if plan.cast else None
-            plan.dst_code = native_dtype(dst_dtype) if plan.cast else None
-        items = plan.items
-        for item, out, numel in zip(items, outs, plan.out_numels):
-            assert out.is_cuda, "gather runs on the GPU only"
-            assert out.dtype == dst_dtype, "one launch takes one dtype pair"
-            assert out.is_contiguous()
-            assert out.numel() == numel, f"output numel {out.numel()} != {W} * shard numel {numel // W}"
-            item.dst = out.data_ptr()
-
-        lib = _native.load()
-        with comm_stream_section("odc.gather") as comm:
+    def _launch(self, entry, world, pg, *call) -> None:
+        """``entry`` (odc_torch.cpp) checks its tensors, fills the item array and launches."""
+        W = world.world_size
+        assert pg is world.group or group_size(pg) == W, f"group size {group_size(pg)} != arena world size {W}"
+        stream = plain_launch_stream(world)
+        if stream is not None:
             if self._conversion is not None:
-                self._order_after_conversion(comm.cuda_stream)
-            stream = ctypes.c_void_p(comm.cuda_stream)
-            if plan.cast:
-                status = lib.odc_gather_cast(
-                    world.arena.handle, items, plan.n, plan.src_code, plan.dst_code, get_rank(), stream
-                )
-            else:
-                status = lib.odc_gather(world.arena.handle, items, plan.n, get_rank(), stream)
+                self._order_after_conversion(stream)
+            status = entry(world.handle, W, world.rank, stream, *call)
+        else:
+            with comm_stream_section("odc.gather") as comm:
+                if self._conversion is not None:
+                    self._order_after_conversion(comm.cuda_stream)
+                status = entry(world.handle, W, world.rank, comm.cuda_stream, *call)
         if status:
             _native.check(status)
 
@@ -169,18 +97,8 @@ class GatherService:
         assert input_tensor.is_cuda and input_tensor.is_contiguous()
         if not len(output_tensors):
             return
-        es = input_tensor.element_size()
-        total = input_tensor.numel()
-        base = SymmBufferRegistry.get_instance().symmetric_offset_of(input_tensor)
-        outs, offsets, numels = [], [], []
-        for out, off, n in zip(output_tensors, slice_offsets, slice_numels):
-            assert 0 <= off and off + n <= total, "slice leaves the buffer"
-            if n or out.numel():
-                outs.append(out)
-                offsets.append(base + off * es)
-                numels.append(n)
-        if outs:
-            self._gather(outs, offsets, numels, input_tensor.dtype, pg)
+        self._launch(_host_path.gather_slices, get_world(), pg, output_tensors, input_tensor, slice_offsets,
+                     slice_numels)
 
     def convert_symm_buffer(self, dst_key, src_key, ranks: Sequence[int] = None) -> None:
         """Rank r's symmetric buffer ``dst_key`` = rank r's ``src_key`` converted to the

@@ -19,9 +19,10 @@ per minibatch it saves the clear's 4 bytes per element and the first read of the
 from an earlier call is not tracked and, in lazy mode only, shows the previous minibatch's sums
 between a clear and the next accumulate.
 
-Launch plans are cached: the ctypes item array of a call (accumulation offsets, shard sizes) is
-built the first time a list of keys and sizes is seen, per host thread, and later calls only
-rewrite the gradient pointers (the reference caches per key too, :599-600).
+The item array of a call (gradient pointers, accumulation offsets, shard sizes) is checked and
+filled in ``odc_torch.cpp`` on every call, from the table of accumulations that ``register`` keeps
+(the reference caches per key too, :599-600); only what the bookkeeping of slice layouts needs is
+remembered from call to call.
 
 Callers on several host threads and streams. In the reference every add into rank r's
 accumulation goes through r's one watcher (:291-310, :386-392), so clients never race on it. Here
@@ -38,7 +39,6 @@ from __future__ import annotations
 
 import collections.abc
 import contextlib
-import ctypes
 import logging
 import os
 import threading
@@ -52,14 +52,17 @@ from odc_amd.primitives.utils import (
     StreamOrder,
     SymmBufferRegistry,
     comm_stream_section,
+    plain_launch_stream,
     wait_for_launches,
-    get_rank,
     get_world,
     group_size,
     native_dtype,
 )
 
 logger = logging.getLogger(__name__)
+
+_host_path = _native.load_torch_binding()
+_is_capturing = torch._C._cuda_isCurrentStreamCapturing  # what _is_capturing() asks
 
 
 class _LiveAccumulations(collections.abc.Sequence):
@@ -90,17 +93,30 @@ class _LiveAccumulations(collections.abc.Sequence):
         return f"<{len(self)} live accumulations>"
 
 
-class _AccumPlan:
-    """The cached part of one scatter-accumulate call: its item array with everything but the
-    gradient pointers filled in."""
+class _SlicePlan:
+    """What a list of slices of one accumulation means for the bookkeeping."""
 
-    __slots__ = ("items", "n", "grad_code", "acc_code", "acc_dtype", "max_numels", "tiles_exactly", "keys",
-                 "layout")
+    __slots__ = ("layout", "disjoint", "tiles_exactly")
 
-    def __init__(self, n):
-        self.items = (_native.AccumItem * n)()
-        self.n = n
+    def __init__(self, slice_offsets, slice_numels, accumulation_numel):
+        self.layout = _host_path.slice_layout(slice_offsets, slice_numels)
+        # The store form overwrites the slices and nothing else, so it can stand in for a
+        # clear only if the slices are disjoint and the rest of the accumulation holds zeros:
+        # either there is no rest (the slices tile the accumulation), or nothing but these
+        # very slices has been written since a kernel last zeroed all of it (self._written).
+        layout = tuple(sorted((int(o), int(m)) for o, m in zip(slice_offsets, slice_numels) if m))
+        end, disjoint, gaps = 0, True, False
+        for o, m in layout:
+            if o < end:
+                disjoint = False
+                break
+            gaps |= o != end
+            end = o + m
+        self.disjoint = layout if disjoint else None
+        self.tiles_exactly = disjoint and not gaps and end == accumulation_numel
 
+
+_MAX_SLICE_PLANS = 16  # per key: one, unless the caller changes which parameters it reduces
 
 _MIXED = "mixed"
 
@@ -123,7 +139,11 @@ class ReductionService:
         # may be folded into a store over slices only while everything outside them is still zero.
         self._written = {}
         self._sliced_keys = set()  # keys ever used through scatter_accumulate_slices
-        self._plans = threading.local()  # per host thread: plan key -> _AccumPlan
+        # key -> (symmetric offset, elements, dtype code) of its accumulation in the arena of the
+        # world with serial number _table_serial: what odc_torch.cpp reads
+        self._table = {}
+        self._table_serial = None
+        self._slice_plans = {}  # key -> [_SlicePlan], for the same arena
         # One lock for the bookkeeping above AND the launches it decides: callers come from several
         # host threads (the autograd device thread in backward), and the order of the bookkeeping
         # must be the order of the launches.
@@ -144,7 +164,7 @@ class ReductionService:
         assert len(output_tensor_shape) == 1
         with self._lock:
             assert key not in self.accumulation_indices
-            if torch.cuda.is_current_stream_capturing():
+            if _is_capturing():
                 raise RuntimeError(
                     "register accumulation keys before capturing: the zeroing of a new accumulation "
                     "would be recorded into the graph and run on every replay"
@@ -154,41 +174,54 @@ class ReductionService:
             accumulation_key = self._acc_key(key)
             assert not registry.has_key(accumulation_key)
             registry.allocate_symm_buffer(accumulation_key, tuple(output_tensor_shape), reduction_dtype)
+            self._accumulation_table(get_world())[key] = (
+                registry.offsets[accumulation_key][0], int(output_tensor_shape[0]), native_dtype(reduction_dtype)
+            )
             self.accumulation_indices[key] = len(self.accumulation_keys)
             self.accumulation_keys.append(key)
             self._clear_keys([key])  # a one-time cost; the buffer never shows arena leftovers
+
+    def _accumulation_table(self, world):
+        """The table of this world's accumulations. A service kept from an earlier arena starts an
+        empty one: its keys do not exist there (caller holds the lock, or only reads)."""
+        if self._table_serial != world.serial:
+            with self._lock:
+                if self._table_serial != world.serial:
+                    self._table, self._slice_plans = {}, {}
+                    self._table_serial = world.serial
+        return self._table
 
     def _clear_keys(self, keys):
         """Launch the clear kernel over ``keys`` (caller holds the lock)."""
         keys = list(keys)
         self._owed_zero.difference_update(keys)
-        if self._capture_scope and torch.cuda.is_current_stream_capturing():
+        if self._capture_scope and _is_capturing():
             self._capture_scope.difference_update(keys)
         if not keys:
             return
         for key in keys:
             self._written[key] = None
-        registry = SymmBufferRegistry.get_instance()
-        spans = (_native.Span * len(keys))()
-        for i, key in enumerate(keys):
-            offset, shape, dtype = registry.offsets[self._acc_key(key)]
-            spans[i].offset = offset
-            spans[i].nbytes = shape[0] * dtype.itemsize
-        with comm_stream_section("odc.clear") as comm:
-            self._order_after_writers(keys, comm.cuda_stream)
-            _native.check(
-                _native.load().odc_clear(
-                    get_world().arena.handle, spans, len(spans), ctypes.c_void_p(comm.cuda_stream)
-                )
-            )
+        world = get_world()
+        table = self._accumulation_table(world)
+        stream = plain_launch_stream(world)
+        if stream is not None:
+            self._order_after_writers(keys, stream)
+            status = _host_path.clear(world.handle, stream, table, keys)
+        else:
+            with comm_stream_section("odc.clear") as comm:
+                self._order_after_writers(keys, comm.cuda_stream)
+                status = _host_path.clear(world.handle, comm.cuda_stream, table, keys)
+        if status:
+            _native.check(status)
 
     def _order_after_writers(self, keys, stream_handle) -> None:
         """Before a launch that writes ``keys`` on ``stream_handle``: wait for the launches that
         last wrote them on other streams (caller holds the lock; see the module docstring)."""
-        if torch.cuda.is_current_stream_capturing():
-            return  # a graph runs on the stream it is replayed on: nothing the host could order
-        total = len(self.accumulation_keys)
-        self._order.before_launch(keys, stream_handle, all_keys=len(keys) == total, total=total)
+        order = self._order
+        if not order.settled_on(stream_handle) and not _is_capturing():
+            # (a graph runs on the stream it is replayed on: nothing the host could order)
+            total = len(self.accumulation_keys)
+            order.before_launch(keys, stream_handle, all_keys=len(keys) == total, total=total)
 
     def clear_accumulations(self):
         """Zero every registered accumulation of EVERY virtual rank in one launch
@@ -200,7 +233,7 @@ class ReductionService:
         into: a graph replays the read-modify-write form whatever the host has noted since, so
         those are always cleared by a kernel (captured too, when this call is)."""
         with self._lock:
-            if torch.cuda.is_current_stream_capturing():
+            if _is_capturing():
                 if self._capture_scope is not None:
                     # inside captured_minibatch(): the clear is recorded when (and if) it is needed
                     self._check_no_host_owed(self.accumulation_keys)
@@ -229,7 +262,7 @@ class ReductionService:
         minibatch whatever ran before it. Works with eager and lazy clears alike; a capture
         that starts while a lazy clear still owes zeros is refused, as always."""
         with self._lock:
-            if not torch.cuda.is_current_stream_capturing():
+            if not _is_capturing():
                 raise RuntimeError("captured_minibatch() belongs inside torch.cuda.graph(...)")
             if self._capture_scope is not None:
                 raise RuntimeError("captured_minibatch() blocks do not nest")
@@ -256,14 +289,14 @@ class ReductionService:
 
     def _settle(self, keys):
         """Write the zeros still owed to ``keys`` (before anything reads or adds into them)."""
-        if self._capture_scope and torch.cuda.is_current_stream_capturing():
+        if self._capture_scope and _is_capturing():
             deferred = [k for k in keys if k in self._capture_scope]
             if deferred:
                 self._clear_keys(deferred)  # recorded into the graph, in order
         if self._owed_zero:
             owed = [k for k in keys if k in self._owed_zero]
             if owed:
-                if torch.cuda.is_current_stream_capturing():
+                if _is_capturing():
                     self._check_no_host_owed(owed)
                 self._clear_keys(owed)
 
@@ -274,7 +307,7 @@ class ReductionService:
         read-modify-write form is recorded (or, inside ``captured_minibatch()``, the store form
         for a key whose clear was captured just before), and the keys are from now on cleared by
         kernels outside capture."""
-        if not torch.cuda.is_current_stream_capturing():
+        if not _is_capturing():
             return False
         self._check_no_host_owed(keys)
         self._captured.update(keys)
@@ -289,21 +322,17 @@ class ReductionService:
     def _launch(self, keys, items, n, grad_code, acc_code, store):
         if not n:
             return
-        lib = _native.load()
-        entry = lib.odc_scatter_store if store else lib.odc_scatter_accumulate
-        with comm_stream_section("odc.scatter_store" if store else "odc.scatter_accumulate") as comm:
-            self._order_after_writers(keys, comm.cuda_stream)
-            status = entry(
-                get_world().arena.handle, items, n, grad_code, acc_code, ctypes.c_void_p(comm.cuda_stream)
-            )
+        world = get_world()
+        stream = plain_launch_stream(world)
+        if stream is not None:
+            self._order_after_writers(keys, stream)
+            status = items.launch(world.handle, stream, store)
+        else:
+            with comm_stream_section("odc.scatter_store" if store else "odc.scatter_accumulate") as comm:
+                self._order_after_writers(keys, comm.cuda_stream)
+                status = items.launch(world.handle, comm.cuda_stream, store)
         if status:
             _native.check(status)
-
-    def _plan_cache(self):
-        cache = getattr(self._plans, "cache", None)
-        if cache is None:
-            cache = self._plans.cache = {}
-        return cache
 
     # -- the primitive ----------------------------------------------------------------------
     def infer_output_shape(self, input_tensor, pg):
@@ -315,41 +344,17 @@ class ReductionService:
         """``acc_r[key] += input_tensor.view(W, -1)[r]`` for every rank r."""
         self.scatter_accumulate_multi([key], [input_tensor], pg)
 
-    def _plan_multi(self, keys, input_tensors, pg, valid_numels, W):
-        """Validate a (keys, gradients) list once and build its item array."""
-        registry = SymmBufferRegistry.get_instance()
-        grad_dtype = input_tensors[0].dtype
-        plan = _AccumPlan(len(keys))
-        plan.keys = tuple(keys)
-        acc_dtype = None
-        for i, (key, grad) in enumerate(zip(keys, input_tensors)):
-            assert grad.dtype == grad_dtype, "one launch takes one gradient dtype"
-            if valid_numels is None:
-                shard_shape = self.infer_output_shape(grad, pg)
-                valid = grad.numel()
-            else:
-                assert key in self.accumulation_indices, "padded form needs a registered key"
-                shard_shape = registry.offsets[self._acc_key(key)][1]
-                valid = int(valid_numels[i])
-                assert valid <= grad.numel() and valid <= W * shard_shape[0]
-            if key not in self.accumulation_indices:
-                accum_dtype = (
-                    self.accumulation_dtype if self.accumulation_dtype is not None else grad.dtype
-                )
-                self.register(key, shard_shape, grad.dtype, accum_dtype, pg)
-            offset, acc_shape, this_acc_dtype = registry.offsets[self._acc_key(key)]
-            assert tuple(acc_shape) == tuple(
-                shard_shape
-            ), f"key {key}: registered shard {acc_shape}, gradient implies {shard_shape}"
-            assert acc_dtype in (None, this_acc_dtype), "one launch takes one accumulation dtype"
-            acc_dtype = this_acc_dtype
-            plan.items[i].grad_elems = valid
-            plan.items[i].acc_offset = offset
-            plan.items[i].shard_elems = shard_shape[0]
-        plan.grad_code = native_dtype(grad_dtype)
-        plan.acc_code = native_dtype(acc_dtype)
-        plan.acc_dtype = acc_dtype
-        return plan
+    def _register_missing(self, keys, input_tensors, pg, padded):
+        """Register the keys of a call that the table does not hold yet."""
+        with self._lock:
+            for key, grad in zip(keys, input_tensors):
+                if key in self._table:
+                    continue
+                if key in self.accumulation_indices:  # registered in an arena that is gone
+                    raise KeyError(self._acc_key(key))
+                assert not padded, "padded form needs a registered key"
+                accum_dtype = self.accumulation_dtype if self.accumulation_dtype is not None else grad.dtype
+                self.register(key, self.infer_output_shape(grad, pg), grad.dtype, accum_dtype, pg)
 
     def scatter_accumulate_multi(
         self, keys: Sequence, input_tensors: Sequence[torch.Tensor], pg, valid_numels=None
@@ -366,22 +371,13 @@ class ReductionService:
         if not n:
             return
         world = get_world()
-        W = group_size(pg)
-        assert W == world.world_size, f"group size {W} != arena world size {world.world_size}"
-        grad_dtype = input_tensors[0].dtype
-        numels = tuple(t.numel() for t in input_tensors)
-        plan_key = ("multi", world.serial, tuple(keys), numels, grad_dtype,
-                    None if valid_numels is None else tuple(int(v) for v in valid_numels))
-        cache = self._plan_cache()
-        plan = cache.get(plan_key)
-        if plan is None:
-            plan = cache[plan_key] = self._plan_multi(keys, input_tensors, pg, valid_numels, W)
-        items = plan.items
-        for i, grad in enumerate(input_tensors):
-            assert grad.is_cuda, "scatter-accumulate runs on the GPU only"
-            assert grad.dtype == grad_dtype, "one launch takes one gradient dtype"
-            assert grad.is_contiguous()
-            items[i].grad = grad.data_ptr()
+        W = world.world_size
+        assert pg is world.group or group_size(pg) == W, f"group size {group_size(pg)} != arena world size {W}"
+        table = self._accumulation_table(world)
+        items = _host_path.accumulate_batch(table, W, keys, input_tensors, valid_numels)
+        if items is None:
+            self._register_missing(keys, input_tensors, pg, valid_numels is not None)
+            items = _host_path.accumulate_batch(table, W, keys, input_tensors, valid_numels)
 
         with self._lock:
             if self._sliced_keys and not self._sliced_keys.isdisjoint(keys):
@@ -390,9 +386,9 @@ class ReductionService:
             # the keys that count as zero without holding zeros: owed by a lazy clear, or, in a
             # captured minibatch, by the clear captured just before
             zero = self._capture_scope if self._under_capture(keys) else self._owed_zero
-            duplicates = len(set(keys)) != n
+            duplicates = n > 1 and len(set(keys)) != n
             if not duplicates and (not zero or zero.isdisjoint(keys)):
-                self._launch(keys, items, n, plan.grad_code, plan.acc_code, False)  # the steady state
+                self._launch(keys, items, n, items.grad_code, items.acc_code, False)  # the steady state
             else:
                 # Keys that still count as zero take the store form (no read of the accumulation).
                 # A key listed k times goes into k consecutive launches, so its gradients add up
@@ -410,8 +406,8 @@ class ReductionService:
                         picked = [i for i in members if (k == 0 and keys[i] in zero) == store]
                         if not picked:
                             continue
-                        part = (_native.AccumItem * len(picked))(*[items[i] for i in picked])
-                        self._launch([keys[i] for i in picked], part, len(picked), plan.grad_code, plan.acc_code,
+                        part = items if len(picked) == n else items.pick(picked)
+                        self._launch([keys[i] for i in picked], part, len(picked), items.grad_code, items.acc_code,
                                      store)
                 if zero:
                     zero.difference_update(keys)
@@ -441,61 +437,22 @@ class ReductionService:
         if not n:
             return
         world = get_world()
-        W = group_size(pg)
-        assert W == world.world_size, f"group size {W} != arena world size {world.world_size}"
-        grad_dtype = input_tensors[0].dtype
-        plan_key = ("slices", world.serial, key, tuple(slice_offsets), tuple(slice_numels), grad_dtype)
-        cache = self._plan_cache()
-        plan = cache.get(plan_key)
+        W = world.world_size
+        assert pg is world.group or group_size(pg) == W, f"group size {group_size(pg)} != arena world size {W}"
+        table = self._accumulation_table(world)
+        plan = None
+        for known in self._slice_plans.get(key, ()):
+            if known.layout.matches(slice_offsets, slice_numels):
+                plan = known
+                break
         if plan is None:
-            registry = SymmBufferRegistry.get_instance()
-            if key not in self._sliced_keys:
-                self._sliced_keys.add(key)
-                self._written[key] = _MIXED  # whatever whole-key calls wrote before was not tracked
-            if key not in self.accumulation_indices:
-                total = accumulation_numel
-                if total is None:
-                    total = max(o + m for o, m in zip(slice_offsets, slice_numels))
-                accum_dtype = accumulation_dtype or self.accumulation_dtype or grad_dtype
-                self.register(key, (total,), grad_dtype, accum_dtype, pg)  # zeroes it: nothing written
-            offset, acc_shape, acc_dtype = registry.offsets[self._acc_key(key)]
-            plan = _AccumPlan(n)
-            plan.keys = (key,)
-            plan.max_numels = []
-            for i, (off, m) in enumerate(zip(slice_offsets, slice_numels)):
-                assert 0 <= off and off + m <= acc_shape[0], "slice leaves the accumulation"
-                plan.items[i].acc_offset = offset + off * acc_dtype.itemsize
-                plan.items[i].shard_elems = m
-                plan.max_numels.append(W * m)
-            # The store form overwrites the slices and nothing else, so it can stand in for a
-            # clear only if the slices are disjoint and the rest of the accumulation holds zeros:
-            # either there is no rest (the slices tile the accumulation), or nothing but these
-            # very slices has been written since a kernel last zeroed all of it (self._written).
-            layout = tuple(sorted((int(o), int(m)) for o, m in zip(slice_offsets, slice_numels) if m))
-            end, disjoint, gaps = 0, True, False
-            for o, m in layout:
-                if o < end:
-                    disjoint = False
-                    break
-                gaps |= o != end
-                end = o + m
-            plan.layout = layout if disjoint else None
-            plan.tiles_exactly = disjoint and not gaps and end == acc_shape[0]
-            plan.grad_code = native_dtype(grad_dtype)
-            plan.acc_code = native_dtype(acc_dtype)
-            plan.acc_dtype = acc_dtype
-            cache[plan_key] = plan
-        items = plan.items
-        for i, grad in enumerate(input_tensors):
-            numel = grad.numel()
-            assert grad.is_cuda and grad.is_contiguous() and grad.dtype == grad_dtype
-            assert numel <= plan.max_numels[i], f"gradient {i} has {numel} > {W} * {slice_numels[i]} elements"
-            items[i].grad = grad.data_ptr()
-            items[i].grad_elems = numel
+            plan = self._plan_slices(key, slice_offsets, slice_numels, input_tensors[0].dtype, pg, accumulation_numel,
+                                     accumulation_dtype)
+        items = plan.layout.batch(table[key], W, input_tensors)
         with self._lock:
             store = False
             written = self._written.get(key, _MIXED)
-            if self._under_capture(plan.keys):
+            if self._under_capture((key,)):
                 # In a captured minibatch the store form stands in for the captured clear only
                 # when the slices tile the accumulation: what lies between the slices of a gapped
                 # layout at the time of a replay is not known when the graph is recorded.
@@ -507,15 +464,38 @@ class ReductionService:
                         self._settle([key])
                         written = None
             elif key in self._owed_zero:
-                store = plan.tiles_exactly or (plan.layout is not None and written in (None, plan.layout))
+                store = plan.tiles_exactly or (plan.disjoint is not None and written in (None, plan.disjoint))
                 if store:
                     self._owed_zero.discard(key)
                 else:
                     self._settle([key])
                     written = None
-            self._written[key] = plan.layout if plan.layout is not None and written in (None, plan.layout) else _MIXED
-            self._launch(plan.keys, items, n, plan.grad_code, plan.acc_code, store)
+            self._written[key] = plan.disjoint if plan.disjoint is not None and written in (None, plan.disjoint) else _MIXED
+            self._launch((key,), items, n, items.grad_code, items.acc_code, store)
             self.dispatched_tasks += 1
+
+    def _plan_slices(self, key, slice_offsets, slice_numels, grad_dtype, pg, accumulation_numel, accumulation_dtype):
+        """First call with these slices of ``key``: registers the key when it is new."""
+        with self._lock:
+            if key not in self._sliced_keys:
+                self._sliced_keys.add(key)
+                self._written[key] = _MIXED  # whatever whole-key calls wrote before was not tracked
+            if key not in self.accumulation_indices:
+                total = accumulation_numel
+                if total is None:
+                    total = max(o + m for o, m in zip(slice_offsets, slice_numels))
+                accum_dtype = accumulation_dtype or self.accumulation_dtype or grad_dtype
+                self.register(key, (total,), grad_dtype, accum_dtype, pg)  # zeroes it: nothing written
+            if key not in self._table:  # registered in an arena that is gone
+                raise KeyError(self._acc_key(key))
+            numel = self._table[key][1]
+            for off, m in zip(slice_offsets, slice_numels):
+                assert 0 <= off and off + m <= numel, "slice leaves the accumulation"
+            plan = _SlicePlan(slice_offsets, slice_numels, numel)
+            # plans are replaced, not appended to: other threads may be walking the tuple
+            known = self._slice_plans.get(key, ())
+            self._slice_plans[key] = (*known[-(_MAX_SLICE_PLANS - 1):], plan)
+            return plan
 
     # -- results ----------------------------------------------------------------------------
     def get_accumulation(self, key, within_slices: bool = False):
@@ -553,39 +533,33 @@ class ReductionService:
             return []
         with self._lock:
             self._settle(keys)
+            world = get_world()
+            table = self._accumulation_table(world)
             registry = SymmBufferRegistry.get_instance()
-            items = (_native.PublishItem * len(keys))()
-            results, acc_dtype = [], None
-            for i, key in enumerate(keys):
-                offset, shape, dtype = registry.offsets[self._acc_key(key)]
+            outs, results, acc_dtype = [], [], None
+            for key in keys:
+                _offset, shape, dtype = registry.offsets[self._acc_key(key)]
                 assert acc_dtype in (None, dtype), "one launch takes one accumulation dtype"
                 acc_dtype = dtype
-                acc = registry.get_symm_buffer(self._acc_key(key))
-                items[i].acc_offset = offset
-                items[i].elems = shape[0]
                 if out_dtype is None or out_dtype == dtype:
-                    items[i].out = None
-                    results.append(acc)
+                    outs.append(None)
+                    results.append(registry.get_symm_buffer(self._acc_key(key)))
                     self._handed_out([key], within_slices)
                 else:
-                    out = torch.empty(shape, dtype=out_dtype, device=acc.device)
-                    items[i].out = out.data_ptr()
+                    out = torch.empty(shape, dtype=out_dtype, device=torch.device("cuda", world.device))
+                    outs.append(out)
                     results.append(out)
-            target = acc_dtype if out_dtype is None else out_dtype
-            with comm_stream_section("odc.publish") as comm:
-                self._order_after_writers(keys, comm.cuda_stream)
-                _native.check(
-                    _native.load().odc_publish(
-                        get_world().arena.handle,
-                        get_rank(),
-                        items,
-                        len(items),
-                        native_dtype(acc_dtype),
-                        native_dtype(target),
-                        float(divisor),
-                        ctypes.c_void_p(comm.cuda_stream),
-                    )
-                )
+            call = (table, keys, outs, native_dtype(out_dtype or acc_dtype), divisor)
+            stream = plain_launch_stream(world)
+            if stream is not None:
+                self._order_after_writers(keys, stream)
+                status = _host_path.publish(world.handle, world.rank, stream, *call)
+            else:
+                with comm_stream_section("odc.publish") as comm:
+                    self._order_after_writers(keys, comm.cuda_stream)
+                    status = _host_path.publish(world.handle, world.rank, comm.cuda_stream, *call)
+            if status:
+                _native.check(status)
         return results
 
     def accumulation_dtype_of(self, key) -> torch.dtype:

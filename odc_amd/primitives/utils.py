@@ -184,13 +184,20 @@ _world_serial = 0
 
 class _VirtualWorld:
     def __init__(self, arena: SymmetricArena):
-        global _world_serial
-        _world_serial += 1
-        self.serial = _world_serial  # tells one arena from the next in caches that outlive it
+        self.renew_serial()
         self.arena = arena
+        self.handle = arena.handle.value  # the odc_arena, for the calls made through odc_torch.cpp
+        self.device = arena.device
         self.world_size = arena.world_size
         self.rank = 0
         self.group = VirtualGroup(self.world_size)
+
+    def renew_serial(self):
+        """A new number: what a service noted about the buffers of the old one is void. Given to
+        every arena, and to an arena whose registry has freed its buffers."""
+        global _world_serial
+        _world_serial += 1
+        self.serial = _world_serial
 
 
 _world: Optional[_VirtualWorld] = None
@@ -441,6 +448,8 @@ class SymmBufferRegistry:
         return off + inner
 
     def _forget(self):
+        if self._arena is None and _world is not None:
+            _world.renew_serial()
         self.offsets.clear()
         self.local_tensor_to_keys.clear()
         self.updated.clear()
@@ -521,6 +530,11 @@ class StreamOrder:
     def forget(self):
         self._base = None
         self._last.clear()
+
+    def settled_on(self, handle: int) -> bool:
+        """Every key was last written on ``handle``: a launch there has nothing to wait for and
+        nothing to note."""
+        return self._base == handle and not self._last
 
     def before_launch(self, keys, handle: int, all_keys: bool = False, total: int = 0) -> None:
         """Call before launching work that writes ``keys`` on stream ``handle``. ``all_keys``:
@@ -609,6 +623,23 @@ if _current_raw_stream is None:  # a torch without the raw accessor: ask for the
 
     def _current_raw_stream(device: int) -> int:
         return torch.cuda.current_stream(device).cuda_stream
+
+
+_SECTION_KEYS = tuple(_ENCODE_KEY(name) for name in ("ODC_COMM_STREAM", "ODC_TRACE")) if isinstance(
+    _ENVIRON_DATA, dict) and _ENCODE_KEY is not None else None
+
+
+def plain_launch_stream(world):
+    """The handle of the stream a launch goes to when it needs nothing around it: neither of the
+    two environment switches is set, so it is the caller's current stream. None: the caller opens
+    a ``comm_stream_section`` instead, which honours both."""
+    if _SECTION_KEYS is None or _SECTION_KEYS[0] in _ENVIRON_DATA or _SECTION_KEYS[1] in _ENVIRON_DATA:
+        return None
+    handle = _current_raw_stream(world.device)
+    if handle not in _launch_streams:
+        with _launch_lock:
+            _launch_streams.setdefault(handle, None)
+    return handle
 
 
 class comm_stream_section:
