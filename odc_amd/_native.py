@@ -56,7 +56,7 @@ EXPORTED_SYMBOLS = (
 )
 
 ABI_VERSION = 3
-MAX_ITEMS_PER_LAUNCH = 64
+MAX_ITEMS_PER_LAUNCH = 112
 
 ODC_OK = 0
 ODC_ERR_INVALID = -1

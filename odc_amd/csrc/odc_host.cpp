@@ -76,6 +76,8 @@ struct Options {
   int64_t cached_arena_bytes = 192ll << 20;   // see cache_policy
   int64_t cached_output_bytes = 64ll << 20;
   int64_t cached_gradient_bytes = 128ll << 20;
+  int64_t short_tiles_below = 32;             // see wants_short_tiles
+  int64_t dry_run_short_tiles = 0;  // read when an arena without a device is created: 1 = plan short tiles too
 };
 Options g_opt;
 std::mutex g_opt_mu;
@@ -103,6 +105,8 @@ int64_t* option_slot(const char* name) {
   if (!strcmp(name, "cached_arena_bytes")) return &g_opt.cached_arena_bytes;
   if (!strcmp(name, "cached_output_bytes")) return &g_opt.cached_output_bytes;
   if (!strcmp(name, "cached_gradient_bytes")) return &g_opt.cached_gradient_bytes;
+  if (!strcmp(name, "short_tiles_below")) return &g_opt.short_tiles_below;
+  if (!strcmp(name, "dry_run_short_tiles")) return &g_opt.dry_run_short_tiles;
   return nullptr;
 }
 
@@ -132,6 +136,7 @@ struct odc_arena {
   uint8_t* base = nullptr;    // rank 0's region: the allocation rounded up to the stride alignment
   uint8_t* origin = nullptr;  // what launches are planned against: base, or a fictitious address on a dry-run arena
   bool dry_run = false;
+  bool short_tiles = true;  // launches may be cut into short tiles (a dry run counts whole ones unless asked)
   std::map<uint64_t, uint64_t> live;  // offset -> size (rounded)
   std::map<uint64_t, uint64_t> free_; // offset -> size, coalesced
   std::atomic<uint64_t> in_use{0};  // changed under mu, read by launches without it
@@ -243,6 +248,31 @@ CachePolicy cache_policy(const odc_arena* a, const Options& opt, uint64_t read_b
 }
 constexpr int64_t kSymmetric = -1;  // a line: the stream lies in symmetric memory
 
+// Whether the next launch over items [next, n_items) is cut into short tiles (256 vectors, done by
+// 128-thread workgroups): when its segments, one item on one rank, average fewer than `below` = 32
+// whole tiles. A workgroup of 256 or 512 threads whose segment holds a few hundred elements keeps the
+// wave slots of its CU from others and does nothing with them, and a launch of a few dozen whole tiles
+// leaves most CUs idle. Graph-replayed launches, us, whole -> short:
+//   300 slices of 64 .. 65 536 elements, gather + accumulate: W = 4 31.7 -> 29.4, W = 16 46.5 -> 31.8,
+//     W = 64 122 -> 56;
+//   60 items at W = 8, gather: 300 elements per segment 3.6 -> 2.9, 10 000 6.5 -> 5.6, 40 000 14.0 -> 13.8;
+//   one item at W = 8, gather: 19 000 elements per segment 2.5 -> 2.2, 300 000 (37 tiles) 3.3 -> 3.2,
+//     600 000 (73) 4.55 -> 4.65; converting gather level from there on, store 5.0 -> 5.5 at 600 000.
+// Launches of longer segments stream best in whole tiles, with one exception (accum_streams_short).
+template <class Units>
+bool wants_short_tiles(const odc_arena* a, uint32_t n_items, uint32_t next, uint64_t tile_units, Units units,
+                       int64_t below) {
+  if (!a->short_tiles) return false;
+  uint64_t segments = 0, tiles = 0;
+  for (uint32_t i = next; i < n_items && segments < (uint64_t)kMaxItems; ++i) {
+    const uint64_t n = units(i);
+    if (n == 0) continue;
+    tiles += tiles_for(n, tile_units);
+    ++segments;
+  }
+  return tiles < (uint64_t)below * segments;
+}
+
 // One-workgroup-per-tile launches are dealt out by the hardware dispatcher, which keeps as many
 // workgroups resident as fit. Fewer resident workgroups (a smaller window of memory in flight)
 // can stream faster; the only lever is to make each workgroup claim a share of the CU's LDS that
@@ -310,6 +340,7 @@ int odc_arena_create(uint32_t world_size, uint64_t bytes_per_rank, uint32_t flag
   const uint64_t stride_align = std::max<uint64_t>(round_up((uint64_t)opt.rank_stride_align, kAlign), kAlign);
   a->alloc_align = std::max<uint64_t>(round_up((uint64_t)opt.alloc_align, kAlign), kAlign);
   a->bytes_per_rank = round_up(bytes_per_rank, kAlign);
+  a->short_tiles = !(flags & ODC_ARENA_NO_BACKING) || opt.dry_run_short_tiles != 0;
   a->rank_stride = round_up(a->bytes_per_rank + round_up((uint64_t)opt.rank_stagger_bytes, kAlign), stride_align);
   // the device allocation promises 256 B alignment only; the regions shall start on stride_align
   // boundaries, so the allocation is that much larger: the whole sum must fit 64 bits
@@ -491,6 +522,9 @@ int dtype_bytes(int dt) {
   }
 }
 
+// Units of one tile of a launch.
+uint64_t tile_units(uint64_t whole, bool short_tiles) { return short_tiles ? whole / kShortTileParts : whole; }
+
 // odc_tiles::fill_tile_table with its failure turned into an error message.
 // `order`, when given, maps positions of the launch order to the caller's item indices (for the
 // message only: units and take already work on positions).
@@ -564,8 +598,10 @@ int odc_gather(odc_arena* a, const odc_gather_item* items, uint32_t n_items, uin
     L.rank_stride = a->rank_stride;
     L.tt.order = (uint32_t)opt.rank_major;
     L.tt.first_rank = first_rank;
+    const auto units = [&](uint32_t i) { return items[i].shard_bytes; };
+    L.short_tiles = wants_short_tiles(a, n_items, next, kTileBytes, units, opt.short_tiles_below);
     const int n = fill_launch(
-        L.tt, a->world, n_items, &next, kTileBytes, [&](uint32_t i) { return items[i].shard_bytes; },
+        L.tt, a->world, n_items, &next, tile_units(kTileBytes, L.short_tiles), units,
         [&](uint32_t slot, uint32_t i) {
           L.item[slot] = {static_cast<uint8_t*>(items[i].dst), items[i].src_offset, items[i].shard_bytes};
         });
@@ -614,8 +650,10 @@ int odc_gather_cast(odc_arena* a, const odc_gather_cast_item* items, uint32_t n_
     L.rank_stride = a->rank_stride;
     L.tt.order = (uint32_t)opt.rank_major;
     L.tt.first_rank = first_rank;
+    const auto units = [&](uint32_t i) { return items[i].shard_elems; };
+    L.short_tiles = wants_short_tiles(a, n_items, next, kTileElems, units, opt.short_tiles_below);
     const int n = fill_launch(
-        L.tt, a->world, n_items, &next, kTileElems, [&](uint32_t i) { return items[i].shard_elems; },
+        L.tt, a->world, n_items, &next, tile_units(kTileElems, L.short_tiles), units,
         [&](uint32_t slot, uint32_t i) {
           L.item[slot] = {static_cast<uint8_t*>(items[i].dst), items[i].shard_elems * (uint64_t)db,
                           items[i].src_offset, items[i].shard_elems};
@@ -661,8 +699,10 @@ int odc_convert(odc_arena* a, const odc_convert_item* items, uint32_t n_items, i
     L.rank_stride = a->rank_stride;
     L.tt.order = (uint32_t)opt.rank_major;
     L.tt.first_rank = 0;
+    const auto units = [&](uint32_t i) { return items[i].elems; };
+    L.short_tiles = wants_short_tiles(a, n_items, next, kTileElems, units, opt.short_tiles_below);
     const int n = fill_launch(
-        L.tt, a->world, n_items, &next, kTileElems, [&](uint32_t i) { return items[i].elems; },
+        L.tt, a->world, n_items, &next, tile_units(kTileElems, L.short_tiles), units,
         [&](uint32_t slot, uint32_t i) {
           // the gather-with-cast kernel with every rank's output in that rank's own region
           L.item[slot] = {a->origin + items[i].dst_offset, a->rank_stride, items[i].src_offset, items[i].elems};
@@ -771,8 +811,11 @@ int scatter_launch(odc_arena* a, const odc_accum_item* items, uint32_t n_items, 
     L.rank_stride = a->rank_stride;
     L.tt.order = (uint32_t)opt.rank_major;
     L.tt.first_rank = 0;
+    const auto units = [&](uint32_t i) { return items[order[i]].shard_elems; };
+    L.short_tiles = (a->short_tiles && odc_launch::accum_streams_short(grad_dtype, acc_dtype)) ||
+                    wants_short_tiles(a, n_items, next, kTileElems, units, opt.short_tiles_below);
     const int n = fill_launch(
-        L.tt, a->world, n_items, &next, kTileElems, [&](uint32_t i) { return items[order[i]].shard_elems; },
+        L.tt, a->world, n_items, &next, tile_units(kTileElems, L.short_tiles), units,
         [&](uint32_t slot, uint32_t i) {
           const odc_accum_item& it = items[order[i]];
           L.item[slot] = {static_cast<const uint8_t*>(it.grad), it.grad_elems, it.acc_offset, it.shard_elems};
@@ -788,8 +831,9 @@ int scatter_launch(odc_arena* a, const odc_accum_item* items, uint32_t n_items, 
     // rank-outermost: +1.1 % at W=4, +1.6 % at W=16 (370 tiles per segment on average), -1.9 % at
     // W=32 (185), -6 % at W=64, -10 % at W=128.
     const uint64_t segments = (uint64_t)L.tt.n_items * a->world;
+    const uint64_t whole_tiles = L.short_tiles ? L.tt.n_tiles / kShortTileParts : L.tt.n_tiles;
     if (opt.accum_tile_order == 3)
-      L.tt.order = L.tt.n_tiles < (uint64_t)opt.accum_short_segment_tiles * segments ? kRankOutermost : kItemMajor;
+      L.tt.order = whole_tiles < (uint64_t)opt.accum_short_segment_tiles * segments ? kRankOutermost : kItemMajor;
     else
       L.tt.order = (uint32_t)opt.accum_tile_order;
     // Launch shape: one workgroup per tile. A persistent shape (one workgroup per CU,
@@ -811,7 +855,7 @@ int scatter_launch(odc_arena* a, const odc_accum_item* items, uint32_t n_items, 
     L.policy = cache_policy(a, opt, grad_elems * gb, opt.cached_gradient_bytes, 0, kSymmetric);
     int64_t blocks_per_cu = store ? opt.store_blocks_per_cu : opt.accum_blocks_per_cu;
     if (blocks_per_cu < 0)
-      blocks_per_cu = L.tt.n_tiles < (uint64_t)opt.accum_persistent_below_tiles * segments ? 1 : 0;
+      blocks_per_cu = whole_tiles < (uint64_t)opt.accum_persistent_below_tiles * segments ? 1 : 0;
     const uint32_t grid = grid_for(a, blocks_per_cu, L.tt.n_tiles, ragged);
     const int64_t cap = store ? opt.store_resident_cap : opt.accum_resident_cap;
     const uint32_t lds = lds_claim_for(a, cap, grid, L.tt.n_tiles);

@@ -11,9 +11,11 @@
 //   clear_kernel        : zero a span in every rank region            (write 1 B per byte)
 //   publish_kernel      : one rank's acc /= divisor, plus a cast copy (end of a minibatch)
 //
-// Launch model shared by the kernels: the work of one launch is cut into tiles of
-// kThreads * kUnroll = 1024 vectors (16 KiB); workgroups of 256 threads (512 for the two
-// gathers and the scatter-store) walk the tiles with a grid-stride loop, by default one workgroup per tile, so that,
+// Launch model shared by the kernels: the work of one launch is cut into tiles of 1024 vectors
+// (16 KiB), done by workgroups of 256 threads (512 for the two gathers), or into short tiles of 256
+// vectors, done by 128 threads: launches of short segments (wants_short_tiles in odc_host.cpp) and
+// every accumulate and store of 16-bit gradients into fp32 (accum_streams_short in odc_launch.h).
+// Workgroups walk the tiles with a grid-stride loop, by default one workgroup per tile, so that,
 // at any instant, the whole chip streams one compact window of memory. Per-item
 // descriptors (<= ODC_MAX_ITEMS_PER_LAUNCH) travel BY VALUE in the kernel argument segment and
 // are read with scalar loads, so a call needs no device-side work list, no host->device copy and
@@ -38,18 +40,22 @@
 namespace {
 
 // Workgroup shape of the two gathers and of the scatter-store (the kernels that read one stream
-// and write one): 512 threads x 2 steps over the same 16 KiB tile as the 256 x 4 of the other
-// kernels. Four such workgroups fill a CU's wave slots, which is the residency these kernels
+// and write one) on whole tiles: 512 threads x 2 steps over the same 16 KiB tile as the 256 x 4 of
+// the other kernels. Four such workgroups fill a CU's wave slots, which is the residency these kernels
 // stream best at (measured: gathers +1.4..2.6 % over 256 x 4 with a residency cap of 4, which
-// had to be enforced by claiming LDS; scatter-store level with it on per-parameter shards at W=8
-// and +2..3 % on flat shards and at W=64; 256 x 4 without a cap loses 6..8 %; 1024 x 1 loses
-// 20 %). The read-modify-write keeps 256 x 4 (512 x 2: equal on long segments, -3 % in the
-// persistent shape at W=64), and so does the clear (512 x 2: -25 % on per-parameter spans).
+// had to be enforced by claiming LDS; 256 x 4 without a cap loses 6..8 %; 1024 x 1 loses
+// 20 %; short tiles lose 1 %). The read-modify-write of equally wide types keeps 256 x 4 (512 x 2:
+// equal on long segments), and so does the clear (512 x 2: -25 % on per-parameter spans).
 constexpr int kCopyThreads = 512;
 constexpr int kCopyUnroll = (int)odc_tiles::kTileVecs / kCopyThreads;  // 2 for the 16 KiB tile
 constexpr int kStoreThreads = 512;
 constexpr int kStoreUnroll = (int)odc_tiles::kTileVecs / kStoreThreads;
 static_assert(kCopyUnroll >= 1 && kStoreUnroll >= 1, "a tile holds at least one vector per thread");
+// Shape for short tiles: two vectors per lane, and few enough threads that a segment of a few hundred elements does not hold the wave slots of a CU for nothing
+// (300 slices at W = 16, gather + accumulate: 31.9 us; 256 threads x 1: 40.1; 128 x 1 on eighths:
+// 35.2; 128 x 4 on halves: 33.1; whole tiles: 46.6).
+constexpr int kShortThreads = 128;
+constexpr int kShortUnroll = (int)odc_tiles::kShortTileVecs / kShortThreads;
 
 // ------------------------------------------------------------------------------------------------
 // device side
@@ -89,15 +95,16 @@ __device__ __forceinline__ void store_vec(V* p, V v) {  // aligned
 }
 
 // ---- gather -------------------------------------------------------------------------------
-// Everything of a tile that is not a run of kTileVecs whole vectors: the last partial run, the
-// head and the tail. Kept out of line so that the streaming loop stays tight.
+// Everything of a tile that is not a run of T * U whole vectors: the last partial run, the
+// head and the tail. Kept out of line so that the streaming loop stays tight (inline, the
+// short-segment kernels, which come here for most of their tiles, were 5 % slower too).
 template <bool kSrcCached, bool kDstCached, int T, int U>
 __device__ __attribute__((noinline)) void gather_edges(uint8_t* d, const uint8_t* s, uint32_t chunk, SegShape g) {
   // Every load of the tile is issued before its first store (a lone resident workgroup would
-  // otherwise pay one memory round trip per step).
+  // otherwise pay one memory round trip per vector).
   const uint32_t tid = threadIdx.x;
-  const TileWork w = tile_work(chunk, g);
-  const uint32_t left = is_whole(w) ? 0u : w.nv;
+  const TileWork w = tile_work<T * U>(chunk, g);
+  const uint32_t left = is_whole<T * U>(w) ? 0u : w.nv;
   const uint8_t* sb = s + g.head + w.v0 * 16;
   u32x4* db = reinterpret_cast<u32x4*>(d + g.head) + w.v0;
   const bool do_head = w.head && tid < g.head;
@@ -117,11 +124,13 @@ __device__ __attribute__((noinline)) void gather_edges(uint8_t* d, const uint8_t
   if (do_tail) d[tail_at] = tail_byte;
 }
 
-// T threads do a tile in U steps of T vectors (T * U = kTileVecs, so the geometry is that of every
-// other kernel); the copies stream best from 512-thread workgroups, of which 4 fit a CU.
+// T threads do a tile of T * U vectors in one step; the copies stream best from 512-thread
+// workgroups, of which 4 fit a CU.
 template <bool kSrcCached, bool kDstCached, int T, int U>
 __global__ __launch_bounds__(T) void gather_kernel(const GatherLaunch launch) {
-  static_assert(T * U == (int)kTileVecs, "one tile per workgroup step");
+  constexpr uint32_t kVecs = T * U;
+  static_assert(kVecs == kTileVecs || kVecs == kShortTileVecs, "a whole tile or a short one");
+  static_assert(T >= ODC_BODY_ALIGN - 1, "one lane per head byte");
   const uint32_t tid = threadIdx.x;
   TileCursor cur;
   GatherDesc it = {};
@@ -135,9 +144,9 @@ __global__ __launch_bounds__(T) void gather_kernel(const GatherLaunch launch) {
     const uint64_t seg = it.seg_bytes;
     const uint8_t* s = launch.base + (uint64_t)c.rank * launch.rank_stride + it.src_off;
     uint8_t* d = it.dst + (uint64_t)c.rank * seg;
-    const SegShape g = seg_shape((uintptr_t)d, seg, 1, 16);
-    const TileWork w = tile_work(c.chunk, g);
-    if (is_whole(w)) {
+    const SegShape g = seg_shape<kVecs>((uintptr_t)d, seg, 1, 16);
+    const TileWork w = tile_work<kVecs>(c.chunk, g);
+    if (is_whole<kVecs>(w)) {
       const uint8_t* sb = s + g.head + (w.v0 + tid) * 16;
       u32x4* db = reinterpret_cast<u32x4*>(d + g.head) + w.v0 + tid;
       u32x4 v[U];
@@ -155,7 +164,7 @@ __global__ __launch_bounds__(T) void gather_kernel(const GatherLaunch launch) {
       for (int u = 0; u < U; ++u) store_vec<kDstCached>(db + u * T, v[u]);
       if (do_head) d[tid] = head_byte;
       if (do_tail) d[tail_at] = tail_byte;
-    } else if (has_edges(w)) {
+    } else if (has_edges<kVecs>(w)) {
       gather_edges<kSrcCached, kDstCached, T, U>(d, s, c.chunk, g);
     }
   }
@@ -301,7 +310,7 @@ __device__ __attribute__((noinline)) void accum_edges(uint8_t* acc, const uint8_
   typedef typename Codec<A>::raw_t araw_t;
   constexpr uint32_t kAB = Codec<A>::kBytes, kGB = Codec<G>::kBytes;
   const uint32_t tid = threadIdx.x;
-  const TileWork w = tile_work(chunk, g);
+  const TileWork w = tile_work<T * U>(chunk, g);
   const uint32_t left = body ? w.nv : 0u;
   const uint64_t e0 = g.head + w.v0 * 4;
   avec_t* ap = reinterpret_cast<avec_t*>(acc + e0 * kAB);
@@ -313,8 +322,8 @@ __device__ __attribute__((noinline)) void accum_edges(uint8_t* acc, const uint8_
   // valid gradient elements from the tile's first body element on: whole quads, and what is left
   const uint64_t g0 = g_seg + e0;
   const uint64_t valid = grad_elems > g0 ? grad_elems - g0 : 0;
-  const uint32_t whole_quads = valid >= kTileElems ? kTileVecs : (uint32_t)(valid / 4);
-  const uint32_t cut = valid >= kTileElems ? 0u : (uint32_t)(valid & 3u);
+  const uint32_t whole_quads = valid >= 4 * T * U ? T * U : (uint32_t)(valid / 4);
+  const uint32_t cut = valid >= 4 * T * U ? 0u : (uint32_t)(valid & 3u);
   const bool has_cut = cut != 0 && whole_quads < left && tid == whole_quads % T;
 
   gvec_t graw[U] = {};
@@ -367,10 +376,12 @@ __device__ __attribute__((noinline)) void accum_edges(uint8_t* acc, const uint8_
 
 template <class G, class A, bool kStore, bool kGradCached, bool kAccCached, int T, int U>
 __global__ __launch_bounds__(T) void accum_kernel(const AccumLaunch launch) {
-  static_assert(T * U == (int)kTileVecs, "one tile per workgroup step");
+  constexpr uint32_t kVecs = T * U;  // quads
+  static_assert(kVecs == kTileVecs || kVecs == kShortTileVecs, "a whole tile or a short one");
   typedef typename Quad<G>::vec_t gvec_t;
   typedef typename Quad<A>::vec_t avec_t;
   constexpr uint32_t kAB = Codec<A>::kBytes, kGB = Codec<G>::kBytes;
+  static_assert(T >= ODC_BODY_ALIGN / kAB, "one lane per head element");
   const uint32_t tid = threadIdx.x;
   TileCursor cur;
   AccumDesc it = {};
@@ -384,11 +395,11 @@ __global__ __launch_bounds__(T) void accum_kernel(const AccumLaunch launch) {
     const uint64_t seg = it.seg_elems;
     uint8_t* acc = launch.base + (uint64_t)c.rank * launch.rank_stride + it.acc_off;
     const uint64_t g_seg = (uint64_t)c.rank * seg;  // gradient index of the segment's first element
-    const SegShape g = seg_shape((uintptr_t)acc, seg, kAB, 4);
-    const TileWork w = tile_work(c.chunk, g);
+    const SegShape g = seg_shape<kVecs>((uintptr_t)acc, seg, kAB, 4);
+    const TileWork w = tile_work<kVecs>(c.chunk, g);
     const uint64_t e0 = g.head + w.v0 * 4;  // the tile's first body element within the segment
-    // whole: all kTileVecs quads exist in the accumulation AND in the valid part of the gradient
-    const bool whole = is_whole(w) && g_seg + e0 + kTileElems <= it.grad_elems;
+    // whole: all its quads exist in the accumulation AND in the valid part of the gradient
+    const bool whole = is_whole<kVecs>(w) && g_seg + e0 + 4 * kVecs <= it.grad_elems;
     if (whole) {
       const uint8_t* gb = it.grad + (g_seg + e0) * kGB + (size_t)tid * sizeof(gvec_t);
       avec_t* ap = reinterpret_cast<avec_t*>(acc + e0 * kAB) + tid;
@@ -429,8 +440,8 @@ __device__ __attribute__((noinline)) void cast_edges(uint8_t* d, const uint8_t* 
   typedef typename Codec<D>::raw_t draw_t;
   constexpr uint32_t kSB = Codec<S>::kBytes, kDB = Codec<D>::kBytes;
   const uint32_t tid = threadIdx.x;
-  const TileWork w = tile_work(chunk, g);
-  const uint32_t left = is_whole(w) ? 0u : w.nv;
+  const TileWork w = tile_work<T * U>(chunk, g);
+  const uint32_t left = is_whole<T * U>(w) ? 0u : w.nv;
   const uint64_t e0 = g.head + w.v0 * 4;
   const uint8_t* sb = s + e0 * kSB;
   dvec_t* dp = reinterpret_cast<dvec_t*>(d + e0 * kDB);
@@ -464,7 +475,9 @@ __device__ __attribute__((noinline)) void cast_edges(uint8_t* d, const uint8_t* 
 
 template <class S, class D, bool kCached, int T, int U>
 __global__ __launch_bounds__(T) void cast_gather_kernel(const CastGatherLaunch launch) {
-  static_assert(T * U == (int)kTileVecs, "one tile per workgroup step");
+  constexpr uint32_t kVecs = T * U;  // quads
+  static_assert(kVecs == kTileVecs || kVecs == kShortTileVecs, "a whole tile or a short one");
+  static_assert(T >= ODC_BODY_ALIGN / Codec<D>::kBytes, "one lane per head element");
   typedef typename Quad<S>::vec_t svec_t;
   typedef typename Quad<D>::vec_t dvec_t;
   constexpr uint32_t kSB = Codec<S>::kBytes, kDB = Codec<D>::kBytes;
@@ -481,9 +494,9 @@ __global__ __launch_bounds__(T) void cast_gather_kernel(const CastGatherLaunch l
     const uint64_t seg = it.seg_elems;
     const uint8_t* s = launch.base + (uint64_t)c.rank * launch.rank_stride + it.src_off;
     uint8_t* d = it.dst + (uint64_t)c.rank * it.dst_stride;
-    const SegShape g = seg_shape((uintptr_t)d, seg, kDB, 4);
-    const TileWork w = tile_work(c.chunk, g);
-    if (is_whole(w)) {
+    const SegShape g = seg_shape<kVecs>((uintptr_t)d, seg, kDB, 4);
+    const TileWork w = tile_work<kVecs>(c.chunk, g);
+    if (is_whole<kVecs>(w)) {
       const uint64_t e0 = g.head + w.v0 * 4;
       const uint8_t* sb = s + e0 * kSB + (size_t)tid * sizeof(svec_t);
       dvec_t* dp = reinterpret_cast<dvec_t*>(d + e0 * kDB) + tid;
@@ -509,7 +522,7 @@ __global__ __launch_bounds__(T) void cast_gather_kernel(const CastGatherLaunch l
       }
       if (do_head) ds[tid] = Codec<D>::narrow(Codec<S>::widen(head_raw));
       if (do_tail) ds[tail_at] = Codec<D>::narrow(Codec<S>::widen(tail_raw));
-    } else if (has_edges(w)) {
+    } else if (has_edges<kVecs>(w)) {
       cast_edges<S, D, kCached, T, U>(d, s, c.chunk, g);
     }
   }
@@ -656,40 +669,58 @@ typedef void (*publish_fn)(const PublishLaunch);
 
 // (gradient dtype, accumulation dtype). The store form never reads the accumulation and keeps it
 // nontemporal; the read-modify-write keeps it cached only together with the gradient.
-template <class G, class A>
-accum_fn pick_accum_policy(bool store, CachePolicy policy) {
-  if (store)
-    return policy.read ? accum_kernel<G, A, true, true, false, kStoreThreads, kStoreUnroll>
-                       : accum_kernel<G, A, true, false, false, kStoreThreads, kStoreUnroll>;
-  if (policy.read && policy.written) return accum_kernel<G, A, false, true, true, kThreads, kUnroll>;
-  return policy.read ? accum_kernel<G, A, false, true, false, kThreads, kUnroll>
-                     : accum_kernel<G, A, false, false, false, kThreads, kUnroll>;
+template <class G, class A, int T, int U>
+accum_fn pick_rmw(CachePolicy policy) {
+  if (policy.read && policy.written) return accum_kernel<G, A, false, true, true, T, U>;
+  return policy.read ? accum_kernel<G, A, false, true, false, T, U> : accum_kernel<G, A, false, false, false, T, U>;
 }
 
-accum_fn pick_accum(int g, int a, bool store, CachePolicy policy) {
-#define X(E1, T1, E2, T2) if (g == E1 && a == E2) return pick_accum_policy<T1, T2>(store, policy);
+template <class G, class A, int T, int U>
+accum_fn pick_store(CachePolicy policy) {
+  return policy.read ? accum_kernel<G, A, true, true, false, T, U> : accum_kernel<G, A, true, false, false, T, U>;
+}
+
+// kShortOnly: accum_streams_short says so, there is no kernel of whole tiles.
+template <class G, class A, bool kShortOnly>
+accum_fn pick_accum_form(bool store, CachePolicy policy, bool short_tiles) {
+  if (short_tiles)
+    return store ? pick_store<G, A, kShortThreads, kShortUnroll>(policy) : pick_rmw<G, A, kShortThreads, kShortUnroll>(policy);
+  if constexpr (kShortOnly) return nullptr;
+  else return store ? pick_store<G, A, kStoreThreads, kStoreUnroll>(policy) : pick_rmw<G, A, kThreads, kUnroll>(policy);
+}
+
+accum_fn pick_accum(int g, int a, bool store, CachePolicy policy, bool short_tiles) {
+#define X(E1, T1, E2, T2) \
+  if (g == E1 && a == E2) return pick_accum_form<T1, T2, accum_streams_short(E1, E2)>(store, policy, short_tiles);
   ODC_FOR_EACH_DTYPE_PAIR(X)
 #undef X
   return nullptr;
 }
 
-gather_fn pick_gather(CachePolicy policy) {
+template <bool kSrcCached, bool kDstCached>
+gather_fn pick_gather_threads(bool short_tiles) {
+  return short_tiles ? gather_kernel<kSrcCached, kDstCached, kShortThreads, kShortUnroll>
+                     : gather_kernel<kSrcCached, kDstCached, kCopyThreads, kCopyUnroll>;
+}
+
+gather_fn pick_gather(CachePolicy policy, bool short_tiles) {
   if (policy.read)
-    return policy.written ? gather_kernel<true, true, kCopyThreads, kCopyUnroll>
-                          : gather_kernel<true, false, kCopyThreads, kCopyUnroll>;
-  return policy.written ? gather_kernel<false, true, kCopyThreads, kCopyUnroll>
-                        : gather_kernel<false, false, kCopyThreads, kCopyUnroll>;
+    return policy.written ? pick_gather_threads<true, true>(short_tiles) : pick_gather_threads<true, false>(short_tiles);
+  return policy.written ? pick_gather_threads<false, true>(short_tiles) : pick_gather_threads<false, false>(short_tiles);
 }
 
 // Shards and output of the converting gather are cached together or not at all.
 template <class S, class D>
-cast_gather_fn pick_cast_gather_policy(CachePolicy policy) {
+cast_gather_fn pick_cast_gather_form(CachePolicy policy, bool short_tiles) {
+  if (short_tiles)
+    return policy.read ? cast_gather_kernel<S, D, true, kShortThreads, kShortUnroll>
+                       : cast_gather_kernel<S, D, false, kShortThreads, kShortUnroll>;
   return policy.read ? cast_gather_kernel<S, D, true, kCopyThreads, kCopyUnroll>
                      : cast_gather_kernel<S, D, false, kCopyThreads, kCopyUnroll>;
 }
 
-cast_gather_fn pick_cast_gather(int s, int d, CachePolicy policy) {  // (shard dtype, output dtype)
-#define X(E1, T1, E2, T2) if (s == E1 && d == E2) return pick_cast_gather_policy<T1, T2>(policy);
+cast_gather_fn pick_cast_gather(int s, int d, CachePolicy policy, bool short_tiles) {  // (shard dtype, output dtype)
+#define X(E1, T1, E2, T2) if (s == E1 && d == E2) return pick_cast_gather_form<T1, T2>(policy, short_tiles);
   ODC_FOR_EACH_DTYPE_PAIR(X)
 #undef X
   return nullptr;
@@ -752,20 +783,23 @@ bool is_out_of_memory(int code) { return code == (int)hipErrorOutOfMemory; }
 
 const char* error_string(int code) { return hipGetErrorString(static_cast<hipError_t>(code)); }
 
-bool has_accum(int g, int a) { return pick_accum(g, a, false, {}) != nullptr; }
-bool has_cast_gather(int s, int d) { return pick_cast_gather(s, d, {}) != nullptr; }
+bool has_accum(int g, int a) { return pick_accum(g, a, false, {}, true) != nullptr; }
+bool has_cast_gather(int s, int d) { return pick_cast_gather(s, d, {}, false) != nullptr; }
 bool has_publish(int a, int o) { return pick_publish(a, o) != nullptr; }
 
 int launch_gather(const GatherLaunch& L, uint32_t grid, uint32_t lds_bytes, void* stream) {
-  return launch(pick_gather(L.policy), L, grid, kCopyThreads, lds_bytes, stream);
+  return launch(pick_gather(L.policy, L.short_tiles), L, grid, L.short_tiles ? kShortThreads : kCopyThreads, lds_bytes,
+                stream);
 }
 
 int launch_cast_gather(int s, int d, const CastGatherLaunch& L, uint32_t grid, uint32_t lds_bytes, void* stream) {
-  return launch(pick_cast_gather(s, d, L.policy), L, grid, kCopyThreads, lds_bytes, stream);
+  return launch(pick_cast_gather(s, d, L.policy, L.short_tiles), L, grid, L.short_tiles ? kShortThreads : kCopyThreads,
+                lds_bytes, stream);
 }
 
 int launch_accum(int g, int a, bool store, const AccumLaunch& L, uint32_t grid, uint32_t lds_bytes, void* stream) {
-  return launch(pick_accum(g, a, store, L.policy), L, grid, store ? kStoreThreads : kThreads, lds_bytes, stream);
+  const uint32_t threads = L.short_tiles ? kShortThreads : store ? kStoreThreads : kThreads;
+  return launch(pick_accum(g, a, store, L.policy, L.short_tiles), L, grid, threads, lds_bytes, stream);
 }
 
 int launch_clear(const ClearLaunch& L, uint32_t grid, void* stream) {

@@ -12,6 +12,7 @@
 
 #include <stdint.h>
 
+#include "odc_hip.h"
 #include "odc_tiles.h"
 
 namespace odc_launch {
@@ -27,6 +28,19 @@ struct CachePolicy {
   bool written = false;
 };
 
+// 16-bit gradients into fp32 accumulations are accumulated and stored in short tiles whatever the
+// sizes. What bounds these streams is how reads and writes mix in HBM, and 16 workgroups of 128
+// threads with 2 quads per lane in flight (98 KB of loads per CU) mix them better than 8 of 256 with
+// 4 (196 KB), the more so the oftener the launch hops between segments. The decoder layer, us,
+// 256 x 4 -> 128 x 2: accumulate 344 -> 341 at W = 8, 354 -> 349 at W = 16, 365 -> 352 at W = 32,
+// 373 -> 352 at W = 64, 374 -> 370 at W = 128; a 525 M element embedding 863 -> 852; the store
+// 206 -> 198 at W = 8, 209 -> 205 at W = 64. (128 x 1: 386, 64 x 2: 371, 64 x 4: 348 and 357 at
+// W = 64, 128 x 4: 349 and 372, 256 x 1: 367, 256 x 2: 360.) fp32 gradients move the same bytes per
+// lane in both streams and keep 256 x 4 (421; 128 x 2: 429), and so do 16-bit accumulations.
+constexpr bool accum_streams_short(int grad_dtype, int acc_dtype) {
+  return grad_dtype != ODC_DTYPE_F32 && acc_dtype == ODC_DTYPE_F32;
+}
+
 // One record per item, read with scalar loads by the workgroup that works on the item.
 struct GatherDesc {
   uint8_t* dst;
@@ -37,7 +51,8 @@ struct GatherLaunch {
   TileTable tt;
   const uint8_t* base;  // arena base (rank 0 region)
   uint64_t rank_stride;
-  CachePolicy policy;  // picks the kernel
+  CachePolicy policy;    // these two pick the kernel
+  bool short_tiles = false;
   GatherDesc item[kMaxItems];
 };
 
@@ -51,7 +66,8 @@ struct CastGatherLaunch {
   TileTable tt;
   const uint8_t* base;
   uint64_t rank_stride;
-  CachePolicy policy;  // picks the kernel
+  CachePolicy policy;    // these two pick the kernel
+  bool short_tiles = false;
   CastGatherDesc item[kMaxItems];
 };
 
@@ -65,7 +81,8 @@ struct AccumLaunch {
   TileTable tt;
   uint8_t* base;
   uint64_t rank_stride;
-  CachePolicy policy;  // picks the kernel
+  CachePolicy policy;    // these two pick the kernel
+  bool short_tiles = false;
   AccumDesc item[kMaxItems];
 };
 

@@ -29,7 +29,7 @@
 #define ODC_BODY_ALIGN 128  // bytes: alignment of a segment's vector body on the written side
 #endif
 #ifndef ODC_MAX_ITEMS_PER_LAUNCH
-#define ODC_MAX_ITEMS_PER_LAUNCH 64
+#define ODC_MAX_ITEMS_PER_LAUNCH 112
 #endif
 
 namespace odc_tiles {
@@ -41,6 +41,9 @@ constexpr uint32_t kTileVecs = kThreads * kUnroll;  // vectors per tile
 constexpr uint32_t kTileBytes = kTileVecs * 16;     // gather / clear: 16 KiB of destination
 constexpr uint32_t kTileElems = kTileVecs * 4;      // accumulate / cast / publish: 4096 elements
 constexpr uint64_t kMaxTilesPerLaunch = 1ull << 31;
+// Launches of short segments are cut finer: into quarters of a tile (see short_tiles in odc_host.cpp).
+constexpr uint32_t kShortTileParts = 4;
+constexpr uint32_t kShortTileVecs = kTileVecs / kShortTileParts;
 
 // Tile order of a launch (TileTable::order).
 //   kRanksInterleaved : item by item; within an item tile c of rank 0, of rank 1, ..., then c+1
@@ -163,7 +166,9 @@ struct SegShape {
   uint64_t last;  // tile that owns the tail
 };
 
-// unit_bytes: size of one unit on the written side; vec_units: units per vector
+// unit_bytes: size of one unit on the written side; vec_units: units per vector; kVecs: vectors per
+// tile of the launch
+template <uint32_t kVecs = kTileVecs>
 ODC_HD SegShape seg_shape(uintptr_t written_addr, uint64_t n, uint32_t unit_bytes, uint32_t vec_units) {
   // The body starts on a 128 B line of the written side, not merely on a vector boundary: a
   // wavefront's 64 vector stores then cover whole lines, none shared with the next wavefront.
@@ -176,7 +181,7 @@ ODC_HD SegShape seg_shape(uintptr_t written_addr, uint64_t n, uint32_t unit_byte
   g.head = (uint32_t)head;
   g.nvec = (n - head) / vec_units;
   g.tail = (uint32_t)((n - head) - g.nvec * vec_units);
-  g.last = g.nvec ? (g.nvec - 1) / kTileVecs : 0;
+  g.last = g.nvec ? (g.nvec - 1) / kVecs : 0;
   return g;
 }
 
@@ -191,19 +196,22 @@ struct TileWork {
   bool head, tail; // also does the segment's head / tail
 };
 
+template <uint32_t kVecs = kTileVecs>
 ODC_HD TileWork tile_work(uint32_t chunk, const SegShape& g) {
   TileWork w;
-  w.v0 = (uint64_t)chunk * kTileVecs;
-  w.nv = w.v0 >= g.nvec ? 0u : (g.nvec - w.v0 >= kTileVecs ? kTileVecs : (uint32_t)(g.nvec - w.v0));
+  w.v0 = (uint64_t)chunk * kVecs;
+  w.nv = w.v0 >= g.nvec ? 0u : (g.nvec - w.v0 >= kVecs ? kVecs : (uint32_t)(g.nvec - w.v0));
   w.head = chunk == 0 && g.head != 0;
   w.tail = chunk == g.last && g.tail != 0;
   return w;
 }
 
-// A tile is a whole run when all its kTileVecs vectors exist: the unrolled, unguarded loop.
-ODC_HD bool is_whole(const TileWork& w) { return w.nv == kTileVecs; }
+// A tile is a whole run when all its vectors exist: the unrolled, unguarded loop.
+template <uint32_t kVecs = kTileVecs>
+ODC_HD bool is_whole(const TileWork& w) { return w.nv == kVecs; }
 // True when the tile has anything else to do: a partial run, the head or the tail.
-ODC_HD bool has_edges(const TileWork& w) { return (w.nv != 0 && w.nv != kTileVecs) || w.head || w.tail; }
+template <uint32_t kVecs = kTileVecs>
+ODC_HD bool has_edges(const TileWork& w) { return (w.nv != 0 && w.nv != kVecs) || w.head || w.tail; }
 
 // Cuts items [*next, n_items) into one launch: at most kMaxItems non-empty items and fewer than
 // kMaxTilesPerLaunch tiles. units(i) is item i's per-rank size in tile units (0 = skip);

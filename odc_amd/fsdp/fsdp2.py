@@ -609,7 +609,7 @@ def update_gradients(fsdp_param_group) -> None:
 def update_all_gradients(fsdp_param_groups) -> None:
     """``update_gradients`` for every group of a model with as few passes as possible: the
     groups whose accumulations share (accumulation dtype, gradient dtype, divisor) are divided
-    and cast by ONE launch (per 64 groups) instead of one short launch each."""
+    and cast by ONE launch (per 112 groups) instead of one short launch each."""
     scatter = get_reduction_service()
     batches = {}
     for group in fsdp_param_groups:

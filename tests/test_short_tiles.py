@@ -1,0 +1,86 @@
+"""Short tiles: their geometry by brute force on the CPU, how launches are planned in them on a
+dry-run arena, and the kernels at the edges of a short tile against the oracle."""
+
+import ctypes
+import subprocess
+from pathlib import Path
+
+import pytest
+import torch
+
+from helpers import assert_bit_equal, put_shards
+from odc_amd import _native
+from oracle import odc_oracle as oracle
+
+ROOT = Path(__file__).resolve().parent.parent
+
+
+def test_short_tile_geometry(tmp_path):
+    exe = tmp_path / "short_tile_check"
+    subprocess.run(["g++", "-std=c++17", "-O2", "-Wall", "-Wextra", "-fsanitize=address,undefined",
+                    "-fno-sanitize-recover=all", "-Wno-unknown-pragmas", f"-I{ROOT / 'odc_amd' / 'csrc'}",
+                    str(ROOT / "tests" / "cpu" / "short_tile_check.cpp"), "-o", str(exe)], check=True)
+    proc = subprocess.run([str(exe)], capture_output=True, text=True, timeout=300)
+    assert proc.returncode == 0 and "short tiles ok" in proc.stdout, proc.stdout + proc.stderr
+
+
+@pytest.mark.parametrize("shard,acc_dtype,tiles", [
+    (1024, _native.DTYPE_F32, 1), (1025, _native.DTYPE_F32, 2), (200_000, _native.DTYPE_F32, 196),  # always short
+    (4096, _native.DTYPE_BF16, 4), (40 * 4096, _native.DTYPE_BF16, 40),  # short below 32 whole tiles per segment
+])
+def test_plans_in_short_tiles(shard, acc_dtype, tiles):
+    W, lib, handle = 4, _native.load(), ctypes.c_void_p()
+    _native.set_option("dry_run_short_tiles", 1)
+    try:
+        _native.check(lib.odc_arena_create(W, 1 << 30, _native.ODC_ARENA_DRY_RUN, ctypes.byref(handle)))
+    finally:
+        _native.set_option("dry_run_short_tiles", 0)
+    _native.set_option("dry_run_reset", 0)
+    item = (_native.AccumItem * 1)(_native.AccumItem(1 << 33, W * shard, 0, shard))
+    _native.check(lib.odc_scatter_accumulate(handle, item, 1, _native.DTYPE_BF16, acc_dtype, None))
+    assert _native.get_option("dry_run_tiles") == _native.get_option("dry_run_workgroups") == W * tiles
+    _native.check(lib.odc_arena_destroy(handle))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("below", [0, 1 << 30])  # whole tiles where there is a choice, short tiles everywhere
+@pytest.mark.parametrize("dtypes", [
+    (torch.bfloat16, torch.bfloat16, torch.float32), (torch.float32, torch.bfloat16, torch.bfloat16),
+    (torch.float32, torch.float32, torch.float32), (torch.float16, torch.float32, torch.float16),
+], ids=lambda d: "-".join(str(x).rsplit(".", 1)[-1] for x in d))
+def test_kernels_at_the_edges_of_a_short_tile(make_world, below, dtypes):
+    from odc_amd import GatherService, ReductionService, SymmBufferRegistry
+
+    shard_dtype, compute_dtype, acc_dtype = dtypes
+    saved = _native.get_option("short_tiles_below")
+    _native.set_option("short_tiles_below", below)
+    try:
+        W, sizes = 3, [1, 63, 1023, 1024, 1025, 2047, 2049, 4095, 4097, 20_481]
+        group = make_world(W, 4 << 20)
+        registry = SymmBufferRegistry.get_instance()
+        gather, red = GatherService(), ReductionService(accumulation_dtype=acc_dtype, lazy_clear=True)
+        gen = torch.Generator().manual_seed(11)
+        shards = [[torch.randn(n, generator=gen).to(shard_dtype) for _ in range(W)] for n in sizes]
+        sources = [put_shards(registry, ("p", i), s) for i, s in enumerate(shards)]
+        outs = [torch.full((W * n,), float("nan"), dtype=compute_dtype, device="cuda") for n in sizes]
+        gather.gather_into_tensors(outs, sources, group)
+        for out, s in zip(outs, shards):
+            assert_bit_equal(out, oracle.gather(s) if shard_dtype == compute_dtype else oracle.gather_cast(s, compute_dtype))
+
+        keys = list(range(len(sizes)))
+        for key, n in zip(keys, sizes):
+            red.register(key, (n,), compute_dtype, acc_dtype, group)
+        want = [[torch.zeros(n, dtype=acc_dtype) for _ in range(W)] for n in sizes]
+        red.clear_accumulations()
+        for m in range(3):  # the store form, then read-modify-write; gradients that end early
+            valid = [max(0, W * n - m) for n in sizes]
+            grads = [torch.randn(v, generator=gen).to(compute_dtype) for v in valid]
+            red.scatter_accumulate_multi(keys, [g.cuda() for g in grads], group, valid_numels=valid)
+            for accs, g, n in zip(want, grads, sizes):
+                oracle.scatter_accumulate(accs, torch.nn.functional.pad(g, [0, W * n - g.numel()]))
+        red.sync(group)
+        for key, accs in zip(keys, want):
+            for r, got in enumerate(red.get_peer_accumulations(key)):
+                assert_bit_equal(got, accs[r], f"size {sizes[key]} rank {r}")
+    finally:
+        _native.set_option("short_tiles_below", saved)
