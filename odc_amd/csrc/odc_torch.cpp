@@ -14,8 +14,6 @@
 #include <Python.h>
 
 #include <ATen/core/Tensor.h>
-#include <ATen/ops/as_strided.h>
-#include <ATen/ops/empty.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <cstddef>
@@ -101,19 +99,29 @@ void expect_args(Py_ssize_t n, Py_ssize_t want) {
   if (n != want) raise(PyExc_TypeError, "expected %zd arguments, got %zd", want, n);
 }
 
-uint64_t as_u64(PyObject* o) {
-  const unsigned long long v = PyLong_AsUnsignedLongLong(o);
+// The value of an int object; the reference to it is given up. Negative ones fail like the size
+// checks they come from.
+uint64_t take_u64(PyObject* i) {
+  if (!i) throw Failed();
+  const unsigned long long v = PyLong_AsUnsignedLongLong(i);
+  Py_DECREF(i);
   if (v == (unsigned long long)-1 && PyErr_Occurred()) {
-    PyErr_Clear();  // not an int object: anything with __index__ (numpy integers)
-    PyObject* i = PyNumber_Index(o);
-    if (!i) throw Failed();
-    const unsigned long long w = PyLong_AsUnsignedLongLong(i);
-    Py_DECREF(i);
-    if (w == (unsigned long long)-1 && PyErr_Occurred()) throw Failed();
-    return w;
+    PyErr_Clear();
+    raise(PyExc_AssertionError, "an offset or a size is negative or does not fit 64 bits");
   }
   return v;
 }
+
+uint64_t as_u64(PyObject* o) {
+  if (PyLong_CheckExact(o)) {
+    Py_INCREF(o);
+    return take_u64(o);
+  }
+  return take_u64(PyNumber_Index(o));  // anything with __index__ (numpy integers)
+}
+
+// int(o): a count that the caller may have left a float or a tensor of one element
+uint64_t as_count(PyObject* o) { return PyLong_CheckExact(o) ? as_u64(o) : take_u64(PyNumber_Long(o)); }
 
 void* as_pointer(PyObject* o) { return reinterpret_cast<void*>((uintptr_t)as_u64(o)); }
 
@@ -222,6 +230,7 @@ PyObject* gather(PyObject*, PyObject* const* args, Py_ssize_t n) {
   return guarded([&] {
     expect_args(n, 6);
     const Sequence outs(args[4], "outputs are a sequence"), shards(args[5], "shards are a sequence");
+    ODC_ASSERT(outs.size() == shards.size() && shards.size() > 0, "one output per shard");
     GatherCall call{static_cast<odc_arena*>(as_pointer(args[0])), (uint32_t)as_u64(args[1]), (uint32_t)as_u64(args[2]),
                     as_pointer(args[3]), as_tensor(shards[0]).scalar_type()};
     call.plain.reserve((size_t)shards.size());
@@ -246,6 +255,7 @@ PyObject* gather_slices(PyObject*, PyObject* const* args, Py_ssize_t n) {
     expect_args(n, 8);
     const Sequence outs(args[4], "outputs are a sequence"), offsets(args[6], "slice offsets are a sequence"),
         numels(args[7], "slice sizes are a sequence");
+    ODC_ASSERT(outs.size() == offsets.size() && outs.size() == numels.size(), "one offset and size per output");
     const at::Tensor& input = as_tensor(args[5]);
     GatherCall call{static_cast<odc_arena*>(as_pointer(args[0])), (uint32_t)as_u64(args[1]), (uint32_t)as_u64(args[2]),
                     as_pointer(args[3]), input.scalar_type()};
@@ -330,7 +340,9 @@ PyObject* accumulate_batch(PyObject*, PyObject* const* args, Py_ssize_t n) {
     const Sequence keys(args[2], "keys are a sequence"), grads(args[3], "gradients are a sequence");
     const bool padded = args[4] != Py_None;
     const Sequence valid(padded ? args[4] : args[2], "valid_numels is a sequence");
-    ODC_ASSERT(valid.size() == keys.size(), "one valid_numel per key");
+    ODC_ASSERT(grads.size() == keys.size(), "one gradient per key");
+    ODC_ASSERT(valid.size() >= keys.size(), "one valid_numel per key");
+    if (!keys.size()) Py_RETURN_NONE;
     BatchRef ref;
     std::vector<odc_accum_item>& items = *ref.b->items;
     items.reserve((size_t)keys.size());
@@ -348,7 +360,7 @@ PyObject* accumulate_batch(PyObject*, PyObject* const* args, Py_ssize_t n) {
       const uint64_t numel = (uint64_t)grad.numel();
       uint64_t elems = numel;
       if (padded) {
-        elems = as_u64(valid[k]);
+        elems = as_count(valid[k]);
         ODC_ASSERT(elems <= numel && elems <= world * acc.numel,
                    "valid_numel %llu exceeds the gradient (%llu) or the %llu elements of the key's shards",
                    (unsigned long long)elems, (unsigned long long)numel, (unsigned long long)(world * acc.numel));
@@ -474,7 +486,7 @@ PyObject* slice_layout_batch(PyObject* self, PyObject* const* args, Py_ssize_t n
     const Accumulation acc = as_accumulation(args[0]);
     const uint64_t world = as_u64(args[1]), bytes = dtype_bytes(acc.code);
     const Sequence grads(args[2], "gradients are a sequence");
-    ODC_ASSERT((size_t)grads.size() == s->offsets->size(), "one gradient per slice");
+    ODC_ASSERT((size_t)grads.size() == s->offsets->size() && grads.size() > 0, "one gradient per slice");
     BatchRef ref;
     ref.b->acc_code = acc.code;
     ref.b->items->reserve((size_t)grads.size());
@@ -541,6 +553,7 @@ PyObject* publish(PyObject*, PyObject* const* args, Py_ssize_t n) {
   return guarded([&] {
     expect_args(n, 8);
     const Sequence keys(args[4], "keys are a sequence"), outs(args[5], "outputs are a sequence");
+    ODC_ASSERT(outs.size() == keys.size(), "one output per key");
     std::vector<odc_publish_item> items;
     items.reserve((size_t)keys.size());
     int acc_code = -1;

@@ -69,6 +69,34 @@ def test_refusals(make_world):
         assert not peer.any()
 
 
+def test_counts_and_their_limits(make_world):
+    """Valid sizes go through int() and the list may be longer than the keys; negative sizes and
+    offsets are assertions, and nothing is written by a refused call."""
+    from odc_amd import GatherService, ReductionService, SymmBufferRegistry
+
+    W = 2
+    group = make_world(W, 1 << 20)
+    gather, red = GatherService(), ReductionService(accumulation_dtype=torch.float32)
+    red.register("k", (4,), torch.bfloat16, torch.float32, group)
+    grad = torch.arange(8, dtype=torch.bfloat16, device="cuda")
+    for count in (7.0, torch.tensor(7), np.int32(7)):
+        red.scatter_accumulate_multi(["k"], [grad], group, valid_numels=[count, 99])
+    want = torch.arange(8, dtype=torch.float32) * 3
+    want[7] = 0
+    for r, got in enumerate(red.get_peer_accumulations("k")):
+        assert_bit_equal(got, want.view(W, -1)[r])
+    shard = SymmBufferRegistry.get_instance().allocate_symm_buffer("s", (8,), torch.bfloat16)
+    for call in (lambda: gather.gather_slices([grad], shard, [-1], [4], group),
+                 lambda: gather.gather_slices([grad], shard, [5], [4], group),
+                 lambda: red.scatter_accumulate_slices("k", [grad], [-1], [4], group),
+                 lambda: red.scatter_accumulate_multi(["k"], [grad], group, valid_numels=[-1]),
+                 lambda: red.scatter_accumulate_multi(["k"], [grad], group, valid_numels=[])):
+        with pytest.raises(AssertionError):
+            call()
+    for r, got in enumerate(red.get_peer_accumulations("k")):
+        assert_bit_equal(got, want.view(W, -1)[r])
+
+
 def test_buffers_that_are_gone_are_not_used(make_world):
     """A registry that freed its buffers voids what services noted about them, in the same arena."""
     from odc_amd import ReductionService, SymmBufferRegistry
