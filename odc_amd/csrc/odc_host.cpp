@@ -911,17 +911,18 @@ int odc_publish(odc_arena* a, uint32_t rank, const odc_publish_item* items, uint
   uint32_t next = 0;
   while (next < n_items) {
     PublishLaunch L;
-    L.region = region;
-    L.divisor = divisor;
-    L.divide = divisor != 1.0f;
-    L.reciprocal = 1.0f;
+    L.base = region;
+    L.rank_stride = 0;
+    L.scale.divisor = divisor;
+    L.scale.divide = divisor != 1.0f;
+    L.scale.reciprocal = 1.0f;
     // Dividing by a power of two whose reciprocal is a normal number is the same correctly
     // rounded result as multiplying by that reciprocal (both round one exact real value), and
     // costs one instruction instead of the division sequence.
     int exponent = 0;
-    if (L.divide && std::fabs(std::frexp(divisor, &exponent)) == 0.5f && exponent > -120 && exponent < 120) {
-      L.reciprocal = 1.0f / divisor;
-      L.divide = 2;
+    if (L.scale.divide && std::fabs(std::frexp(divisor, &exponent)) == 0.5f && exponent > -120 && exponent < 120) {
+      L.scale.reciprocal = 1.0f / divisor;
+      L.scale.divide = 2;
     }
     L.tt.order = kItemMajor;
     L.tt.first_rank = 0;

@@ -33,6 +33,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "odc_hip.h"
 #include "odc_launch.h"
 #include "odc_tiles.h"
@@ -94,12 +96,87 @@ __device__ __forceinline__ void store_vec(V* p, V v) {  // aligned
   if constexpr (kCached) *p = v; else __builtin_nontemporal_store(v, p);
 }
 
+// An address in device memory. Of an address that comes as an argument of a function, or as a number,
+// the compiler must assume that it may lie in LDS or scratch, and it takes the slower flat accesses.
+template <class P>
+__device__ __forceinline__ P* as_global(P* p) {
+  return (P*)(__attribute__((address_space(1))) P*)(uintptr_t)p;
+}
+
+// ---- finding a tile's work ------------------------------------------------------------------
+// The walk of a workgroup over the tiles of its launch; all its lanes come along.
+template <class Launch>
+struct TileWalk {
+  typedef typename Launch::Desc Desc;
+  TileCursor cur;
+  Desc it = {};  // the item of the tile located last
+
+  __device__ __forceinline__ explicit TileWalk(const Launch&) {}
+  __device__ __forceinline__ uint32_t n_tiles(const Launch& launch) const { return launch.tt.n_tiles; }
+  __device__ __forceinline__ uint8_t* region(const Launch& launch, uint32_t rank) const {
+    return launch.base + (uint64_t)rank * launch.rank_stride;
+  }
+  __device__ __forceinline__ TileCoord locate(const Launch& launch, uint32_t t) {
+    if (!cursor_holds(cur, t)) {
+      cursor_seek(launch.tt, t, cur);
+      it = launch.item[cur.item];  // issued together with the loads of cursor_enter
+      cursor_enter(launch.tt, cur);
+    }
+    return cursor_coord(launch.tt, cur, t);
+  }
+};
+
+// A launch of one item: a small one is a chain of memory latencies, a third of which was reading
+// the arguments in four dependent steps, from memory that no cache has seen. Here all of them are
+// read at once. Kernel times, us: gather and accumulate of a 4096-element vector at W = 8 3.0 -> 2.5
+// and 3.4 -> 2.8 (an empty kernel takes 1.4); gather, accumulate and publish of 4 Mi elements at
+// W = 4 4.6 -> 3.9, 7.1 -> 6.8, 5.2 -> 4.7. Launches of hundreds of megabytes are level.
+template <class D>
+struct SingleWalk {
+  typedef D Desc;
+  TileHead tt;
+  uint8_t* base;
+  uint64_t rank_stride;
+  Desc it;
+
+  __device__ __forceinline__ explicit SingleWalk(const SingleLaunch<D>& launch) {
+    static_assert(sizeof(D) % 8 == 0 && sizeof(D) >= 16 && sizeof(D) <= 32, "2 to 4 words");
+    constexpr int kWords = sizeof(D) / 8;
+    tt = launch.tt;
+    uint64_t b = (uint64_t)(uintptr_t)launch.base, stride = launch.rank_stride;
+    uint64_t w[4] = {0, 0, 0, 0};
+#pragma unroll
+    for (int i = 0; i < kWords; ++i) w[i] = reinterpret_cast<const uint64_t*>(launch.item)[i];
+    // (left alone, the compiler reads each value where it is first used)
+    asm volatile("" : "+s"(tt.world), "+s"(tt.n_tiles), "+s"(tt.order), "+s"(tt.first_rank), "+s"(tt.tiles_per_rank),
+                      "+s"(b), "+s"(stride), "+s"(w[0]), "+s"(w[1]), "+s"(w[2]), "+s"(w[3]));
+    base = as_global(reinterpret_cast<uint8_t*>((uintptr_t)b));
+    rank_stride = stride;
+    __builtin_memcpy(&it, w, sizeof(D));
+  }
+  __device__ __forceinline__ uint32_t n_tiles(const SingleLaunch<D>&) const { return tt.n_tiles; }
+  __device__ __forceinline__ uint8_t* region(const SingleLaunch<D>&, uint32_t rank) const {
+    return base + (uint64_t)rank * rank_stride;
+  }
+  __device__ __forceinline__ TileCoord locate(const SingleLaunch<D>&, uint32_t t) const { return single_item_coord(tt, t); }
+};
+template <class D>
+struct TileWalk<SingleLaunch<D>> : SingleWalk<D> {
+  using SingleWalk<D>::SingleWalk;
+};
+template <>
+struct TileWalk<PublishSingle> : SingleWalk<PublishDesc> {
+  using SingleWalk<PublishDesc>::SingleWalk;
+};
+
 // ---- gather -------------------------------------------------------------------------------
 // Everything of a tile that is not a run of T * U whole vectors: the last partial run, the
 // head and the tail. Kept out of line so that the streaming loop stays tight (inline, the
 // short-segment kernels, which come here for most of their tiles, were 5 % slower too).
 template <bool kSrcCached, bool kDstCached, int T, int U>
 __device__ __attribute__((noinline)) void gather_edges(uint8_t* d, const uint8_t* s, uint32_t chunk, SegShape g) {
+  d = as_global(d);
+  s = as_global(s);
   // Every load of the tile is issued before its first store (a lone resident workgroup would
   // otherwise pay one memory round trip per vector).
   const uint32_t tid = threadIdx.x;
@@ -126,24 +203,19 @@ __device__ __attribute__((noinline)) void gather_edges(uint8_t* d, const uint8_t
 
 // T threads do a tile of T * U vectors in one step; the copies stream best from 512-thread
 // workgroups, of which 4 fit a CU.
-template <bool kSrcCached, bool kDstCached, int T, int U>
-__global__ __launch_bounds__(T) void gather_kernel(const GatherLaunch launch) {
+template <class Launch, bool kSrcCached, bool kDstCached, int T, int U>
+__global__ __launch_bounds__(T) void gather_kernel(const Launch launch) {
   constexpr uint32_t kVecs = T * U;
   static_assert(kVecs == kTileVecs || kVecs == kShortTileVecs, "a whole tile or a short one");
   static_assert(T >= ODC_BODY_ALIGN - 1, "one lane per head byte");
   const uint32_t tid = threadIdx.x;
-  TileCursor cur;
-  GatherDesc it = {};
-  for (uint32_t t = blockIdx.x; t < launch.tt.n_tiles; t += gridDim.x) {
-    if (!cursor_holds(cur, t)) {
-      cursor_seek(launch.tt, t, cur);
-      it = launch.item[cur.item];  // issued together with the loads of cursor_enter
-      cursor_enter(launch.tt, cur);
-    }
-    const TileCoord c = cursor_coord(launch.tt, cur, t);
+  TileWalk<Launch> walk(launch);
+  for (uint32_t t = blockIdx.x; t < walk.n_tiles(launch); t += gridDim.x) {
+    const TileCoord c = walk.locate(launch, t);
+    const GatherDesc it = walk.it;
     const uint64_t seg = it.seg_bytes;
-    const uint8_t* s = launch.base + (uint64_t)c.rank * launch.rank_stride + it.src_off;
-    uint8_t* d = it.dst + (uint64_t)c.rank * seg;
+    const uint8_t* s = walk.region(launch, c.rank) + it.src_off;
+    uint8_t* d = as_global(it.dst) + (uint64_t)c.rank * seg;
     const SegShape g = seg_shape<kVecs>((uintptr_t)d, seg, 1, 16);
     const TileWork w = tile_work<kVecs>(c.chunk, g);
     if (is_whole<kVecs>(w)) {
@@ -173,6 +245,7 @@ __global__ __launch_bounds__(T) void gather_kernel(const GatherLaunch launch) {
 // ---- clear --------------------------------------------------------------------------------
 // Plain (not nontemporal) stores: for a write-only stream they measure faster here.
 __device__ __attribute__((noinline)) void clear_edges(uint8_t* d, uint32_t chunk, SegShape g) {
+  d = as_global(d);
   const u32x4 zero = {0u, 0u, 0u, 0u};
   const uint32_t tid = threadIdx.x;
   const TileWork w = tile_work(chunk, g);
@@ -186,19 +259,15 @@ __device__ __attribute__((noinline)) void clear_edges(uint8_t* d, uint32_t chunk
   if (w.tail && tid < g.tail) d[g.head + g.nvec * 16 + tid] = 0;
 }
 
-__global__ __launch_bounds__(kThreads) void clear_kernel(const ClearLaunch launch) {
+template <class Launch>
+__global__ __launch_bounds__(kThreads) void clear_kernel(const Launch launch) {
   const u32x4 zero = {0u, 0u, 0u, 0u};
   const uint32_t tid = threadIdx.x;
-  TileCursor cur;
-  ClearDesc it = {};
-  for (uint32_t t = blockIdx.x; t < launch.tt.n_tiles; t += gridDim.x) {
-    if (!cursor_holds(cur, t)) {
-      cursor_seek(launch.tt, t, cur);
-      it = launch.item[cur.item];  // issued together with the loads of cursor_enter
-      cursor_enter(launch.tt, cur);
-    }
-    const TileCoord c = cursor_coord(launch.tt, cur, t);
-    uint8_t* d = launch.base + (uint64_t)c.rank * launch.rank_stride + it.off;
+  TileWalk<Launch> walk(launch);
+  for (uint32_t t = blockIdx.x; t < walk.n_tiles(launch); t += gridDim.x) {
+    const TileCoord c = walk.locate(launch, t);
+    const ClearDesc it = walk.it;
+    uint8_t* d = walk.region(launch, c.rank) + it.off;
     const SegShape g = seg_shape((uintptr_t)d, it.seg_bytes, 1, 16);
     const TileWork w = tile_work(c.chunk, g);
     if (is_whole(w)) {
@@ -304,6 +373,8 @@ template <class G, class A, bool kStore, bool kGradCached, bool kAccCached, int 
 __device__ __attribute__((noinline)) void accum_edges(uint8_t* acc, const uint8_t* grad, uint64_t g_seg,
                                                       uint64_t grad_elems, uint32_t chunk, SegShape g,
                                                       bool body) {
+  acc = as_global(acc);
+  grad = as_global(grad);
   typedef typename Quad<G>::vec_t gvec_t;
   typedef typename Quad<A>::vec_t avec_t;
   typedef typename Codec<G>::raw_t graw_t;
@@ -374,8 +445,8 @@ __device__ __attribute__((noinline)) void accum_edges(uint8_t* acc, const uint8_
   if (do_tail) as[tail_at] = Codec<A>::narrow(Codec<A>::widen(tail_araw) + Codec<G>::widen(tail_graw));
 }
 
-template <class G, class A, bool kStore, bool kGradCached, bool kAccCached, int T, int U>
-__global__ __launch_bounds__(T) void accum_kernel(const AccumLaunch launch) {
+template <class Launch, class G, class A, bool kStore, bool kGradCached, bool kAccCached, int T, int U>
+__global__ __launch_bounds__(T) void accum_kernel(const Launch launch) {
   constexpr uint32_t kVecs = T * U;  // quads
   static_assert(kVecs == kTileVecs || kVecs == kShortTileVecs, "a whole tile or a short one");
   typedef typename Quad<G>::vec_t gvec_t;
@@ -383,17 +454,12 @@ __global__ __launch_bounds__(T) void accum_kernel(const AccumLaunch launch) {
   constexpr uint32_t kAB = Codec<A>::kBytes, kGB = Codec<G>::kBytes;
   static_assert(T >= ODC_BODY_ALIGN / kAB, "one lane per head element");
   const uint32_t tid = threadIdx.x;
-  TileCursor cur;
-  AccumDesc it = {};
-  for (uint32_t t = blockIdx.x; t < launch.tt.n_tiles; t += gridDim.x) {
-    if (!cursor_holds(cur, t)) {
-      cursor_seek(launch.tt, t, cur);
-      it = launch.item[cur.item];  // issued together with the loads of cursor_enter
-      cursor_enter(launch.tt, cur);
-    }
-    const TileCoord c = cursor_coord(launch.tt, cur, t);
+  TileWalk<Launch> walk(launch);
+  for (uint32_t t = blockIdx.x; t < walk.n_tiles(launch); t += gridDim.x) {
+    const TileCoord c = walk.locate(launch, t);
+    const AccumDesc it = walk.it;
     const uint64_t seg = it.seg_elems;
-    uint8_t* acc = launch.base + (uint64_t)c.rank * launch.rank_stride + it.acc_off;
+    uint8_t* acc = walk.region(launch, c.rank) + it.acc_off;
     const uint64_t g_seg = (uint64_t)c.rank * seg;  // gradient index of the segment's first element
     const SegShape g = seg_shape<kVecs>((uintptr_t)acc, seg, kAB, 4);
     const TileWork w = tile_work<kVecs>(c.chunk, g);
@@ -401,7 +467,7 @@ __global__ __launch_bounds__(T) void accum_kernel(const AccumLaunch launch) {
     // whole: all its quads exist in the accumulation AND in the valid part of the gradient
     const bool whole = is_whole<kVecs>(w) && g_seg + e0 + 4 * kVecs <= it.grad_elems;
     if (whole) {
-      const uint8_t* gb = it.grad + (g_seg + e0) * kGB + (size_t)tid * sizeof(gvec_t);
+      const uint8_t* gb = as_global(it.grad) + (g_seg + e0) * kGB + (size_t)tid * sizeof(gvec_t);
       avec_t* ap = reinterpret_cast<avec_t*>(acc + e0 * kAB) + tid;
       gvec_t graw[U];
       avec_t araw[U];
@@ -434,6 +500,8 @@ __global__ __launch_bounds__(T) void accum_kernel(const AccumLaunch launch) {
 // a second symmetric buffer.
 template <class S, class D, bool kCached, int T, int U>
 __device__ __attribute__((noinline)) void cast_edges(uint8_t* d, const uint8_t* s, uint32_t chunk, SegShape g) {
+  d = as_global(d);
+  s = as_global(s);
   typedef typename Quad<S>::vec_t svec_t;
   typedef typename Quad<D>::vec_t dvec_t;
   typedef typename Codec<S>::raw_t sraw_t;
@@ -473,8 +541,8 @@ __device__ __attribute__((noinline)) void cast_edges(uint8_t* d, const uint8_t* 
   if (do_tail) ds[tail_at] = Codec<D>::narrow(Codec<S>::widen(tail_raw));
 }
 
-template <class S, class D, bool kCached, int T, int U>
-__global__ __launch_bounds__(T) void cast_gather_kernel(const CastGatherLaunch launch) {
+template <class Launch, class S, class D, bool kCached, int T, int U>
+__global__ __launch_bounds__(T) void cast_gather_kernel(const Launch launch) {
   constexpr uint32_t kVecs = T * U;  // quads
   static_assert(kVecs == kTileVecs || kVecs == kShortTileVecs, "a whole tile or a short one");
   static_assert(T >= ODC_BODY_ALIGN / Codec<D>::kBytes, "one lane per head element");
@@ -482,18 +550,13 @@ __global__ __launch_bounds__(T) void cast_gather_kernel(const CastGatherLaunch l
   typedef typename Quad<D>::vec_t dvec_t;
   constexpr uint32_t kSB = Codec<S>::kBytes, kDB = Codec<D>::kBytes;
   const uint32_t tid = threadIdx.x;
-  TileCursor cur;
-  CastGatherDesc it = {};
-  for (uint32_t t = blockIdx.x; t < launch.tt.n_tiles; t += gridDim.x) {
-    if (!cursor_holds(cur, t)) {
-      cursor_seek(launch.tt, t, cur);
-      it = launch.item[cur.item];  // issued together with the loads of cursor_enter
-      cursor_enter(launch.tt, cur);
-    }
-    const TileCoord c = cursor_coord(launch.tt, cur, t);
+  TileWalk<Launch> walk(launch);
+  for (uint32_t t = blockIdx.x; t < walk.n_tiles(launch); t += gridDim.x) {
+    const TileCoord c = walk.locate(launch, t);
+    const CastGatherDesc it = walk.it;
     const uint64_t seg = it.seg_elems;
-    const uint8_t* s = launch.base + (uint64_t)c.rank * launch.rank_stride + it.src_off;
-    uint8_t* d = it.dst + (uint64_t)c.rank * it.dst_stride;
+    const uint8_t* s = walk.region(launch, c.rank) + it.src_off;
+    uint8_t* d = as_global(it.dst) + (uint64_t)c.rank * it.dst_stride;
     const SegShape g = seg_shape<kVecs>((uintptr_t)d, seg, kDB, 4);
     const TileWork w = tile_work<kVecs>(c.chunk, g);
     if (is_whole<kVecs>(w)) {
@@ -533,24 +596,24 @@ __global__ __launch_bounds__(T) void cast_gather_kernel(const CastGatherLaunch l
 // rounded IEEE division, rounded to the accumulation dtype) and out[i] = narrow_O(acc[i]).
 template <class A>
 __device__ __forceinline__ typename Codec<A>::raw_t publish_scale(typename Codec<A>::raw_t raw,
-                                                                  const PublishLaunch& launch) {
+                                                                  const PublishScale& by) {
   const float x = Codec<A>::widen(raw);
-  return Codec<A>::narrow(launch.divide == 2 ? x * launch.reciprocal : x / launch.divisor);
+  return Codec<A>::narrow(by.divide == 2 ? x * by.reciprocal : x / by.divisor);
 }
 
 // Four elements: scales `raw` in place when the launch divides and returns the cast copy.
 template <class A, class O>
 __device__ __forceinline__ typename Quad<O>::vec_t publish_quad(typename Quad<A>::vec_t& raw,
-                                                                const PublishLaunch& launch) {
+                                                                const PublishScale& by) {
   float f[4];
   Quad<A>::widen(raw, f);
-  if (launch.divide) {
-    if (launch.divide == 2) {
+  if (by.divide) {
+    if (by.divide == 2) {
 #pragma unroll
-      for (int k = 0; k < 4; ++k) f[k] = f[k] * launch.reciprocal;
+      for (int k = 0; k < 4; ++k) f[k] = f[k] * by.reciprocal;
     } else {
 #pragma unroll
-      for (int k = 0; k < 4; ++k) f[k] = f[k] / launch.divisor;
+      for (int k = 0; k < 4; ++k) f[k] = f[k] / by.divisor;
     }
     raw = Quad<A>::narrow(f);
     Quad<A>::widen(raw, f);  // the copy is a cast of the ROUNDED accumulation
@@ -558,26 +621,21 @@ __device__ __forceinline__ typename Quad<O>::vec_t publish_quad(typename Quad<A>
   return Quad<O>::narrow(f);
 }
 
-template <class A, class O>
-__global__ __launch_bounds__(kThreads) void publish_kernel(const PublishLaunch launch) {
+template <class Launch, class A, class O>
+__global__ __launch_bounds__(kThreads) void publish_kernel(const Launch launch) {
   typedef typename Codec<A>::raw_t araw_t;
   typedef typename Codec<O>::raw_t oraw_t;
   typedef typename Quad<A>::vec_t avec_t;
   typedef typename Quad<O>::vec_t ovec_t;
   const uint32_t tid = threadIdx.x;
-  TileCursor cur;
-  PublishDesc it = {};
-  for (uint32_t t = blockIdx.x; t < launch.tt.n_tiles; t += gridDim.x) {
-    if (!cursor_holds(cur, t)) {
-      cursor_seek(launch.tt, t, cur);
-      it = launch.item[cur.item];  // issued together with the loads of cursor_enter
-      cursor_enter(launch.tt, cur);
-    }
-    const TileCoord c = cursor_coord(launch.tt, cur, t);
+  TileWalk<Launch> walk(launch);
+  for (uint32_t t = blockIdx.x; t < walk.n_tiles(launch); t += gridDim.x) {
+    const TileCoord c = walk.locate(launch, t);
+    const PublishDesc it = walk.it;
     const uint64_t seg = it.seg_elems;
     const uint64_t in_seg = (uint64_t)c.chunk * kTileElems;
-    araw_t* acc = reinterpret_cast<araw_t*>(launch.region + it.acc_off) + in_seg;
-    oraw_t* out = it.out ? reinterpret_cast<oraw_t*>(it.out) + in_seg : nullptr;
+    araw_t* acc = reinterpret_cast<araw_t*>(walk.region(launch, 0) + it.acc_off) + in_seg;
+    oraw_t* out = it.out ? reinterpret_cast<oraw_t*>(as_global(it.out)) + in_seg : nullptr;
     const uint64_t left = seg - in_seg;
     if (left >= kTileElems && (((uintptr_t)acc) & (sizeof(avec_t) - 1)) == 0 &&
         (((uintptr_t)out) & (sizeof(ovec_t) - 1)) == 0) {
@@ -589,11 +647,11 @@ __global__ __launch_bounds__(kThreads) void publish_kernel(const PublishLaunch l
       for (int u = 0; u < kUnroll; ++u) raw[u] = __builtin_nontemporal_load(ap + u * kThreads);
 #pragma unroll
       for (int u = 0; u < kUnroll; ++u) {
-        cast[u] = publish_quad<A, O>(raw[u], launch);
+        cast[u] = publish_quad<A, O>(raw[u], launch.scale);
       }
       // The two written streams go out one after the other, not interleaved vector by vector
       // (measured: +6..12 %; plain instead of nontemporal stores for the copy change nothing then).
-      if (launch.divide) {
+      if (launch.scale.divide) {
 #pragma unroll
         for (int u = 0; u < kUnroll; ++u) __builtin_nontemporal_store(raw[u], ap + u * kThreads);
       }
@@ -618,13 +676,13 @@ __global__ __launch_bounds__(kThreads) void publish_kernel(const PublishLaunch l
 #pragma unroll
       for (int u = 0; u < kUnroll; ++u) {
         if (u * kThreads + tid < quads) {
-          const ovec_t cast = publish_quad<A, O>(raw[u], launch);
-          if (launch.divide) __builtin_nontemporal_store(raw[u], ap + u * kThreads);
+          const ovec_t cast = publish_quad<A, O>(raw[u], launch.scale);
+          if (launch.scale.divide) __builtin_nontemporal_store(raw[u], ap + u * kThreads);
           if (out) __builtin_nontemporal_store(cast, op + u * kThreads);
         }
       }
       if (tid < rest) {
-        if (launch.divide) acc[quads * 4 + tid] = rest_raw = publish_scale<A>(rest_raw, launch);
+        if (launch.scale.divide) acc[quads * 4 + tid] = rest_raw = publish_scale<A>(rest_raw, launch.scale);
         if (out) out[quads * 4 + tid] = Codec<O>::narrow(Codec<A>::widen(rest_raw));
       }
     } else {
@@ -640,7 +698,7 @@ __global__ __launch_bounds__(kThreads) void publish_kernel(const PublishLaunch l
       for (int j = 0; j < kPerLane; ++j) {
         const uint32_t i = j * kThreads + tid;
         if (i < n) {
-          if (launch.divide) acc[i] = raw[j] = publish_scale<A>(raw[j], launch);
+          if (launch.scale.divide) acc[i] = raw[j] = publish_scale<A>(raw[j], launch.scale);
           if (out) out[i] = Codec<O>::narrow(Codec<A>::widen(raw[j]));
         }
       }
@@ -651,10 +709,7 @@ __global__ __launch_bounds__(kThreads) void publish_kernel(const PublishLaunch l
 // ------------------------------------------------------------------------------------------------
 // dtype dispatch
 // ------------------------------------------------------------------------------------------------
-typedef void (*gather_fn)(const GatherLaunch);
-typedef void (*accum_fn)(const AccumLaunch);
-typedef void (*cast_gather_fn)(const CastGatherLaunch);
-typedef void (*publish_fn)(const PublishLaunch);
+template <class Launch> using kernel_fn = void (*)(const Launch);
 
 #define ODC_FOR_EACH_DTYPE_PAIR(X)                    \
   X(ODC_DTYPE_BF16, bf16_tag, ODC_DTYPE_BF16, bf16_tag) \
@@ -669,68 +724,91 @@ typedef void (*publish_fn)(const PublishLaunch);
 
 // (gradient dtype, accumulation dtype). The store form never reads the accumulation and keeps it
 // nontemporal; the read-modify-write keeps it cached only together with the gradient.
-template <class G, class A, int T, int U>
-accum_fn pick_rmw(CachePolicy policy) {
-  if (policy.read && policy.written) return accum_kernel<G, A, false, true, true, T, U>;
-  return policy.read ? accum_kernel<G, A, false, true, false, T, U> : accum_kernel<G, A, false, false, false, T, U>;
+template <class L, class G, class A, int T, int U>
+kernel_fn<L> pick_rmw(CachePolicy policy) {
+  if (policy.read && policy.written) return accum_kernel<L, G, A, false, true, true, T, U>;
+  return policy.read ? accum_kernel<L, G, A, false, true, false, T, U> : accum_kernel<L, G, A, false, false, false, T, U>;
 }
 
-template <class G, class A, int T, int U>
-accum_fn pick_store(CachePolicy policy) {
-  return policy.read ? accum_kernel<G, A, true, true, false, T, U> : accum_kernel<G, A, true, false, false, T, U>;
+template <class L, class G, class A, int T, int U>
+kernel_fn<L> pick_store(CachePolicy policy) {
+  return policy.read ? accum_kernel<L, G, A, true, true, false, T, U> : accum_kernel<L, G, A, true, false, false, T, U>;
 }
 
 // kShortOnly: accum_streams_short says so, there is no kernel of whole tiles.
-template <class G, class A, bool kShortOnly>
-accum_fn pick_accum_form(bool store, CachePolicy policy, bool short_tiles) {
+template <class L, class G, class A, bool kShortOnly>
+kernel_fn<L> pick_accum_form(bool store, CachePolicy policy, bool short_tiles) {
   if (short_tiles)
-    return store ? pick_store<G, A, kShortThreads, kShortUnroll>(policy) : pick_rmw<G, A, kShortThreads, kShortUnroll>(policy);
+    return store ? pick_store<L, G, A, kShortThreads, kShortUnroll>(policy)
+                 : pick_rmw<L, G, A, kShortThreads, kShortUnroll>(policy);
   if constexpr (kShortOnly) return nullptr;
-  else return store ? pick_store<G, A, kStoreThreads, kStoreUnroll>(policy) : pick_rmw<G, A, kThreads, kUnroll>(policy);
+  else return store ? pick_store<L, G, A, kStoreThreads, kStoreUnroll>(policy) : pick_rmw<L, G, A, kThreads, kUnroll>(policy);
 }
 
-accum_fn pick_accum(int g, int a, bool store, CachePolicy policy, bool short_tiles) {
+template <class L>
+kernel_fn<L> pick_accum(int g, int a, bool store, CachePolicy policy, bool short_tiles) {
 #define X(E1, T1, E2, T2) \
-  if (g == E1 && a == E2) return pick_accum_form<T1, T2, accum_streams_short(E1, E2)>(store, policy, short_tiles);
+  if (g == E1 && a == E2) return pick_accum_form<L, T1, T2, accum_streams_short(E1, E2)>(store, policy, short_tiles);
   ODC_FOR_EACH_DTYPE_PAIR(X)
 #undef X
   return nullptr;
 }
 
-template <bool kSrcCached, bool kDstCached>
-gather_fn pick_gather_threads(bool short_tiles) {
-  return short_tiles ? gather_kernel<kSrcCached, kDstCached, kShortThreads, kShortUnroll>
-                     : gather_kernel<kSrcCached, kDstCached, kCopyThreads, kCopyUnroll>;
+template <class L, bool kSrcCached, bool kDstCached>
+kernel_fn<L> pick_gather_threads(bool short_tiles) {
+  return short_tiles ? gather_kernel<L, kSrcCached, kDstCached, kShortThreads, kShortUnroll>
+                     : gather_kernel<L, kSrcCached, kDstCached, kCopyThreads, kCopyUnroll>;
 }
 
-gather_fn pick_gather(CachePolicy policy, bool short_tiles) {
+template <class L>
+kernel_fn<L> pick_gather(CachePolicy policy, bool short_tiles) {
   if (policy.read)
-    return policy.written ? pick_gather_threads<true, true>(short_tiles) : pick_gather_threads<true, false>(short_tiles);
-  return policy.written ? pick_gather_threads<false, true>(short_tiles) : pick_gather_threads<false, false>(short_tiles);
+    return policy.written ? pick_gather_threads<L, true, true>(short_tiles) : pick_gather_threads<L, true, false>(short_tiles);
+  return policy.written ? pick_gather_threads<L, false, true>(short_tiles) : pick_gather_threads<L, false, false>(short_tiles);
 }
 
 // Shards and output of the converting gather are cached together or not at all.
-template <class S, class D>
-cast_gather_fn pick_cast_gather_form(CachePolicy policy, bool short_tiles) {
+template <class L, class S, class D>
+kernel_fn<L> pick_cast_gather_form(CachePolicy policy, bool short_tiles) {
   if (short_tiles)
-    return policy.read ? cast_gather_kernel<S, D, true, kShortThreads, kShortUnroll>
-                       : cast_gather_kernel<S, D, false, kShortThreads, kShortUnroll>;
-  return policy.read ? cast_gather_kernel<S, D, true, kCopyThreads, kCopyUnroll>
-                     : cast_gather_kernel<S, D, false, kCopyThreads, kCopyUnroll>;
+    return policy.read ? cast_gather_kernel<L, S, D, true, kShortThreads, kShortUnroll>
+                       : cast_gather_kernel<L, S, D, false, kShortThreads, kShortUnroll>;
+  return policy.read ? cast_gather_kernel<L, S, D, true, kCopyThreads, kCopyUnroll>
+                     : cast_gather_kernel<L, S, D, false, kCopyThreads, kCopyUnroll>;
 }
 
-cast_gather_fn pick_cast_gather(int s, int d, CachePolicy policy, bool short_tiles) {  // (shard dtype, output dtype)
-#define X(E1, T1, E2, T2) if (s == E1 && d == E2) return pick_cast_gather_form<T1, T2>(policy, short_tiles);
+template <class L>
+kernel_fn<L> pick_cast_gather(int s, int d, CachePolicy policy, bool short_tiles) {  // (shard dtype, output dtype)
+#define X(E1, T1, E2, T2) if (s == E1 && d == E2) return pick_cast_gather_form<L, T1, T2>(policy, short_tiles);
   ODC_FOR_EACH_DTYPE_PAIR(X)
 #undef X
   return nullptr;
 }
 
-publish_fn pick_publish(int a, int o) {  // (accumulation dtype, output dtype)
-#define X(E1, T1, E2, T2) if (a == E1 && o == E2) return publish_kernel<T1, T2>;
+template <class L>
+kernel_fn<L> pick_publish(int a, int o) {  // (accumulation dtype, output dtype)
+#define X(E1, T1, E2, T2) if (a == E1 && o == E2) return publish_kernel<L, T1, T2>;
   ODC_FOR_EACH_DTYPE_PAIR(X)
 #undef X
   return nullptr;
+}
+
+// A launch of one item in its own form.
+template <class Launch>
+SingleLaunch<typename Launch::Desc> single_form(const Launch& L) {
+  SingleLaunch<typename Launch::Desc> s;
+  s.tt = L.tt;
+  s.base = L.base;
+  s.rank_stride = L.rank_stride;
+  s.item[0] = L.item[0];
+  return s;
+}
+
+PublishSingle single_form(const PublishLaunch& L) {
+  PublishSingle s;
+  static_cast<SingleLaunch<PublishDesc>&>(s) = single_form<PublishLaunch>(L);
+  s.scale = L.scale;
+  return s;
 }
 
 // The launch's own status, not hipGetLastError(): that one also reports what an earlier,
@@ -742,6 +820,17 @@ int launch(void (*kernel)(const Launch), const Launch& L, uint32_t grid, uint32_
   void* args[] = {const_cast<Launch*>(&L)};
   return (int)hipLaunchKernel(reinterpret_cast<const void*>(kernel), dim3(grid), dim3(threads), args, lds_bytes,
                               static_cast<hipStream_t>(stream));
+}
+
+template <class L> struct Form { typedef L type; };
+
+// pick(Form<L>) names the kernel for launches of type L.
+template <class Launch, class Pick>
+int launch_form(const Launch& L, uint32_t grid, uint32_t threads, uint32_t lds_bytes, void* stream, Pick pick) {
+  if (L.tt.n_items != 1) return launch<Launch>(pick(Form<Launch>{}), L, grid, threads, lds_bytes, stream);
+  const auto single = single_form(L);
+  typedef std::remove_const_t<decltype(single)> Single;
+  return launch<Single>(pick(Form<Single>{}), single, grid, threads, lds_bytes, stream);
 }
 
 }  // namespace
@@ -783,31 +872,37 @@ bool is_out_of_memory(int code) { return code == (int)hipErrorOutOfMemory; }
 
 const char* error_string(int code) { return hipGetErrorString(static_cast<hipError_t>(code)); }
 
-bool has_accum(int g, int a) { return pick_accum(g, a, false, {}, true) != nullptr; }
-bool has_cast_gather(int s, int d) { return pick_cast_gather(s, d, {}, false) != nullptr; }
-bool has_publish(int a, int o) { return pick_publish(a, o) != nullptr; }
+bool has_accum(int g, int a) { return pick_accum<AccumLaunch>(g, a, false, {}, true) != nullptr; }
+bool has_cast_gather(int s, int d) { return pick_cast_gather<CastGatherLaunch>(s, d, {}, false) != nullptr; }
+bool has_publish(int a, int o) { return pick_publish<PublishLaunch>(a, o) != nullptr; }
 
 int launch_gather(const GatherLaunch& L, uint32_t grid, uint32_t lds_bytes, void* stream) {
-  return launch(pick_gather(L.policy, L.short_tiles), L, grid, L.short_tiles ? kShortThreads : kCopyThreads, lds_bytes,
-                stream);
+  return launch_form(L, grid, L.short_tiles ? kShortThreads : kCopyThreads, lds_bytes, stream, [&](auto form) {
+    return pick_gather<typename decltype(form)::type>(L.policy, L.short_tiles);
+  });
 }
 
 int launch_cast_gather(int s, int d, const CastGatherLaunch& L, uint32_t grid, uint32_t lds_bytes, void* stream) {
-  return launch(pick_cast_gather(s, d, L.policy, L.short_tiles), L, grid, L.short_tiles ? kShortThreads : kCopyThreads,
-                lds_bytes, stream);
+  return launch_form(L, grid, L.short_tiles ? kShortThreads : kCopyThreads, lds_bytes, stream, [&](auto form) {
+    return pick_cast_gather<typename decltype(form)::type>(s, d, L.policy, L.short_tiles);
+  });
 }
 
 int launch_accum(int g, int a, bool store, const AccumLaunch& L, uint32_t grid, uint32_t lds_bytes, void* stream) {
   const uint32_t threads = L.short_tiles ? kShortThreads : store ? kStoreThreads : kThreads;
-  return launch(pick_accum(g, a, store, L.policy, L.short_tiles), L, grid, threads, lds_bytes, stream);
+  return launch_form(L, grid, threads, lds_bytes, stream, [&](auto form) {
+    return pick_accum<typename decltype(form)::type>(g, a, store, L.policy, L.short_tiles);
+  });
 }
 
 int launch_clear(const ClearLaunch& L, uint32_t grid, void* stream) {
-  return launch(clear_kernel, L, grid, kThreads, 0u, stream);
+  return launch_form(L, grid, kThreads, 0u, stream,
+                     [](auto form) { return &clear_kernel<typename decltype(form)::type>; });
 }
 
 int launch_publish(int a, int o, const PublishLaunch& L, uint32_t grid, uint32_t lds_bytes, void* stream) {
-  return launch(pick_publish(a, o), L, grid, kThreads, lds_bytes, stream);
+  return launch_form(L, grid, kThreads, lds_bytes, stream,
+                     [&](auto form) { return pick_publish<typename decltype(form)::type>(a, o); });
 }
 
 }  // namespace odc_device

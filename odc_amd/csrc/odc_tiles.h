@@ -51,17 +51,21 @@ constexpr uint32_t kShortTileVecs = kTileVecs / kShortTileParts;
 //   kRankOutermost    : rank by rank; within a rank item by item
 enum TileOrder : uint32_t { kRanksInterleaved = 0, kItemMajor = 1, kRankOutermost = 2 };
 
-// Travels by value in the kernel-argument segment. seg_prefix[i] is the number of tiles that
-// the items before item i have in ONE rank segment each, so item i has
-// seg_prefix[i+1] - seg_prefix[i] tiles per rank segment and world times that in the launch.
-// Entries past n_items hold tiles_per_rank, so a search never lands on them.
-struct TileTable {
+// What a launch of any number of items says about its tiles; all there is to say about one item.
+struct TileHead {
   uint32_t world;
   uint32_t n_items;
   uint32_t n_tiles;         // world * tiles_per_rank
   uint32_t order;           // TileOrder
   uint32_t first_rank;      // rotation of the rank walk (never changes the result)
   uint32_t tiles_per_rank;  // seg_prefix[n_items]
+};
+
+// Travels by value in the kernel-argument segment. seg_prefix[i] is the number of tiles that
+// the items before item i have in ONE rank segment each, so item i has
+// seg_prefix[i+1] - seg_prefix[i] tiles per rank segment and world times that in the launch.
+// Entries past n_items hold tiles_per_rank, so a search never lands on them.
+struct TileTable : TileHead {
   uint32_t seg_prefix[kMaxItems + 1];
 };
 
@@ -150,6 +154,22 @@ ODC_HD bool locate_tile(const TileTable& tt, uint32_t t, TileCursor& cur, TileCo
   }
   c = cursor_coord(tt, cur, t);
   return moved;
+}
+
+// The same for the tiles of a launch of one item, whose two rank by rank orders are one.
+ODC_HD TileCoord single_item_coord(const TileHead& tt, uint32_t t) {
+  TileCoord c;
+  c.item = 0;
+  if (tt.order == kRanksInterleaved) {
+    c.chunk = t / tt.world;
+    c.rank = t - c.chunk * tt.world;
+  } else {
+    c.rank = t / tt.tiles_per_rank;
+    c.chunk = t - c.rank * tt.tiles_per_rank;
+  }
+  c.rank += tt.first_rank;
+  if (c.rank >= tt.world) c.rank -= tt.world;
+  return c;
 }
 
 // Shape of one rank segment of `n` units whose WRITTEN side starts at address D:
