@@ -77,6 +77,7 @@ struct Options {
   int64_t cached_output_bytes = 64ll << 20;
   int64_t cached_gradient_bytes = 128ll << 20;
   int64_t short_tiles_below = 32;             // see wants_short_tiles
+  int64_t few_tiles = 32768;                  // see tile_form
   int64_t dry_run_short_tiles = 0;  // read when an arena without a device is created: 1 = plan short tiles too
 };
 Options g_opt;
@@ -106,6 +107,7 @@ int64_t* option_slot(const char* name) {
   if (!strcmp(name, "cached_output_bytes")) return &g_opt.cached_output_bytes;
   if (!strcmp(name, "cached_gradient_bytes")) return &g_opt.cached_gradient_bytes;
   if (!strcmp(name, "short_tiles_below")) return &g_opt.short_tiles_below;
+  if (!strcmp(name, "few_tiles")) return &g_opt.few_tiles;
   if (!strcmp(name, "dry_run_short_tiles")) return &g_opt.dry_run_short_tiles;
   return nullptr;
 }
@@ -271,6 +273,19 @@ bool wants_short_tiles(const odc_arena* a, uint32_t n_items, uint32_t next, uint
     ++segments;
   }
   return tiles < (uint64_t)below * segments;
+}
+
+// How the workgroups of a launch find their items. Up to eight fills of the chip (4096 workgroups of
+// 128 threads each) a launch is mostly the latency from its arguments to its first loads, and the
+// whole prefix table read at once pays off; in longer ones the other workgroups of the CU hide that
+// latency and the extra loads only cost. Graph-replayed gather + accumulate of one group of slices,
+// us, binary search -> table read at once:
+//   300 of 64 .. 65 536 elements: W = 4 27.4 -> 23.2, W = 8 28.6 -> 24.3, W = 64 55.6 -> 45.0;
+//   112 of 4096: 6.0 -> 5.1, 6.3 -> 5.7, 17.8 -> 13.5; 10 of 256 .. 262 144: 6.1 -> 5.9, 6.5 -> 6.2, 7.2 -> 6.9;
+//   112 of 160 000 (17 900 tiles): 41.2 -> 39.7, 41.1 -> 40.2; 112 of 640 000 (70 000 tiles): 156 -> 159,
+//   159 -> 162; 60 of 900 000 (53 000 tiles): 115 -> 115, 116.5 -> 117.6.
+TileForm tile_form(bool short_tiles, uint32_t n_tiles, int64_t few) {
+  return !short_tiles ? kWholeTiles : n_tiles <= (uint64_t)few ? kFewShortTiles : kShortTiles;
 }
 
 // One-workgroup-per-tile launches are dealt out by the hardware dispatcher, which keeps as many
@@ -599,14 +614,15 @@ int odc_gather(odc_arena* a, const odc_gather_item* items, uint32_t n_items, uin
     L.tt.order = (uint32_t)opt.rank_major;
     L.tt.first_rank = first_rank;
     const auto units = [&](uint32_t i) { return items[i].shard_bytes; };
-    L.short_tiles = wants_short_tiles(a, n_items, next, kTileBytes, units, opt.short_tiles_below);
+    const bool short_tiles = wants_short_tiles(a, n_items, next, kTileBytes, units, opt.short_tiles_below);
     const int n = fill_launch(
-        L.tt, a->world, n_items, &next, tile_units(kTileBytes, L.short_tiles), units,
+        L.tt, a->world, n_items, &next, tile_units(kTileBytes, short_tiles), units,
         [&](uint32_t slot, uint32_t i) {
           L.item[slot] = {static_cast<uint8_t*>(items[i].dst), items[i].src_offset, items[i].shard_bytes};
         });
     if (n < 0) return n;
     if (n == 0) continue;
+    L.form = tile_form(short_tiles, L.tt.n_tiles, opt.few_tiles);
     bool ragged = false;
     uint64_t shard_bytes = 0;
     for (uint32_t k = 0; k < L.tt.n_items; ++k) shard_bytes += L.item[k].seg_bytes;
@@ -651,15 +667,16 @@ int odc_gather_cast(odc_arena* a, const odc_gather_cast_item* items, uint32_t n_
     L.tt.order = (uint32_t)opt.rank_major;
     L.tt.first_rank = first_rank;
     const auto units = [&](uint32_t i) { return items[i].shard_elems; };
-    L.short_tiles = wants_short_tiles(a, n_items, next, kTileElems, units, opt.short_tiles_below);
+    const bool short_tiles = wants_short_tiles(a, n_items, next, kTileElems, units, opt.short_tiles_below);
     const int n = fill_launch(
-        L.tt, a->world, n_items, &next, tile_units(kTileElems, L.short_tiles), units,
+        L.tt, a->world, n_items, &next, tile_units(kTileElems, short_tiles), units,
         [&](uint32_t slot, uint32_t i) {
           L.item[slot] = {static_cast<uint8_t*>(items[i].dst), items[i].shard_elems * (uint64_t)db,
                           items[i].src_offset, items[i].shard_elems};
         });
     if (n < 0) return n;
     if (n == 0) continue;
+    L.form = tile_form(short_tiles, L.tt.n_tiles, opt.few_tiles);
     L.policy = cache_policy(a, opt, 0, kSymmetric, 0, kSymmetric);
     const uint32_t grid = grid_for(a, opt.gather_blocks_per_cu, L.tt.n_tiles);
     const uint32_t lds = lds_claim_for(a, opt.cast_resident_cap, grid, L.tt.n_tiles);
@@ -700,15 +717,16 @@ int odc_convert(odc_arena* a, const odc_convert_item* items, uint32_t n_items, i
     L.tt.order = (uint32_t)opt.rank_major;
     L.tt.first_rank = 0;
     const auto units = [&](uint32_t i) { return items[i].elems; };
-    L.short_tiles = wants_short_tiles(a, n_items, next, kTileElems, units, opt.short_tiles_below);
+    const bool short_tiles = wants_short_tiles(a, n_items, next, kTileElems, units, opt.short_tiles_below);
     const int n = fill_launch(
-        L.tt, a->world, n_items, &next, tile_units(kTileElems, L.short_tiles), units,
+        L.tt, a->world, n_items, &next, tile_units(kTileElems, short_tiles), units,
         [&](uint32_t slot, uint32_t i) {
           // the gather-with-cast kernel with every rank's output in that rank's own region
           L.item[slot] = {a->origin + items[i].dst_offset, a->rank_stride, items[i].src_offset, items[i].elems};
         });
     if (n < 0) return n;
     if (n == 0) continue;
+    L.form = tile_form(short_tiles, L.tt.n_tiles, opt.few_tiles);
     L.policy = cache_policy(a, opt, 0, kSymmetric, 0, kSymmetric);
     const uint32_t grid = grid_for(a, opt.gather_blocks_per_cu, L.tt.n_tiles);
     const uint32_t lds = lds_claim_for(a, opt.cast_resident_cap, grid, L.tt.n_tiles);
@@ -812,10 +830,10 @@ int scatter_launch(odc_arena* a, const odc_accum_item* items, uint32_t n_items, 
     L.tt.order = (uint32_t)opt.rank_major;
     L.tt.first_rank = 0;
     const auto units = [&](uint32_t i) { return items[order[i]].shard_elems; };
-    L.short_tiles = (a->short_tiles && odc_launch::accum_streams_short(grad_dtype, acc_dtype)) ||
-                    wants_short_tiles(a, n_items, next, kTileElems, units, opt.short_tiles_below);
+    const bool short_tiles = (a->short_tiles && odc_launch::accum_streams_short(grad_dtype, acc_dtype)) ||
+                             wants_short_tiles(a, n_items, next, kTileElems, units, opt.short_tiles_below);
     const int n = fill_launch(
-        L.tt, a->world, n_items, &next, tile_units(kTileElems, L.short_tiles), units,
+        L.tt, a->world, n_items, &next, tile_units(kTileElems, short_tiles), units,
         [&](uint32_t slot, uint32_t i) {
           const odc_accum_item& it = items[order[i]];
           L.item[slot] = {static_cast<const uint8_t*>(it.grad), it.grad_elems, it.acc_offset, it.shard_elems};
@@ -823,6 +841,7 @@ int scatter_launch(odc_arena* a, const odc_accum_item* items, uint32_t n_items, 
         order);
     if (n < 0) return n;
     if (n == 0) continue;
+    L.form = tile_form(short_tiles, L.tt.n_tiles, opt.few_tiles);
     // Tile order. Item-major (a rank's segment, then the next rank's, item by item) walks the
     // gradient contiguously and hops between rank regions at every segment; rank-outermost walks
     // one rank region from accumulation to accumulation (they are neighbours when registered
@@ -831,7 +850,7 @@ int scatter_launch(odc_arena* a, const odc_accum_item* items, uint32_t n_items, 
     // rank-outermost: +1.1 % at W=4, +1.6 % at W=16 (370 tiles per segment on average), -1.9 % at
     // W=32 (185), -6 % at W=64, -10 % at W=128.
     const uint64_t segments = (uint64_t)L.tt.n_items * a->world;
-    const uint64_t whole_tiles = L.short_tiles ? L.tt.n_tiles / kShortTileParts : L.tt.n_tiles;
+    const uint64_t whole_tiles = short_tiles ? L.tt.n_tiles / kShortTileParts : L.tt.n_tiles;
     if (opt.accum_tile_order == 3)
       L.tt.order = whole_tiles < (uint64_t)opt.accum_short_segment_tiles * segments ? kRankOutermost : kItemMajor;
     else

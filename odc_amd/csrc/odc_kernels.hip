@@ -106,12 +106,12 @@ __device__ __forceinline__ P* as_global(P* p) {
 // ---- finding a tile's work ------------------------------------------------------------------
 // The walk of a workgroup over the tiles of its launch; all its lanes come along.
 template <class Launch>
-struct TileWalk {
+struct TableWalk {
   typedef typename Launch::Desc Desc;
   TileCursor cur;
   Desc it = {};  // the item of the tile located last
 
-  __device__ __forceinline__ explicit TileWalk(const Launch&) {}
+  __device__ __forceinline__ explicit TableWalk(const Launch&) {}
   __device__ __forceinline__ uint32_t n_tiles(const Launch& launch) const { return launch.tt.n_tiles; }
   __device__ __forceinline__ uint8_t* region(const Launch& launch, uint32_t rank) const {
     return launch.base + (uint64_t)rank * launch.rank_stride;
@@ -160,14 +160,51 @@ struct SingleWalk {
   }
   __device__ __forceinline__ TileCoord locate(const SingleLaunch<D>&, uint32_t t) const { return single_item_coord(tt, t); }
 };
-template <class D>
-struct TileWalk<SingleLaunch<D>> : SingleWalk<D> {
-  using SingleWalk<D>::SingleWalk;
+// Few short tiles of several items (tile_form in odc_host.cpp): again a chain of latencies, the binary
+// search being most of it. The whole prefix table is read together with the header instead, one entry per lane (two for its second
+// half), and the item found by counting the entries that are not greater than the tile's position:
+// two round trips to the item in place of up to nine.
+template <class Launch>
+struct FewTilesWalk {
+  typedef typename Launch::Desc Desc;
+  TileHead tt;
+  uint8_t* base;
+  uint64_t rank_stride;
+  TileCursor cur;
+  Desc it = {};
+  uint32_t bound[2];  // lane l: seg_prefix[1 + l] and seg_prefix[65 + l]
+
+  __device__ __forceinline__ explicit FewTilesWalk(const Launch& launch) {
+    static_assert(kMaxItems > 64 && kMaxItems <= 128, "two prefix entries per lane of a wavefront");
+    const uint32_t lane = threadIdx.x & 63u;
+    bound[0] = launch.tt.seg_prefix[1 + lane];
+    bound[1] = launch.tt.seg_prefix[65 + lane < kMaxItems ? 65 + lane : kMaxItems];
+    tt = launch.tt;
+    uint64_t b = (uint64_t)(uintptr_t)launch.base, stride = launch.rank_stride;
+    asm volatile("" : "+s"(tt.world), "+s"(tt.n_tiles), "+s"(tt.order), "+s"(tt.first_rank), "+s"(tt.tiles_per_rank),
+                      "+s"(b), "+s"(stride), "+v"(bound[0]), "+v"(bound[1]));
+    base = as_global(reinterpret_cast<uint8_t*>((uintptr_t)b));
+    rank_stride = stride;
+  }
+  __device__ __forceinline__ uint32_t n_tiles(const Launch&) const { return tt.n_tiles; }
+  __device__ __forceinline__ uint8_t* region(const Launch&, uint32_t rank) const {
+    return base + (uint64_t)rank * rank_stride;
+  }
+  __device__ __forceinline__ TileCoord locate(const Launch& launch, uint32_t t) {
+    if (!cursor_holds(cur, t)) {
+      const uint32_t x = cursor_position(tt, t, cur);
+      // (entries past the last item, the doubled ones among them, hold tiles_per_rank > x)
+      cur.item = (uint32_t)__popcll(__ballot(bound[0] <= x)) + (uint32_t)__popcll(__ballot(bound[1] <= x));
+      it = launch.item[cur.item];
+      cursor_bounds(tt, launch.tt.seg_prefix[cur.item], launch.tt.seg_prefix[cur.item + 1], cur);
+    }
+    return cursor_coord(tt, cur, t);
+  }
 };
-template <>
-struct TileWalk<PublishSingle> : SingleWalk<PublishDesc> {
-  using SingleWalk<PublishDesc>::SingleWalk;
-};
+
+template <class Launch, bool kFew = false>
+using TileWalk = std::conditional_t<!std::is_same_v<decltype(Launch::tt), TileTable>, SingleWalk<typename Launch::Desc>,
+                                    std::conditional_t<kFew, FewTilesWalk<Launch>, TableWalk<Launch>>>;
 
 // ---- gather -------------------------------------------------------------------------------
 // Everything of a tile that is not a run of T * U whole vectors: the last partial run, the
@@ -203,13 +240,13 @@ __device__ __attribute__((noinline)) void gather_edges(uint8_t* d, const uint8_t
 
 // T threads do a tile of T * U vectors in one step; the copies stream best from 512-thread
 // workgroups, of which 4 fit a CU.
-template <class Launch, bool kSrcCached, bool kDstCached, int T, int U>
+template <class Launch, bool kSrcCached, bool kDstCached, bool kFew, int T, int U>
 __global__ __launch_bounds__(T) void gather_kernel(const Launch launch) {
   constexpr uint32_t kVecs = T * U;
   static_assert(kVecs == kTileVecs || kVecs == kShortTileVecs, "a whole tile or a short one");
   static_assert(T >= ODC_BODY_ALIGN - 1, "one lane per head byte");
   const uint32_t tid = threadIdx.x;
-  TileWalk<Launch> walk(launch);
+  TileWalk<Launch, kFew> walk(launch);
   for (uint32_t t = blockIdx.x; t < walk.n_tiles(launch); t += gridDim.x) {
     const TileCoord c = walk.locate(launch, t);
     const GatherDesc it = walk.it;
@@ -445,7 +482,7 @@ __device__ __attribute__((noinline)) void accum_edges(uint8_t* acc, const uint8_
   if (do_tail) as[tail_at] = Codec<A>::narrow(Codec<A>::widen(tail_araw) + Codec<G>::widen(tail_graw));
 }
 
-template <class Launch, class G, class A, bool kStore, bool kGradCached, bool kAccCached, int T, int U>
+template <class Launch, class G, class A, bool kStore, bool kGradCached, bool kAccCached, bool kFew, int T, int U>
 __global__ __launch_bounds__(T) void accum_kernel(const Launch launch) {
   constexpr uint32_t kVecs = T * U;  // quads
   static_assert(kVecs == kTileVecs || kVecs == kShortTileVecs, "a whole tile or a short one");
@@ -454,7 +491,7 @@ __global__ __launch_bounds__(T) void accum_kernel(const Launch launch) {
   constexpr uint32_t kAB = Codec<A>::kBytes, kGB = Codec<G>::kBytes;
   static_assert(T >= ODC_BODY_ALIGN / kAB, "one lane per head element");
   const uint32_t tid = threadIdx.x;
-  TileWalk<Launch> walk(launch);
+  TileWalk<Launch, kFew> walk(launch);
   for (uint32_t t = blockIdx.x; t < walk.n_tiles(launch); t += gridDim.x) {
     const TileCoord c = walk.locate(launch, t);
     const AccumDesc it = walk.it;
@@ -541,7 +578,7 @@ __device__ __attribute__((noinline)) void cast_edges(uint8_t* d, const uint8_t* 
   if (do_tail) ds[tail_at] = Codec<D>::narrow(Codec<S>::widen(tail_raw));
 }
 
-template <class Launch, class S, class D, bool kCached, int T, int U>
+template <class Launch, class S, class D, bool kCached, bool kFew, int T, int U>
 __global__ __launch_bounds__(T) void cast_gather_kernel(const Launch launch) {
   constexpr uint32_t kVecs = T * U;  // quads
   static_assert(kVecs == kTileVecs || kVecs == kShortTileVecs, "a whole tile or a short one");
@@ -550,7 +587,7 @@ __global__ __launch_bounds__(T) void cast_gather_kernel(const Launch launch) {
   typedef typename Quad<D>::vec_t dvec_t;
   constexpr uint32_t kSB = Codec<S>::kBytes, kDB = Codec<D>::kBytes;
   const uint32_t tid = threadIdx.x;
-  TileWalk<Launch> walk(launch);
+  TileWalk<Launch, kFew> walk(launch);
   for (uint32_t t = blockIdx.x; t < walk.n_tiles(launch); t += gridDim.x) {
     const TileCoord c = walk.locate(launch, t);
     const CastGatherDesc it = walk.it;
@@ -710,6 +747,8 @@ __global__ __launch_bounds__(kThreads) void publish_kernel(const Launch launch) 
 // dtype dispatch
 // ------------------------------------------------------------------------------------------------
 template <class Launch> using kernel_fn = void (*)(const Launch);
+// A launch of one item has nothing to search: one kernel serves both short forms.
+template <class Launch> constexpr bool kSearches = std::is_same_v<decltype(Launch::tt), TileTable>;
 
 #define ODC_FOR_EACH_DTYPE_PAIR(X)                    \
   X(ODC_DTYPE_BF16, bf16_tag, ODC_DTYPE_BF16, bf16_tag) \
@@ -724,62 +763,70 @@ template <class Launch> using kernel_fn = void (*)(const Launch);
 
 // (gradient dtype, accumulation dtype). The store form never reads the accumulation and keeps it
 // nontemporal; the read-modify-write keeps it cached only together with the gradient.
-template <class L, class G, class A, int T, int U>
+template <class L, class G, class A, bool kFew, int T, int U>
 kernel_fn<L> pick_rmw(CachePolicy policy) {
-  if (policy.read && policy.written) return accum_kernel<L, G, A, false, true, true, T, U>;
-  return policy.read ? accum_kernel<L, G, A, false, true, false, T, U> : accum_kernel<L, G, A, false, false, false, T, U>;
+  if (policy.read && policy.written) return accum_kernel<L, G, A, false, true, true, kFew, T, U>;
+  return policy.read ? accum_kernel<L, G, A, false, true, false, kFew, T, U>
+                     : accum_kernel<L, G, A, false, false, false, kFew, T, U>;
 }
 
-template <class L, class G, class A, int T, int U>
+template <class L, class G, class A, bool kFew, int T, int U>
 kernel_fn<L> pick_store(CachePolicy policy) {
-  return policy.read ? accum_kernel<L, G, A, true, true, false, T, U> : accum_kernel<L, G, A, true, false, false, T, U>;
+  return policy.read ? accum_kernel<L, G, A, true, true, false, kFew, T, U>
+                     : accum_kernel<L, G, A, true, false, false, kFew, T, U>;
 }
 
 // kShortOnly: accum_streams_short says so, there is no kernel of whole tiles.
 template <class L, class G, class A, bool kShortOnly>
-kernel_fn<L> pick_accum_form(bool store, CachePolicy policy, bool short_tiles) {
-  if (short_tiles)
-    return store ? pick_store<L, G, A, kShortThreads, kShortUnroll>(policy)
-                 : pick_rmw<L, G, A, kShortThreads, kShortUnroll>(policy);
+kernel_fn<L> pick_accum_form(bool store, CachePolicy policy, TileForm form) {
+  if (form == kFewShortTiles)
+    return store ? pick_store<L, G, A, kSearches<L>, kShortThreads, kShortUnroll>(policy)
+                 : pick_rmw<L, G, A, kSearches<L>, kShortThreads, kShortUnroll>(policy);
+  if (form == kShortTiles)
+    return store ? pick_store<L, G, A, false, kShortThreads, kShortUnroll>(policy)
+                 : pick_rmw<L, G, A, false, kShortThreads, kShortUnroll>(policy);
   if constexpr (kShortOnly) return nullptr;
-  else return store ? pick_store<L, G, A, kStoreThreads, kStoreUnroll>(policy) : pick_rmw<L, G, A, kThreads, kUnroll>(policy);
+  else
+    return store ? pick_store<L, G, A, false, kStoreThreads, kStoreUnroll>(policy)
+                 : pick_rmw<L, G, A, false, kThreads, kUnroll>(policy);
 }
 
 template <class L>
-kernel_fn<L> pick_accum(int g, int a, bool store, CachePolicy policy, bool short_tiles) {
+kernel_fn<L> pick_accum(int g, int a, bool store, CachePolicy policy, TileForm form) {
 #define X(E1, T1, E2, T2) \
-  if (g == E1 && a == E2) return pick_accum_form<L, T1, T2, accum_streams_short(E1, E2)>(store, policy, short_tiles);
+  if (g == E1 && a == E2) return pick_accum_form<L, T1, T2, accum_streams_short(E1, E2)>(store, policy, form);
   ODC_FOR_EACH_DTYPE_PAIR(X)
 #undef X
   return nullptr;
 }
 
 template <class L, bool kSrcCached, bool kDstCached>
-kernel_fn<L> pick_gather_threads(bool short_tiles) {
-  return short_tiles ? gather_kernel<L, kSrcCached, kDstCached, kShortThreads, kShortUnroll>
-                     : gather_kernel<L, kSrcCached, kDstCached, kCopyThreads, kCopyUnroll>;
+kernel_fn<L> pick_gather_form(TileForm form) {
+  if (form == kFewShortTiles) return gather_kernel<L, kSrcCached, kDstCached, kSearches<L>, kShortThreads, kShortUnroll>;
+  if (form == kShortTiles) return gather_kernel<L, kSrcCached, kDstCached, false, kShortThreads, kShortUnroll>;
+  return gather_kernel<L, kSrcCached, kDstCached, false, kCopyThreads, kCopyUnroll>;
 }
 
 template <class L>
-kernel_fn<L> pick_gather(CachePolicy policy, bool short_tiles) {
+kernel_fn<L> pick_gather(CachePolicy policy, TileForm form) {
   if (policy.read)
-    return policy.written ? pick_gather_threads<L, true, true>(short_tiles) : pick_gather_threads<L, true, false>(short_tiles);
-  return policy.written ? pick_gather_threads<L, false, true>(short_tiles) : pick_gather_threads<L, false, false>(short_tiles);
+    return policy.written ? pick_gather_form<L, true, true>(form) : pick_gather_form<L, true, false>(form);
+  return policy.written ? pick_gather_form<L, false, true>(form) : pick_gather_form<L, false, false>(form);
 }
 
 // Shards and output of the converting gather are cached together or not at all.
-template <class L, class S, class D>
-kernel_fn<L> pick_cast_gather_form(CachePolicy policy, bool short_tiles) {
-  if (short_tiles)
-    return policy.read ? cast_gather_kernel<L, S, D, true, kShortThreads, kShortUnroll>
-                       : cast_gather_kernel<L, S, D, false, kShortThreads, kShortUnroll>;
-  return policy.read ? cast_gather_kernel<L, S, D, true, kCopyThreads, kCopyUnroll>
-                     : cast_gather_kernel<L, S, D, false, kCopyThreads, kCopyUnroll>;
+template <class L, class S, class D, bool kCached>
+kernel_fn<L> pick_cast_gather_form(TileForm form) {
+  if (form == kFewShortTiles) return cast_gather_kernel<L, S, D, kCached, kSearches<L>, kShortThreads, kShortUnroll>;
+  if (form == kShortTiles) return cast_gather_kernel<L, S, D, kCached, false, kShortThreads, kShortUnroll>;
+  return cast_gather_kernel<L, S, D, kCached, false, kCopyThreads, kCopyUnroll>;
 }
 
 template <class L>
-kernel_fn<L> pick_cast_gather(int s, int d, CachePolicy policy, bool short_tiles) {  // (shard dtype, output dtype)
-#define X(E1, T1, E2, T2) if (s == E1 && d == E2) return pick_cast_gather_form<L, T1, T2>(policy, short_tiles);
+kernel_fn<L> pick_cast_gather(int s, int d, CachePolicy policy, TileForm form) {  // (shard dtype, output dtype)
+#define X(E1, T1, E2, T2) \
+  if (s == E1 && d == E2) \
+    return policy.read ? pick_cast_gather_form<L, T1, T2, true>(form) : pick_cast_gather_form<L, T1, T2, false>(form);
   ODC_FOR_EACH_DTYPE_PAIR(X)
 #undef X
   return nullptr;
@@ -872,26 +919,26 @@ bool is_out_of_memory(int code) { return code == (int)hipErrorOutOfMemory; }
 
 const char* error_string(int code) { return hipGetErrorString(static_cast<hipError_t>(code)); }
 
-bool has_accum(int g, int a) { return pick_accum<AccumLaunch>(g, a, false, {}, true) != nullptr; }
-bool has_cast_gather(int s, int d) { return pick_cast_gather<CastGatherLaunch>(s, d, {}, false) != nullptr; }
+bool has_accum(int g, int a) { return pick_accum<AccumLaunch>(g, a, false, {}, kShortTiles) != nullptr; }
+bool has_cast_gather(int s, int d) { return pick_cast_gather<CastGatherLaunch>(s, d, {}, kWholeTiles) != nullptr; }
 bool has_publish(int a, int o) { return pick_publish<PublishLaunch>(a, o) != nullptr; }
 
 int launch_gather(const GatherLaunch& L, uint32_t grid, uint32_t lds_bytes, void* stream) {
-  return launch_form(L, grid, L.short_tiles ? kShortThreads : kCopyThreads, lds_bytes, stream, [&](auto form) {
-    return pick_gather<typename decltype(form)::type>(L.policy, L.short_tiles);
+  return launch_form(L, grid, L.form != kWholeTiles ? kShortThreads : kCopyThreads, lds_bytes, stream, [&](auto form) {
+    return pick_gather<typename decltype(form)::type>(L.policy, L.form);
   });
 }
 
 int launch_cast_gather(int s, int d, const CastGatherLaunch& L, uint32_t grid, uint32_t lds_bytes, void* stream) {
-  return launch_form(L, grid, L.short_tiles ? kShortThreads : kCopyThreads, lds_bytes, stream, [&](auto form) {
-    return pick_cast_gather<typename decltype(form)::type>(s, d, L.policy, L.short_tiles);
+  return launch_form(L, grid, L.form != kWholeTiles ? kShortThreads : kCopyThreads, lds_bytes, stream, [&](auto form) {
+    return pick_cast_gather<typename decltype(form)::type>(s, d, L.policy, L.form);
   });
 }
 
 int launch_accum(int g, int a, bool store, const AccumLaunch& L, uint32_t grid, uint32_t lds_bytes, void* stream) {
-  const uint32_t threads = L.short_tiles ? kShortThreads : store ? kStoreThreads : kThreads;
+  const uint32_t threads = L.form != kWholeTiles ? kShortThreads : store ? kStoreThreads : kThreads;
   return launch_form(L, grid, threads, lds_bytes, stream, [&](auto form) {
-    return pick_accum<typename decltype(form)::type>(g, a, store, L.policy, L.short_tiles);
+    return pick_accum<typename decltype(form)::type>(g, a, store, L.policy, L.form);
   });
 }
 

@@ -28,6 +28,10 @@ struct CachePolicy {
   bool written = false;
 };
 
+// How a launch is cut, and how its workgroups find their items (wants_short_tiles and tile_form in
+// odc_host.cpp).
+enum TileForm : uint32_t { kWholeTiles, kShortTiles, kFewShortTiles };
+
 // 16-bit gradients into fp32 accumulations are accumulated and stored in short tiles whatever the
 // sizes. What bounds these streams is how reads and writes mix in HBM, and 16 workgroups of 128
 // threads with 2 quads per lane in flight (98 KB of loads per CU) mix them better than 8 of 256 with
@@ -44,7 +48,7 @@ constexpr bool accum_streams_short(int grad_dtype, int acc_dtype) {
 // A launch carries up to kMaxItems items. One of a single item, a flat parameter on its own, goes out
 // in a form without the tables: 56 .. 72 bytes of arguments instead of 3 to 4 KB, which the host
 // hands over in 2.6 us instead of 4.0 (512 bytes: 3.4), and all of it is read at once instead of
-// along the item search (SingleLaunch, TileWalk in odc_kernels.hip).
+// along the item search (SingleWalk in odc_kernels.hip).
 template <class D>
 struct SingleLaunch {
   typedef D Desc;
@@ -66,7 +70,7 @@ struct GatherLaunch {
   uint8_t* base;  // arena base (rank 0 region)
   uint64_t rank_stride;
   CachePolicy policy;    // these two pick the kernel
-  bool short_tiles = false;
+  TileForm form = kWholeTiles;
   GatherDesc item[kMaxItems];
 };
 
@@ -82,7 +86,7 @@ struct CastGatherLaunch {
   uint8_t* base;
   uint64_t rank_stride;
   CachePolicy policy;    // these two pick the kernel
-  bool short_tiles = false;
+  TileForm form = kWholeTiles;
   CastGatherDesc item[kMaxItems];
 };
 
@@ -98,7 +102,7 @@ struct AccumLaunch {
   uint8_t* base;
   uint64_t rank_stride;
   CachePolicy policy;    // these two pick the kernel
-  bool short_tiles = false;
+  TileForm form = kWholeTiles;
   AccumDesc item[kMaxItems];
 };
 

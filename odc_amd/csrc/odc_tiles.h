@@ -102,19 +102,23 @@ struct TileCursor {
 
 ODC_HD bool cursor_holds(const TileCursor& cur, uint32_t t) { return t >= cur.lo && t < cur.hi; }
 
-ODC_HD void cursor_seek(const TileTable& tt, uint32_t t, TileCursor& cur) {
+// The position of tile t along the items of one rank: seg_prefix[item] <= position < seg_prefix[item + 1].
+ODC_HD uint32_t cursor_position(const TileHead& tt, uint32_t t, TileCursor& cur) {
   if (tt.order == kRankOutermost) {
     cur.rank = t / tt.tiles_per_rank;
-    cur.item = find_item(tt, t - cur.rank * tt.tiles_per_rank);
-  } else {
-    // item i owns tiles [seg_prefix[i] * world, seg_prefix[i+1] * world)
-    cur.rank = 0;
-    cur.item = find_item(tt, t / tt.world);
+    return t - cur.rank * tt.tiles_per_rank;
   }
+  // item i owns tiles [seg_prefix[i] * world, seg_prefix[i+1] * world)
+  cur.rank = 0;
+  return t / tt.world;
 }
 
-ODC_HD void cursor_enter(const TileTable& tt, TileCursor& cur) {
-  const uint32_t first = tt.seg_prefix[cur.item], next = tt.seg_prefix[cur.item + 1];
+ODC_HD void cursor_seek(const TileTable& tt, uint32_t t, TileCursor& cur) {
+  cur.item = find_item(tt, cursor_position(tt, t, cur));
+}
+
+// The run's bounds, from the two entries of seg_prefix around cur.item.
+ODC_HD void cursor_bounds(const TileHead& tt, uint32_t first, uint32_t next, TileCursor& cur) {
   cur.tps = next - first;
   if (tt.order == kRankOutermost) {
     cur.lo = cur.rank * tt.tiles_per_rank + first;
@@ -125,8 +129,12 @@ ODC_HD void cursor_enter(const TileTable& tt, TileCursor& cur) {
   }
 }
 
+ODC_HD void cursor_enter(const TileTable& tt, TileCursor& cur) {
+  cursor_bounds(tt, tt.seg_prefix[cur.item], tt.seg_prefix[cur.item + 1], cur);
+}
+
 // Tile t (inside the cursor's run) -> (item, rank, chunk). Everything here is wave-uniform.
-ODC_HD TileCoord cursor_coord(const TileTable& tt, const TileCursor& cur, uint32_t t) {
+ODC_HD TileCoord cursor_coord(const TileHead& tt, const TileCursor& cur, uint32_t t) {
   TileCoord c;
   const uint32_t lt = t - cur.lo;
   c.item = cur.item;

@@ -43,17 +43,18 @@ def test_plans_in_short_tiles(shard, acc_dtype, tiles):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("below", [0, 1 << 30])  # whole tiles where there is a choice, short tiles everywhere
+@pytest.mark.parametrize("below,few", [(0, 0), (1 << 30, 0), (1 << 30, 1 << 30)])  # whole tiles, short ones, few short ones
 @pytest.mark.parametrize("dtypes", [
     (torch.bfloat16, torch.bfloat16, torch.float32), (torch.float32, torch.bfloat16, torch.bfloat16),
     (torch.float32, torch.float32, torch.float32), (torch.float16, torch.float32, torch.float16),
 ], ids=lambda d: "-".join(str(x).rsplit(".", 1)[-1] for x in d))
-def test_kernels_at_the_edges_of_a_short_tile(make_world, below, dtypes):
+def test_kernels_at_the_edges_of_a_short_tile(make_world, below, few, dtypes):
     from odc_amd import GatherService, ReductionService, SymmBufferRegistry
 
     shard_dtype, compute_dtype, acc_dtype = dtypes
-    saved = _native.get_option("short_tiles_below")
+    saved = {name: _native.get_option(name) for name in ("short_tiles_below", "few_tiles")}
     _native.set_option("short_tiles_below", below)
+    _native.set_option("few_tiles", few)
     try:
         W, sizes = 3, [1, 63, 1023, 1024, 1025, 2047, 2049, 4095, 4097, 20_481]
         group = make_world(W, 4 << 20)
@@ -83,4 +84,40 @@ def test_kernels_at_the_edges_of_a_short_tile(make_world, below, dtypes):
             for r, got in enumerate(red.get_peer_accumulations(key)):
                 assert_bit_equal(got, accs[r], f"size {sizes[key]} rank {r}")
     finally:
-        _native.set_option("short_tiles_below", saved)
+        for name, value in saved.items():
+            _native.set_option(name, value)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("order", [0, 1, 2])  # of the tiles: interleaved ranks, item major, rank outermost
+@pytest.mark.parametrize("n", [2, 63, 64, 65, 66, 111, 112, 113])
+def test_every_item_is_found_among_few_tiles(make_world, n, order):
+    """The search of launches of few tiles reads the prefix table in two halves of one entry per lane:
+    item counts around a half and around a whole launch, items of none to three tiles."""
+    from odc_amd import GatherService, ReductionService
+
+    options = {"rank_major": order, "accum_tile_order": order, "few_tiles": 1 << 30}
+    saved = {name: _native.get_option(name) for name in options}
+    try:
+        for name, value in options.items():
+            _native.set_option(name, value)
+        from odc_amd import SymmBufferRegistry
+
+        W, sizes = 3, [(701 * i + 5) % 2500 for i in range(n)]
+        offsets = [sum(sizes[:i]) for i in range(n)]
+        group = make_world(W, 4 << 20)
+        gather, red = GatherService(), ReductionService(accumulation_dtype=torch.float32)
+        gen = torch.Generator().manual_seed(n)
+        shards = [torch.randn(sum(sizes), generator=gen).bfloat16() for _ in range(W)]
+        source = put_shards(SymmBufferRegistry.get_instance(), "p", shards)
+        outs = [torch.full((W * m,), float("nan"), dtype=torch.bfloat16, device="cuda") for m in sizes]
+        gather.gather_slices(outs, source, offsets, sizes, group)
+        for out, off, m in zip(outs, offsets, sizes):
+            assert_bit_equal(out, oracle.gather([s[off : off + m] for s in shards]))
+        grads = [torch.randn(W * m, generator=gen).bfloat16() for m in sizes]
+        red.scatter_accumulate_slices("g", [g.cuda() for g in grads], offsets, sizes, group)
+        for r, got in enumerate(red.get_peer_accumulations("g")):
+            assert_bit_equal(got, torch.cat([g.view(W, -1)[r] if g.numel() else g for g in grads]).float(), f"rank {r}")
+    finally:
+        for name, value in saved.items():
+            _native.set_option(name, value)
