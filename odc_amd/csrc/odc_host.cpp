@@ -275,6 +275,28 @@ bool wants_short_tiles(const odc_arena* a, uint32_t n_items, uint32_t next, uint
   return tiles < (uint64_t)below * segments;
 }
 
+// Whether a publish of items [next, n_items) is cut into short tiles. It sees a W-th of the elements
+// that the other launches see, and a launch of a few hundred whole tiles leaves most of a CU idle;
+// two written streams per read one also stream better from 128 x 2 than from 256 x 4. So
+// fp32 accumulations always are. 16-bit ones move 4 to 6 KB per short tile, too little for the cost of
+// a workgroup, and are only up to 1024 whole tiles (4 workgroups per CU). Graph-replayed
+// launches over buffers in turn, us, whole -> short:
+//   fp32 into bf16: ten slices of 98 816 elements 3.5 -> 2.9, one of 1 Mi 4.2 -> 3.65, 112 of 3 640 5.2 -> 3.65, one of
+//     3.1 M 9.65 -> 7.1, a decoder layer's 27 M at W = 8 45.8 -> 44.0, eight layers 369 -> 335, one of 66 M 108.7 -> 103.4;
+//   fp32 in place: 3.2 -> 2.65, 3.8 -> 3.35, 4.35 -> 3.3, 7.65 -> 6.1, 35.8 -> 34.5, 284 -> 267, 81.2 -> 82.0;
+//   bf16 in place: 3.05 -> 2.7, 3.25 -> 3.05, 4.1 -> 3.0, 4.4 -> 4.2, but 19.5 -> 22.6, 134 -> 173, and 42.0 -> 41.4.
+template <class Units>
+bool publish_in_short_tiles(const odc_arena* a, uint32_t n_items, uint32_t next, Units units, int acc_bytes) {
+  if (!a->short_tiles || acc_bytes == 4) return a->short_tiles;
+  uint64_t tiles = 0;
+  uint32_t taken = 0;
+  for (uint32_t i = next; i < n_items && taken < (uint32_t)kMaxItems; ++i) {
+    tiles += tiles_for(units(i), kTileElems);
+    taken += units(i) != 0;
+  }
+  return tiles <= 1024;
+}
+
 // How the workgroups of a launch find their items. Up to eight fills of the chip (4096 workgroups of
 // 128 threads each) a launch is mostly the latency from its arguments to its first loads, and the
 // whole prefix table read at once pays off; in longer ones the other workgroups of the CU hide that
@@ -945,13 +967,16 @@ int odc_publish(odc_arena* a, uint32_t rank, const odc_publish_item* items, uint
     }
     L.tt.order = kItemMajor;
     L.tt.first_rank = 0;
+    const auto units = [&](uint32_t i) { return items[i].elems; };
+    const bool short_tiles = publish_in_short_tiles(a, n_items, next, units, ab);
     const int n = fill_launch(
-        L.tt, 1u, n_items, &next, kTileElems, [&](uint32_t i) { return items[i].elems; },
+        L.tt, 1u, n_items, &next, tile_units(kTileElems, short_tiles), units,
         [&](uint32_t slot, uint32_t i) {
           L.item[slot] = {static_cast<uint8_t*>(items[i].out), items[i].acc_offset, items[i].elems};
         });
     if (n < 0) return n;
     if (n == 0) continue;
+    L.form = tile_form(short_tiles, L.tt.n_tiles, opt.few_tiles);
     // one workgroup per tile: the division sequence wants the occupancy, and the launch is short
     const uint32_t grid = grid_for(a, opt.publish_blocks_per_cu, L.tt.n_tiles);
     const uint32_t lds = lds_claim_for(a, opt.publish_resident_cap, grid, L.tt.n_tiles);

@@ -14,7 +14,8 @@
 // Launch model shared by the kernels: the work of one launch is cut into tiles of 1024 vectors
 // (16 KiB), done by workgroups of 256 threads (512 for the two gathers), or into short tiles of 256
 // vectors, done by 128 threads: launches of short segments (wants_short_tiles in odc_host.cpp) and
-// every accumulate and store of 16-bit gradients into fp32 (accum_streams_short in odc_launch.h).
+// every accumulate and store of 16-bit gradients into fp32 (accum_streams_short in odc_launch.h), and
+// every publish of fp32 accumulations (publish_in_short_tiles in odc_host.cpp).
 // Workgroups walk the tiles with a grid-stride loop, by default one workgroup per tile, so that,
 // at any instant, the whole chip streams one compact window of memory. Per-item
 // descriptors (<= ODC_MAX_ITEMS_PER_LAUNCH) travel BY VALUE in the kernel argument segment and
@@ -658,64 +659,70 @@ __device__ __forceinline__ typename Quad<O>::vec_t publish_quad(typename Quad<A>
   return Quad<O>::narrow(f);
 }
 
-template <class Launch, class A, class O>
-__global__ __launch_bounds__(kThreads) void publish_kernel(const Launch launch) {
+// Bound by HBM in long launches, by latency and idle CUs in short ones; which tiles it takes is
+// publish_in_short_tiles in odc_host.cpp. Everything is nontemporal in both forms (plain accesses: 3.1 M
+// elements 7.0 -> 10.8 us, 8 Mi 15.5 -> 23.2).
+template <class Launch, class A, class O, bool kFew, int T, int U>
+__global__ __launch_bounds__(T) void publish_kernel(const Launch launch) {
+  constexpr uint32_t kVecs = T * U, kElems = kVecs * 4;
+  static_assert(kVecs == kTileVecs || kVecs == kShortTileVecs, "a whole tile or a short one");
   typedef typename Codec<A>::raw_t araw_t;
   typedef typename Codec<O>::raw_t oraw_t;
   typedef typename Quad<A>::vec_t avec_t;
   typedef typename Quad<O>::vec_t ovec_t;
   const uint32_t tid = threadIdx.x;
-  TileWalk<Launch> walk(launch);
+  TileWalk<Launch, kFew> walk(launch);
   for (uint32_t t = blockIdx.x; t < walk.n_tiles(launch); t += gridDim.x) {
     const TileCoord c = walk.locate(launch, t);
     const PublishDesc it = walk.it;
     const uint64_t seg = it.seg_elems;
-    const uint64_t in_seg = (uint64_t)c.chunk * kTileElems;
+    const uint64_t in_seg = (uint64_t)c.chunk * kElems;
     araw_t* acc = reinterpret_cast<araw_t*>(walk.region(launch, 0) + it.acc_off) + in_seg;
     oraw_t* out = it.out ? reinterpret_cast<oraw_t*>(as_global(it.out)) + in_seg : nullptr;
     const uint64_t left = seg - in_seg;
-    if (left >= kTileElems && (((uintptr_t)acc) & (sizeof(avec_t) - 1)) == 0 &&
+    if (left >= kElems && (((uintptr_t)acc) & (sizeof(avec_t) - 1)) == 0 &&
         (((uintptr_t)out) & (sizeof(ovec_t) - 1)) == 0) {
       avec_t* ap = reinterpret_cast<avec_t*>(acc) + tid;
       ovec_t* op = reinterpret_cast<ovec_t*>(out) + tid;
-      avec_t raw[kUnroll];
-      ovec_t cast[kUnroll];
+      avec_t raw[U];
+      ovec_t cast[U];
 #pragma unroll
-      for (int u = 0; u < kUnroll; ++u) raw[u] = __builtin_nontemporal_load(ap + u * kThreads);
+      for (int u = 0; u < U; ++u) raw[u] = __builtin_nontemporal_load(ap + u * T);
 #pragma unroll
-      for (int u = 0; u < kUnroll; ++u) {
+      for (int u = 0; u < U; ++u) {
         cast[u] = publish_quad<A, O>(raw[u], launch.scale);
       }
       // The two written streams go out one after the other, not interleaved vector by vector
       // (measured: +6..12 %; plain instead of nontemporal stores for the copy change nothing then).
       if (launch.scale.divide) {
 #pragma unroll
-        for (int u = 0; u < kUnroll; ++u) __builtin_nontemporal_store(raw[u], ap + u * kThreads);
+        for (int u = 0; u < U; ++u) __builtin_nontemporal_store(raw[u], ap + u * T);
       }
       if (out) {
 #pragma unroll
-        for (int u = 0; u < kUnroll; ++u) __builtin_nontemporal_store(cast[u], op + u * kThreads);
+        for (int u = 0; u < U; ++u) __builtin_nontemporal_store(cast[u], op + u * T);
       }
     } else if ((((uintptr_t)acc) & (sizeof(avec_t) - 1)) == 0 && (((uintptr_t)out) & (sizeof(ovec_t) - 1)) == 0) {
       // A partial tile (every accumulation's last one): the same vectors under a lane mask, and
       // the up to three elements behind the last whole vector. The whole tile is one memory round
       // trip; element by element it was sixteen loads per lane and stores of 2 or 4 bytes
-      // (nine accumulations of 3 640 elements: 4.2 us instead of 5.9; of 233 016: 5.9 instead of 7.3).
+      // (256 x 4, nine accumulations of 3 640 elements: 4.2 us instead of 5.9; of 233 016: 5.9 instead
+      // of 7.3).
       const uint32_t quads = (uint32_t)left / 4, rest = (uint32_t)left & 3u;
       avec_t* ap = reinterpret_cast<avec_t*>(acc) + tid;
       ovec_t* op = reinterpret_cast<ovec_t*>(out) + tid;
-      avec_t raw[kUnroll] = {};
+      avec_t raw[U] = {};
       araw_t rest_raw = 0;
 #pragma unroll
-      for (int u = 0; u < kUnroll; ++u)
-        if (u * kThreads + tid < quads) raw[u] = __builtin_nontemporal_load(ap + u * kThreads);
+      for (int u = 0; u < U; ++u)
+        if (u * T + tid < quads) raw[u] = __builtin_nontemporal_load(ap + u * T);
       if (tid < rest) rest_raw = acc[quads * 4 + tid];
 #pragma unroll
-      for (int u = 0; u < kUnroll; ++u) {
-        if (u * kThreads + tid < quads) {
+      for (int u = 0; u < U; ++u) {
+        if (u * T + tid < quads) {
           const ovec_t cast = publish_quad<A, O>(raw[u], launch.scale);
-          if (launch.scale.divide) __builtin_nontemporal_store(raw[u], ap + u * kThreads);
-          if (out) __builtin_nontemporal_store(cast, op + u * kThreads);
+          if (launch.scale.divide) __builtin_nontemporal_store(raw[u], ap + u * T);
+          if (out) __builtin_nontemporal_store(cast, op + u * T);
         }
       }
       if (tid < rest) {
@@ -725,15 +732,15 @@ __global__ __launch_bounds__(kThreads) void publish_kernel(const Launch launch) 
     } else {
       // accumulations or outputs that are not aligned to their vectors: element by element, all
       // loads before the first store
-      constexpr int kPerLane = kTileElems / kThreads;
-      const uint32_t n = left < kTileElems ? (uint32_t)left : kTileElems;
+      constexpr int kPerLane = kElems / T;
+      const uint32_t n = left < kElems ? (uint32_t)left : kElems;
       araw_t raw[kPerLane];
 #pragma unroll
       for (int j = 0; j < kPerLane; ++j)
-        if (j * kThreads + tid < n) raw[j] = acc[j * kThreads + tid];
+        if (j * T + tid < n) raw[j] = acc[j * T + tid];
 #pragma unroll
       for (int j = 0; j < kPerLane; ++j) {
-        const uint32_t i = j * kThreads + tid;
+        const uint32_t i = j * T + tid;
         if (i < n) {
           if (launch.scale.divide) acc[i] = raw[j] = publish_scale<A>(raw[j], launch.scale);
           if (out) out[i] = Codec<O>::narrow(Codec<A>::widen(raw[j]));
@@ -832,9 +839,20 @@ kernel_fn<L> pick_cast_gather(int s, int d, CachePolicy policy, TileForm form) {
   return nullptr;
 }
 
+// publish_in_short_tiles: fp32 accumulations have no kernel of whole tiles.
+template <class L, class A, class O>
+kernel_fn<L> pick_publish_form(TileForm form) {
+  if (form == kFewShortTiles) return publish_kernel<L, A, O, kSearches<L>, kShortThreads, kShortUnroll>;
+  if (form == kShortTiles) return publish_kernel<L, A, O, false, kShortThreads, kShortUnroll>;
+  if constexpr (Codec<A>::kBytes == 4) return nullptr;
+  else return publish_kernel<L, A, O, false, kThreads, kUnroll>;
+}
+
 template <class L>
-kernel_fn<L> pick_publish(int a, int o) {  // (accumulation dtype, output dtype)
-#define X(E1, T1, E2, T2) if (a == E1 && o == E2) return publish_kernel<L, T1, T2>;
+kernel_fn<L> pick_publish(int a, int o, TileForm form) {  // (accumulation dtype, output dtype)
+#define X(E1, T1, E2, T2) \
+  if (a == E1 && o == E2) \
+    return pick_publish_form<L, T1, T2>(form);
   ODC_FOR_EACH_DTYPE_PAIR(X)
 #undef X
   return nullptr;
@@ -921,7 +939,7 @@ const char* error_string(int code) { return hipGetErrorString(static_cast<hipErr
 
 bool has_accum(int g, int a) { return pick_accum<AccumLaunch>(g, a, false, {}, kShortTiles) != nullptr; }
 bool has_cast_gather(int s, int d) { return pick_cast_gather<CastGatherLaunch>(s, d, {}, kWholeTiles) != nullptr; }
-bool has_publish(int a, int o) { return pick_publish<PublishLaunch>(a, o) != nullptr; }
+bool has_publish(int a, int o) { return pick_publish<PublishLaunch>(a, o, kShortTiles) != nullptr; }
 
 int launch_gather(const GatherLaunch& L, uint32_t grid, uint32_t lds_bytes, void* stream) {
   return launch_form(L, grid, L.form != kWholeTiles ? kShortThreads : kCopyThreads, lds_bytes, stream, [&](auto form) {
@@ -948,8 +966,8 @@ int launch_clear(const ClearLaunch& L, uint32_t grid, void* stream) {
 }
 
 int launch_publish(int a, int o, const PublishLaunch& L, uint32_t grid, uint32_t lds_bytes, void* stream) {
-  return launch_form(L, grid, kThreads, lds_bytes, stream,
-                     [&](auto form) { return pick_publish<typename decltype(form)::type>(a, o); });
+  return launch_form(L, grid, L.form != kWholeTiles ? kShortThreads : kThreads, lds_bytes, stream,
+                     [&](auto form) { return pick_publish<typename decltype(form)::type>(a, o, L.form); });
 }
 
 }  // namespace odc_device

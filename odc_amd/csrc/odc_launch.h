@@ -134,6 +134,7 @@ struct PublishLaunch {  // one rank's region only: tt.world == 1
   uint8_t* base;        // of the publishing rank's region
   uint64_t rank_stride; // not used
   PublishScale scale;
+  TileForm form = kWholeTiles;  // picks the kernel
   PublishDesc item[kMaxItems];
 };
 struct PublishSingle : SingleLaunch<PublishDesc> {

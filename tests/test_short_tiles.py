@@ -121,3 +121,60 @@ def test_every_item_is_found_among_few_tiles(make_world, n, order):
     finally:
         for name, value in saved.items():
             _native.set_option(name, value)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("few", [0, 1 << 30])  # the binary search, the table read at once
+@pytest.mark.parametrize("acc_dtype,out_dtype", [
+    (torch.float32, torch.bfloat16), (torch.float32, torch.float32), (torch.bfloat16, torch.float16),
+])
+@pytest.mark.parametrize("n", [1, 2, 64, 66, 112, 113])
+def test_publish_of_many_items_in_short_tiles(make_world, n, acc_dtype, out_dtype, few):
+    """Items of none to a few tiles and around the edges of one, in one launch and in two."""
+    from odc_amd import SymmBufferRegistry
+    from odc_amd.primitives.utils import get_world, native_dtype
+
+    make_world(2, 8 << 20)
+    registry = SymmBufferRegistry.get_instance()
+    sizes = [[1023, 1024, 1025, 2049, 4097, 0, 5, 3070][i % 8] for i in range(n)]
+    starts = [sum(-(-m // 64) * 64 for m in sizes[:i]) for i in range(n)]
+    total = starts[-1] + sizes[-1] + 64
+    registry.allocate_symm_buffer("acc", (total,), acc_dtype)
+    acc = registry.peer_tensors["acc"][1]
+    start = torch.randn(total, generator=torch.Generator().manual_seed(n)).to(acc_dtype)
+    saved = _native.get_option("few_tiles")
+    _native.set_option("few_tiles", few)
+    try:
+        for divisor in (8.0, 3.0, 1.0):
+            acc.copy_(start)
+            outs = [torch.full((m + 8,), 7.0, dtype=out_dtype, device="cuda") for m in sizes]
+            items = (_native.PublishItem * n)(*[
+                _native.PublishItem(registry.get_offset("acc") + at * acc_dtype.itemsize, m, out.data_ptr())
+                for at, m, out in zip(starts, sizes, outs)])
+            _native.check(_native.load().odc_publish(
+                get_world().arena.handle, 1, items, n, native_dtype(acc_dtype), native_dtype(out_dtype), divisor,
+                ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+            want = start.clone()
+            for at, m, out in zip(starts, sizes, outs):
+                copy = torch.full((m + 8,), 7.0, dtype=out_dtype)
+                if m:
+                    copy[:m] = oracle.fsdp1_publish(want[at : at + m], divisor, out_dtype)
+                assert_bit_equal(out, copy, f"output at {at} / {divisor}")
+            assert_bit_equal(acc, want, f"accumulations / {divisor}")
+    finally:
+        _native.set_option("few_tiles", saved)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1024 * 4096, 1024 * 4096 + 1, 1025 * 4096 + 1027])  # the longest in short tiles, then whole ones
+def test_publish_of_16_bit_accumulations_around_the_line(make_world, n):
+    from odc_amd import ReductionService
+
+    group = make_world(2, 32 << 20)
+    red = ReductionService(accumulation_dtype=torch.bfloat16)
+    red.register("k", (n,), torch.bfloat16, torch.bfloat16, group)
+    start = torch.randn(n, generator=torch.Generator().manual_seed(n)).bfloat16()
+    red.get_accumulation("k").copy_(start)
+    (out,) = red.publish(["k"], out_dtype=torch.float32, divisor=3.0)
+    assert_bit_equal(out, oracle.fsdp1_publish(start, 3.0, torch.float32))
+    assert_bit_equal(red.get_accumulation("k"), start)
