@@ -78,7 +78,6 @@ struct Options {
   int64_t cached_gradient_bytes = 128ll << 20;
   int64_t short_tiles_below = 32;             // see wants_short_tiles
   int64_t few_tiles = 32768;                  // see tile_form
-  int64_t dry_run_short_tiles = 0;  // read when an arena without a device is created: 1 = plan short tiles too
 };
 Options g_opt;
 std::mutex g_opt_mu;
@@ -108,7 +107,6 @@ int64_t* option_slot(const char* name) {
   if (!strcmp(name, "cached_gradient_bytes")) return &g_opt.cached_gradient_bytes;
   if (!strcmp(name, "short_tiles_below")) return &g_opt.short_tiles_below;
   if (!strcmp(name, "few_tiles")) return &g_opt.few_tiles;
-  if (!strcmp(name, "dry_run_short_tiles")) return &g_opt.dry_run_short_tiles;
   return nullptr;
 }
 
@@ -138,7 +136,6 @@ struct odc_arena {
   uint8_t* base = nullptr;    // rank 0's region: the allocation rounded up to the stride alignment
   uint8_t* origin = nullptr;  // what launches are planned against: base, or a fictitious address on a dry-run arena
   bool dry_run = false;
-  bool short_tiles = true;  // launches may be cut into short tiles (a dry run counts whole ones unless asked)
   std::map<uint64_t, uint64_t> live;  // offset -> size (rounded)
   std::map<uint64_t, uint64_t> free_; // offset -> size, coalesced
   std::atomic<uint64_t> in_use{0};  // changed under mu, read by launches without it
@@ -187,6 +184,10 @@ int check_compute(odc_arena* a, DeviceGuard& guard) {
 
 // What dry-run arenas have "launched" (process-wide, reset by odc_set_option("dry_run_reset", 0)).
 std::atomic<int64_t> g_dry_launches{0}, g_dry_tiles{0}, g_dry_workgroups{0};
+std::atomic<int64_t> g_dry_short{0}, g_dry_few{0};  // of the launches: those in kShortTiles, in kFewShortTiles
+
+template <class Launch> TileForm form_of(const Launch& L) { return L.form; }
+TileForm form_of(const ClearLaunch&) { return kWholeTiles; }
 
 // The one place kernels are launched from: `issue` is the odc_device launch of the entry point.
 // On a dry-run arena the launch is only counted: the host-side validation, work-list splitting
@@ -199,6 +200,8 @@ int launch_tiles(const odc_arena* a, const Launch& L, uint32_t grid, Issue issue
     g_dry_launches += 1;
     g_dry_tiles += L.tt.n_tiles;
     g_dry_workgroups += grid;
+    g_dry_short += form_of(L) == kShortTiles;
+    g_dry_few += form_of(L) == kFewShortTiles;
     return ODC_OK;
   }
   const int e = issue();
@@ -262,9 +265,7 @@ constexpr int64_t kSymmetric = -1;  // a line: the stream lies in symmetric memo
 //     600 000 (73) 4.55 -> 4.65; converting gather level from there on, store 5.0 -> 5.5 at 600 000.
 // Launches of longer segments stream best in whole tiles, with one exception (accum_streams_short).
 template <class Units>
-bool wants_short_tiles(const odc_arena* a, uint32_t n_items, uint32_t next, uint64_t tile_units, Units units,
-                       int64_t below) {
-  if (!a->short_tiles) return false;
+bool wants_short_tiles(uint32_t n_items, uint32_t next, uint64_t tile_units, Units units, int64_t below) {
   uint64_t segments = 0, tiles = 0;
   for (uint32_t i = next; i < n_items && segments < (uint64_t)kMaxItems; ++i) {
     const uint64_t n = units(i);
@@ -286,8 +287,8 @@ bool wants_short_tiles(const odc_arena* a, uint32_t n_items, uint32_t next, uint
 //   fp32 in place: 3.2 -> 2.65, 3.8 -> 3.35, 4.35 -> 3.3, 7.65 -> 6.1, 35.8 -> 34.5, 284 -> 267, 81.2 -> 82.0;
 //   bf16 in place: 3.05 -> 2.7, 3.25 -> 3.05, 4.1 -> 3.0, 4.4 -> 4.2, but 19.5 -> 22.6, 134 -> 173, and 42.0 -> 41.4.
 template <class Units>
-bool publish_in_short_tiles(const odc_arena* a, uint32_t n_items, uint32_t next, Units units, int acc_bytes) {
-  if (!a->short_tiles || acc_bytes == 4) return a->short_tiles;
+bool publish_in_short_tiles(uint32_t n_items, uint32_t next, Units units, int acc_bytes) {
+  if (acc_bytes == 4) return true;
   uint64_t tiles = 0;
   uint32_t taken = 0;
   for (uint32_t i = next; i < n_items && taken < (uint32_t)kMaxItems; ++i) {
@@ -330,7 +331,7 @@ int odc_abi_version(void) { return ODC_HIP_ABI_VERSION; }
 
 int odc_set_option(const char* name, int64_t value) {
   if (name && !strcmp(name, "dry_run_reset")) {
-    g_dry_launches = 0; g_dry_tiles = 0; g_dry_workgroups = 0;
+    g_dry_launches = 0; g_dry_tiles = 0; g_dry_workgroups = 0; g_dry_short = 0; g_dry_few = 0;
     return ODC_OK;
   }
   std::lock_guard<std::mutex> lk(g_opt_mu);
@@ -351,6 +352,8 @@ int odc_get_option(const char* name, int64_t* value) {
     if (!strcmp(name, "dry_run_launches")) { *value = g_dry_launches.load(); return ODC_OK; }
     if (!strcmp(name, "dry_run_tiles")) { *value = g_dry_tiles.load(); return ODC_OK; }
     if (!strcmp(name, "dry_run_workgroups")) { *value = g_dry_workgroups.load(); return ODC_OK; }
+    if (!strcmp(name, "dry_run_short_launches")) { *value = g_dry_short.load(); return ODC_OK; }
+    if (!strcmp(name, "dry_run_few_launches")) { *value = g_dry_few.load(); return ODC_OK; }
   }
   std::lock_guard<std::mutex> lk(g_opt_mu);
   int64_t* s = option_slot(name);
@@ -377,7 +380,6 @@ int odc_arena_create(uint32_t world_size, uint64_t bytes_per_rank, uint32_t flag
   const uint64_t stride_align = std::max<uint64_t>(round_up((uint64_t)opt.rank_stride_align, kAlign), kAlign);
   a->alloc_align = std::max<uint64_t>(round_up((uint64_t)opt.alloc_align, kAlign), kAlign);
   a->bytes_per_rank = round_up(bytes_per_rank, kAlign);
-  a->short_tiles = !(flags & ODC_ARENA_NO_BACKING) || opt.dry_run_short_tiles != 0;
   a->rank_stride = round_up(a->bytes_per_rank + round_up((uint64_t)opt.rank_stagger_bytes, kAlign), stride_align);
   // the device allocation promises 256 B alignment only; the regions shall start on stride_align
   // boundaries, so the allocation is that much larger: the whole sum must fit 64 bits
@@ -636,7 +638,7 @@ int odc_gather(odc_arena* a, const odc_gather_item* items, uint32_t n_items, uin
     L.tt.order = (uint32_t)opt.rank_major;
     L.tt.first_rank = first_rank;
     const auto units = [&](uint32_t i) { return items[i].shard_bytes; };
-    const bool short_tiles = wants_short_tiles(a, n_items, next, kTileBytes, units, opt.short_tiles_below);
+    const bool short_tiles = wants_short_tiles(n_items, next, kTileBytes, units, opt.short_tiles_below);
     const int n = fill_launch(
         L.tt, a->world, n_items, &next, tile_units(kTileBytes, short_tiles), units,
         [&](uint32_t slot, uint32_t i) {
@@ -689,7 +691,7 @@ int odc_gather_cast(odc_arena* a, const odc_gather_cast_item* items, uint32_t n_
     L.tt.order = (uint32_t)opt.rank_major;
     L.tt.first_rank = first_rank;
     const auto units = [&](uint32_t i) { return items[i].shard_elems; };
-    const bool short_tiles = wants_short_tiles(a, n_items, next, kTileElems, units, opt.short_tiles_below);
+    const bool short_tiles = wants_short_tiles(n_items, next, kTileElems, units, opt.short_tiles_below);
     const int n = fill_launch(
         L.tt, a->world, n_items, &next, tile_units(kTileElems, short_tiles), units,
         [&](uint32_t slot, uint32_t i) {
@@ -739,7 +741,7 @@ int odc_convert(odc_arena* a, const odc_convert_item* items, uint32_t n_items, i
     L.tt.order = (uint32_t)opt.rank_major;
     L.tt.first_rank = 0;
     const auto units = [&](uint32_t i) { return items[i].elems; };
-    const bool short_tiles = wants_short_tiles(a, n_items, next, kTileElems, units, opt.short_tiles_below);
+    const bool short_tiles = wants_short_tiles(n_items, next, kTileElems, units, opt.short_tiles_below);
     const int n = fill_launch(
         L.tt, a->world, n_items, &next, tile_units(kTileElems, short_tiles), units,
         [&](uint32_t slot, uint32_t i) {
@@ -852,8 +854,8 @@ int scatter_launch(odc_arena* a, const odc_accum_item* items, uint32_t n_items, 
     L.tt.order = (uint32_t)opt.rank_major;
     L.tt.first_rank = 0;
     const auto units = [&](uint32_t i) { return items[order[i]].shard_elems; };
-    const bool short_tiles = (a->short_tiles && odc_launch::accum_streams_short(grad_dtype, acc_dtype)) ||
-                             wants_short_tiles(a, n_items, next, kTileElems, units, opt.short_tiles_below);
+    const bool short_tiles = odc_launch::accum_streams_short(grad_dtype, acc_dtype) ||
+                             wants_short_tiles(n_items, next, kTileElems, units, opt.short_tiles_below);
     const int n = fill_launch(
         L.tt, a->world, n_items, &next, tile_units(kTileElems, short_tiles), units,
         [&](uint32_t slot, uint32_t i) {
@@ -968,7 +970,7 @@ int odc_publish(odc_arena* a, uint32_t rank, const odc_publish_item* items, uint
     L.tt.order = kItemMajor;
     L.tt.first_rank = 0;
     const auto units = [&](uint32_t i) { return items[i].elems; };
-    const bool short_tiles = publish_in_short_tiles(a, n_items, next, units, ab);
+    const bool short_tiles = publish_in_short_tiles(n_items, next, units, ab);
     const int n = fill_launch(
         L.tt, 1u, n_items, &next, tile_units(kTileElems, short_tiles), units,
         [&](uint32_t slot, uint32_t i) {

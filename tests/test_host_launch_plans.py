@@ -14,6 +14,8 @@ from odc_amd import _native
 
 TILE_BYTES = 16 * 1024
 TILE_ELEMS = 4096
+SHORT_TILE_BYTES = TILE_BYTES // 4
+SHORT_TILE_ELEMS = TILE_ELEMS // 4
 N_CU = 256  # what a dry-run arena assumes
 
 
@@ -30,6 +32,11 @@ class DryArena:
 
     def counters(self):
         return tuple(_native.get_option(n) for n in ("dry_run_launches", "dry_run_tiles", "dry_run_workgroups"))
+
+    def forms(self):
+        """Launches in whole tiles, in short tiles, in few short tiles."""
+        launches, short, few = (_native.get_option(f"dry_run_{n}") for n in ("launches", "short_launches", "few_launches"))
+        return launches - short - few, short, few
 
     def close(self):
         _native.check(self.lib.odc_arena_destroy(self.handle))
@@ -87,7 +94,7 @@ def test_long_item_lists_are_split_over_launches(arena, n_items):
     nonempty = [s for s in sizes if s]
     launches, tiles, workgroups = a.counters()
     assert launches == math.ceil(len(nonempty) / _native.MAX_ITEMS_PER_LAUNCH)
-    assert tiles == W * sum(math.ceil(s / TILE_BYTES) for s in nonempty)
+    assert tiles == W * sum(math.ceil(s / SHORT_TILE_BYTES) for s in nonempty)  # segments of 3 whole tiles at most
     assert workgroups == tiles  # the gather runs one workgroup per tile
 
 
@@ -102,9 +109,10 @@ def test_accumulate_launch_shapes(arena):
     )
     _native.check(a.lib.odc_scatter_accumulate(a.handle, items, 2, _native.DTYPE_BF16, _native.DTYPE_F32, None))
     launches, tiles, workgroups = a.counters()
-    assert (launches, tiles, workgroups) == (1, 2 * W * shard // TILE_ELEMS, 2 * W * shard // TILE_ELEMS)
+    # (16-bit gradients into fp32 go in short tiles whatever the sizes)
+    assert (launches, tiles, workgroups) == (1, 2 * W * shard // SHORT_TILE_ELEMS, 2 * W * shard // SHORT_TILE_ELEMS)
     _native.set_option("dry_run_reset", 0)
-    _native.set_option("accum_persistent_below_tiles", 128)  # segments of 64 tiles are below it
+    _native.set_option("accum_persistent_below_tiles", 128)  # segments of 64 whole tiles are below it
     try:
         _native.check(a.lib.odc_scatter_accumulate(a.handle, items, 2, _native.DTYPE_BF16, _native.DTYPE_F32, None))
         assert a.counters() == (1, tiles, N_CU)
@@ -125,7 +133,7 @@ def test_accumulate_launch_shapes(arena):
         _native.AccumItem(OUTSIDE, W * shard, 0, shard), _native.AccumItem(OUTSIDE + (1 << 30), W * shard, 4 * shard, shard)
     )
     _native.check(a.lib.odc_scatter_accumulate(a.handle, long_items, 2, _native.DTYPE_BF16, _native.DTYPE_F32, None))
-    long_tiles = 2 * W * shard // TILE_ELEMS
+    long_tiles = 2 * W * shard // SHORT_TILE_ELEMS
     assert a.counters() == (1, long_tiles, long_tiles)
     _native.set_option("dry_run_reset", 0)
     _native.set_option("accum_blocks_per_cu", 2)
@@ -138,7 +146,7 @@ def test_accumulate_launch_shapes(arena):
     _native.set_option("dry_run_reset", 0)
     small = (_native.AccumItem * 1)(_native.AccumItem(OUTSIDE, W * 4096, 0, 4096))
     _native.check(a.lib.odc_scatter_accumulate(a.handle, small, 1, _native.DTYPE_BF16, _native.DTYPE_F32, None))
-    assert a.counters() == (1, W, W)
+    assert a.counters() == (1, 4 * W, 4 * W)
 
 
 def test_clear_cast_gather_and_publish_plan(arena):
@@ -150,11 +158,11 @@ def test_clear_cast_gather_and_publish_plan(arena):
     _native.set_option("dry_run_reset", 0)
     cast = (_native.GatherCastItem * 1)(_native.GatherCastItem(OUTSIDE, 0, 10_000))
     _native.check(a.lib.odc_gather_cast(a.handle, cast, 1, _native.DTYPE_F32, _native.DTYPE_BF16, 2, None))
-    assert a.counters() == (1, W * 3, W * 3)
+    assert a.counters() == (1, W * 10, W * 10)  # 3 whole tiles per segment: cut into short ones
     _native.set_option("dry_run_reset", 0)
     pub = (_native.PublishItem * 2)(_native.PublishItem(0, 10_000, OUTSIDE), _native.PublishItem(1 << 20, 4096, None))
     _native.check(a.lib.odc_publish(a.handle, 1, pub, 2, _native.DTYPE_F32, _native.DTYPE_BF16, ctypes.c_float(8.0), None))
-    assert a.counters() == (1, 3 + 1, 4)  # one rank only
+    assert a.counters() == (1, 10 + 4, 14)  # one rank only; fp32 accumulations go in short tiles
 
 
 def _error(lib, status):
@@ -294,10 +302,95 @@ def test_accumulate_item_lists_with_tiny_items_keep_every_item(arena, n_items):
     nonempty = [s for s in sizes if s]
     launches, tiles, _ = a.counters()
     assert launches == math.ceil(len(nonempty) / _native.MAX_ITEMS_PER_LAUNCH)
-    assert tiles == W * sum(math.ceil(s / TILE_ELEMS) for s in nonempty)
+    assert tiles == W * sum(math.ceil(s / SHORT_TILE_ELEMS) for s in nonempty)
     bad = n_items - 2  # position in the caller's list; in launch order it sits elsewhere
     items[bad].shard_elems = (1 << 31) * TILE_ELEMS // W  # 2^31 tiles in all: one too many for a launch
     items[bad].grad_elems, items[bad].acc_offset = 0, 0
     status = a.lib.odc_scatter_accumulate(a.handle, items, n_items, _native.DTYPE_BF16, _native.DTYPE_F32, None)
     message = a.lib.odc_last_error().decode()
     assert status == _native.ODC_ERR_INVALID and f"item {bad}:" in message and "too large for one launch" in message
+
+
+BF16, F16, F32 = _native.DTYPE_BF16, _native.DTYPE_F16, _native.DTYPE_F32
+# entry point -> (item type, an item of n units at symmetric offset off, the call, elements (or bytes) of a whole tile)
+PLANNED = {
+    "gather": (_native.GatherItem, lambda W, off, n: (OUTSIDE, off, n),
+               lambda lib, a, items, n: lib.odc_gather(a, items, n, 0, None), TILE_BYTES),
+    "gather_cast": (_native.GatherCastItem, lambda W, off, n: (OUTSIDE, off, n),
+                    lambda lib, a, items, n: lib.odc_gather_cast(a, items, n, F32, BF16, 0, None), TILE_ELEMS),
+    "convert": (_native.ConvertItem, lambda W, off, n: (off, (1 << 34) + off, n),
+                lambda lib, a, items, n: lib.odc_convert(a, items, n, F32, BF16, None), TILE_ELEMS),
+    "accumulate": (_native.AccumItem, lambda W, off, n: (OUTSIDE, W * n, off, n),
+                   lambda lib, a, items, n: lib.odc_scatter_accumulate(a, items, n, F32, F32, None), TILE_ELEMS),
+    "store": (_native.AccumItem, lambda W, off, n: (OUTSIDE, W * n, off, n),
+              lambda lib, a, items, n: lib.odc_scatter_store(a, items, n, F32, F32, None), TILE_ELEMS),
+}
+
+
+def _plan(a, what, sizes):
+    kind, item, call, _tile = PLANNED[what]
+    items, off = (kind * len(sizes))(), 0
+    for k, n in enumerate(sizes):
+        items[k] = kind(*item(a.world, off, n))
+        off += -(-4 * n // 256) * 256
+    _native.set_option("dry_run_reset", 0)
+    _native.check(call(a.lib, a.handle, items, len(sizes)))
+    return a.counters(), a.forms()
+
+
+@pytest.mark.parametrize("what", PLANNED)
+def test_launches_are_cut_as_on_a_device(arena, what):
+    """Short segments go in short tiles, long ones in whole tiles, launch by launch; up to 32768
+    short tiles in a launch are 'few'."""
+    W, tile = 4, PLANNED[what][3]
+    a = arena(W, 1 << 36)
+    long, edge = 32 * tile, 31 * tile  # segments that average 32 whole tiles and more are long
+    assert _plan(a, what, [1]) == ((1, W, W), (0, 0, 1))
+    assert _plan(a, what, [edge]) == ((1, W * 4 * 31, W * 4 * 31), (0, 0, 1))
+    assert _plan(a, what, [long]) == ((1, W * 32, W * 32), (1, 0, 0))
+    assert _plan(a, what, [long, 0, edge])[1] == (0, 0, 1)  # 31.5 on average
+    assert _plan(a, what, [long + tile, 0, edge])[1] == (1, 0, 0)
+    many = [edge] * 67  # 67 * 4 * 124 short tiles: more than 32768
+    assert _plan(a, what, many) == ((1, W * 4 * 31 * 67, W * 4 * 31 * 67), (0, 1, 0))
+    assert _plan(a, what, many[1:])[1] == (0, 0, 1)
+    # every launch of a longer list is cut by its own items: 112 long ones, 112 of one whole tile
+    # each, 70 shorter ones that 42 longer ones outweigh, and three long ones
+    mixed = [long] * 112 + [tile] * 112 + [edge] * 70 + [8 * long] * 42 + [2 * long] * 3
+    tiles = W * (32 * 112 + 4 * 112 + (31 * 70 + 8 * 32 * 42) + 64 * 3)
+    assert _plan(a, what, mixed) == ((4, tiles, tiles), (3, 0, 1))
+
+
+def test_publish_is_cut_as_on_a_device(arena):
+    a = arena(2, 1 << 36)
+
+    def plan(sizes, acc, out):
+        items, off = (_native.PublishItem * len(sizes))(), 0
+        for k, n in enumerate(sizes):
+            items[k] = _native.PublishItem(off, n, OUTSIDE)
+            off += -(-4 * n // 256) * 256
+        _native.set_option("dry_run_reset", 0)
+        _native.check(a.lib.odc_publish(a.handle, 1, items, len(items), acc, out, ctypes.c_float(2.0), None))
+        return a.counters(), a.forms()
+
+    # fp32 accumulations always in short tiles, few of them up to 32768
+    assert plan([1, 4096], F32, BF16) == ((1, 5, 5), (0, 0, 1))
+    assert plan([32768 * 1024], F32, F16) == ((1, 32768, 32768), (0, 0, 1))
+    assert plan([32768 * 1024 + 1], F32, F32) == ((1, 32769, 32769), (0, 1, 0))
+    # 16-bit ones up to 1024 whole tiles per launch
+    assert plan([1000 * 4096, 24 * 4096], BF16, BF16) == ((1, 4096, 4096), (0, 0, 1))
+    assert plan([1000 * 4096, 24 * 4096 + 1], BF16, BF16) == ((1, 1025, 1025), (1, 0, 0))
+    # launch by launch: 112 items of 10 whole tiles, then 5 of one
+    assert plan([10 * 4096] * 112 + [0, 0] + [4096] * 5, F16, F32) == ((2, 1120 + 20, 1140), (1, 0, 1))
+
+
+@pytest.mark.parametrize("grad", [BF16, F16])
+def test_16_bit_gradients_into_fp32_always_go_in_short_tiles(arena, grad):
+    W = 4
+    a = arena(W, 1 << 36)
+    for call in (a.lib.odc_scatter_accumulate, a.lib.odc_scatter_store):
+        for n, form in ((1, (0, 0, 1)), (8192 * 1024, (0, 0, 1)), (8192 * 1024 + 1, (0, 1, 0))):
+            _native.set_option("dry_run_reset", 0)
+            items = (_native.AccumItem * 1)(_native.AccumItem(OUTSIDE, W * n, 0, n))
+            _native.check(call(a.handle, items, 1, grad, F32, None))
+            tiles = W * math.ceil(n / SHORT_TILE_ELEMS)
+            assert (a.counters(), a.forms()) == ((1, tiles, tiles), form)

@@ -30,11 +30,7 @@ def test_short_tile_geometry(tmp_path):
 ])
 def test_plans_in_short_tiles(shard, acc_dtype, tiles):
     W, lib, handle = 4, _native.load(), ctypes.c_void_p()
-    _native.set_option("dry_run_short_tiles", 1)
-    try:
-        _native.check(lib.odc_arena_create(W, 1 << 30, _native.ODC_ARENA_DRY_RUN, ctypes.byref(handle)))
-    finally:
-        _native.set_option("dry_run_short_tiles", 0)
+    _native.check(lib.odc_arena_create(W, 1 << 30, _native.ODC_ARENA_DRY_RUN, ctypes.byref(handle)))
     _native.set_option("dry_run_reset", 0)
     item = (_native.AccumItem * 1)(_native.AccumItem(1 << 33, W * shard, 0, shard))
     _native.check(lib.odc_scatter_accumulate(handle, item, 1, _native.DTYPE_BF16, acc_dtype, None))
