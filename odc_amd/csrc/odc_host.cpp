@@ -217,10 +217,11 @@ Options options_snapshot() {
 // blocks_per_cu > 0 asks for that many persistent workgroups per CU. Ragged launches (uneven
 // shards: unaligned reads, heads and tails) never get them: they hide their extra latency better
 // with one workgroup per tile, i.e. full occupancy (measured: +5..10 %).
-uint32_t grid_for(const odc_arena* a, int64_t blocks_per_cu, uint32_t n_tiles, bool ragged = false) {
-  if (blocks_per_cu <= 0 || ragged) return n_tiles;
-  const uint64_t g = (uint64_t)a->n_cu * (uint64_t)blocks_per_cu;
-  return (uint32_t)std::min<uint64_t>(g, n_tiles);
+uint32_t grid_for(const odc_arena* a, int64_t blocks_per_cu, uint32_t n_tiles, uint32_t threads, bool ragged = false) {
+  const uint32_t most = std::min(n_tiles, most_workgroups(threads));
+  if (blocks_per_cu <= 0 || ragged) return most;
+  const uint64_t cu = (uint64_t)a->n_cu, per_cu = (uint64_t)blocks_per_cu;
+  return per_cu >= most ? most : (uint32_t)std::min<uint64_t>(cu * per_cu, most);
 }
 
 // What a launch leaves in the caches. Nontemporal accesses stream fastest when nothing will be
@@ -653,7 +654,7 @@ int odc_gather(odc_arena* a, const odc_gather_item* items, uint32_t n_items, uin
     L.policy = cache_policy(a, opt, 0, kSymmetric, shard_bytes * a->world, opt.cached_output_bytes);
     for (uint32_t k = 0; k < L.tt.n_items; ++k)
       ragged |= (((uintptr_t)L.item[k].dst | L.item[k].src_off | L.item[k].seg_bytes) & 15u) != 0;
-    const uint32_t grid = grid_for(a, opt.gather_blocks_per_cu, L.tt.n_tiles, ragged);
+    const uint32_t grid = grid_for(a, opt.gather_blocks_per_cu, L.tt.n_tiles, copy_threads(L.form), ragged);
     const uint32_t lds = lds_claim_for(a, opt.gather_resident_cap, grid, L.tt.n_tiles);
     if (int rc = launch_tiles(a, L, grid, [&] { return odc_device::launch_gather(L, grid, lds, stream); })) return rc;
   }
@@ -702,7 +703,7 @@ int odc_gather_cast(odc_arena* a, const odc_gather_cast_item* items, uint32_t n_
     if (n == 0) continue;
     L.form = tile_form(short_tiles, L.tt.n_tiles, opt.few_tiles);
     L.policy = cache_policy(a, opt, 0, kSymmetric, 0, kSymmetric);
-    const uint32_t grid = grid_for(a, opt.gather_blocks_per_cu, L.tt.n_tiles);
+    const uint32_t grid = grid_for(a, opt.gather_blocks_per_cu, L.tt.n_tiles, copy_threads(L.form));
     const uint32_t lds = lds_claim_for(a, opt.cast_resident_cap, grid, L.tt.n_tiles);
     if (int rc = launch_tiles(a, L, grid, [&] {
           return odc_device::launch_cast_gather(src_dtype, dst_dtype, L, grid, lds, stream);
@@ -752,7 +753,7 @@ int odc_convert(odc_arena* a, const odc_convert_item* items, uint32_t n_items, i
     if (n == 0) continue;
     L.form = tile_form(short_tiles, L.tt.n_tiles, opt.few_tiles);
     L.policy = cache_policy(a, opt, 0, kSymmetric, 0, kSymmetric);
-    const uint32_t grid = grid_for(a, opt.gather_blocks_per_cu, L.tt.n_tiles);
+    const uint32_t grid = grid_for(a, opt.gather_blocks_per_cu, L.tt.n_tiles, copy_threads(L.form));
     const uint32_t lds = lds_claim_for(a, opt.cast_resident_cap, grid, L.tt.n_tiles);
     if (int rc = launch_tiles(a, L, grid, [&] {
           return odc_device::launch_cast_gather(src_dtype, dst_dtype, L, grid, lds, stream);
@@ -785,7 +786,7 @@ int odc_clear(odc_arena* a, const odc_span* spans, uint32_t n_spans, void* strea
         });
     if (n < 0) return n;
     if (n == 0) continue;
-    const uint32_t grid = grid_for(a, opt.clear_blocks_per_cu, L.tt.n_tiles);
+    const uint32_t grid = grid_for(a, opt.clear_blocks_per_cu, L.tt.n_tiles, kThreads);
     if (int rc = launch_tiles(a, L, grid, [&] { return odc_device::launch_clear(L, grid, stream); })) return rc;
   }
   return ODC_OK;
@@ -899,7 +900,8 @@ int scatter_launch(odc_arena* a, const odc_accum_item* items, uint32_t n_items, 
     int64_t blocks_per_cu = store ? opt.store_blocks_per_cu : opt.accum_blocks_per_cu;
     if (blocks_per_cu < 0)
       blocks_per_cu = whole_tiles < (uint64_t)opt.accum_persistent_below_tiles * segments ? 1 : 0;
-    const uint32_t grid = grid_for(a, blocks_per_cu, L.tt.n_tiles, ragged);
+    const uint32_t threads = accum_threads(grad_dtype, acc_dtype, store, L.policy, L.form);
+    const uint32_t grid = grid_for(a, blocks_per_cu, L.tt.n_tiles, threads, ragged);
     const int64_t cap = store ? opt.store_resident_cap : opt.accum_resident_cap;
     const uint32_t lds = lds_claim_for(a, cap, grid, L.tt.n_tiles);
     if (int rc = launch_tiles(a, L, grid, [&] {
@@ -980,7 +982,7 @@ int odc_publish(odc_arena* a, uint32_t rank, const odc_publish_item* items, uint
     if (n == 0) continue;
     L.form = tile_form(short_tiles, L.tt.n_tiles, opt.few_tiles);
     // one workgroup per tile: the division sequence wants the occupancy, and the launch is short
-    const uint32_t grid = grid_for(a, opt.publish_blocks_per_cu, L.tt.n_tiles);
+    const uint32_t grid = grid_for(a, opt.publish_blocks_per_cu, L.tt.n_tiles, publish_threads(L.form));
     const uint32_t lds = lds_claim_for(a, opt.publish_resident_cap, grid, L.tt.n_tiles);
     if (int rc = launch_tiles(a, L, grid, [&] {
           return odc_device::launch_publish(acc_dtype, out_dtype, L, grid, lds, stream);

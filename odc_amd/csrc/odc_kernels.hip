@@ -42,34 +42,6 @@
 
 namespace {
 
-// Workgroup shape of the two gathers and of the scatter-store (the kernels that read one stream
-// and write one) on whole tiles: 512 threads x 2 steps over the same 16 KiB tile as the 256 x 4 of
-// the other kernels. Four such workgroups fill a CU's wave slots, which is the residency these kernels
-// stream best at (measured: gathers +1.4..2.6 % over 256 x 4 with a residency cap of 4, which
-// had to be enforced by claiming LDS; 256 x 4 without a cap loses 6..8 %; 1024 x 1 loses
-// 20 %; short tiles lose 1 %). The read-modify-write with fp32 gradients keeps 256 x 4 (512 x 2:
-// equal on long segments), and so does the clear (512 x 2: -25 % on per-parameter spans).
-constexpr int kCopyThreads = 512;
-constexpr int kCopyUnroll = (int)odc_tiles::kTileVecs / kCopyThreads;  // 2 for the 16 KiB tile
-constexpr int kStoreThreads = 512;
-constexpr int kStoreUnroll = (int)odc_tiles::kTileVecs / kStoreThreads;
-static_assert(kCopyUnroll >= 1 && kStoreUnroll >= 1, "a tile holds at least one vector per thread");
-// 16-bit gradients into 16-bit accumulations have 8-byte vectors in both streams, half a tile's bytes,
-// and whole tiles take the other two shapes: the store 256 x 4 (64 KB of loads in flight per CU, as the
-// gathers have; 512 x 2 has half of that), the read-modify-write 512 x 2 where its gradient is streamed
-// (where the gradient is cached, up to 64 Mi elements, 256 x 4 is level or ahead). Graph-replayed launches, us, before ->
-// after, then 128 x 8 for both: a decoder layer's store at W = 8 174 -> 136, 138; at W = 64 167 -> 140, 143; 12 uneven
-// ranks 177 -> 141, 144; one of 525 M elements 326 -> 328, 333; 4 Mi 4.9 -> 4.5, 4.7; the layer's
-// read-modify-write at W = 8 209 -> 199, 210; at W = 64 218 -> 204.5, 218; 525 M elements 516 -> 489, 517. (Pairs
-// of vectors, 16 bytes per lane, in the old shapes: 213 and 178 for the layer at W = 8, 524 and 341 for 525 M.)
-constexpr int kNarrowRmwThreads = 512;
-constexpr int kNarrowRmwUnroll = (int)odc_tiles::kTileVecs / kNarrowRmwThreads;
-// Shape for short tiles: two vectors per lane, and few enough threads that a segment of a few hundred elements does not hold the wave slots of a CU for nothing
-// (300 slices at W = 16, gather + accumulate: 31.9 us; 256 threads x 1: 40.1; 128 x 1 on eighths:
-// 35.2; 128 x 4 on halves: 33.1; whole tiles: 46.6).
-constexpr int kShortThreads = 128;
-constexpr int kShortUnroll = (int)odc_tiles::kShortTileVecs / kShortThreads;
-
 // ------------------------------------------------------------------------------------------------
 // device side
 // ------------------------------------------------------------------------------------------------
@@ -956,23 +928,19 @@ bool has_cast_gather(int s, int d) { return pick_cast_gather<CastGatherLaunch>(s
 bool has_publish(int a, int o) { return pick_publish<PublishLaunch>(a, o, kShortTiles) != nullptr; }
 
 int launch_gather(const GatherLaunch& L, uint32_t grid, uint32_t lds_bytes, void* stream) {
-  return launch_form(L, grid, L.form != kWholeTiles ? kShortThreads : kCopyThreads, lds_bytes, stream, [&](auto form) {
+  return launch_form(L, grid, copy_threads(L.form), lds_bytes, stream, [&](auto form) {
     return pick_gather<typename decltype(form)::type>(L.policy, L.form);
   });
 }
 
 int launch_cast_gather(int s, int d, const CastGatherLaunch& L, uint32_t grid, uint32_t lds_bytes, void* stream) {
-  return launch_form(L, grid, L.form != kWholeTiles ? kShortThreads : kCopyThreads, lds_bytes, stream, [&](auto form) {
+  return launch_form(L, grid, copy_threads(L.form), lds_bytes, stream, [&](auto form) {
     return pick_cast_gather<typename decltype(form)::type>(s, d, L.policy, L.form);
   });
 }
 
 int launch_accum(int g, int a, bool store, const AccumLaunch& L, uint32_t grid, uint32_t lds_bytes, void* stream) {
-  const bool narrow = g != ODC_DTYPE_F32 && a != ODC_DTYPE_F32;
-  uint32_t threads = store ? kStoreThreads : kThreads;  // as pick_accum_form
-  if (narrow) threads = store || L.policy.read ? kThreads : kNarrowRmwThreads;
-  if (L.form != kWholeTiles) threads = kShortThreads;
-  return launch_form(L, grid, threads, lds_bytes, stream, [&](auto form) {
+  return launch_form(L, grid, accum_threads(g, a, store, L.policy, L.form), lds_bytes, stream, [&](auto form) {
     return pick_accum<typename decltype(form)::type>(g, a, store, L.policy, L.form);
   });
 }
@@ -983,7 +951,7 @@ int launch_clear(const ClearLaunch& L, uint32_t grid, void* stream) {
 }
 
 int launch_publish(int a, int o, const PublishLaunch& L, uint32_t grid, uint32_t lds_bytes, void* stream) {
-  return launch_form(L, grid, L.form != kWholeTiles ? kShortThreads : kThreads, lds_bytes, stream,
+  return launch_form(L, grid, publish_threads(L.form), lds_bytes, stream,
                      [&](auto form) { return pick_publish<typename decltype(form)::type>(a, o, L.form); });
 }
 

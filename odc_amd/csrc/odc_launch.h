@@ -18,6 +18,9 @@
 namespace odc_launch {
 
 using odc_tiles::kMaxItems;
+using odc_tiles::kShortTileVecs;
+using odc_tiles::kThreads;
+using odc_tiles::kTileVecs;
 using odc_tiles::TileTable;
 
 // Whether a launch leaves what it reads / what it writes in the caches (plain accesses) or streams
@@ -44,6 +47,48 @@ enum TileForm : uint32_t { kWholeTiles, kShortTiles, kFewShortTiles };
 constexpr bool accum_streams_short(int grad_dtype, int acc_dtype) {
   return grad_dtype != ODC_DTYPE_F32 && acc_dtype == ODC_DTYPE_F32;
 }
+
+// Workgroup shape of the two gathers and of the scatter-store (the kernels that read one stream
+// and write one) on whole tiles: 512 threads x 2 steps over the same 16 KiB tile as the 256 x 4 of
+// the other kernels. Four such workgroups fill a CU's wave slots, which is the residency these kernels
+// stream best at (measured: gathers +1.4..2.6 % over 256 x 4 with a residency cap of 4, which
+// had to be enforced by claiming LDS; 256 x 4 without a cap loses 6..8 %; 1024 x 1 loses
+// 20 %; short tiles lose 1 %). The read-modify-write with fp32 gradients keeps 256 x 4 (512 x 2:
+// equal on long segments), and so does the clear (512 x 2: -25 % on per-parameter spans).
+constexpr int kCopyThreads = 512;
+constexpr int kCopyUnroll = (int)kTileVecs / kCopyThreads;  // 2 for the 16 KiB tile
+constexpr int kStoreThreads = 512;
+constexpr int kStoreUnroll = (int)kTileVecs / kStoreThreads;
+static_assert(kCopyUnroll >= 1 && kStoreUnroll >= 1, "a tile holds at least one vector per thread");
+// 16-bit gradients into 16-bit accumulations have 8-byte vectors in both streams, half a tile's bytes,
+// and whole tiles take the other two shapes: the store 256 x 4 (64 KB of loads in flight per CU, as the
+// gathers have; 512 x 2 has half of that), the read-modify-write 512 x 2 where its gradient is streamed
+// (where the gradient is cached, up to 64 Mi elements, 256 x 4 is level or ahead). Graph-replayed launches, us, before ->
+// after, then 128 x 8 for both: a decoder layer's store at W = 8 174 -> 136, 138; at W = 64 167 -> 140, 143; 12 uneven
+// ranks 177 -> 141, 144; one of 525 M elements 326 -> 328, 333; 4 Mi 4.9 -> 4.5, 4.7; the layer's
+// read-modify-write at W = 8 209 -> 199, 210; at W = 64 218 -> 204.5, 218; 525 M elements 516 -> 489, 517. (Pairs
+// of vectors, 16 bytes per lane, in the old shapes: 213 and 178 for the layer at W = 8, 524 and 341 for 525 M.)
+constexpr int kNarrowRmwThreads = 512;
+constexpr int kNarrowRmwUnroll = (int)kTileVecs / kNarrowRmwThreads;
+// Shape for short tiles: two vectors per lane, and few enough threads that a segment of a few hundred elements does not hold the wave slots of a CU for nothing
+// (300 slices at W = 16, gather + accumulate: 31.9 us; 256 threads x 1: 40.1; 128 x 1 on eighths:
+// 35.2; 128 x 4 on halves: 33.1; whole tiles: 46.6).
+constexpr int kShortThreads = 128;
+constexpr int kShortUnroll = (int)kShortTileVecs / kShortThreads;
+
+// The workgroup sizes of the launches, as the pick_* functions of odc_kernels.hip take them.
+inline uint32_t copy_threads(TileForm form) { return form != kWholeTiles ? kShortThreads : kCopyThreads; }
+inline uint32_t publish_threads(TileForm form) { return form != kWholeTiles ? kShortThreads : kThreads; }
+inline uint32_t accum_threads(int grad_dtype, int acc_dtype, bool store, CachePolicy policy, TileForm form) {
+  if (form != kWholeTiles) return kShortThreads;
+  if (grad_dtype != ODC_DTYPE_F32 && acc_dtype != ODC_DTYPE_F32)
+    return store || policy.read ? kThreads : kNarrowRmwThreads;
+  return store ? kStoreThreads : kThreads;
+}
+
+// A dispatch counts its work-items in 32 bits. Launches of more tiles than that leaves workgroups for
+// (2^25 of 128 threads, 2^23 of 512) get the largest grid there is, which walks them.
+constexpr uint32_t most_workgroups(uint32_t threads) { return 0xffffffffu / threads; }
 
 // A launch carries up to kMaxItems items. One of a single item, a flat parameter on its own, goes out
 // in a form without the tables: 56 .. 72 bytes of arguments instead of 3 to 4 KB, which the host

@@ -17,6 +17,7 @@ TILE_ELEMS = 4096
 SHORT_TILE_BYTES = TILE_BYTES // 4
 SHORT_TILE_ELEMS = TILE_ELEMS // 4
 N_CU = 256  # what a dry-run arena assumes
+MOST_WORK_ITEMS = (1 << 32) - 1  # of one dispatch
 
 
 class DryArena:
@@ -223,7 +224,7 @@ def test_an_item_too_large_for_one_launch_is_refused_not_truncated(arena):
     _native.set_option("dry_run_reset", 0)
     items[0].shard_bytes = ((1 << 31) - 1) * TILE_BYTES
     _native.check(a.lib.odc_gather(a.handle, items, 1, 0, None))
-    assert a.counters() == (1, (1 << 31) - 1, (1 << 31) - 1)
+    assert a.counters() == (1, (1 << 31) - 1, MOST_WORK_ITEMS // 512)
 
 
 def test_many_large_items_split_when_the_tile_count_would_overflow(arena):
@@ -394,3 +395,46 @@ def test_16_bit_gradients_into_fp32_always_go_in_short_tiles(arena, grad):
             _native.check(call(a.handle, items, 1, grad, F32, None))
             tiles = W * math.ceil(n / SHORT_TILE_ELEMS)
             assert (a.counters(), a.forms()) == ((1, tiles, tiles), form)
+
+
+@pytest.mark.parametrize("call,grad,acc,tile,threads", [
+    ("odc_scatter_accumulate", BF16, F32, SHORT_TILE_ELEMS, 128), ("odc_scatter_store", F16, F32, SHORT_TILE_ELEMS, 128),
+    ("odc_scatter_accumulate", BF16, BF16, TILE_ELEMS, 512), ("odc_scatter_store", BF16, BF16, TILE_ELEMS, 256),
+    ("odc_scatter_accumulate", F32, F32, TILE_ELEMS, 256), ("odc_scatter_store", F32, F32, TILE_ELEMS, 512),
+])
+def test_a_grid_never_exceeds_the_work_items_of_a_dispatch(arena, call, grad, acc, tile, threads):
+    """Launches of more tiles than a dispatch has workgroups for are walked by the largest grid."""
+    W = 2
+    a = arena(W, 1 << 46)
+    most = MOST_WORK_ITEMS // threads
+    for tiles_per_rank in (most // W, most // W + 1, 1 << 28):
+        n, tiles = tiles_per_rank * tile, W * tiles_per_rank
+        for items in ([(0, n)], [(0, n - tile), (1 << 45, tile)]):  # one item, the same work in two
+            arr = (_native.AccumItem * len(items))(*[_native.AccumItem(FAR_OUTSIDE, W * m, off, m) for off, m in items])
+            _native.set_option("dry_run_reset", 0)
+            _native.check(getattr(a.lib, call)(a.handle, arr, len(arr), grad, acc, None))
+            assert a.counters() == (1, tiles, min(tiles, most))
+
+
+def test_grids_of_the_other_entry_points_are_bounded_too(arena):
+    a = arena(1, 1 << 46)
+    n = 1 << 28  # whole tiles
+    span = (_native.Span * 1)(_native.Span(0, n * TILE_BYTES))
+    _native.check(a.lib.odc_clear(a.handle, span, 1, None))
+    assert a.counters() == (1, n, MOST_WORK_ITEMS // 256)
+    for out, acc, tiles, threads in ((F32, F32, 4 * n, 128), (BF16, BF16, n, 256)):
+        pub = (_native.PublishItem * 1)(_native.PublishItem(0, n * TILE_ELEMS, FAR_OUTSIDE))
+        _native.set_option("dry_run_reset", 0)
+        _native.check(a.lib.odc_publish(a.handle, 0, pub, 1, acc, out, ctypes.c_float(3.0), None))
+        assert a.counters() == (1, tiles, MOST_WORK_ITEMS // threads)
+    cast = (_native.GatherCastItem * 1)(_native.GatherCastItem(FAR_OUTSIDE, 0, n * TILE_ELEMS))
+    _native.set_option("dry_run_reset", 0)
+    _native.check(a.lib.odc_gather_cast(a.handle, cast, 1, F32, BF16, 0, None))
+    assert a.counters() == (1, n, MOST_WORK_ITEMS // 512)
+    _native.set_option("gather_blocks_per_cu", 1 << 62)  # more workgroups than there are
+    try:
+        _native.set_option("dry_run_reset", 0)
+        _native.check(a.lib.odc_gather_cast(a.handle, cast, 1, F32, BF16, 0, None))
+        assert a.counters() == (1, n, MOST_WORK_ITEMS // 512)
+    finally:
+        _native.set_option("gather_blocks_per_cu", 0)
