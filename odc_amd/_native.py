@@ -12,6 +12,7 @@ import importlib.machinery
 import importlib.util
 import os
 import subprocess
+import sys
 import sysconfig
 import threading
 from pathlib import Path
@@ -173,51 +174,78 @@ def _with_languages(sources) -> list[str]:
     return args
 
 
-def _run_hipcc(cmd, verbose: bool) -> None:
-    proc = subprocess.run(cmd, capture_output=True, text=True)
-    if verbose or proc.returncode != 0:
-        print(" ".join(cmd))
-        print(proc.stdout)
-        print(proc.stderr)
-    if proc.returncode != 0:
-        raise RuntimeError(f"hipcc failed with exit code {proc.returncode}")
+def _compile(target: Path, command, verbose: bool) -> Path:
+    """Run ``command(output)`` and put what it made in ``target``'s place in one step: a process
+    that loads ``target`` meanwhile, or builds it too, never sees half a file."""
+    partial = target.with_name(f".{target.name}.{os.getpid()}.{threading.get_ident()}.partial")
+    cmd = command(partial)
+    try:
+        proc = subprocess.run(cmd, capture_output=True, text=True)
+        if verbose or proc.returncode != 0:
+            print(" ".join(cmd))
+            print(proc.stdout)
+            print(proc.stderr)
+        if proc.returncode != 0:
+            raise RuntimeError(f"building {target.name} failed: {cmd[0]} ended with exit code {proc.returncode}")
+        os.replace(partial, target)
+    finally:
+        partial.unlink(missing_ok=True)
+    return target
 
 
 def build_library(verbose: bool = False) -> Path:
     """Compile libodc_hip.so in-tree for gfx950 (works without a GPU)."""
-    _run_hipcc(hipcc_command(), verbose)
-    return LIB_PATH
+    return _compile(LIB_PATH, hipcc_command, verbose)
 
 
 def build_ceiling_library(verbose: bool = False) -> Path:
     """Compile libodc_ceiling.so (bench.py's bare streaming kernels) in-tree for gfx950."""
-    _run_hipcc(hipcc_command(CEILING_LIB_PATH, CEILING_SOURCES), verbose)
-    return CEILING_LIB_PATH
+    return _compile(CEILING_LIB_PATH, lambda output: hipcc_command(output, CEILING_SOURCES), verbose)
+
+
+def _torch_binding_target() -> str:
+    """What odc_torch.so is built for: it reads at::Tensor and CPython objects by their layout."""
+    import torch
+
+    return f"ABI {ABI_VERSION}, torch {torch.__version__}, CPython {sys.version_info.major}.{sys.version_info.minor}"
+
+
+def torch_binding_command(output: Path = TORCH_BINDING_PATH) -> list[str]:
+    import torch
+
+    root = Path(torch.__file__).resolve().parent
+    return [
+        os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
+        f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+        f'-DODC_TORCH_VERSION="{torch.__version__}"',
+        f"-I{INCLUDE_DIR}", f"-I{root / 'include'}", f"-I{root / 'include' / 'torch' / 'csrc' / 'api' / 'include'}",
+        f"-I{sysconfig.get_paths()['include']}", str(TORCH_BINDING_SOURCE), "-o", str(output),
+        f"-L{root / 'lib'}", "-ltorch_python", "-ltorch_cpu", "-lc10",
+    ]
 
 
 def build_torch_binding(verbose: bool = False) -> Path:
     """Compile odc_torch.so in-tree: host code only, against the torch that is importable here."""
-    import torch
-
-    root = Path(torch.__file__).resolve().parent
-    cmd = [
-        os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
-        f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
-        f"-I{INCLUDE_DIR}", f"-I{root / 'include'}", f"-I{root / 'include' / 'torch' / 'csrc' / 'api' / 'include'}",
-        f"-I{sysconfig.get_paths()['include']}", str(TORCH_BINDING_SOURCE), "-o", str(TORCH_BINDING_PATH),
-        f"-L{root / 'lib'}", "-ltorch_python", "-ltorch_cpu", "-lc10",
-    ]
-    proc = subprocess.run(cmd, capture_output=True, text=True)
-    if verbose or proc.returncode != 0:
-        print(" ".join(cmd))
-        print(proc.stdout)
-        print(proc.stderr)
-    if proc.returncode != 0:
-        raise RuntimeError(f"building {TORCH_BINDING_PATH.name} failed with exit code {proc.returncode}")
-    return TORCH_BINDING_PATH
+    return _compile(TORCH_BINDING_PATH, torch_binding_command, verbose)
 
 
+_REBUILD = "run `python -c 'import __graft_entry__ as g; g.build()'`"
 _torch_binding = None
+
+
+def _load_torch_binding_file(path: Path):
+    """The extension module at ``path``; ImportError when it was built for something else."""
+    loader = importlib.machinery.ExtensionFileLoader("odc_torch", str(path))
+    spec = importlib.util.spec_from_file_location("odc_torch", path, loader=loader)
+    try:
+        module = importlib.util.module_from_spec(spec)
+        loader.exec_module(module)
+    except ImportError as e:  # a symbol of another torch, or not a library at all
+        raise ImportError(f"{path} cannot be loaded ({e}): {_REBUILD}") from None
+    built_for, wanted = getattr(module, "built_for", "something older"), _torch_binding_target()
+    if built_for != wanted:
+        raise ImportError(f"{path} is stale: built for {built_for}, this is {wanted}: {_REBUILD}")
+    return module
 
 
 def load_torch_binding():
@@ -228,11 +256,11 @@ def load_torch_binding():
     with _lib_lock:
         if _torch_binding is None:
             if not TORCH_BINDING_PATH.exists():
-                build_torch_binding()
-            loader = importlib.machinery.ExtensionFileLoader("odc_torch", str(TORCH_BINDING_PATH))
-            spec = importlib.util.spec_from_file_location("odc_torch", TORCH_BINDING_PATH, loader=loader)
-            module = importlib.util.module_from_spec(spec)
-            loader.exec_module(module)
+                try:
+                    build_torch_binding()
+                except (OSError, RuntimeError) as e:
+                    raise ImportError(f"{TORCH_BINDING_PATH} is missing and could not be built ({e}): {_REBUILD}") from None
+            module = _load_torch_binding_file(TORCH_BINDING_PATH)
             entry_points = []
             for name in ("odc_gather", "odc_gather_cast", "odc_scatter_accumulate", "odc_scatter_store", "odc_clear",
                          "odc_publish", "odc_arena_locate", "odc_last_error"):
@@ -311,8 +339,7 @@ def load() -> ctypes.CDLL:
                     build_library()
                 except (OSError, RuntimeError) as e:
                     raise ImportError(
-                        f"{LIB_PATH} is missing and could not be built ({e}): run "
-                        "`python -c 'import __graft_entry__ as g; g.build()'` (needs hipcc)"
+                        f"{LIB_PATH} is missing and could not be built ({e}): {_REBUILD} (needs hipcc)"
                     ) from None
             # torch ships a HIP runtime of its own and must load it before this library pulls in
             # the system's by name: two HIP runtimes in one process do not both see the device

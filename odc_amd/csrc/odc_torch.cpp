@@ -2,7 +2,8 @@
 // reads tensors and Python lists, fills the item arrays and makes the call. A CPython extension
 // module (no pybind), plain C++ against torch's headers; it links no HIP code and no libodc_hip.so:
 // the entry points are bound by address (bind()), so that it always calls the library that
-// odc_amd/_native.py loaded.
+// odc_amd/_native.py loaded. It reads at::Tensor and CPython objects by their layout and fills the
+// structures of the C ABI, so it says what it was built for (built_for) and the loader compares.
 //
 // What bounds small calls is this path: a launch itself costs the host 2.5-3.5 us and the device
 // 2-3 us, while reading the tensors of a call attribute by attribute in Python took 3-5 us for one
@@ -23,6 +24,10 @@
 #include <vector>
 
 #include "odc_hip.h"
+
+#ifndef ODC_TORCH_VERSION
+#error "ODC_TORCH_VERSION: the torch.__version__ that this is compiled against"
+#endif
 
 namespace {
 
@@ -596,5 +601,14 @@ PyMODINIT_FUNC PyInit_odc_torch(void) {
   batch_type = reinterpret_cast<PyTypeObject*>(PyType_FromSpec(&batch_spec));
   slice_layout_type = reinterpret_cast<PyTypeObject*>(PyType_FromSpec(&slice_layout_spec));
   if (!batch_type || !slice_layout_type) return nullptr;
-  return PyModule_Create(&module_def);
+  PyObject* module = PyModule_Create(&module_def);
+#define ODC_TEXT_(x) #x
+#define ODC_TEXT(x) ODC_TEXT_(x)
+  if (module && PyModule_AddStringConstant(module, "built_for",
+                                           "ABI " ODC_TEXT(ODC_HIP_ABI_VERSION) ", torch " ODC_TORCH_VERSION
+                                           ", CPython " ODC_TEXT(PY_MAJOR_VERSION) "." ODC_TEXT(PY_MINOR_VERSION)) < 0) {
+    Py_DECREF(module);
+    return nullptr;
+  }
+  return module;
 }
