@@ -160,10 +160,9 @@ int dtype_code(at::ScalarType t) {
   }
 }
 
-int supported_dtype_code(at::ScalarType t) {
+int supported_dtype_code(const char* what, at::ScalarType t) {
   const int code = dtype_code(t);
-  if (code < 0)
-    raise(PyExc_TypeError, "scatter-accumulate supports bf16/fp16/fp32, not %s", at::toString(t));
+  if (code < 0) raise(PyExc_TypeError, "%s supports bf16/fp16/fp32, not %s", what, at::toString(t));
   return code;
 }
 
@@ -220,7 +219,7 @@ struct GatherCall {
                       offsetof(odc_gather_item, src_offset) == offsetof(odc_gather_cast_item, src_offset) &&
                       offsetof(odc_gather_item, shard_bytes) == offsetof(odc_gather_cast_item, shard_elems),
                   "one item array serves both gathers");
-    const int s = supported_dtype_code(src), d = supported_dtype_code(dst);
+    const int s = supported_dtype_code("a converting gather", src), d = supported_dtype_code("a converting gather", dst);
     const auto* items = reinterpret_cast<const odc_gather_cast_item*>(plain.data());
     int status;
     Py_BEGIN_ALLOW_THREADS
@@ -352,7 +351,7 @@ PyObject* accumulate_batch(PyObject*, PyObject* const* args, Py_ssize_t n) {
     std::vector<odc_accum_item>& items = *ref.b->items;
     items.reserve((size_t)keys.size());
     const at::ScalarType dtype = as_tensor(grads[0]).scalar_type();
-    ref.b->grad_code = supported_dtype_code(dtype);
+    ref.b->grad_code = supported_dtype_code("scatter-accumulate", dtype);
     for (Py_ssize_t k = 0; k < keys.size(); ++k) {
       PyObject* entry = PyDict_GetItemWithError(args[0], keys[k]);
       if (!entry) {
@@ -496,7 +495,7 @@ PyObject* slice_layout_batch(PyObject* self, PyObject* const* args, Py_ssize_t n
     ref.b->acc_code = acc.code;
     ref.b->items->reserve((size_t)grads.size());
     const at::ScalarType dtype = as_tensor(grads[0]).scalar_type();
-    ref.b->grad_code = supported_dtype_code(dtype);
+    ref.b->grad_code = supported_dtype_code("scatter-accumulate", dtype);
     for (Py_ssize_t k = 0; k < grads.size(); ++k) {
       const at::Tensor& grad = as_tensor(grads[k]);
       check_grad(grad, dtype);

@@ -432,21 +432,6 @@ class SymmBufferRegistry:
         """Symmetric byte offset of a registered buffer (what the kernels take)."""
         return self.offsets[key][0]
 
-    def symmetric_offset_of(self, tensor: torch.Tensor) -> int:
-        """Symmetric byte offset of ``tensor``, which must be (a contiguous view into) a
-        registered buffer of any rank. Exact buffer starts resolve through the data_ptr map
-        (``utils.py:158-161``); inner views through ``odc_arena_locate``."""
-        key = self.local_tensor_to_keys.get(tensor.data_ptr())
-        if key is not None:
-            return self.offsets[key][0]
-        if not tensor.is_cuda:
-            raise ValueError("tensor is not in the symmetric arena")
-        try:
-            _rank, off, inner = self.arena.locate(tensor.data_ptr())
-        except _native.OdcNativeError as e:
-            raise ValueError(f"tensor is not in the symmetric arena: {e.message}") from None
-        return off + inner
-
     def _forget(self):
         if self._arena is None and _world is not None:
             _world.renew_serial()

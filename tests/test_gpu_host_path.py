@@ -56,6 +56,8 @@ def test_refusals(make_world):
         gather.gather_into_tensor(full, torch.zeros(8, dtype=torch.bfloat16, device="cuda"), group)
     with pytest.raises(TypeError):
         gather.gather_into_tensors([None], [shard], group)
+    with pytest.raises(TypeError, match="gather supports bf16/fp16/fp32, not Double"):
+        gather.gather_into_tensor(full.double(), shard, group)
     red.register("k", (8,), torch.bfloat16, torch.float32, group)
     for grads, valid in (([full.cpu()], None), ([full[:-1]], None), ([full.view(2, -1)], None),
                          ([torch.cat([full, full])], None), ([full], [W * 8 + 1])):
