@@ -68,12 +68,12 @@ class GatherService:
         if stream is not None:
             if self._conversion is not None:
                 self._order_after_conversion(stream)
-            status = entry(world.handle, W, world.rank, stream, *call)
+            status = entry(world.arena.raw_handle, W, world.rank, stream, *call)
         else:
             with comm_stream_section("odc.gather") as comm:
                 if self._conversion is not None:
                     self._order_after_conversion(comm.cuda_stream)
-                status = entry(world.handle, W, world.rank, comm.cuda_stream, *call)
+                status = entry(world.arena.raw_handle, W, world.rank, comm.cuda_stream, *call)
         if status:
             _native.check(status)
 

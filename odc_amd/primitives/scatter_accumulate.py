@@ -206,11 +206,11 @@ class ReductionService:
         stream = plain_launch_stream(world)
         if stream is not None:
             self._order_after_writers(keys, stream)
-            status = _host_path.clear(world.handle, stream, table, keys)
+            status = _host_path.clear(world.arena.raw_handle, stream, table, keys)
         else:
             with comm_stream_section("odc.clear") as comm:
                 self._order_after_writers(keys, comm.cuda_stream)
-                status = _host_path.clear(world.handle, comm.cuda_stream, table, keys)
+                status = _host_path.clear(world.arena.raw_handle, comm.cuda_stream, table, keys)
         if status:
             _native.check(status)
 
@@ -326,11 +326,11 @@ class ReductionService:
         stream = plain_launch_stream(world)
         if stream is not None:
             self._order_after_writers(keys, stream)
-            status = items.launch(world.handle, stream, store)
+            status = items.launch(world.arena.raw_handle, stream, store)
         else:
             with comm_stream_section("odc.scatter_store" if store else "odc.scatter_accumulate") as comm:
                 self._order_after_writers(keys, comm.cuda_stream)
-                status = items.launch(world.handle, comm.cuda_stream, store)
+                status = items.launch(world.arena.raw_handle, comm.cuda_stream, store)
         if status:
             _native.check(status)
 
@@ -553,11 +553,11 @@ class ReductionService:
             stream = plain_launch_stream(world)
             if stream is not None:
                 self._order_after_writers(keys, stream)
-                status = _host_path.publish(world.handle, world.rank, stream, *call)
+                status = _host_path.publish(world.arena.raw_handle, world.rank, stream, *call)
             else:
                 with comm_stream_section("odc.publish") as comm:
                     self._order_after_writers(keys, comm.cuda_stream)
-                    status = _host_path.publish(world.handle, world.rank, comm.cuda_stream, *call)
+                    status = _host_path.publish(world.arena.raw_handle, world.rank, comm.cuda_stream, *call)
             if status:
                 _native.check(status)
         return results

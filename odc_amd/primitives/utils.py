@@ -91,6 +91,13 @@ class _ArenaMemory:
         }
 
 
+class _Finalized:
+    """The handle of an arena that is gone, for the calls made through odc_torch.cpp."""
+
+    def __index__(self):
+        raise RuntimeError("the symmetric arena has been finalized")
+
+
 class SymmetricArena:
     """Python handle of one ``odc_arena`` (include/odc_hip.h)."""
 
@@ -103,6 +110,7 @@ class SymmetricArena:
                 int(world_size), int(bytes_per_rank), flags, ctypes.byref(self._handle)
             )
         )
+        self.raw_handle = self._handle.value  # what odc_torch.cpp takes: the address, while there is one
         info = self.info()
         self.world_size = info.world_size
         self.bytes_per_rank = info.bytes_per_rank
@@ -175,6 +183,7 @@ class SymmetricArena:
     def destroy(self) -> None:
         if self._handle is not None and self._handle.value:
             self._bytes = None
+            self.raw_handle = _Finalized()
             handle, self._handle = self._handle, None
             _native.check(self._lib.odc_arena_destroy(handle))
 
@@ -186,7 +195,6 @@ class _VirtualWorld:
     def __init__(self, arena: SymmetricArena):
         self.renew_serial()
         self.arena = arena
-        self.handle = arena.handle.value  # the odc_arena, for the calls made through odc_torch.cpp
         self.device = arena.device
         self.world_size = arena.world_size
         self.rank = 0
