@@ -254,6 +254,22 @@ CachePolicy cache_policy(const odc_arena* a, const Options& opt, uint64_t read_b
 }
 constexpr int64_t kSymmetric = -1;  // a line: the stream lies in symmetric memory
 
+// The items that the next launch over [next, n_items) can take, and their whole tiles on one rank.
+struct LaunchSize {
+  uint32_t items = 0;
+  uint64_t tiles = 0;
+};
+template <class Units>
+LaunchSize launch_size(uint32_t n_items, uint32_t next, uint64_t tile_units, Units units) {
+  LaunchSize size;
+  for (uint32_t i = next; i < n_items && size.items < (uint32_t)kMaxItems; ++i) {
+    const uint64_t n = units(i);
+    size.tiles += tiles_for(n, tile_units);
+    size.items += n != 0;
+  }
+  return size;
+}
+
 // Whether the next launch over items [next, n_items) is cut into short tiles (256 vectors, done by
 // 128-thread workgroups): when its segments, one item on one rank, average fewer than `below` = 32
 // whole tiles. A workgroup of 256 or 512 threads whose segment holds a few hundred elements keeps the
@@ -267,14 +283,29 @@ constexpr int64_t kSymmetric = -1;  // a line: the stream lies in symmetric memo
 // Launches of longer segments stream best in whole tiles, with one exception (accum_streams_short).
 template <class Units>
 bool wants_short_tiles(uint32_t n_items, uint32_t next, uint64_t tile_units, Units units, int64_t below) {
-  uint64_t segments = 0, tiles = 0;
-  for (uint32_t i = next; i < n_items && segments < (uint64_t)kMaxItems; ++i) {
-    const uint64_t n = units(i);
-    if (n == 0) continue;
-    tiles += tiles_for(n, tile_units);
-    ++segments;
-  }
-  return tiles < (uint64_t)below * segments;
+  const LaunchSize size = launch_size(n_items, next, tile_units, units);
+  return size.tiles < (uint64_t)below * size.items;
+}
+
+// The same for an accumulate or a store. One that would take short tiles does not where 16-bit
+// gradients are stored into 16-bit accumulations and the launch has more than 1536 whole tiles: a short
+// tile of theirs moves 4 KB, too little for the cost of a workgroup once there are enough others.
+// Graph-replayed stores over 900 MB of buffers in turn, bf16 into bf16, us, short -> whole:
+//   W = 8, segments of 31 tiles: 9 items 9.8 -> 9.3, 30 items 24.8 -> 23.1, 60 items 49.7 -> 42.7; of 16 tiles: 30 items
+//     14.6 -> 13.6, 60 items 25.1 -> 23.4; of 8: 30 items (1920 tiles in all) 8.76 -> 8.45;
+//   W = 32, 9 items of 16 tiles 17.1 -> 16.3, 60 of 4 25.3 -> 23.9; the gradient nontemporal: 16.5 -> 15.2, 24.7 -> 22.8;
+//   960 tiles in all: 5.0 -> 4.9 .. 5.3, nontemporal 5.45 -> 5.8; 1152: 6.5 -> 6.25, nontemporal 6.1 -> 6.2; 576: 4.1 -> 4.3.
+// The read-modify-write of the same types has no such line: nontemporal short tiles are ahead or level
+// throughout (60 items of 16 tiles at W = 8 30.1, whole 33.5; 9 of 31 11.3 and 11.0), cached ones are
+// behind by up to 7 % at 4 to 17 Mi elements and ahead by as much at 57 Mi.
+template <class Units>
+bool scatter_in_short_tiles(const odc_arena* a, uint32_t n_items, uint32_t next, Units units, int64_t below, int grad_dtype,
+                            int acc_dtype, bool store) {
+  if (accum_streams_short(grad_dtype, acc_dtype)) return true;
+  const LaunchSize size = launch_size(n_items, next, kTileElems, units);
+  if (size.tiles >= (uint64_t)below * size.items) return false;
+  const bool narrow = grad_dtype != ODC_DTYPE_F32 && acc_dtype != ODC_DTYPE_F32;
+  return !(store && narrow) || size.tiles * a->world <= 1536;
 }
 
 // Whether a publish of items [next, n_items) is cut into short tiles. It sees a W-th of the elements
@@ -289,14 +320,7 @@ bool wants_short_tiles(uint32_t n_items, uint32_t next, uint64_t tile_units, Uni
 //   bf16 in place: 3.05 -> 2.7, 3.25 -> 3.05, 4.1 -> 3.0, 4.4 -> 4.2, but 19.5 -> 22.6, 134 -> 173, and 42.0 -> 41.4.
 template <class Units>
 bool publish_in_short_tiles(uint32_t n_items, uint32_t next, Units units, int acc_bytes) {
-  if (acc_bytes == 4) return true;
-  uint64_t tiles = 0;
-  uint32_t taken = 0;
-  for (uint32_t i = next; i < n_items && taken < (uint32_t)kMaxItems; ++i) {
-    tiles += tiles_for(units(i), kTileElems);
-    taken += units(i) != 0;
-  }
-  return tiles <= 1024;
+  return acc_bytes == 4 || launch_size(n_items, next, kTileElems, units).tiles <= 1024;
 }
 
 // How the workgroups of a launch find their items. Up to eight fills of the chip (4096 workgroups of
@@ -855,8 +879,7 @@ int scatter_launch(odc_arena* a, const odc_accum_item* items, uint32_t n_items, 
     L.tt.order = (uint32_t)opt.rank_major;
     L.tt.first_rank = 0;
     const auto units = [&](uint32_t i) { return items[order[i]].shard_elems; };
-    const bool short_tiles = odc_launch::accum_streams_short(grad_dtype, acc_dtype) ||
-                             wants_short_tiles(n_items, next, kTileElems, units, opt.short_tiles_below);
+    const bool short_tiles = scatter_in_short_tiles(a, n_items, next, units, opt.short_tiles_below, grad_dtype, acc_dtype, store);
     const int n = fill_launch(
         L.tt, a->world, n_items, &next, tile_units(kTileElems, short_tiles), units,
         [&](uint32_t slot, uint32_t i) {

@@ -438,3 +438,20 @@ def test_grids_of_the_other_entry_points_are_bounded_too(arena):
         assert a.counters() == (1, n, MOST_WORK_ITEMS // 512)
     finally:
         _native.set_option("gather_blocks_per_cu", 0)
+
+
+@pytest.mark.parametrize("grad,acc", [(BF16, BF16), (F16, BF16), (F16, F16)])
+def test_long_stores_of_16_bit_types_stay_in_whole_tiles(arena, grad, acc):
+    """Up to 1536 whole tiles in the launch a store of short segments goes in short tiles; the
+    read-modify-write always does."""
+    W = 4
+    a = arena(W, 1 << 36)
+    for sizes, store_form in (([24 * 4096] * 16, (0, 0, 1)), ([24 * 4096] * 15 + [24 * 4096 + 1], (1, 0, 0)), ([4096] * 112, (0, 0, 1))):
+        items, off = (_native.AccumItem * len(sizes))(), 0
+        for k, n in enumerate(sizes):
+            items[k] = _native.AccumItem(OUTSIDE, W * n, off, n)
+            off += 4 * n + 256
+        for call, form in ((a.lib.odc_scatter_store, store_form), (a.lib.odc_scatter_accumulate, (0, 0, 1))):
+            _native.set_option("dry_run_reset", 0)
+            _native.check(call(a.handle, items, len(items), grad, acc, None))
+            assert a.forms() == form
