@@ -75,6 +75,7 @@ struct Options {
   int64_t alloc_align = 16384;        // so do symmetric allocations at least this large
   int64_t cached_arena_bytes = 192ll << 20;   // see cache_policy
   int64_t cached_output_bytes = 64ll << 20;
+  int64_t plain_output_bytes = 24ll << 20;    // see output_form
   int64_t cached_gradient_bytes = 128ll << 20;
   int64_t short_tiles_below = 32;             // see wants_short_tiles
   int64_t few_tiles = 32768;                  // see tile_form
@@ -104,6 +105,7 @@ int64_t* option_slot(const char* name) {
   if (!strcmp(name, "publish_resident_cap")) return &g_opt.publish_resident_cap;
   if (!strcmp(name, "cached_arena_bytes")) return &g_opt.cached_arena_bytes;
   if (!strcmp(name, "cached_output_bytes")) return &g_opt.cached_output_bytes;
+  if (!strcmp(name, "plain_output_bytes")) return &g_opt.plain_output_bytes;
   if (!strcmp(name, "cached_gradient_bytes")) return &g_opt.cached_gradient_bytes;
   if (!strcmp(name, "short_tiles_below")) return &g_opt.short_tiles_below;
   if (!strcmp(name, "few_tiles")) return &g_opt.few_tiles;
@@ -236,6 +238,10 @@ uint32_t grid_for(const odc_arena* a, int64_t blocks_per_cu, uint32_t n_tiles, u
 //   * the gathers' output, read by the forward or backward just after: gather + read 20.3 -> 18.7 /
 //     19.2 -> 17.5, still 64.7 -> 62.3 at 64 Mi elements, but the gather alone is then 42.1 -> 45.8
 //     (22.1 -> 19.1 at 32 Mi): the line is 64 MiB of output.
+//     What reads it in earnest are products: of a decoder layer's step (gather, forward products, gather,
+//     backward products, accumulate) the cached output takes 234 -> 213 at 14 MiB and 512 tokens, 592 ->
+//     565 at 35 MiB and 2048, 762 -> 713 at 59 MiB and 2048, 1535 -> 1511 at 8192. It costs where nothing reads it: a
+//     gather and accumulate of 17 MiB 21.0 -> 24.0, of 48 MiB 40.4 -> 41.7 (written through, 41.1: output_form).
 //   * shards and accumulations come back only in the next microbatch, so what counts is whether ALL
 //     symmetric memory in use stays in the cache from one to the next: with 72 MB of it (4 Mi
 //     elements, 3 sets) fill + accumulate 12.7 -> 10.8 and accumulate alone 8.9 -> 7.9, with 144 MB
@@ -253,6 +259,17 @@ CachePolicy cache_policy(const odc_arena* a, const Options& opt, uint64_t read_b
   return p;
 }
 constexpr int64_t kSymmetric = -1;  // a line: the stream lies in symmetric memory
+
+// How a gather writes an output that stays in the caches. Up to what the L2s hold (8 x 4 MB) plain
+// stores leave it there for the reader; beyond that it is written through to the last-level cache (store_output
+// in odc_kernels.hip has the figures). Below the line of 24 MiB plain stores are ahead: passes of gather
+// and accumulate over three sets of buffers in turn, us, plain -> written through: 18 MiB of output at W = 16 41.2 -> 42.1,
+// 20 MiB at W = 8 41.0 -> 42.0; above it 29 MiB 61.2 -> 60.4, 34 MiB 98.7 -> 95.9, 42 MiB at W = 32
+// 130.7 -> 125.0, 48 MiB 47.8 -> 45.6 (nontemporal stores: 57.9, 97.0, 124.5, 43.0).
+OutputForm output_form(const Options& opt, bool cached, uint64_t bytes) {
+  if (!cached) return kStream;
+  return bytes <= (uint64_t)opt.plain_output_bytes ? kKeep : kWriteThrough;
+}
 
 // The items that the next launch over [next, n_items) can take, and their whole tiles on one rank.
 struct LaunchSize {
@@ -676,6 +693,7 @@ int odc_gather(odc_arena* a, const odc_gather_item* items, uint32_t n_items, uin
     uint64_t shard_bytes = 0;
     for (uint32_t k = 0; k < L.tt.n_items; ++k) shard_bytes += L.item[k].seg_bytes;
     L.policy = cache_policy(a, opt, 0, kSymmetric, shard_bytes * a->world, opt.cached_output_bytes);
+    L.output = output_form(opt, L.policy.written, shard_bytes * a->world);
     for (uint32_t k = 0; k < L.tt.n_items; ++k)
       ragged |= (((uintptr_t)L.item[k].dst | L.item[k].src_off | L.item[k].seg_bytes) & 15u) != 0;
     const uint32_t grid = grid_for(a, opt.gather_blocks_per_cu, L.tt.n_tiles, copy_threads(L.form), ragged);

@@ -79,6 +79,24 @@ __device__ __forceinline__ void store_vec(V* p, V v) {  // aligned
   if constexpr (kCached) *p = v; else __builtin_nontemporal_store(v, p);
 }
 
+// A whole tile of a gather's output: vector `i` of the kVecs that start at `tile`, an address that all
+// lanes agree on. Outputs that the next kernel is to find in the last-level cache, but that are more
+// than the L2s hold, are written through the L2: left in it by plain stores they went to memory only as other
+// lines pushed them out, between the reads of whatever ran next. us, nontemporal / plain / written
+// through (a decoder layer's nine parameters, bf16, W = 8, three sets of buffers in turn):
+//   gather alone: 35 MiB of output 14.4 / 15.7 / 13.2, 48 MiB 18.6 / 16.7 / 15.4;
+//   an accumulate behind it, nothing reads the output: 32.1 / 31.9 / 29.4, 40.4 / 41.7 / 41.1;
+//   the products that read the parameters behind it (1024 tokens): 141 / 129 / 126.5, 184 / 160 / 158.5.
+constexpr int kSc1 = 16;  // of a buffer store: write through
+template <OutputForm kForm, uint32_t kVecs>
+__device__ __forceinline__ void store_output(u32x4* tile, uint32_t i, u32x4 v) {
+  if constexpr (kForm == kWriteThrough)
+    __builtin_amdgcn_raw_buffer_store_b128(v, __builtin_amdgcn_make_buffer_rsrc(tile, 0, kVecs * 16, 0x00027000),
+                                           (int)(i * 16), 0, kSc1);
+  else
+    store_vec<kForm == kKeep>(tile + i, v);
+}
+
 // An address in device memory. Of an address that comes as an argument of a function, or as a number,
 // the compiler must assume that it may lie in LDS or scratch, and it takes the slower flat accesses.
 template <class P>
@@ -223,7 +241,7 @@ __device__ __attribute__((noinline)) void gather_edges(uint8_t* d, const uint8_t
 
 // T threads do a tile of T * U vectors in one step; the copies stream best from 512-thread
 // workgroups, of which 4 fit a CU.
-template <class Launch, bool kSrcCached, bool kDstCached, bool kFew, int T, int U>
+template <class Launch, bool kSrcCached, OutputForm kDst, bool kFew, int T, int U>
 __global__ __launch_bounds__(T) void gather_kernel(const Launch launch) {
   constexpr uint32_t kVecs = T * U;
   static_assert(kVecs == kTileVecs || kVecs == kShortTileVecs, "a whole tile or a short one");
@@ -240,7 +258,7 @@ __global__ __launch_bounds__(T) void gather_kernel(const Launch launch) {
     const TileWork w = tile_work<kVecs>(c.chunk, g);
     if (is_whole<kVecs>(w)) {
       const uint8_t* sb = s + g.head + (w.v0 + tid) * 16;
-      u32x4* db = reinterpret_cast<u32x4*>(d + g.head) + w.v0 + tid;
+      u32x4* db = reinterpret_cast<u32x4*>(d + g.head) + w.v0;
       u32x4 v[U];
 #pragma unroll
       for (int u = 0; u < U; ++u) v[u] = load_any<kSrcCached, u32x4>(sb + (size_t)u * T * 16);
@@ -253,11 +271,11 @@ __global__ __launch_bounds__(T) void gather_kernel(const Launch launch) {
       if (do_head) head_byte = s[tid];
       if (do_tail) tail_byte = s[tail_at];
 #pragma unroll
-      for (int u = 0; u < U; ++u) store_vec<kDstCached>(db + u * T, v[u]);
+      for (int u = 0; u < U; ++u) store_output<kDst, kVecs>(db, u * T + tid, v[u]);
       if (do_head) d[tid] = head_byte;
       if (do_tail) d[tail_at] = tail_byte;
     } else if (has_edges<kVecs>(w)) {
-      gather_edges<kSrcCached, kDstCached, T, U>(d, s, c.chunk, g);
+      gather_edges<kSrcCached, kDst != kStream, T, U>(d, s, c.chunk, g);
     }
   }
 }
@@ -793,18 +811,22 @@ kernel_fn<L> pick_accum(int g, int a, bool store, CachePolicy policy, TileForm f
   return nullptr;
 }
 
-template <class L, bool kSrcCached, bool kDstCached>
+template <class L, bool kSrcCached, OutputForm kDst>
 kernel_fn<L> pick_gather_form(TileForm form) {
-  if (form == kFewShortTiles) return gather_kernel<L, kSrcCached, kDstCached, kSearches<L>, kShortThreads, kShortUnroll>;
-  if (form == kShortTiles) return gather_kernel<L, kSrcCached, kDstCached, false, kShortThreads, kShortUnroll>;
-  return gather_kernel<L, kSrcCached, kDstCached, false, kCopyThreads, kCopyUnroll>;
+  if (form == kFewShortTiles) return gather_kernel<L, kSrcCached, kDst, kSearches<L>, kShortThreads, kShortUnroll>;
+  if (form == kShortTiles) return gather_kernel<L, kSrcCached, kDst, false, kShortThreads, kShortUnroll>;
+  return gather_kernel<L, kSrcCached, kDst, false, kCopyThreads, kCopyUnroll>;
+}
+
+template <class L, bool kSrcCached>
+kernel_fn<L> pick_gather_output(OutputForm output, TileForm form) {
+  if (output == kStream) return pick_gather_form<L, kSrcCached, kStream>(form);
+  return output == kKeep ? pick_gather_form<L, kSrcCached, kKeep>(form) : pick_gather_form<L, kSrcCached, kWriteThrough>(form);
 }
 
 template <class L>
-kernel_fn<L> pick_gather(CachePolicy policy, TileForm form) {
-  if (policy.read)
-    return policy.written ? pick_gather_form<L, true, true>(form) : pick_gather_form<L, true, false>(form);
-  return policy.written ? pick_gather_form<L, false, true>(form) : pick_gather_form<L, false, false>(form);
+kernel_fn<L> pick_gather(bool shards_cached, OutputForm output, TileForm form) {
+  return shards_cached ? pick_gather_output<L, true>(output, form) : pick_gather_output<L, false>(output, form);
 }
 
 // Shards and output of the converting gather are cached together or not at all.
@@ -929,7 +951,7 @@ bool has_publish(int a, int o) { return pick_publish<PublishLaunch>(a, o, kShort
 
 int launch_gather(const GatherLaunch& L, uint32_t grid, uint32_t lds_bytes, void* stream) {
   return launch_form(L, grid, copy_threads(L.form), lds_bytes, stream, [&](auto form) {
-    return pick_gather<typename decltype(form)::type>(L.policy, L.form);
+    return pick_gather<typename decltype(form)::type>(L.policy.read, L.output, L.form);
   });
 }
 

@@ -25,11 +25,16 @@ using odc_tiles::TileTable;
 
 // Whether a launch leaves what it reads / what it writes in the caches (plain accesses) or streams
 // past them (nontemporal ones). For the accumulate "read" is the gradient and "written" the
-// accumulation, read and written; for the gathers they are the shards and the output.
+// accumulation, read and written; for the gathers they are the shards and the output (OutputForm for
+// the plain gather's).
 struct CachePolicy {
   bool read = false;
   bool written = false;
 };
+
+// How a gather writes its output: past the caches, through the L2 into the last-level cache, or with
+// plain stores (store_output in odc_kernels.hip, output_form in odc_host.cpp).
+enum OutputForm : uint32_t { kStream, kWriteThrough, kKeep };
 
 // How a launch is cut, and how its workgroups find their items (wants_short_tiles and tile_form in
 // odc_host.cpp).
@@ -114,7 +119,8 @@ struct GatherLaunch {
   TileTable tt;
   uint8_t* base;  // arena base (rank 0 region)
   uint64_t rank_stride;
-  CachePolicy policy;    // these two pick the kernel
+  CachePolicy policy;    // these three pick the kernel
+  OutputForm output = kStream;
   TileForm form = kWholeTiles;
   GatherDesc item[kMaxItems];
 };
