@@ -241,6 +241,10 @@ const char* odc_last_error(void);
 int odc_abi_version(void);
 
 /* Launch-shape knobs, for measurement.
+ * The work of a launch is cut into tiles (1024 vectors of 16 bytes of output, or 4096 elements), done by
+ * workgroups of 256 or 512 threads, or into short tiles, a quarter of that, done by 128 threads. Knobs that
+ * count workgroups count those of the launch: for short tiles, which 16-bit gradients into fp32 always
+ * take, one persistent workgroup per CU is two wavefronts. Thresholds in tiles mean whole ones.
  *  - "gather_blocks_per_cu", "accum_blocks_per_cu", "store_blocks_per_cu", "clear_blocks_per_cu",
  *    "publish_blocks_per_cu": persistent workgroups per CU walking the tiles with a grid-stride
  *    loop; 0 = one workgroup per tile, dealt out by the hardware dispatcher. accum_blocks_per_cu
@@ -256,6 +260,14 @@ int odc_abi_version(void);
  *    tiles and 1 otherwise.
  *  - "accum_small_items_last" (default 1): scatter-accumulate and scatter-store launch the items
  *    of less than one tile per rank after the others; 0 keeps the caller's order.
+ *  - "short_tiles_below" (default 32): launches whose segments average fewer whole tiles are cut into
+ *    short ones (0: none but those that always are). "few_tiles" (32768): up to so many short tiles
+ *    a workgroup reads the whole table of the launch's items at once instead of searching it.
+ *  - what a launch leaves in the caches: gathers of at most "cached_output_bytes" (64 MiB) of output
+ *    leave it there, with plain stores up to "plain_output_bytes" (24 MiB) and written through the L2
+ *    above; gradients of at most "cached_gradient_bytes" (128 MiB) per launch are read through the
+ *    caches; so are shards and accumulations while all symmetric memory in use, over all ranks, is at most
+ *    "cached_arena_bytes" (192 MiB). 0 streams past the caches.
  *  - "rank_stagger_bytes" (extra distance between rank regions), "rank_stride_align" (rank regions
  *    start on multiples of it, default 16384 = one tile) and "alloc_align" (allocations of at
  *    least this many bytes start on multiples of it, default 16384; smaller ones on 256): read

@@ -5,7 +5,8 @@
 // against an odc_device that has no device, this file runs under AddressSanitizer and UBSan on
 // bookkeeping-only and dry-run arenas.
 //
-// Launch model: the work of one launch is cut into tiles of 1024 vectors (16 KiB, odc_tiles.h);
+// Launch model: the work of one launch is cut into tiles of 1024 vectors (16 KiB, odc_tiles.h), or of
+// 256 (scatter_in_short_tiles, wants_short_tiles, publish_in_short_tiles);
 // per-item descriptors (<= ODC_MAX_ITEMS_PER_LAUNCH) travel BY VALUE in the kernel argument
 // segment, so a call needs no device-side work list, no host->device copy and no allocation;
 // longer item lists are split over several launches.
@@ -64,7 +65,7 @@ struct Options {
   int64_t accum_persistent_below_tiles = 0;  // segments averaging fewer tiles: persistent launch shape (0: never)
   int64_t accum_small_items_last = 1;  // scatter launches: items of less than one tile per rank go last
   int64_t store_blocks_per_cu = 0;  // the scatter-store (no read of the accumulation)
-  int64_t store_resident_cap = 0;  // 512-thread workgroups, like the gathers
+  int64_t store_resident_cap = 0;
   int64_t clear_blocks_per_cu = 0;
   int64_t publish_blocks_per_cu = 0;
   int64_t publish_resident_cap = 0;
@@ -73,7 +74,7 @@ struct Options {
   int64_t rank_stagger_bytes = 0;
   int64_t rank_stride_align = 16384;  // rank regions start on multiples of this (read when an arena is created)
   int64_t alloc_align = 16384;        // so do symmetric allocations at least this large
-  int64_t cached_arena_bytes = 192ll << 20;   // see cache_policy
+  int64_t cached_arena_bytes = 192ll << 20;   // these and the next two: see cache_policy
   int64_t cached_output_bytes = 64ll << 20;
   int64_t plain_output_bytes = 24ll << 20;    // see output_form
   int64_t cached_gradient_bytes = 128ll << 20;
@@ -219,7 +220,8 @@ Options options_snapshot() {
 // blocks_per_cu > 0 asks for that many persistent workgroups per CU. Ragged launches (uneven
 // shards: unaligned reads, heads and tails) never get them: they hide their extra latency better
 // with one workgroup per tile, i.e. full occupancy (measured: +5..10 %).
-uint32_t grid_for(const odc_arena* a, int64_t blocks_per_cu, uint32_t n_tiles, uint32_t threads, bool ragged = false) {
+uint32_t grid_for(const odc_arena* a, int64_t blocks_per_cu, uint32_t n_tiles, uint32_t threads,
+                  bool ragged = false) {
   const uint32_t most = std::min(n_tiles, most_workgroups(threads));
   if (blocks_per_cu <= 0 || ragged) return most;
   const uint64_t cu = (uint64_t)a->n_cu, per_cu = (uint64_t)blocks_per_cu;
@@ -240,8 +242,9 @@ uint32_t grid_for(const odc_arena* a, int64_t blocks_per_cu, uint32_t n_tiles, u
 //     (22.1 -> 19.1 at 32 Mi): the line is 64 MiB of output.
 //     What reads it in earnest are products: of a decoder layer's step (gather, forward products, gather,
 //     backward products, accumulate) the cached output takes 234 -> 213 at 14 MiB and 512 tokens, 592 ->
-//     565 at 35 MiB and 2048, 762 -> 713 at 59 MiB and 2048, 1535 -> 1511 at 8192. It costs where nothing reads it: a
-//     gather and accumulate of 17 MiB 21.0 -> 24.0, of 48 MiB 40.4 -> 41.7 (written through, 41.1: output_form).
+//     565 at 35 MiB and 2048, 762 -> 713 at 59 MiB and 2048, 1535 -> 1511 at 8192. It costs where
+//     nothing reads it: a gather and accumulate of 17 MiB 21.0 -> 24.0, of 48 MiB 40.4 -> 41.7 (written
+//     through, 41.1: output_form).
 //   * shards and accumulations come back only in the next microbatch, so what counts is whether ALL
 //     symmetric memory in use stays in the cache from one to the next: with 72 MB of it (4 Mi
 //     elements, 3 sets) fill + accumulate 12.7 -> 10.8 and accumulate alone 8.9 -> 7.9, with 144 MB
@@ -261,11 +264,12 @@ CachePolicy cache_policy(const odc_arena* a, const Options& opt, uint64_t read_b
 constexpr int64_t kSymmetric = -1;  // a line: the stream lies in symmetric memory
 
 // How a gather writes an output that stays in the caches. Up to what the L2s hold (8 x 4 MB) plain
-// stores leave it there for the reader; beyond that it is written through to the last-level cache (store_output
-// in odc_kernels.hip has the figures). Below the line of 24 MiB plain stores are ahead: passes of gather
-// and accumulate over three sets of buffers in turn, us, plain -> written through: 18 MiB of output at W = 16 41.2 -> 42.1,
-// 20 MiB at W = 8 41.0 -> 42.0; above it 29 MiB 61.2 -> 60.4, 34 MiB 98.7 -> 95.9, 42 MiB at W = 32
-// 130.7 -> 125.0, 48 MiB 47.8 -> 45.6 (nontemporal stores: 57.9, 97.0, 124.5, 43.0).
+// stores leave it there for the reader; beyond that it is written through to the last-level cache
+// (store_output in odc_kernels.hip has the figures). Below the line of 24 MiB plain stores are ahead:
+// passes of gather and accumulate over three sets of buffers in turn, us, plain -> written through: 18
+// MiB of output at W = 16 41.2 -> 42.1, 20 MiB at W = 8 41.0 -> 42.0; above it 29 MiB 61.2 -> 60.4, 34
+// MiB 98.7 -> 95.9, 42 MiB at W = 32 130.7 -> 125.0, 48 MiB 47.8 -> 45.6 (nontemporal stores: 57.9,
+// 97.0, 124.5, 43.0).
 OutputForm output_form(const Options& opt, bool cached, uint64_t bytes) {
   if (!cached) return kStream;
   return bytes <= (uint64_t)opt.plain_output_bytes ? kKeep : kWriteThrough;
@@ -308,16 +312,17 @@ bool wants_short_tiles(uint32_t n_items, uint32_t next, uint64_t tile_units, Uni
 // gradients are stored into 16-bit accumulations and the launch has more than 1536 whole tiles: a short
 // tile of theirs moves 4 KB, too little for the cost of a workgroup once there are enough others.
 // Graph-replayed stores over 900 MB of buffers in turn, bf16 into bf16, us, short -> whole:
-//   W = 8, segments of 31 tiles: 9 items 9.8 -> 9.3, 30 items 24.8 -> 23.1, 60 items 49.7 -> 42.7; of 16 tiles: 30 items
-//     14.6 -> 13.6, 60 items 25.1 -> 23.4; of 8: 30 items (1920 tiles in all) 8.76 -> 8.45;
-//   W = 32, 9 items of 16 tiles 17.1 -> 16.3, 60 of 4 25.3 -> 23.9; the gradient nontemporal: 16.5 -> 15.2, 24.7 -> 22.8;
-//   960 tiles in all: 5.0 -> 4.9 .. 5.3, nontemporal 5.45 -> 5.8; 1152: 6.5 -> 6.25, nontemporal 6.1 -> 6.2; 576: 4.1 -> 4.3.
+//   W = 8, segments of 31 tiles: 9 items 9.8 -> 9.3, 30 items 24.8 -> 23.1, 60 items 49.7 -> 42.7;
+//   of 16 tiles: 30 items 14.6 -> 13.6, 60 items 25.1 -> 23.4; of 8: 30 items (1920 tiles) 8.76 -> 8.45;
+//   W = 32: 9 items of 16 tiles 17.1 -> 16.3, 60 of 4 25.3 -> 23.9, nontemporal 16.5 -> 15.2, 24.7 -> 22.8;
+//   1152 tiles in all: 6.5 -> 6.25, nontemporal 6.1 -> 6.2; 960: 5.0 -> 4.9 .. 5.3, nontemporal 5.45 ->
+//   5.8; 576: 4.1 -> 4.3.
 // The read-modify-write of the same types has no such line: nontemporal short tiles are ahead or level
 // throughout (60 items of 16 tiles at W = 8 30.1, whole 33.5; 9 of 31 11.3 and 11.0), cached ones are
 // behind by up to 7 % at 4 to 17 Mi elements and ahead by as much at 57 Mi.
 template <class Units>
-bool scatter_in_short_tiles(const odc_arena* a, uint32_t n_items, uint32_t next, Units units, int64_t below, int grad_dtype,
-                            int acc_dtype, bool store) {
+bool scatter_in_short_tiles(const odc_arena* a, uint32_t n_items, uint32_t next, Units units, int64_t below,
+                            int grad_dtype, int acc_dtype, bool store) {
   if (accum_streams_short(grad_dtype, acc_dtype)) return true;
   const LaunchSize size = launch_size(n_items, next, kTileElems, units);
   if (size.tiles >= (uint64_t)below * size.items) return false;
@@ -331,10 +336,13 @@ bool scatter_in_short_tiles(const odc_arena* a, uint32_t n_items, uint32_t next,
 // fp32 accumulations always are. 16-bit ones move 4 to 6 KB per short tile, too little for the cost of
 // a workgroup, and are only up to 1024 whole tiles (4 workgroups per CU). Graph-replayed
 // launches over buffers in turn, us, whole -> short:
-//   fp32 into bf16: ten slices of 98 816 elements 3.5 -> 2.9, one of 1 Mi 4.2 -> 3.65, 112 of 3 640 5.2 -> 3.65, one of
-//     3.1 M 9.65 -> 7.1, a decoder layer's 27 M at W = 8 45.8 -> 44.0, eight layers 369 -> 335, one of 66 M 108.7 -> 103.4;
-//   fp32 in place: 3.2 -> 2.65, 3.8 -> 3.35, 4.35 -> 3.3, 7.65 -> 6.1, 35.8 -> 34.5, 284 -> 267, 81.2 -> 82.0;
-//   bf16 in place: 3.05 -> 2.7, 3.25 -> 3.05, 4.1 -> 3.0, 4.4 -> 4.2, but 19.5 -> 22.6, 134 -> 173, and 42.0 -> 41.4.
+//   fp32 into bf16: ten slices of 98 816 elements 3.5 -> 2.9, one of 1 Mi 4.2 -> 3.65, 112 of 3 640
+//     5.2 -> 3.65, one of 3.1 M 9.65 -> 7.1, a decoder layer's 27 M at W = 8 45.8 -> 44.0, eight layers
+//     369 -> 335, one of 66 M 108.7 -> 103.4;
+//   fp32 in place: 3.2 -> 2.65, 3.8 -> 3.35, 4.35 -> 3.3, 7.65 -> 6.1, 35.8 -> 34.5, 284 -> 267,
+//     81.2 -> 82.0;
+//   bf16 in place: 3.05 -> 2.7, 3.25 -> 3.05, 4.1 -> 3.0, 4.4 -> 4.2, but 19.5 -> 22.6, 134 -> 173,
+//     and 42.0 -> 41.4.
 template <class Units>
 bool publish_in_short_tiles(uint32_t n_items, uint32_t next, Units units, int acc_bytes) {
   return acc_bytes == 4 || launch_size(n_items, next, kTileElems, units).tiles <= 1024;
@@ -346,7 +354,8 @@ bool publish_in_short_tiles(uint32_t n_items, uint32_t next, Units units, int ac
 // latency and the extra loads only cost. Graph-replayed gather + accumulate of one group of slices,
 // us, binary search -> table read at once:
 //   300 of 64 .. 65 536 elements: W = 4 27.4 -> 23.2, W = 8 28.6 -> 24.3, W = 64 55.6 -> 45.0;
-//   112 of 4096: 6.0 -> 5.1, 6.3 -> 5.7, 17.8 -> 13.5; 10 of 256 .. 262 144: 6.1 -> 5.9, 6.5 -> 6.2, 7.2 -> 6.9;
+//   112 of 4096: 6.0 -> 5.1, 6.3 -> 5.7, 17.8 -> 13.5;
+//   10 of 256 .. 262 144: 6.1 -> 5.9, 6.5 -> 6.2, 7.2 -> 6.9;
 //   112 of 160 000 (17 900 tiles): 41.2 -> 39.7, 41.1 -> 40.2; 112 of 640 000 (70 000 tiles): 156 -> 159,
 //   159 -> 162; 60 of 900 000 (53 000 tiles): 115 -> 115, 116.5 -> 117.6.
 TileForm tile_form(bool short_tiles, uint32_t n_tiles, int64_t few) {
@@ -712,7 +721,8 @@ int odc_gather_cast(odc_arena* a, const odc_gather_cast_item* items, uint32_t n_
     return fail(ODC_ERR_INVALID, "first_rank %u >= world size %u", first_rank, a->world);
   const int sb = dtype_bytes(src_dtype), db = dtype_bytes(dst_dtype);
   if (!sb || !db) return fail(ODC_ERR_INVALID, "unknown dtype code (src %d, dst %d)", src_dtype, dst_dtype);
-  if (!odc_device::has_cast_gather(src_dtype, dst_dtype)) return fail(ODC_ERR_UNSUPPORTED, "gather from dtype %d into dtype %d is not implemented", src_dtype, dst_dtype);
+  if (!odc_device::has_cast_gather(src_dtype, dst_dtype))
+    return fail(ODC_ERR_UNSUPPORTED, "gather from dtype %d into dtype %d is not implemented", src_dtype, dst_dtype);
   for (uint32_t i = 0; i < n_items; ++i) {
     const odc_gather_cast_item& it = items[i];
     if (it.shard_elems == 0) continue;
@@ -897,7 +907,8 @@ int scatter_launch(odc_arena* a, const odc_accum_item* items, uint32_t n_items, 
     L.tt.order = (uint32_t)opt.rank_major;
     L.tt.first_rank = 0;
     const auto units = [&](uint32_t i) { return items[order[i]].shard_elems; };
-    const bool short_tiles = scatter_in_short_tiles(a, n_items, next, units, opt.short_tiles_below, grad_dtype, acc_dtype, store);
+    const bool short_tiles = scatter_in_short_tiles(a, n_items, next, units, opt.short_tiles_below, grad_dtype,
+                                                    acc_dtype, store);
     const int n = fill_launch(
         L.tt, a->world, n_items, &next, tile_units(kTileElems, short_tiles), units,
         [&](uint32_t slot, uint32_t i) {
@@ -976,7 +987,8 @@ int odc_publish(odc_arena* a, uint32_t rank, const odc_publish_item* items, uint
   const int ab = dtype_bytes(acc_dtype), ob = dtype_bytes(out_dtype);
   if (!ab || !ob) return fail(ODC_ERR_INVALID, "unknown dtype code (acc %d, out %d)", acc_dtype, out_dtype);
   if (!(divisor == divisor) || divisor == 0.0f) return fail(ODC_ERR_INVALID, "divisor must be a non-zero number");
-  if (!odc_device::has_publish(acc_dtype, out_dtype)) return fail(ODC_ERR_UNSUPPORTED, "publish from dtype %d into dtype %d is not implemented", acc_dtype, out_dtype);
+  if (!odc_device::has_publish(acc_dtype, out_dtype))
+    return fail(ODC_ERR_UNSUPPORTED, "publish from dtype %d into dtype %d is not implemented", acc_dtype, out_dtype);
   uint8_t* region = a->origin + (uint64_t)rank * a->rank_stride;
   for (uint32_t i = 0; i < n_items; ++i) {
     const odc_publish_item& it = items[i];

@@ -12,7 +12,7 @@
 //   publish_kernel      : one rank's acc /= divisor, plus a cast copy (end of a minibatch)
 //
 // Launch model shared by the kernels: the work of one launch is cut into tiles of 1024 vectors
-// (16 KiB), done by workgroups of 256 threads (512 for the two gathers), or into short tiles of 256
+// (16 KiB), done by workgroups of 256 threads or 512 (odc_launch.h says which), or into short tiles of 256
 // vectors, done by 128 threads: launches of short segments (wants_short_tiles in odc_host.cpp) and
 // every accumulate and store of 16-bit gradients into fp32 (accum_streams_short in odc_launch.h), and
 // every publish of fp32 accumulations (publish_in_short_tiles in odc_host.cpp).
@@ -162,8 +162,9 @@ struct SingleWalk {
   __device__ __forceinline__ TileCoord locate(const SingleLaunch<D>&, uint32_t t) const { return single_item_coord(tt, t); }
 };
 // Few short tiles of several items (tile_form in odc_host.cpp): again a chain of latencies, the binary
-// search being most of it. The whole prefix table is read together with the header instead, one entry per lane (two for its second
-// half), and the item found by counting the entries that are not greater than the tile's position:
+// search being most of it. The whole prefix table is read together with the header instead, one entry
+// per lane (two for its second half), and the item found by counting the entries that are not greater
+// than the tile's position:
 // two round trips to the item in place of up to nine.
 template <class Launch>
 struct FewTilesWalk {
@@ -821,7 +822,8 @@ kernel_fn<L> pick_gather_form(TileForm form) {
 template <class L, bool kSrcCached>
 kernel_fn<L> pick_gather_output(OutputForm output, TileForm form) {
   if (output == kStream) return pick_gather_form<L, kSrcCached, kStream>(form);
-  return output == kKeep ? pick_gather_form<L, kSrcCached, kKeep>(form) : pick_gather_form<L, kSrcCached, kWriteThrough>(form);
+  if (output == kKeep) return pick_gather_form<L, kSrcCached, kKeep>(form);
+  return pick_gather_form<L, kSrcCached, kWriteThrough>(form);
 }
 
 template <class L>

@@ -48,7 +48,10 @@ enum TileForm : uint32_t { kWholeTiles, kShortTiles, kFewShortTiles };
 // 373 -> 352 at W = 64, 374 -> 370 at W = 128; a 525 M element embedding 863 -> 852; the store
 // 206 -> 198 at W = 8, 209 -> 205 at W = 64. (128 x 1: 386, 64 x 2: 371, 64 x 4: 348 and 357 at
 // W = 64, 128 x 4: 349 and 372, 256 x 1: 367, 256 x 2: 360.) fp32 gradients move the same bytes per
-// lane in both streams and keep 256 x 4 (421; 128 x 2: 429), and so do 16-bit accumulations.
+// lane in both streams and keep 256 x 4 (421; 128 x 2: 429); 16-bit accumulations have the shapes of
+// kNarrowRmwThreads below. Where rank segments start on no line boundary neighbouring tiles share a
+// line of gradient, and a short one holds a quarter of a whole one's: 1.4 % instead of 0.5 % more traffic
+// over 40 uneven parameters at W = 12, in 619 us instead of 631.
 constexpr bool accum_streams_short(int grad_dtype, int acc_dtype) {
   return grad_dtype != ODC_DTYPE_F32 && acc_dtype == ODC_DTYPE_F32;
 }
@@ -68,16 +71,17 @@ static_assert(kCopyUnroll >= 1 && kStoreUnroll >= 1, "a tile holds at least one 
 // 16-bit gradients into 16-bit accumulations have 8-byte vectors in both streams, half a tile's bytes,
 // and whole tiles take the other two shapes: the store 256 x 4 (64 KB of loads in flight per CU, as the
 // gathers have; 512 x 2 has half of that), the read-modify-write 512 x 2 where its gradient is streamed
-// (where the gradient is cached, up to 64 Mi elements, 256 x 4 is level or ahead). Graph-replayed launches, us, before ->
-// after, then 128 x 8 for both: a decoder layer's store at W = 8 174 -> 136, 138; at W = 64 167 -> 140, 143; 12 uneven
-// ranks 177 -> 141, 144; one of 525 M elements 326 -> 328, 333; 4 Mi 4.9 -> 4.5, 4.7; the layer's
-// read-modify-write at W = 8 209 -> 199, 210; at W = 64 218 -> 204.5, 218; 525 M elements 516 -> 489, 517. (Pairs
-// of vectors, 16 bytes per lane, in the old shapes: 213 and 178 for the layer at W = 8, 524 and 341 for 525 M.)
+// (where the gradient is cached, up to 64 Mi elements, 256 x 4 is level or ahead). Graph-replayed
+// launches, us, before -> after, then 128 x 8 for both: a decoder layer's store at W = 8 174 -> 136, 138;
+// at W = 64 167 -> 140, 143; 12 uneven ranks 177 -> 141, 144; one of 525 M elements 326 -> 328, 333;
+// 4 Mi 4.9 -> 4.5, 4.7; the layer's read-modify-write at W = 8 209 -> 199, 210; at W = 64 218 -> 204.5,
+// 218; 525 M elements 516 -> 489, 517. (Pairs of vectors, 16 bytes per lane, in the old shapes: 213 and
+// 178 for the layer at W = 8, 524 and 341 for 525 M.)
 constexpr int kNarrowRmwThreads = 512;
 constexpr int kNarrowRmwUnroll = (int)kTileVecs / kNarrowRmwThreads;
-// Shape for short tiles: two vectors per lane, and few enough threads that a segment of a few hundred elements does not hold the wave slots of a CU for nothing
-// (300 slices at W = 16, gather + accumulate: 31.9 us; 256 threads x 1: 40.1; 128 x 1 on eighths:
-// 35.2; 128 x 4 on halves: 33.1; whole tiles: 46.6).
+// Shape for short tiles: two vectors per lane, and few enough threads that a segment of a few hundred
+// elements does not hold the wave slots of a CU for nothing (300 slices at W = 16, gather + accumulate:
+// 31.9 us; 256 threads x 1: 40.1; 128 x 1 on eighths: 35.2; 128 x 4 on halves: 33.1; whole tiles: 46.6).
 constexpr int kShortThreads = 128;
 constexpr int kShortUnroll = (int)kShortTileVecs / kShortThreads;
 
@@ -96,7 +100,7 @@ inline uint32_t accum_threads(int grad_dtype, int acc_dtype, bool store, CachePo
 constexpr uint32_t most_workgroups(uint32_t threads) { return 0xffffffffu / threads; }
 
 // A launch carries up to kMaxItems items. One of a single item, a flat parameter on its own, goes out
-// in a form without the tables: 56 .. 72 bytes of arguments instead of 3 to 4 KB, which the host
+// in a form without the tables: 56 to 80 bytes of arguments instead of 2.3 to 4 KB, which the host
 // hands over in 2.6 us instead of 4.0 (512 bytes: 3.4), and all of it is read at once instead of
 // along the item search (SingleWalk in odc_kernels.hip).
 template <class D>
@@ -191,6 +195,7 @@ struct PublishLaunch {  // one rank's region only: tt.world == 1
 struct PublishSingle : SingleLaunch<PublishDesc> {
   PublishScale scale;
 };
+static_assert(sizeof(SingleLaunch<ClearDesc>) == 56 && sizeof(PublishSingle) == 80, "as SingleLaunch says");
 static_assert(sizeof(GatherLaunch) <= 4096 && sizeof(AccumLaunch) <= 4096 && sizeof(PublishLaunch) <= 4096 &&
                   sizeof(CastGatherLaunch) <= 4096 && sizeof(ClearLaunch) <= 4096,
               "launch descriptors must fit the kernel-argument segment");

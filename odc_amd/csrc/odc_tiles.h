@@ -6,8 +6,8 @@
 //
 // Vocabulary. A launch carries up to kMaxItems ITEMS (one shard of one tensor). An item has one
 // SEGMENT per rank: `n` units (bytes or elements) at the same symmetric offset of every rank
-// region. A segment is cut into TILES of kTileVecs vectors; a 256-thread workgroup does one tile
-// at a time.
+// region. A segment is cut into TILES of kTileVecs vectors (or of kShortTileVecs, a launch of short
+// ones); a workgroup of 128, 256 or 512 threads does one tile at a time.
 #ifndef ODC_TILES_H_
 #define ODC_TILES_H_
 
@@ -41,7 +41,8 @@ constexpr uint32_t kTileVecs = kThreads * kUnroll;  // vectors per tile
 constexpr uint32_t kTileBytes = kTileVecs * 16;     // gather / clear: 16 KiB of destination
 constexpr uint32_t kTileElems = kTileVecs * 4;      // accumulate / cast / publish: 4096 elements
 constexpr uint64_t kMaxTilesPerLaunch = 1ull << 31;
-// Launches of short segments are cut finer: into quarters of a tile (see short_tiles in odc_host.cpp).
+// Launches of short segments are cut finer: into quarters of a tile (wants_short_tiles and its
+// neighbours in odc_host.cpp).
 constexpr uint32_t kShortTileParts = 4;
 constexpr uint32_t kShortTileVecs = kTileVecs / kShortTileParts;
 

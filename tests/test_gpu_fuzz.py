@@ -118,6 +118,12 @@ KNOBS = [
     {"accum_blocks_per_cu": 1, "accum_resident_cap": 4},
     {"accum_persistent_below_tiles": 1 << 30, "accum_short_segment_tiles": 0},
     {"accum_persistent_below_tiles": 0, "accum_short_segment_tiles": 1 << 30},
+    # how launches are cut, with the tiles walked by few workgroups too, and what they leave in the caches
+    {"short_tiles_below": 0, "accum_small_items_last": 0},
+    {"short_tiles_below": 1 << 30, "few_tiles": 0, "gather_blocks_per_cu": 1, "accum_blocks_per_cu": 1},
+    {"short_tiles_below": 1 << 30, "few_tiles": 1 << 30, "store_blocks_per_cu": 1, "publish_blocks_per_cu": 1},
+    {"cached_output_bytes": 0, "cached_gradient_bytes": 0, "cached_arena_bytes": 0},
+    {"cached_output_bytes": 1 << 40, "plain_output_bytes": 0, "cached_gradient_bytes": 1 << 40, "cached_arena_bytes": 1 << 40},
     # arena layout (read when the world is created): packed buffers and staggered, unaligned rank
     # regions; coarse alignment
     {"alloc_align": 256, "rank_stride_align": 256, "rank_stagger_bytes": 4352},
@@ -135,7 +141,8 @@ def test_results_do_not_depend_on_launch_knobs(make_world, knobs):
     names = ["gather_blocks_per_cu", "accum_blocks_per_cu", "store_blocks_per_cu", "clear_blocks_per_cu",
              "publish_blocks_per_cu", "gather_resident_cap", "cast_resident_cap", "accum_resident_cap",
              "store_resident_cap", "rank_major", "accum_tile_order", "accum_persistent_below_tiles",
-             "accum_short_segment_tiles", "alloc_align", "rank_stride_align", "rank_stagger_bytes"]
+             "accum_short_segment_tiles", "accum_small_items_last", "short_tiles_below", "few_tiles",
+             "cached_output_bytes", "plain_output_bytes", "cached_gradient_bytes", "cached_arena_bytes", "alloc_align", "rank_stride_align", "rank_stagger_bytes"]
     saved = {n: _native.get_option(n) for n in names}
     try:
         for name, value in knobs.items():
