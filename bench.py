@@ -82,12 +82,13 @@ def parse_args():
                          "timed scatter-accumulate is the 10N read-modify-write")
     ap.add_argument("--calibrate", action="store_true",
                     help="also run one torch copy of 1 GiB (counter calibration under rocprofv3)")
-    ap.add_argument("--probe", choices=["alignment", "overlap", "tiny-items"],
-                    help="instead of the benchmark, print one of three measurement tables: alignment (what a buffer "
+    ap.add_argument("--probe", choices=["alignment", "overlap", "tiny-items", "launch-forms"],
+                    help="instead of the benchmark, print one of four measurement tables: alignment (what a buffer "
                          "shifted off the 16 KiB tile grid costs the scatter-accumulate and the gather), overlap (how "
                          "much of a gather / scatter-accumulate hides behind a co-running GEMM, by launch shape), "
                          "tiny-items (what items of less than one tile per rank cost the scatter-accumulate by their "
-                         "place in the launch order; run it with --world-size 64)")
+                         "place in the launch order; run it with --world-size 64), launch-forms (smaller decoder "
+                         "layers by what their launches leave in the caches and by the tiles they are cut into)")
     ap.add_argument("--option", action="append", default=[], metavar="NAME=VALUE",
                     help="libodc_hip launch knob, e.g. accum_blocks_per_cu=4")
     return ap.parse_args()
@@ -581,7 +582,8 @@ def probe_tiny_items(args, launches=40):
     """`--probe tiny-items`: the 9-parameter layer's scatter-accumulate, launched back to back, with
     its two norm items (64 elements per rank at W=64: less than one tile) where the caller lists
     them (between the projection matrices), launched last (the library's default), and left out;
-    one workgroup per tile and one persistent workgroup per CU; rank-outermost and item-major."""
+    one workgroup per tile and 16 persistent workgroups per CU (as many of 128 threads as fit);
+    rank-outermost and item-major."""
     import torch
 
     import odc_amd as odc
@@ -620,7 +622,7 @@ def probe_tiny_items(args, launches=40):
             for last in ((0, 1) if len(keys) == 9 else (1,)):
                 for order, order_name in ((2, "rank-outermost"), (1, "item-major")):
                     row = []
-                    for blocks_per_cu in (0, 1):
+                    for blocks_per_cu in (0, 16):
                         _native.set_option("accum_small_items_last", last)
                         _native.set_option("accum_tile_order", order)
                         _native.set_option("accum_blocks_per_cu", blocks_per_cu)
@@ -634,6 +636,103 @@ def probe_tiny_items(args, launches=40):
     torch.cuda.synchronize()
     odc.SymmBufferRegistry.get_instance().finalize()
     odc.finalize_distributed()
+
+
+def probe_launch_forms(args, tokens=1024, replays=7):
+    """`--probe launch-forms`: the rules that choose how a launch is cut into tiles and what it leaves
+    in the caches, each against its alternatives. The nine parameters of decoder layers of several
+    widths, bf16, three or more sets of buffers in turn (so that only what the caches can hold from one
+    launch to the next is found there), replayed from HIP graphs; microseconds per pass, median."""
+    import torch
+
+    import odc_amd as odc
+    from odc_amd import _native
+    from odc_amd.workloads import numel
+
+    W = args.world_size
+    torch.cuda.set_device(0)
+    torch.manual_seed(0)
+    far, names = 1 << 40, ("plain_output_bytes", "cached_output_bytes", "cached_gradient_bytes", "short_tiles_below")
+    defaults = {name: _native.get_option(name) for name in names}
+    outputs = {"streamed": {"cached_output_bytes": 0}, "written through": {"cached_output_bytes": far, "plain_output_bytes": 0},
+               "plain": {"cached_output_bytes": far, "plain_output_bytes": far}, "by rule": {}}
+    gradients = {"streamed": {"cached_gradient_bytes": 0}, "cached": {"cached_gradient_bytes": far}, "by rule": {}}
+    tiles = {"whole tiles": {"short_tiles_below": 0}, "short tiles": {"short_tiles_below": far}, "by rule": {}}
+
+    def timed(step, sets, options):
+        for name, value in {**defaults, **options}.items():
+            _native.set_option(name, value)
+        step(sets[0])
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            for _ in range(2):
+                for s in sets:
+                    step(s)
+        start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        times = []
+        for _ in range(replays):
+            graph.replay()  # leaves the caches as a long run of this form does
+            start.record()
+            graph.replay()
+            end.record()
+            end.synchronize()
+            times.append(start.elapsed_time(end) * 1e3 / (2 * len(sets)))
+        return statistics.median(times)
+
+    print(f"decoder layers at W={W}, microseconds per pass")
+    for hidden in (512, 1024, 1536, 2048):
+        ffn, kv = 2560 * hidden // 1024, hidden // 4
+        shapes = [(hidden,), (hidden, hidden), (kv, hidden), (kv, hidden), (hidden, hidden), (hidden,), (ffn, hidden),
+                  (ffn, hidden), (hidden, ffn)]
+        numels = [numel(s) for s in shapes]
+        nbytes = 2 * sum(numels)
+        n_sets = max(3, min(16, (1 << 30) // (5 * nbytes)))
+        group = odc.init_nvshmem(world_size=W, symmetric_size=n_sets * sum(n // W * 8 + 3 * 16384 for n in numels) + (8 << 20))
+        registry, gather = odc.SymmBufferRegistry.get_instance(), odc.GatherService()
+        wide = odc.ReductionService(accumulation_dtype=torch.float32)
+        narrow = odc.ReductionService(accumulation_dtype=torch.bfloat16)
+        sets = []
+        for k in range(n_sets):
+            s = {"source": [registry.allocate_symm_buffer(("p", k, i), (n // W,), torch.bfloat16) for i, n in enumerate(numels)],
+                 "out": [torch.empty(shape, dtype=torch.bfloat16, device="cuda") for shape in shapes],
+                 "grad": [torch.empty(n, dtype=torch.bfloat16, device="cuda").normal_(0, 1e-3) for n in numels],
+                 "keys": [(k, i) for i in range(len(numels))]}
+            s["flat"] = [o.view(-1) for o in s["out"]]
+            for i, n in enumerate(numels):
+                for service, kind, dtype in ((wide, "w", torch.float32), (narrow, "n", torch.bfloat16)):
+                    service.register((kind, k, i), (n // W,), torch.bfloat16, dtype, group)
+            sets.append(s)
+        x = {d: torch.randn(tokens, d, device="cuda").bfloat16() for d in {hidden, ffn, kv}}
+        y = {d: torch.empty(tokens, d, dtype=torch.bfloat16, device="cuda") for d in x}
+
+        def gathered(s):
+            gather.gather_into_tensors(s["flat"], s["source"], group)
+
+        def accumulated(s, service=wide, kind="w"):
+            service.scatter_accumulate_multi([(kind, *key) for key in s["keys"]], s["grad"], group)
+
+        def products(s):
+            for o in s["out"]:
+                if o.dim() == 2:
+                    torch.mm(x[o.shape[0]], o, out=y[o.shape[1]])
+
+        print(f"hidden {hidden}: {nbytes / 2**20:.0f} MiB of parameters, {n_sets} sets of buffers")
+        table = [("gather", gathered, outputs, "output"), ("gather, accumulate", lambda s: (gathered(s), accumulated(s)), outputs, "output"),
+                 (f"gather, products of {tokens} tokens", lambda s: (gathered(s), products(s)), outputs, "output"),
+                 ("accumulate, bf16 into fp32", accumulated, gradients, "gradient"),
+                 ("accumulate, bf16 into bf16", lambda s: accumulated(s, narrow, "n"), gradients, "gradient"),
+                 ("gather", gathered, tiles, "tiles"),
+                 ("accumulate, bf16 into bf16", lambda s: accumulated(s, narrow, "n"), tiles, "tiles")]
+        for label, step, arms, what in table:
+            figures = ", ".join(f"{name} {timed(step, sets, options):.1f}" for name, options in arms.items())
+            print(f"  {label + ' (' + what + ')':44s} {figures}", flush=True)
+        for name, value in defaults.items():
+            _native.set_option(name, value)
+        del sets
+        torch.cuda.synchronize()
+        registry.finalize()
+        odc.finalize_distributed()
 
 
 def probe_overlap(args, gemm=8192, launches=8, repeats=5):
@@ -719,9 +818,9 @@ def probe_overlap(args, gemm=8192, launches=8, repeats=5):
     _native.set_option("gather_resident_cap", 0)
     report("scatter-accumulate, one workgroup per tile, no cap (default)", run_accum,
            {"accum_blocks_per_cu": 0, "accum_resident_cap": 0})
-    report("scatter-accumulate, one workgroup per tile, <= 4 resident per CU", run_accum,
-           {"accum_blocks_per_cu": 0, "accum_resident_cap": 4})
-    report("scatter-accumulate, 1 persistent workgroup per CU", run_accum, {"accum_blocks_per_cu": 1})
+    report("scatter-accumulate, one workgroup per tile, <= 8 resident per CU", run_accum,
+           {"accum_blocks_per_cu": 0, "accum_resident_cap": 8})
+    report("scatter-accumulate, 16 persistent workgroups per CU", run_accum, {"accum_blocks_per_cu": 16})
     _native.set_option("accum_blocks_per_cu", -1)
     _native.set_option("accum_resident_cap", 0)
     torch.cuda.synchronize()
@@ -736,7 +835,8 @@ def main():
               "second GPU. Run with --gpus 1.", file=sys.stderr)
         sys.exit(2)
     if args.probe:
-        return {"alignment": probe_alignment, "overlap": probe_overlap, "tiny-items": probe_tiny_items}[args.probe](args)
+        return {"alignment": probe_alignment, "overlap": probe_overlap, "tiny-items": probe_tiny_items,
+                "launch-forms": probe_launch_forms}[args.probe](args)
     if args.workload == "model":
         return model_sweep(args)
 

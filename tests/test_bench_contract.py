@@ -33,7 +33,10 @@ def test_a_launcher_that_sets_world_size_is_refused_too():
 
 def test_the_committed_traffic_table_is_what_the_bench_line_cites():
     """profiles/traffic.json: every entry names the summary it comes from, that summary exists,
-    and the HBM bytes per launch are within 1 % of the algorithmic bytes (no wasted traffic)."""
+    and the HBM bytes per launch are within 1 % of the algorithmic bytes (no wasted traffic). Segments
+    that start on no 128-byte line add to that in the accumulate and the store of the uneven workload: a
+    short tile reads 2048 bytes of gradient and shares a line with the next, at most 128 / 2048 of the
+    gradient's 2 of 10 bytes per element (1.25 %) and of its 2 of 6 (2.1 %)."""
     table = json.loads((ROOT / "profiles" / "traffic.json").read_text())
     assert table["entries"]
     seen = set()
@@ -42,7 +45,8 @@ def test_the_committed_traffic_table_is_what_the_bench_line_cites():
         key = (e["workload"], e["layout"], e["world_size"], e["kernel"], e.get("unit_shape"))
         assert key not in seen, f"duplicate entry {key}"
         seen.add(key)
-        assert 0.99 < e["hbm_bytes_per_launch"] / e["algorithmic_bytes"] < 1.01, key
+        shared = {"accum": 0.0125, "store": 0.021}.get(e["kernel"], 0) if e["workload"] == "uneven" else 0
+        assert 0.99 < e["hbm_bytes_per_launch"] / e["algorithmic_bytes"] < 1.01 + shared, key
     assert ("layer", "per-param", 8, "accum", None) in seen
     assert ("model", "per-param", 8, "accum", "embedding") in seen
 
@@ -51,5 +55,5 @@ def test_the_committed_traffic_table_is_what_the_bench_line_cites():
 def test_help_lists_the_workloads_and_probes(flag):
     proc = run_bench(flag)
     assert proc.returncode == 0
-    for word in ("--workload", "model", "uneven", "--probe", "tiny-items", "--lazy-clear", "--no-graph"):
+    for word in ("--workload", "model", "uneven", "--probe", "tiny-items", "launch-forms", "--lazy-clear", "--no-graph"):
         assert word in proc.stdout
