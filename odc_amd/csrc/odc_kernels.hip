@@ -18,8 +18,8 @@
 // every publish of fp32 accumulations (publish_in_short_tiles in odc_host.cpp).
 // Workgroups walk the tiles with a grid-stride loop, by default one workgroup per tile, so that,
 // at any instant, the whole chip streams one compact window of memory. Per-item
-// descriptors (<= ODC_MAX_ITEMS_PER_LAUNCH) travel BY VALUE in the kernel argument segment and
-// are read with scalar loads, so a call needs no device-side work list, no host->device copy and
+// descriptors (<= ODC_MAX_ITEMS_PER_LAUNCH; launches of one item and of up to 16 have smaller tables) travel
+// BY VALUE in the kernel argument segment and are read with scalar loads, so a call needs no device-side work list, no host->device copy and
 // no allocation; longer item lists are split over several launches.
 //
 // Each wavefront issues its 2 or 4 independent 128-bit loads per stream before the first store.
@@ -34,6 +34,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <iterator>
 #include <type_traits>
 
 #include "odc_hip.h"
@@ -49,6 +51,7 @@ using namespace odc_tiles;
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x16 __attribute__((ext_vector_type(16)));
 
 using namespace odc_launch;
 
@@ -109,6 +112,7 @@ __device__ __forceinline__ P* as_global(P* p) {
 template <class Launch>
 struct TableWalk {
   typedef typename Launch::Desc Desc;
+  static constexpr bool kOneTile = false;
   TileCursor cur;
   Desc it = {};  // the item of the tile located last
 
@@ -117,6 +121,7 @@ struct TableWalk {
   __device__ __forceinline__ uint8_t* region(const Launch& launch, uint32_t rank) const {
     return launch.base + (uint64_t)rank * launch.rank_stride;
   }
+  template <uint32_t>
   __device__ __forceinline__ TileCoord locate(const Launch& launch, uint32_t t) {
     if (!cursor_holds(cur, t)) {
       cursor_seek(launch.tt, t, cur);
@@ -135,6 +140,7 @@ struct TableWalk {
 template <class D>
 struct SingleWalk {
   typedef D Desc;
+  static constexpr bool kOneTile = true;
   TileHead tt;
   uint8_t* base;
   uint64_t rank_stride;
@@ -149,16 +155,16 @@ struct SingleWalk {
 #pragma unroll
     for (int i = 0; i < kWords; ++i) w[i] = reinterpret_cast<const uint64_t*>(launch.item)[i];
     // (left alone, the compiler reads each value where it is first used)
-    asm volatile("" : "+s"(tt.world), "+s"(tt.n_tiles), "+s"(tt.order), "+s"(tt.first_rank), "+s"(tt.tiles_per_rank),
+    asm volatile("" : "+s"(tt.world), "+s"(tt.order), "+s"(tt.first_rank), "+s"(tt.tiles_per_rank),
                       "+s"(b), "+s"(stride), "+s"(w[0]), "+s"(w[1]), "+s"(w[2]), "+s"(w[3]));
     base = as_global(reinterpret_cast<uint8_t*>((uintptr_t)b));
     rank_stride = stride;
     __builtin_memcpy(&it, w, sizeof(D));
   }
-  __device__ __forceinline__ uint32_t n_tiles(const SingleLaunch<D>&) const { return tt.n_tiles; }
   __device__ __forceinline__ uint8_t* region(const SingleLaunch<D>&, uint32_t rank) const {
     return base + (uint64_t)rank * rank_stride;
   }
+  template <uint32_t>
   __device__ __forceinline__ TileCoord locate(const SingleLaunch<D>&, uint32_t t) const { return single_item_coord(tt, t); }
 };
 // Few short tiles of several items (tile_form in odc_host.cpp): again a chain of latencies, the binary
@@ -169,6 +175,7 @@ struct SingleWalk {
 template <class Launch>
 struct FewTilesWalk {
   typedef typename Launch::Desc Desc;
+  static constexpr bool kOneTile = false;
   TileHead tt;
   uint8_t* base;
   uint64_t rank_stride;
@@ -192,6 +199,7 @@ struct FewTilesWalk {
   __device__ __forceinline__ uint8_t* region(const Launch&, uint32_t rank) const {
     return base + (uint64_t)rank * rank_stride;
   }
+  template <uint32_t>
   __device__ __forceinline__ TileCoord locate(const Launch& launch, uint32_t t) {
     if (!cursor_holds(cur, t)) {
       const uint32_t x = cursor_position(tt, t, cur);
@@ -204,9 +212,62 @@ struct FewTilesWalk {
   }
 };
 
-template <class Launch, bool kFew = false>
-using TileWalk = std::conditional_t<!std::is_same_v<decltype(Launch::tt), TileTable>, SingleWalk<typename Launch::Desc>,
-                                    std::conditional_t<kFew, FewTilesWalk<Launch>, TableWalk<Launch>>>;
+// 2 to kFewItems items, one workgroup per tile, tiles of any size. From its arguments to its first load a
+// workgroup went through eight dependent round trips (two for the header, the binary search, the item) and
+// some 350 scalar instructions, about 1 us of which every short launch is made and which the rest of a
+// long one has to hide. Here header and table are read at once, into scalar registers, the item is found
+// by counting there, and the tiles of a rank segment follow from its size: two round trips and some 200
+// instructions, with one division instead of three and no loop around the tile. Graph-replayed launches of
+// nine items at W = 8, us, gather / accumulate / publish of bf16 into fp32 by elements per rank and item:
+// 4096 2.49 / 2.72 / 2.55 -> 2.43 / 2.70 / 2.36, 30 000 3.59 / 4.47 / 2.71 -> 3.38 / 4.42 / 2.60, 300 000
+// 13.5 / 31.9 / 5.8 -> 13.0 / 30.2 / 5.75, 3 M (HBM bound) level; converting gather 30 000 4.36 -> 4.05.
+template <class Launch>
+struct FewItemsWalk {
+  typedef typename Launch::Desc Desc;
+  static constexpr bool kOneTile = true;
+  TileHead tt;
+  uint8_t* base;
+  uint64_t rank_stride;
+  Desc it = {};
+  u32x16 before;
+
+  __device__ __forceinline__ explicit FewItemsWalk(const Launch& launch) {
+    static_assert(kFewItems == 16, "one scalar load");
+    __builtin_memcpy(&before, launch.tt.tiles_before, sizeof(before));
+    tt = launch.tt;
+    uint64_t b = (uint64_t)(uintptr_t)launch.base, stride = launch.rank_stride;
+    asm volatile("" : "+s"(tt.world), "+s"(tt.order), "+s"(tt.first_rank), "+s"(tt.tiles_per_rank), "+s"(b), "+s"(stride),
+                      "+s"(before));
+    base = as_global(reinterpret_cast<uint8_t*>((uintptr_t)b));
+    rank_stride = stride;
+  }
+  __device__ __forceinline__ uint8_t* region(const Launch&, uint32_t rank) const {
+    return base + (uint64_t)rank * rank_stride;
+  }
+  template <uint32_t kUnits>
+  __device__ __forceinline__ TileCoord locate(const Launch& launch, uint32_t t) {
+    const FewItemsTile f = few_items_find(tt, before, t);
+    it = launch.item[f.item];
+    return few_items_coord(tt, f, launch.tt.tiles_before[f.item], (uint32_t)tiles_for(it.units(), kUnits));
+  }
+};
+
+// The walk that goes with a launch's kind of table.
+template <class Launch, bool kFew, class Table = decltype(Launch::tt)> struct WalkOf;
+template <class Launch, bool kFew> struct WalkOf<Launch, kFew, TileHead> { typedef SingleWalk<typename Launch::Desc> type; };
+template <class Launch, bool kFew> struct WalkOf<Launch, kFew, FewItemsTable> { typedef FewItemsWalk<Launch> type; };
+template <class Launch> struct WalkOf<Launch, false, TileTable> { typedef TableWalk<Launch> type; };
+template <class Launch> struct WalkOf<Launch, true, TileTable> { typedef FewTilesWalk<Launch> type; };
+template <class Launch, bool kFew = false> using TileWalk = typename WalkOf<Launch, kFew>::type;
+
+// Calls body(tile) for the tiles of this workgroup: one of as many as there are tiles has its own.
+template <class Walk, class Launch, class Body>
+__device__ __forceinline__ void each_tile(const Walk& walk, const Launch& launch, Body body) {
+  if constexpr (Walk::kOneTile)
+    body(blockIdx.x);
+  else
+    for (uint32_t t = blockIdx.x; t < walk.n_tiles(launch); t += gridDim.x) body(t);
+}
 
 // ---- gather -------------------------------------------------------------------------------
 // Everything of a tile that is not a run of T * U whole vectors: the last partial run, the
@@ -249,8 +310,8 @@ __global__ __launch_bounds__(T) void gather_kernel(const Launch launch) {
   static_assert(T >= ODC_BODY_ALIGN - 1, "one lane per head byte");
   const uint32_t tid = threadIdx.x;
   TileWalk<Launch, kFew> walk(launch);
-  for (uint32_t t = blockIdx.x; t < walk.n_tiles(launch); t += gridDim.x) {
-    const TileCoord c = walk.locate(launch, t);
+  each_tile(walk, launch, [&](uint32_t t) {
+    const TileCoord c = walk.template locate<kVecs * 16>(launch, t);
     const GatherDesc it = walk.it;
     const uint64_t seg = it.seg_bytes;
     const uint8_t* s = walk.region(launch, c.rank) + it.src_off;
@@ -278,7 +339,7 @@ __global__ __launch_bounds__(T) void gather_kernel(const Launch launch) {
     } else if (has_edges<kVecs>(w)) {
       gather_edges<kSrcCached, kDst != kStream, T, U>(d, s, c.chunk, g);
     }
-  }
+  });
 }
 
 // ---- clear --------------------------------------------------------------------------------
@@ -303,8 +364,8 @@ __global__ __launch_bounds__(kThreads) void clear_kernel(const Launch launch) {
   const u32x4 zero = {0u, 0u, 0u, 0u};
   const uint32_t tid = threadIdx.x;
   TileWalk<Launch> walk(launch);
-  for (uint32_t t = blockIdx.x; t < walk.n_tiles(launch); t += gridDim.x) {
-    const TileCoord c = walk.locate(launch, t);
+  each_tile(walk, launch, [&](uint32_t t) {
+    const TileCoord c = walk.template locate<kTileBytes>(launch, t);
     const ClearDesc it = walk.it;
     uint8_t* d = walk.region(launch, c.rank) + it.off;
     const SegShape g = seg_shape((uintptr_t)d, it.seg_bytes, 1, 16);
@@ -315,7 +376,7 @@ __global__ __launch_bounds__(kThreads) void clear_kernel(const Launch launch) {
       for (int u = 0; u < kUnroll; ++u) db[u * kThreads] = zero;
     }
     if (has_edges(w)) clear_edges(d, c.chunk, g);
-  }
+  });
 }
 
 // ---- scatter-accumulate -------------------------------------------------------------------
@@ -494,8 +555,8 @@ __global__ __launch_bounds__(T) void accum_kernel(const Launch launch) {
   static_assert(T >= ODC_BODY_ALIGN / kAB, "one lane per head element");
   const uint32_t tid = threadIdx.x;
   TileWalk<Launch, kFew> walk(launch);
-  for (uint32_t t = blockIdx.x; t < walk.n_tiles(launch); t += gridDim.x) {
-    const TileCoord c = walk.locate(launch, t);
+  each_tile(walk, launch, [&](uint32_t t) {
+    const TileCoord c = walk.template locate<kVecs * 4>(launch, t);
     const AccumDesc it = walk.it;
     const uint64_t seg = it.seg_elems;
     uint8_t* acc = walk.region(launch, c.rank) + it.acc_off;
@@ -528,7 +589,7 @@ __global__ __launch_bounds__(T) void accum_kernel(const Launch launch) {
     }
     if (!whole ? (w.nv != 0 || w.head || w.tail) : (w.head || w.tail))
       accum_edges<G, A, kStore, kGradCached, kAccCached, T, U>(acc, it.grad, g_seg, it.grad_elems, c.chunk, g, !whole);
-  }
+  });
 }
 
 // ---- gather with cast ---------------------------------------------------------------------
@@ -590,8 +651,8 @@ __global__ __launch_bounds__(T) void cast_gather_kernel(const Launch launch) {
   constexpr uint32_t kSB = Codec<S>::kBytes, kDB = Codec<D>::kBytes;
   const uint32_t tid = threadIdx.x;
   TileWalk<Launch, kFew> walk(launch);
-  for (uint32_t t = blockIdx.x; t < walk.n_tiles(launch); t += gridDim.x) {
-    const TileCoord c = walk.locate(launch, t);
+  each_tile(walk, launch, [&](uint32_t t) {
+    const TileCoord c = walk.template locate<kVecs * 4>(launch, t);
     const CastGatherDesc it = walk.it;
     const uint64_t seg = it.seg_elems;
     const uint8_t* s = walk.region(launch, c.rank) + it.src_off;
@@ -627,7 +688,7 @@ __global__ __launch_bounds__(T) void cast_gather_kernel(const Launch launch) {
     } else if (has_edges<kVecs>(w)) {
       cast_edges<S, D, kCached, T, U>(d, s, c.chunk, g);
     }
-  }
+  });
 }
 
 // ---- publish ------------------------------------------------------------------------------
@@ -673,8 +734,8 @@ __global__ __launch_bounds__(T) void publish_kernel(const Launch launch) {
   typedef typename Quad<O>::vec_t ovec_t;
   const uint32_t tid = threadIdx.x;
   TileWalk<Launch, kFew> walk(launch);
-  for (uint32_t t = blockIdx.x; t < walk.n_tiles(launch); t += gridDim.x) {
-    const TileCoord c = walk.locate(launch, t);
+  each_tile(walk, launch, [&](uint32_t t) {
+    const TileCoord c = walk.template locate<kVecs * 4>(launch, t);
     const PublishDesc it = walk.it;
     const uint64_t seg = it.seg_elems;
     const uint64_t in_seg = (uint64_t)c.chunk * kElems;
@@ -748,14 +809,14 @@ __global__ __launch_bounds__(T) void publish_kernel(const Launch launch) {
         }
       }
     }
-  }
+  });
 }
 
 // ------------------------------------------------------------------------------------------------
 // dtype dispatch
 // ------------------------------------------------------------------------------------------------
 template <class Launch> using kernel_fn = void (*)(const Launch);
-// A launch of one item has nothing to search: one kernel serves both short forms.
+// Launches of one item or of few have one way to find it: one kernel serves both short forms.
 template <class Launch> constexpr bool kSearches = std::is_same_v<decltype(Launch::tt), TileTable>;
 
 #define ODC_FOR_EACH_DTYPE_PAIR(X)                    \
@@ -868,21 +929,16 @@ kernel_fn<L> pick_publish(int a, int o, TileForm form) {  // (accumulation dtype
   return nullptr;
 }
 
-// A launch of one item in its own form.
-template <class Launch>
-SingleLaunch<typename Launch::Desc> single_form(const Launch& L) {
-  SingleLaunch<typename Launch::Desc> s;
-  s.tt = L.tt;
+// A launch of one item, or of up to kFewItems, in its own form.
+template <class Form, class Launch>
+Form short_form(const Launch& L) {
+  Form s;
+  if constexpr (std::is_same_v<decltype(s.tt), FewItemsTable>) s.tt = few_items_table(L.tt);
+  else s.tt = L.tt;
   s.base = L.base;
   s.rank_stride = L.rank_stride;
-  s.item[0] = L.item[0];
-  return s;
-}
-
-PublishSingle single_form(const PublishLaunch& L) {
-  PublishSingle s;
-  static_cast<SingleLaunch<PublishDesc>&>(s) = single_form<PublishLaunch>(L);
-  s.scale = L.scale;
+  std::copy_n(L.item, std::min<size_t>(L.tt.n_items, std::size(s.item)), s.item);
+  if constexpr (std::is_same_v<Launch, PublishLaunch>) s.scale = L.scale;
   return s;
 }
 
@@ -899,13 +955,27 @@ int launch(void (*kernel)(const Launch), const Launch& L, uint32_t grid, uint32_
 
 template <class L> struct Form { typedef L type; };
 
+// The short forms of a launch.
+template <class Launch> struct ShortForms {
+  typedef SingleLaunch<typename Launch::Desc> Single;
+  typedef FewItemsLaunch<typename Launch::Desc> FewItems;
+};
+template <> struct ShortForms<PublishLaunch> {
+  typedef PublishSingle Single;
+  typedef PublishFewItems FewItems;
+};
+
 // pick(Form<L>) names the kernel for launches of type L.
 template <class Launch, class Pick>
 int launch_form(const Launch& L, uint32_t grid, uint32_t threads, uint32_t lds_bytes, void* stream, Pick pick) {
-  if (L.tt.n_items != 1) return launch<Launch>(pick(Form<Launch>{}), L, grid, threads, lds_bytes, stream);
-  const auto single = single_form(L);
-  typedef std::remove_const_t<decltype(single)> Single;
-  return launch<Single>(pick(Form<Single>{}), single, grid, threads, lds_bytes, stream);
+  const auto issue = [&](const auto& form) {
+    typedef std::remove_cv_t<std::remove_reference_t<decltype(form)>> F;
+    return launch<F>(pick(Form<F>{}), form, grid, threads, lds_bytes, stream);
+  };
+  if (grid != L.tt.n_tiles) return issue(L);  // workgroups of more than one tile walk the full tables
+  if (L.tt.n_items == 1) return issue(short_form<typename ShortForms<Launch>::Single>(L));
+  if (L.tt.n_items <= kFewItems) return issue(short_form<typename ShortForms<Launch>::FewItems>(L));
+  return issue(L);
 }
 
 }  // namespace

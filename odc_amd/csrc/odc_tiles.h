@@ -181,6 +181,65 @@ ODC_HD TileCoord single_item_coord(const TileHead& tt, uint32_t t) {
   return c;
 }
 
+// A launch of up to kFewItems items with one workgroup per tile: the table fits one scalar load, and holds
+// what the tile order needs, so that no tile divides twice: the tiles before item i in one rank segment
+// each where ranks are outermost, in the whole launch where items are. Entries past the last item hold
+// the total.
+constexpr uint32_t kFewItems = 16;
+struct FewItemsTable : TileHead {
+  uint32_t tiles_before[kFewItems];
+};
+
+inline FewItemsTable few_items_table(const TileTable& tt) {
+  FewItemsTable few;
+  static_cast<TileHead&>(few) = tt;
+  for (uint32_t i = 0; i < kFewItems; ++i)
+    few.tiles_before[i] = tt.seg_prefix[i] * (tt.order == kRankOutermost ? 1u : tt.world);
+  return few;
+}
+
+// A tile of such a launch: its item, its rank (rank outermost only) and its position, among all the launch's
+// tiles or the rank's.
+struct FewItemsTile {
+  uint32_t item, rank, position;
+};
+
+// before: tiles_before in any form that can be indexed (the kernels hold it in scalar registers). The item is
+// the number of later ones that do not begin behind the position, counted by sign bits: every value
+// is less than 2^31.
+template <class Before>
+ODC_HD FewItemsTile few_items_find(const TileHead& tt, const Before& before, uint32_t t) {
+  static_assert(kMaxTilesPerLaunch <= 1ull << 31, "sign bits");
+  FewItemsTile f = {kFewItems - 1, 0, t};
+  if (tt.order == kRankOutermost) {
+    f.rank = t / tt.tiles_per_rank;
+    f.position = t - f.rank * tt.tiles_per_rank;
+  }
+#pragma unroll
+  for (uint32_t i = 1; i < kFewItems; ++i) f.item -= (f.position - before[i]) >> 31;
+  return f;
+}
+
+// first: tiles_before of the item; per_rank: the item's tiles in one rank segment
+ODC_HD TileCoord few_items_coord(const TileHead& tt, FewItemsTile f, uint32_t first, uint32_t per_rank) {
+  TileCoord c;
+  c.item = f.item;
+  f.position -= first;
+  if (tt.order == kRankOutermost) {
+    c.rank = f.rank;
+    c.chunk = f.position;
+  } else if (tt.order == kItemMajor) {
+    c.rank = f.position / per_rank;
+    c.chunk = f.position - c.rank * per_rank;
+  } else {
+    c.chunk = f.position / tt.world;
+    c.rank = f.position - c.chunk * tt.world;
+  }
+  c.rank += tt.first_rank;
+  if (c.rank >= tt.world) c.rank -= tt.world;
+  return c;
+}
+
 // Shape of one rank segment of `n` units whose WRITTEN side starts at address D:
 //     head  : the units before the first 128-byte line boundary of D (at most 127 bytes),
 //     body  : nvec whole vectors, written with aligned 128-bit (64-bit for 16-bit outputs) stores,
