@@ -267,7 +267,11 @@ int odc_abi_version(void);
  *    leave it there, with plain stores up to "plain_output_bytes" (24 MiB) and written through the L2
  *    above; gradients of at most "cached_gradient_bytes" (128 MiB) per launch are read through the
  *    caches; so are shards and accumulations while all symmetric memory in use, over all ranks, is at most
- *    "cached_arena_bytes" (192 MiB). 0 streams past the caches.
+ *    "cached_arena_bytes" (192 MiB). 0 streams past the caches. Above "resident_above" (640 MiB) in use a
+ *    part of the symmetric memory is kept in the cache: of accumulations the share that
+ *    "resident_accumulation_bytes" (384 MiB) have of what is in use, of gathered shards the share of
+ *    "resident_shard_bytes" (96 MiB); clears leave theirs there from "resident_clear_bytes" (48 MiB) per
+ *    launch on. 0 keeps none.
  *  - "rank_stagger_bytes" (extra distance between rank regions), "rank_stride_align" (rank regions
  *    start on multiples of it, default 16384 = one tile) and "alloc_align" (allocations of at
  *    least this many bytes start on multiples of it, default 16384; smaller ones on 256): read

@@ -78,6 +78,10 @@ struct Options {
   int64_t cached_output_bytes = 64ll << 20;
   int64_t plain_output_bytes = 24ll << 20;    // see output_form
   int64_t cached_gradient_bytes = 128ll << 20;
+  int64_t resident_accumulation_bytes = 384ll << 20;  // these and the next three: see resident_below
+  int64_t resident_shard_bytes = 96ll << 20;
+  int64_t resident_above = 640ll << 20;
+  int64_t resident_clear_bytes = 48ll << 20;
   int64_t short_tiles_below = 32;             // see wants_short_tiles
   int64_t few_tiles = 32768;                  // see tile_form
 };
@@ -108,6 +112,10 @@ int64_t* option_slot(const char* name) {
   if (!strcmp(name, "cached_output_bytes")) return &g_opt.cached_output_bytes;
   if (!strcmp(name, "plain_output_bytes")) return &g_opt.plain_output_bytes;
   if (!strcmp(name, "cached_gradient_bytes")) return &g_opt.cached_gradient_bytes;
+  if (!strcmp(name, "resident_accumulation_bytes")) return &g_opt.resident_accumulation_bytes;
+  if (!strcmp(name, "resident_shard_bytes")) return &g_opt.resident_shard_bytes;
+  if (!strcmp(name, "resident_above")) return &g_opt.resident_above;
+  if (!strcmp(name, "resident_clear_bytes")) return &g_opt.resident_clear_bytes;
   if (!strcmp(name, "short_tiles_below")) return &g_opt.short_tiles_below;
   if (!strcmp(name, "few_tiles")) return &g_opt.few_tiles;
   return nullptr;
@@ -262,6 +270,29 @@ CachePolicy cache_policy(const odc_arena* a, const Options& opt, uint64_t read_b
   return p;
 }
 constexpr int64_t kSymmetric = -1;  // a line: the stream lies in symmetric memory
+
+// The part of symmetric memory that stays in the last-level cache when all of it does not fit. Streams that
+// pass by the cache do not push out what others have left in it (a read-modify-write of 872 MB of which
+// 128 MB are read through the caches takes 307 us instead of 346 with 0.9, 1.7 and 3.5 GB of nontemporal
+// copies between two of them alike), so a fixed subset of the accumulations, touched twice by every
+// accumulate, and of the shards can live there from one kernel to the next (is_resident in odc_tiles.h
+// says which bytes; only their loads, and the stores of launches that do not load, go through the caches).
+// Up to 640 MiB in use there is none: gradients and gathered outputs of such sizes are cached themselves
+// and leave no room (bf16 into fp32, 17 Mi elements, three sets of buffers in turn: gather + accumulate
+// 41.8 us without, 48.8 with; 44 Mi 201.5 without, 190 with). Above it accumulations have 384 MiB's share of
+// the memory in use, shards 96 MiB's: with one unit in the arena as much of it as the cache takes, with
+// many the parts of all of them together still fit. us without -> with, a decoder layer at W = 8, three
+// units in turn: gather + accumulate 481 -> 472; store, 3 accumulates, 4 gathers and publish 1822 -> 1745;
+// FSDP2 minibatch of two microbatches, mixed 1664 -> 1643, bf16 1041 -> 1024; FSDP1 of 25 M elements in
+// fp16 214.5 -> 209; three microbatches of 68 M elements 455 -> 422. Ten units in turn, where a unit's
+// part is small and has to last for 25 GB: 481 -> 480, 1827 -> 1803, 1685 -> 1688, 1045.5 -> 1044.6, 214.4 ->
+// 211, 457 -> 444. (384 MiB's share against 256 and 512: 1643 / 1660 / 1633 and 1749 / 1772 / 1735 in
+// minibatches, 473 / 467 / 485 in single passes. Converting gathers gain nothing.)
+uint32_t resident_below(const odc_arena* a, const Options& opt, int64_t most) {
+  const double in_use = (double)(a->in_use.load(std::memory_order_relaxed) * a->world);
+  if (in_use <= (double)opt.resident_above) return 0;
+  return (uint32_t)std::min(4294967295.0, (double)most / in_use * 4294967296.0);
+}
 
 // How a gather writes an output that stays in the caches. Up to what the L2s hold (8 x 4 MB) plain
 // stores leave it there for the reader; beyond that it is written through to the last-level cache
@@ -703,6 +734,7 @@ int odc_gather(odc_arena* a, const odc_gather_item* items, uint32_t n_items, uin
     for (uint32_t k = 0; k < L.tt.n_items; ++k) shard_bytes += L.item[k].seg_bytes;
     L.policy = cache_policy(a, opt, 0, kSymmetric, shard_bytes * a->world, opt.cached_output_bytes);
     L.output = output_form(opt, L.policy.written, shard_bytes * a->world);
+    L.tt.resident_below = resident_below(a, opt, opt.resident_shard_bytes);
     for (uint32_t k = 0; k < L.tt.n_items; ++k)
       ragged |= (((uintptr_t)L.item[k].dst | L.item[k].src_off | L.item[k].seg_bytes) & 15u) != 0;
     const uint32_t grid = grid_for(a, opt.gather_blocks_per_cu, L.tt.n_tiles, copy_threads(L.form), ragged);
@@ -838,6 +870,15 @@ int odc_clear(odc_arena* a, const odc_span* spans, uint32_t n_spans, void* strea
         });
     if (n < 0) return n;
     if (n == 0) continue;
+    // A clear that leaves the resident part in the cache streams the rest past it, which takes longer (a layer's
+    // 872 MB 118 -> 134 us) than leaving the last 256 MB behind unwritten, and pays from 48 MiB of resident
+    // zeros on: FSDP2 minibatches 1660 -> 1643, 349 -> 339 (three units in turn, 85 MB each), but 352 -> 360
+    // and 331 -> 341 (ten, 26 MB each).
+    uint64_t cleared = 0;
+    for (uint32_t k = 0; k < L.tt.n_items; ++k) cleared += L.item[k].seg_bytes;
+    const uint32_t below = resident_below(a, opt, opt.resident_accumulation_bytes);
+    const double resident = (double)(cleared * a->world) * below / 4294967296.0;
+    L.tt.resident_below = resident >= (double)opt.resident_clear_bytes ? below : 0;
     const uint32_t grid = grid_for(a, opt.clear_blocks_per_cu, L.tt.n_tiles, kThreads);
     if (int rc = launch_tiles(a, L, grid, [&] { return odc_device::launch_clear(L, grid, stream); })) return rc;
   }
@@ -949,6 +990,7 @@ int scatter_launch(odc_arena* a, const odc_accum_item* items, uint32_t n_items, 
     uint64_t grad_elems = 0;
     for (uint32_t k = 0; k < L.tt.n_items; ++k) grad_elems += L.item[k].grad_elems;
     L.policy = cache_policy(a, opt, grad_elems * gb, opt.cached_gradient_bytes, 0, kSymmetric);
+    L.tt.resident_below = resident_below(a, opt, opt.resident_accumulation_bytes);
     int64_t blocks_per_cu = store ? opt.store_blocks_per_cu : opt.accum_blocks_per_cu;
     if (blocks_per_cu < 0)
       blocks_per_cu = whole_tiles < (uint64_t)opt.accum_persistent_below_tiles * segments ? 1 : 0;

@@ -25,7 +25,7 @@
 // Each wavefront issues its 2 or 4 independent 128-bit loads per stream before the first store.
 // Streams larger than the 256 MB last-level cache are nontemporal on both sides (worth ~15 % over
 // plain accesses there); what fits the cache and was just produced, or is about to be consumed, is
-// left in it (cache_policy in odc_host.cpp). Deeper unrolling or prefetching the next tile
+// left in it (cache_policy in odc_host.cpp), and so is a part of what does not fit (resident_below there). Deeper unrolling or prefetching the next tile
 // measured slower: the memory system prefers a small window to more requests in flight.
 // Workgroup i runs on XCD i % 8; binding XCDs to address classes (256 B .. 64 KiB granules)
 // changed nothing measurable and giving every XCD one contiguous eighth of the tiles costs the
@@ -64,6 +64,36 @@ template <class V> struct Unaligned;
 template <> struct Unaligned<u32x4> { typedef u32x4_u type; };
 template <> struct Unaligned<u32x2> { typedef u32x2_u type; };
 
+// An address in device memory. Of an address that comes as an argument of a function, or as a number,
+// the compiler must assume that it may lie in LDS or scratch, and it takes the slower flat accesses.
+template <class P>
+__device__ __forceinline__ P* as_global(P* p) {
+  return (P*)(__attribute__((address_space(1))) P*)(uintptr_t)p;
+}
+
+// The same of an address that all lanes agree on, in scalar registers: an access to it plus a 32-bit
+// lane offset then needs no vector arithmetic of its own.
+template <class P>
+__device__ __forceinline__ P* scalar_base(P* p) {
+  uintptr_t a = (uintptr_t)p;
+  asm("" : "+s"(a));
+  return as_global((P*)a);
+}
+
+// Calls body(std::true_type) or body(std::false_type). The two differ in the cache policy of some
+// accesses and in nothing else, and the compiler would make one of them and drop the policy, so one side
+// begins and ends with something that the other has not.
+template <class Body>
+__device__ __forceinline__ void with_policy(bool resident, Body body) {
+  if (resident) {
+    asm volatile("" ::: "memory");
+    body(std::true_type{});
+    asm volatile("" ::: "memory");
+  } else {
+    body(std::false_type{});
+  }
+}
+
 // kCached: a plain access, which leaves its line in the caches; otherwise nontemporal. Which one a
 // stream of a launch takes is the host's choice (cache_policy in odc_host.cpp).
 template <bool kCached, class V>
@@ -100,13 +130,6 @@ __device__ __forceinline__ void store_output(u32x4* tile, uint32_t i, u32x4 v) {
     store_vec<kForm == kKeep>(tile + i, v);
 }
 
-// An address in device memory. Of an address that comes as an argument of a function, or as a number,
-// the compiler must assume that it may lie in LDS or scratch, and it takes the slower flat accesses.
-template <class P>
-__device__ __forceinline__ P* as_global(P* p) {
-  return (P*)(__attribute__((address_space(1))) P*)(uintptr_t)p;
-}
-
 // ---- finding a tile's work ------------------------------------------------------------------
 // The walk of a workgroup over the tiles of its launch; all its lanes come along.
 template <class Launch>
@@ -118,6 +141,7 @@ struct TableWalk {
 
   __device__ __forceinline__ explicit TableWalk(const Launch&) {}
   __device__ __forceinline__ uint32_t n_tiles(const Launch& launch) const { return launch.tt.n_tiles; }
+  __device__ __forceinline__ uint32_t resident_below(const Launch& launch) const { return launch.tt.resident_below; }
   __device__ __forceinline__ uint8_t* region(const Launch& launch, uint32_t rank) const {
     return launch.base + (uint64_t)rank * launch.rank_stride;
   }
@@ -155,12 +179,13 @@ struct SingleWalk {
 #pragma unroll
     for (int i = 0; i < kWords; ++i) w[i] = reinterpret_cast<const uint64_t*>(launch.item)[i];
     // (left alone, the compiler reads each value where it is first used)
-    asm volatile("" : "+s"(tt.world), "+s"(tt.order), "+s"(tt.first_rank), "+s"(tt.tiles_per_rank),
+    asm volatile("" : "+s"(tt.world), "+s"(tt.order), "+s"(tt.first_rank), "+s"(tt.tiles_per_rank), "+s"(tt.resident_below),
                       "+s"(b), "+s"(stride), "+s"(w[0]), "+s"(w[1]), "+s"(w[2]), "+s"(w[3]));
     base = as_global(reinterpret_cast<uint8_t*>((uintptr_t)b));
     rank_stride = stride;
     __builtin_memcpy(&it, w, sizeof(D));
   }
+  __device__ __forceinline__ uint32_t resident_below(const SingleLaunch<D>&) const { return tt.resident_below; }
   __device__ __forceinline__ uint8_t* region(const SingleLaunch<D>&, uint32_t rank) const {
     return base + (uint64_t)rank * rank_stride;
   }
@@ -190,12 +215,13 @@ struct FewTilesWalk {
     bound[1] = launch.tt.seg_prefix[65 + lane < kMaxItems ? 65 + lane : kMaxItems];
     tt = launch.tt;
     uint64_t b = (uint64_t)(uintptr_t)launch.base, stride = launch.rank_stride;
-    asm volatile("" : "+s"(tt.world), "+s"(tt.n_tiles), "+s"(tt.order), "+s"(tt.first_rank), "+s"(tt.tiles_per_rank),
+    asm volatile("" : "+s"(tt.world), "+s"(tt.n_tiles), "+s"(tt.order), "+s"(tt.first_rank), "+s"(tt.tiles_per_rank), "+s"(tt.resident_below),
                       "+s"(b), "+s"(stride), "+v"(bound[0]), "+v"(bound[1]));
     base = as_global(reinterpret_cast<uint8_t*>((uintptr_t)b));
     rank_stride = stride;
   }
   __device__ __forceinline__ uint32_t n_tiles(const Launch&) const { return tt.n_tiles; }
+  __device__ __forceinline__ uint32_t resident_below(const Launch&) const { return tt.resident_below; }
   __device__ __forceinline__ uint8_t* region(const Launch&, uint32_t rank) const {
     return base + (uint64_t)rank * rank_stride;
   }
@@ -236,11 +262,12 @@ struct FewItemsWalk {
     __builtin_memcpy(&before, launch.tt.tiles_before, sizeof(before));
     tt = launch.tt;
     uint64_t b = (uint64_t)(uintptr_t)launch.base, stride = launch.rank_stride;
-    asm volatile("" : "+s"(tt.world), "+s"(tt.order), "+s"(tt.first_rank), "+s"(tt.tiles_per_rank), "+s"(b), "+s"(stride),
+    asm volatile("" : "+s"(tt.world), "+s"(tt.order), "+s"(tt.first_rank), "+s"(tt.tiles_per_rank), "+s"(tt.resident_below), "+s"(b), "+s"(stride),
                       "+s"(before));
     base = as_global(reinterpret_cast<uint8_t*>((uintptr_t)b));
     rank_stride = stride;
   }
+  __device__ __forceinline__ uint32_t resident_below(const Launch&) const { return tt.resident_below; }
   __device__ __forceinline__ uint8_t* region(const Launch&, uint32_t rank) const {
     return base + (uint64_t)rank * rank_stride;
   }
@@ -319,23 +346,27 @@ __global__ __launch_bounds__(T) void gather_kernel(const Launch launch) {
     const SegShape g = seg_shape<kVecs>((uintptr_t)d, seg, 1, 16);
     const TileWork w = tile_work<kVecs>(c.chunk, g);
     if (is_whole<kVecs>(w)) {
-      const uint8_t* sb = s + g.head + (w.v0 + tid) * 16;
-      u32x4* db = reinterpret_cast<u32x4*>(d + g.head) + w.v0;
-      u32x4 v[U];
+      const uint8_t* sb[U];
 #pragma unroll
-      for (int u = 0; u < U; ++u) v[u] = load_any<kSrcCached, u32x4>(sb + (size_t)u * T * 16);
-      // a whole tile that also owns its segment's head or tail (the first and last tile of a
-      // ragged segment) reads those bytes with the same round trip as its vectors
-      const bool do_head = w.head && tid < g.head;
-      const bool do_tail = w.tail && tid < g.tail;
-      const uint64_t tail_at = g.head + g.nvec * 16 + tid;
-      uint8_t head_byte = 0, tail_byte = 0;
-      if (do_head) head_byte = s[tid];
-      if (do_tail) tail_byte = s[tail_at];
+      for (int u = 0; u < U; ++u) sb[u] = scalar_base(s + g.head + (w.v0 + u * T) * 16);
+      u32x4* db = scalar_base(reinterpret_cast<u32x4*>(d + g.head) + w.v0);
+      with_policy(kSrcCached || is_resident((uintptr_t)(s + g.head + w.v0 * 16), walk.resident_below(launch)), [&](auto cached) {
+        u32x4 v[U];
 #pragma unroll
-      for (int u = 0; u < U; ++u) store_output<kDst, kVecs>(db, u * T + tid, v[u]);
-      if (do_head) d[tid] = head_byte;
-      if (do_tail) d[tail_at] = tail_byte;
+        for (int u = 0; u < U; ++u) v[u] = load_any<cached, u32x4>(sb[u] + tid * 16);
+        // a whole tile that also owns its segment's head or tail (the first and last tile of a
+        // ragged segment) reads those bytes with the same round trip as its vectors
+        const bool do_head = w.head && tid < g.head;
+        const bool do_tail = w.tail && tid < g.tail;
+        const uint64_t tail_at = g.head + g.nvec * 16 + tid;
+        uint8_t head_byte = 0, tail_byte = 0;
+        if (do_head) head_byte = s[tid];
+        if (do_tail) tail_byte = s[tail_at];
+#pragma unroll
+        for (int u = 0; u < U; ++u) store_output<kDst, kVecs>(db, u * T + tid, v[u]);
+        if (do_head) d[tid] = head_byte;
+        if (do_tail) d[tail_at] = tail_byte;
+      });
     } else if (has_edges<kVecs>(w)) {
       gather_edges<kSrcCached, kDst != kStream, T, U>(d, s, c.chunk, g);
     }
@@ -372,8 +403,11 @@ __global__ __launch_bounds__(kThreads) void clear_kernel(const Launch launch) {
     const TileWork w = tile_work(c.chunk, g);
     if (is_whole(w)) {
       u32x4* db = reinterpret_cast<u32x4*>(d + g.head) + w.v0 + tid;
+      const uint32_t below = walk.resident_below(launch);
+      with_policy(!below || is_resident((uintptr_t)(d + g.head + w.v0 * 16), below), [&](auto cached) {
 #pragma unroll
-      for (int u = 0; u < kUnroll; ++u) db[u * kThreads] = zero;
+        for (int u = 0; u < kUnroll; ++u) store_vec<cached>(db + u * kThreads, zero);
+      });
     }
     if (has_edges(w)) clear_edges(d, c.chunk, g);
   });
@@ -567,25 +601,32 @@ __global__ __launch_bounds__(T) void accum_kernel(const Launch launch) {
     // whole: all its quads exist in the accumulation AND in the valid part of the gradient
     const bool whole = is_whole<kVecs>(w) && g_seg + e0 + 4 * kVecs <= it.grad_elems;
     if (whole) {
-      const uint8_t* gb = as_global(it.grad) + (g_seg + e0) * kGB + (size_t)tid * sizeof(gvec_t);
-      avec_t* ap = reinterpret_cast<avec_t*>(acc + e0 * kAB) + tid;
-      gvec_t graw[U];
-      avec_t araw[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) graw[u] = load_any<kGradCached, gvec_t>(gb + (size_t)u * T * sizeof(gvec_t));
-      if constexpr (!kStore) {
-#pragma unroll
-        for (int u = 0; u < U; ++u) araw[u] = load_vec<kAccCached>(ap + u * T);
-      }
+      const uint8_t* gb[U];
+      avec_t* ap[U];
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        float gf[4], af[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-        Quad<G>::widen(graw[u], gf);
-        if constexpr (!kStore) Quad<A>::widen(araw[u], af);
-#pragma unroll
-        for (int k = 0; k < 4; ++k) af[k] = af[k] + gf[k];
-        store_vec<kAccCached>(ap + u * T, Quad<A>::narrow(af));
+        gb[u] = scalar_base(it.grad + (g_seg + e0 + u * T * 4) * kGB);
+        ap[u] = scalar_base(reinterpret_cast<avec_t*>(acc + e0 * kAB) + u * T);
       }
+      with_policy(kAccCached || is_resident((uintptr_t)(acc + e0 * kAB), walk.resident_below(launch)), [&](auto cached) {
+        gvec_t graw[U];
+        avec_t araw[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) graw[u] = load_any<kGradCached, gvec_t>(gb[u] + tid * (uint32_t)sizeof(gvec_t));
+        if constexpr (!kStore) {
+#pragma unroll
+          for (int u = 0; u < U; ++u) araw[u] = load_vec<cached>(ap[u] + tid);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          float gf[4], af[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+          Quad<G>::widen(graw[u], gf);
+          if constexpr (!kStore) Quad<A>::widen(araw[u], af);
+#pragma unroll
+          for (int k = 0; k < 4; ++k) af[k] = af[k] + gf[k];
+          store_vec<cached>(ap[u] + tid, Quad<A>::narrow(af));
+        }
+      });
     }
     if (!whole ? (w.nv != 0 || w.head || w.tail) : (w.head || w.tail))
       accum_edges<G, A, kStore, kGradCached, kAccCached, T, U>(acc, it.grad, g_seg, it.grad_elems, c.chunk, g, !whole);
@@ -966,15 +1007,17 @@ template <> struct ShortForms<PublishLaunch> {
 };
 
 // pick(Form<L>) names the kernel for launches of type L.
+// by_table: several items take the full tables, however few they are.
 template <class Launch, class Pick>
-int launch_form(const Launch& L, uint32_t grid, uint32_t threads, uint32_t lds_bytes, void* stream, Pick pick) {
+int launch_form(const Launch& L, uint32_t grid, uint32_t threads, uint32_t lds_bytes, void* stream, Pick pick,
+                bool by_table = false) {
   const auto issue = [&](const auto& form) {
     typedef std::remove_cv_t<std::remove_reference_t<decltype(form)>> F;
     return launch<F>(pick(Form<F>{}), form, grid, threads, lds_bytes, stream);
   };
   if (grid != L.tt.n_tiles) return issue(L);  // workgroups of more than one tile walk the full tables
   if (L.tt.n_items == 1) return issue(short_form<typename ShortForms<Launch>::Single>(L));
-  if (L.tt.n_items <= kFewItems) return issue(short_form<typename ShortForms<Launch>::FewItems>(L));
+  if (L.tt.n_items <= kFewItems && !by_table) return issue(short_form<typename ShortForms<Launch>::FewItems>(L));
   return issue(L);
 }
 
@@ -1021,16 +1064,19 @@ bool has_accum(int g, int a) { return pick_accum<AccumLaunch>(g, a, false, {}, k
 bool has_cast_gather(int s, int d) { return pick_cast_gather<CastGatherLaunch>(s, d, {}, kWholeTiles) != nullptr; }
 bool has_publish(int a, int o) { return pick_publish<PublishLaunch>(a, o, kShortTiles) != nullptr; }
 
+// Gathers of whole tiles are bound by HBM and stream better from workgroups that come to their loads one
+// after the other along the item search: a layer's 872 MB from bf16 134.1 us by the full tables, 136.4 by the
+// small ones, from fp32 196 and 199 (fewer resident workgroups: 224). The other kernels are level there.
 int launch_gather(const GatherLaunch& L, uint32_t grid, uint32_t lds_bytes, void* stream) {
   return launch_form(L, grid, copy_threads(L.form), lds_bytes, stream, [&](auto form) {
     return pick_gather<typename decltype(form)::type>(L.policy.read, L.output, L.form);
-  });
+  }, L.form == kWholeTiles);
 }
 
 int launch_cast_gather(int s, int d, const CastGatherLaunch& L, uint32_t grid, uint32_t lds_bytes, void* stream) {
   return launch_form(L, grid, copy_threads(L.form), lds_bytes, stream, [&](auto form) {
     return pick_cast_gather<typename decltype(form)::type>(s, d, L.policy, L.form);
-  });
+  }, L.form == kWholeTiles);
 }
 
 int launch_accum(int g, int a, bool store, const AccumLaunch& L, uint32_t grid, uint32_t lds_bytes, void* stream) {

@@ -101,7 +101,7 @@ inline uint32_t accum_threads(int grad_dtype, int acc_dtype, bool store, CachePo
 constexpr uint32_t most_workgroups(uint32_t threads) { return 0xffffffffu / threads; }
 
 // A launch carries up to kMaxItems items. One of a single item, a flat parameter on its own, goes out
-// in a form without the tables: 56 to 80 bytes of arguments instead of 2.3 to 4 KB, which the host
+// in a form without the tables: 64 to 88 bytes of arguments instead of 2.3 to 4 KB, which the host
 // hands over in 2.6 us instead of 4.0 (512 bytes: 3.4), and all of it is read at once instead of
 // along the item search (SingleWalk in odc_kernels.hip).
 template <class D>
@@ -216,7 +216,7 @@ struct PublishSingle : SingleLaunch<PublishDesc> {
 struct PublishFewItems : FewItemsLaunch<PublishDesc> {
   PublishScale scale;
 };
-static_assert(sizeof(SingleLaunch<ClearDesc>) == 56 && sizeof(PublishSingle) == 80, "as SingleLaunch says");
+static_assert(sizeof(SingleLaunch<ClearDesc>) == 64 && sizeof(PublishSingle) == 88, "as SingleLaunch says");
 static_assert(sizeof(GatherLaunch) <= 4096 && sizeof(AccumLaunch) <= 4096 && sizeof(PublishLaunch) <= 4096 &&
                   sizeof(CastGatherLaunch) <= 4096 && sizeof(ClearLaunch) <= 4096,
               "launch descriptors must fit the kernel-argument segment");

@@ -60,6 +60,7 @@ struct TileHead {
   uint32_t order;           // TileOrder
   uint32_t first_rank;      // rotation of the rank walk (never changes the result)
   uint32_t tiles_per_rank;  // seg_prefix[n_items]
+  uint32_t resident_below = 0;  // see is_resident
 };
 
 // Travels by value in the kernel-argument segment. seg_prefix[i] is the number of tiles that
@@ -300,6 +301,14 @@ ODC_HD bool is_whole(const TileWork& w) { return w.nv == kVecs; }
 // True when the tile has anything else to do: a partial run, the head or the tail.
 template <uint32_t kVecs = kTileVecs>
 ODC_HD bool has_edges(const TileWork& w) { return (w.nv != 0 && w.nv != kVecs) || w.head || w.tail; }
+
+// Whether the tile at this address of symmetric memory belongs to the part that stays in the last-level cache
+// (resident_below in odc_host.cpp): its 16 KiB granule's place in a sequence that is spread evenly over
+// [0, 2^32) lies below the line. A function of the address alone, so that launches of every kind agree,
+// spread so that every stretch of memory has its share; a lower line keeps a part of what a higher one does.
+ODC_HD bool is_resident(uintptr_t address, uint32_t below) {
+  return (uint32_t)(address >> 14) * 0x9E3779B1u < below;
+}
 
 // Cuts items [*next, n_items) into one launch: at most kMaxItems non-empty items and fewer than
 // kMaxTilesPerLaunch tiles. units(i) is item i's per-rank size in tile units (0 = skip);
