@@ -6,7 +6,7 @@
 // bookkeeping-only and dry-run arenas.
 //
 // Launch model: the work of one launch is cut into tiles of 1024 vectors (16 KiB, odc_tiles.h), or of
-// 256 (scatter_in_short_tiles, wants_short_tiles, publish_in_short_tiles);
+// 256 (scatter_in_short_tiles, wants_short_tiles, publish_in_short_tiles, stream_form);
 // per-item descriptors (<= ODC_MAX_ITEMS_PER_LAUNCH) travel BY VALUE in the kernel argument
 // segment, so a call needs no device-side work list, no host->device copy and no allocation;
 // longer item lists are split over several launches.
@@ -78,10 +78,11 @@ struct Options {
   int64_t cached_output_bytes = 64ll << 20;
   int64_t plain_output_bytes = 24ll << 20;    // see output_form
   int64_t cached_gradient_bytes = 128ll << 20;
-  int64_t resident_accumulation_bytes = 384ll << 20;  // these and the next three: see resident_below
-  int64_t resident_shard_bytes = 96ll << 20;
+  int64_t resident_accumulation_bytes = 320ll << 20;  // these and the next two: see resident_below
+  int64_t resident_shard_bytes = 80ll << 20;
   int64_t resident_above = 640ll << 20;
   int64_t resident_clear_bytes = 48ll << 20;
+  int64_t stream_bytes = 64ll << 20;  // see stream_form
   int64_t short_tiles_below = 32;             // see wants_short_tiles
   int64_t few_tiles = 32768;                  // see tile_form
 };
@@ -116,6 +117,7 @@ int64_t* option_slot(const char* name) {
   if (!strcmp(name, "resident_shard_bytes")) return &g_opt.resident_shard_bytes;
   if (!strcmp(name, "resident_above")) return &g_opt.resident_above;
   if (!strcmp(name, "resident_clear_bytes")) return &g_opt.resident_clear_bytes;
+  if (!strcmp(name, "stream_bytes")) return &g_opt.stream_bytes;
   if (!strcmp(name, "short_tiles_below")) return &g_opt.short_tiles_below;
   if (!strcmp(name, "few_tiles")) return &g_opt.few_tiles;
   return nullptr;
@@ -195,7 +197,7 @@ int check_compute(odc_arena* a, DeviceGuard& guard) {
 
 // What dry-run arenas have "launched" (process-wide, reset by odc_set_option("dry_run_reset", 0)).
 std::atomic<int64_t> g_dry_launches{0}, g_dry_tiles{0}, g_dry_workgroups{0};
-std::atomic<int64_t> g_dry_short{0}, g_dry_few{0};  // of the launches: those in kShortTiles, in kFewShortTiles
+std::atomic<int64_t> g_dry_short{0}, g_dry_few{0}, g_dry_stream{0};  // of the launches: those in kShortTiles, ...
 
 template <class Launch> TileForm form_of(const Launch& L) { return L.form; }
 TileForm form_of(const ClearLaunch&) { return kWholeTiles; }
@@ -213,6 +215,7 @@ int launch_tiles(const odc_arena* a, const Launch& L, uint32_t grid, Issue issue
     g_dry_workgroups += grid;
     g_dry_short += form_of(L) == kShortTiles;
     g_dry_few += form_of(L) == kFewShortTiles;
+    g_dry_stream += form_of(L) == kStreamTiles;
     return ODC_OK;
   }
   const int e = issue();
@@ -277,17 +280,17 @@ constexpr int64_t kSymmetric = -1;  // a line: the stream lies in symmetric memo
 // copies between two of them alike), so a fixed subset of the accumulations, touched twice by every
 // accumulate, and of the shards can live there from one kernel to the next (is_resident in odc_tiles.h
 // says which bytes; only their loads, and the stores of launches that do not load, go through the caches).
-// Up to 640 MiB in use there is none: gradients and gathered outputs of such sizes are cached themselves
-// and leave no room (bf16 into fp32, 17 Mi elements, three sets of buffers in turn: gather + accumulate
-// 41.8 us without, 48.8 with; 44 Mi 201.5 without, 190 with). Above it accumulations have 384 MiB's share of
-// the memory in use, shards 96 MiB's: with one unit in the arena as much of it as the cache takes, with
-// many the parts of all of them together still fit. us without -> with, a decoder layer at W = 8, three
-// units in turn: gather + accumulate 481 -> 472; store, 3 accumulates, 4 gathers and publish 1822 -> 1745;
-// FSDP2 minibatch of two microbatches, mixed 1664 -> 1643, bf16 1041 -> 1024; FSDP1 of 25 M elements in
-// fp16 214.5 -> 209; three microbatches of 68 M elements 455 -> 422. Ten units in turn, where a unit's
-// part is small and has to last for 25 GB: 481 -> 480, 1827 -> 1803, 1685 -> 1688, 1045.5 -> 1044.6, 214.4 ->
-// 211, 457 -> 444. (384 MiB's share against 256 and 512: 1643 / 1660 / 1633 and 1749 / 1772 / 1735 in
-// minibatches, 473 / 467 / 485 in single passes. Converting gathers gain nothing.)
+// Up to 640 MiB in use there is none, and no accumulation's where the launch's gradient is cached: gradients
+// and gathered outputs of such sizes leave no room (bf16 into fp32, three sets of buffers in turn: gather +
+// accumulate of 17 Mi elements 41.8 us without, 48.8 with; of 40 M 85 and 99). Otherwise accumulations have
+// 320 MiB's share of the memory in use, shards 80 MiB's: with one unit in the arena as much of it as the
+// cache takes, with many the parts of all of them together still fit. us without -> with, at W = 8, three
+// units in turn: gather + accumulate of 75 M elements 165 -> 158, two microbatches of it 329 -> 313; of a
+// decoder layer 473 -> 462; a layer's store, 3 accumulates, 4 gathers and publish 1802 -> 1750; its FSDP2
+// minibatch of two microbatches, mixed 1666 -> 1656, bf16 1044 -> 1033, fp32 2063 -> 2033. (384 MiB's share:
+// 314, 470, 1742, 1651, 1028; 256: 460, 1751, 1658, 1031. Ten units in turn, each part small and to last for
+// 25 GB, at 384: layer 482 -> 481, minibatches 1827 -> 1803, 1685 -> 1688, 1045.5 -> 1044.6. Converting
+// gathers gain nothing.)
 uint32_t resident_below(const odc_arena* a, const Options& opt, int64_t most) {
   const double in_use = (double)(a->in_use.load(std::memory_order_relaxed) * a->world);
   if (in_use <= (double)opt.resident_above) return 0;
@@ -306,17 +309,20 @@ OutputForm output_form(const Options& opt, bool cached, uint64_t bytes) {
   return bytes <= (uint64_t)opt.plain_output_bytes ? kKeep : kWriteThrough;
 }
 
-// The items that the next launch over [next, n_items) can take, and their whole tiles on one rank.
+// The items that the next launch over [next, n_items) can take, and their whole tiles and units on one rank.
 struct LaunchSize {
   uint32_t items = 0;
   uint64_t tiles = 0;
+  uint64_t units = 0;
 };
+constexpr uint64_t kMostStreamTiles = 1u << 24;  // well below a dispatch's most workgroups
 template <class Units>
 LaunchSize launch_size(uint32_t n_items, uint32_t next, uint64_t tile_units, Units units) {
   LaunchSize size;
   for (uint32_t i = next; i < n_items && size.items < (uint32_t)kMaxItems; ++i) {
     const uint64_t n = units(i);
     size.tiles += tiles_for(n, tile_units);
+    size.units += n;
     size.items += n != 0;
   }
   return size;
@@ -333,11 +339,7 @@ LaunchSize launch_size(uint32_t n_items, uint32_t next, uint64_t tile_units, Uni
 //   one item at W = 8, gather: 19 000 elements per segment 2.5 -> 2.2, 300 000 (37 tiles) 3.3 -> 3.2,
 //     600 000 (73) 4.55 -> 4.65; converting gather level from there on, store 5.0 -> 5.5 at 600 000.
 // Launches of longer segments stream best in whole tiles, with one exception (accum_streams_short).
-template <class Units>
-bool wants_short_tiles(uint32_t n_items, uint32_t next, uint64_t tile_units, Units units, int64_t below) {
-  const LaunchSize size = launch_size(n_items, next, tile_units, units);
-  return size.tiles < (uint64_t)below * size.items;
-}
+bool wants_short_tiles(const LaunchSize& size, int64_t below) { return size.tiles < (uint64_t)below * size.items; }
 
 // The same for an accumulate or a store. One that would take short tiles does not where 16-bit
 // gradients are stored into 16-bit accumulations and the launch has more than 1536 whole tiles: a short
@@ -351,12 +353,10 @@ bool wants_short_tiles(uint32_t n_items, uint32_t next, uint64_t tile_units, Uni
 // The read-modify-write of the same types has no such line: nontemporal short tiles are ahead or level
 // throughout (60 items of 16 tiles at W = 8 30.1, whole 33.5; 9 of 31 11.3 and 11.0), cached ones are
 // behind by up to 7 % at 4 to 17 Mi elements and ahead by as much at 57 Mi.
-template <class Units>
-bool scatter_in_short_tiles(const odc_arena* a, uint32_t n_items, uint32_t next, Units units, int64_t below,
-                            int grad_dtype, int acc_dtype, bool store) {
+bool scatter_in_short_tiles(const odc_arena* a, const LaunchSize& size, int64_t below, int grad_dtype, int acc_dtype,
+                            bool store) {
   if (accum_streams_short(grad_dtype, acc_dtype)) return true;
-  const LaunchSize size = launch_size(n_items, next, kTileElems, units);
-  if (size.tiles >= (uint64_t)below * size.items) return false;
+  if (!wants_short_tiles(size, below)) return false;
   const bool narrow = grad_dtype != ODC_DTYPE_F32 && acc_dtype != ODC_DTYPE_F32;
   return !(store && narrow) || size.tiles * a->world <= 1536;
 }
@@ -374,10 +374,7 @@ bool scatter_in_short_tiles(const odc_arena* a, uint32_t n_items, uint32_t next,
 //     81.2 -> 82.0;
 //   bf16 in place: 3.05 -> 2.7, 3.25 -> 3.05, 4.1 -> 3.0, 4.4 -> 4.2, but 19.5 -> 22.6, 134 -> 173,
 //     and 42.0 -> 41.4.
-template <class Units>
-bool publish_in_short_tiles(uint32_t n_items, uint32_t next, Units units, int acc_bytes) {
-  return acc_bytes == 4 || launch_size(n_items, next, kTileElems, units).tiles <= 1024;
-}
+bool publish_in_short_tiles(const LaunchSize& size, int acc_bytes) { return acc_bytes == 4 || size.tiles <= 1024; }
 
 // How the workgroups of a launch find their items. Up to eight fills of the chip (4096 workgroups of
 // 128 threads each) a launch is mostly the latency from its arguments to its first loads, and the
@@ -389,8 +386,38 @@ bool publish_in_short_tiles(uint32_t n_items, uint32_t next, Units units, int ac
 //   10 of 256 .. 262 144: 6.1 -> 5.9, 6.5 -> 6.2, 7.2 -> 6.9;
 //   112 of 160 000 (17 900 tiles): 41.2 -> 39.7, 41.1 -> 40.2; 112 of 640 000 (70 000 tiles): 156 -> 159,
 //   159 -> 162; 60 of 900 000 (53 000 tiles): 115 -> 115, 116.5 -> 117.6.
-TileForm tile_form(bool short_tiles, uint32_t n_tiles, int64_t few) {
-  return !short_tiles ? kWholeTiles : n_tiles <= (uint64_t)few ? kFewShortTiles : kShortTiles;
+TileForm tile_form(TileForm cut, uint32_t n_tiles, int64_t few) {
+  return cut == kShortTiles && n_tiles <= (uint64_t)few ? kFewShortTiles : cut;
+}
+
+// Whether a launch that is otherwise cut as `cut` is a long stream: more than 64 MiB written, past the caches,
+// by at most 64 items. Long streams go in short tiles, of which 12 workgroups are resident per CU
+// (kStreamWaves). They are bound by how HBM mixes reads and writes, and it mixes best with some 70 KB of
+// loads in flight per CU; how many that are had been decided by the time a workgroup took to find its item,
+// and by whole tiles. With the items found early (ItemsWalk) it has to be said. One kernel each on real
+// data, us, as they were -> long streams (16 and 10 workgroups per CU; 2 quads per lane in each):
+//   accumulate bf16 into fp32: a decoder layer at W = 8 354 -> 338 (349, 343), at W = 64 361 -> 350 (357,
+//     356), nine items of 11 .. 27 M elements 260 -> 253 (257, 259), 525 M elements 854 -> 826 (850, 814);
+//   fp32 into fp32: the layer 438 -> 420 (423, 411), nine items of 11 .. 13 M 222 -> 207 (206, 205); store
+//     142 -> 136 (141, 137);
+//   gather: the layer 137.4 -> 135.0 (136.9, 136.9), at W = 64 143.5 -> 139 (143, 143), 525 M 332 -> 327 (335,
+//     333); of fp32 273 -> 268 (271, 266).
+// Passes, gather + accumulate: the layer 482 -> 473, at W = 64 496 -> 481, 40 uneven items at W = 12 728 ->
+// 704, 525 M elements 1184 -> 1157; nine items of 2 .. 2.6 M in fp32 (92 MB written) 75.5 -> 71.5. Behind:
+// converting gathers (204 -> 225), stores of 16-bit gradients into fp32 (157.6 -> 161) and accumulates
+// into 16 bits (205 -> 220), which keep their shapes. Tiles of 128 vectors with 14 workgroups: 342 for the
+// layer's accumulate, 831 for 525 M.
+TileForm stream_form(const odc_arena* a, const Options& opt, const LaunchSize& size, uint64_t written_bytes, TileForm cut) {
+  const bool fits = size.items <= kSomeItems && size.tiles * a->world * tile_parts(kStreamTiles) <= kMostStreamTiles;
+  return fits && written_bytes > (uint64_t)opt.stream_bytes ? kStreamTiles : cut;
+}
+
+// The same for an accumulate or a store.
+TileForm scatter_stream_form(const odc_arena* a, const Options& opt, const LaunchSize& size, int grad_dtype, int acc_dtype,
+                             bool store, CachePolicy policy, TileForm cut) {
+  if (acc_dtype != ODC_DTYPE_F32) return cut;
+  if (grad_dtype == ODC_DTYPE_F32 ? cut != kWholeTiles : store || policy.read) return cut;
+  return stream_form(a, opt, size, size.units * 4 * a->world, cut);
 }
 
 // One-workgroup-per-tile launches are dealt out by the hardware dispatcher, which keeps as many
@@ -413,7 +440,7 @@ int odc_abi_version(void) { return ODC_HIP_ABI_VERSION; }
 
 int odc_set_option(const char* name, int64_t value) {
   if (name && !strcmp(name, "dry_run_reset")) {
-    g_dry_launches = 0; g_dry_tiles = 0; g_dry_workgroups = 0; g_dry_short = 0; g_dry_few = 0;
+    g_dry_launches = 0; g_dry_tiles = 0; g_dry_workgroups = 0; g_dry_short = 0; g_dry_few = 0; g_dry_stream = 0;
     return ODC_OK;
   }
   std::lock_guard<std::mutex> lk(g_opt_mu);
@@ -436,6 +463,7 @@ int odc_get_option(const char* name, int64_t* value) {
     if (!strcmp(name, "dry_run_workgroups")) { *value = g_dry_workgroups.load(); return ODC_OK; }
     if (!strcmp(name, "dry_run_short_launches")) { *value = g_dry_short.load(); return ODC_OK; }
     if (!strcmp(name, "dry_run_few_launches")) { *value = g_dry_few.load(); return ODC_OK; }
+    if (!strcmp(name, "dry_run_stream_launches")) { *value = g_dry_stream.load(); return ODC_OK; }
   }
   std::lock_guard<std::mutex> lk(g_opt_mu);
   int64_t* s = option_slot(name);
@@ -644,7 +672,7 @@ int dtype_bytes(int dt) {
 }
 
 // Units of one tile of a launch.
-uint64_t tile_units(uint64_t whole, bool short_tiles) { return short_tiles ? whole / kShortTileParts : whole; }
+uint64_t tile_units(uint64_t whole, TileForm form) { return whole / tile_parts(form); }
 
 // odc_tiles::fill_tile_table with its failure turned into an error message.
 // `order`, when given, maps positions of the launch order to the caller's item indices (for the
@@ -720,19 +748,23 @@ int odc_gather(odc_arena* a, const odc_gather_item* items, uint32_t n_items, uin
     L.tt.order = (uint32_t)opt.rank_major;
     L.tt.first_rank = first_rank;
     const auto units = [&](uint32_t i) { return items[i].shard_bytes; };
-    const bool short_tiles = wants_short_tiles(n_items, next, kTileBytes, units, opt.short_tiles_below);
+    const LaunchSize size = launch_size(n_items, next, kTileBytes, units);
+    const uint64_t out_bytes = size.units * a->world;
+    L.policy = cache_policy(a, opt, 0, kSymmetric, out_bytes, opt.cached_output_bytes);
+    TileForm cut = wants_short_tiles(size, opt.short_tiles_below) ? kShortTiles : kWholeTiles;
+    if (cut == kWholeTiles && !L.policy.read && !L.policy.written && opt.gather_blocks_per_cu == 0)
+      cut = stream_form(a, opt, size, out_bytes, cut);
     const int n = fill_launch(
-        L.tt, a->world, n_items, &next, tile_units(kTileBytes, short_tiles), units,
+        L.tt, a->world, n_items, &next, tile_units(kTileBytes, cut), units,
         [&](uint32_t slot, uint32_t i) {
           L.item[slot] = {static_cast<uint8_t*>(items[i].dst), items[i].src_offset, items[i].shard_bytes};
         });
     if (n < 0) return n;
     if (n == 0) continue;
-    L.form = tile_form(short_tiles, L.tt.n_tiles, opt.few_tiles);
+    L.form = tile_form(cut, L.tt.n_tiles, opt.few_tiles);
     bool ragged = false;
     uint64_t shard_bytes = 0;
     for (uint32_t k = 0; k < L.tt.n_items; ++k) shard_bytes += L.item[k].seg_bytes;
-    L.policy = cache_policy(a, opt, 0, kSymmetric, shard_bytes * a->world, opt.cached_output_bytes);
     L.output = output_form(opt, L.policy.written, shard_bytes * a->world);
     L.tt.resident_below = resident_below(a, opt, opt.resident_shard_bytes);
     for (uint32_t k = 0; k < L.tt.n_items; ++k)
@@ -776,17 +808,18 @@ int odc_gather_cast(odc_arena* a, const odc_gather_cast_item* items, uint32_t n_
     L.tt.order = (uint32_t)opt.rank_major;
     L.tt.first_rank = first_rank;
     const auto units = [&](uint32_t i) { return items[i].shard_elems; };
-    const bool short_tiles = wants_short_tiles(n_items, next, kTileElems, units, opt.short_tiles_below);
+    const LaunchSize size = launch_size(n_items, next, kTileElems, units);
+    L.policy = cache_policy(a, opt, 0, kSymmetric, 0, kSymmetric);
+    const TileForm cut = wants_short_tiles(size, opt.short_tiles_below) ? kShortTiles : kWholeTiles;
     const int n = fill_launch(
-        L.tt, a->world, n_items, &next, tile_units(kTileElems, short_tiles), units,
+        L.tt, a->world, n_items, &next, tile_units(kTileElems, cut), units,
         [&](uint32_t slot, uint32_t i) {
           L.item[slot] = {static_cast<uint8_t*>(items[i].dst), items[i].shard_elems * (uint64_t)db,
                           items[i].src_offset, items[i].shard_elems};
         });
     if (n < 0) return n;
     if (n == 0) continue;
-    L.form = tile_form(short_tiles, L.tt.n_tiles, opt.few_tiles);
-    L.policy = cache_policy(a, opt, 0, kSymmetric, 0, kSymmetric);
+    L.form = tile_form(cut, L.tt.n_tiles, opt.few_tiles);
     const uint32_t grid = grid_for(a, opt.gather_blocks_per_cu, L.tt.n_tiles, copy_threads(L.form));
     const uint32_t lds = lds_claim_for(a, opt.cast_resident_cap, grid, L.tt.n_tiles);
     if (int rc = launch_tiles(a, L, grid, [&] {
@@ -826,17 +859,18 @@ int odc_convert(odc_arena* a, const odc_convert_item* items, uint32_t n_items, i
     L.tt.order = (uint32_t)opt.rank_major;
     L.tt.first_rank = 0;
     const auto units = [&](uint32_t i) { return items[i].elems; };
-    const bool short_tiles = wants_short_tiles(n_items, next, kTileElems, units, opt.short_tiles_below);
+    const LaunchSize size = launch_size(n_items, next, kTileElems, units);
+    L.policy = cache_policy(a, opt, 0, kSymmetric, 0, kSymmetric);
+    const TileForm cut = wants_short_tiles(size, opt.short_tiles_below) ? kShortTiles : kWholeTiles;
     const int n = fill_launch(
-        L.tt, a->world, n_items, &next, tile_units(kTileElems, short_tiles), units,
+        L.tt, a->world, n_items, &next, tile_units(kTileElems, cut), units,
         [&](uint32_t slot, uint32_t i) {
           // the gather-with-cast kernel with every rank's output in that rank's own region
           L.item[slot] = {a->origin + items[i].dst_offset, a->rank_stride, items[i].src_offset, items[i].elems};
         });
     if (n < 0) return n;
     if (n == 0) continue;
-    L.form = tile_form(short_tiles, L.tt.n_tiles, opt.few_tiles);
-    L.policy = cache_policy(a, opt, 0, kSymmetric, 0, kSymmetric);
+    L.form = tile_form(cut, L.tt.n_tiles, opt.few_tiles);
     const uint32_t grid = grid_for(a, opt.gather_blocks_per_cu, L.tt.n_tiles, copy_threads(L.form));
     const uint32_t lds = lds_claim_for(a, opt.cast_resident_cap, grid, L.tt.n_tiles);
     if (int rc = launch_tiles(a, L, grid, [&] {
@@ -873,12 +907,14 @@ int odc_clear(odc_arena* a, const odc_span* spans, uint32_t n_spans, void* strea
     // A clear that leaves the resident part in the cache streams the rest past it, which takes longer (a layer's
     // 872 MB 118 -> 134 us) than leaving the last 256 MB behind unwritten, and pays from 48 MiB of resident
     // zeros on: FSDP2 minibatches 1660 -> 1643, 349 -> 339 (three units in turn, 85 MB each), but 352 -> 360
-    // and 331 -> 341 (ten, 26 MB each).
+    // and 331 -> 341 (ten, 26 MB each). Accumulations whose gradients are cached have no resident part; the
+    // line is that of 16-bit gradients into fp32.
     uint64_t cleared = 0;
-    for (uint32_t k = 0; k < L.tt.n_items; ++k) cleared += L.item[k].seg_bytes;
+    for (uint32_t k = 0; k < L.tt.n_items; ++k) cleared += L.item[k].seg_bytes * a->world;
     const uint32_t below = resident_below(a, opt, opt.resident_accumulation_bytes);
-    const double resident = (double)(cleared * a->world) * below / 4294967296.0;
-    L.tt.resident_below = resident >= (double)opt.resident_clear_bytes ? below : 0;
+    const double resident = (double)cleared * below / 4294967296.0;
+    if (cleared > 2 * (uint64_t)opt.cached_gradient_bytes && resident >= (double)opt.resident_clear_bytes)
+      L.tt.resident_below = below;
     const uint32_t grid = grid_for(a, opt.clear_blocks_per_cu, L.tt.n_tiles, kThreads);
     if (int rc = launch_tiles(a, L, grid, [&] { return odc_device::launch_clear(L, grid, stream); })) return rc;
   }
@@ -948,10 +984,23 @@ int scatter_launch(odc_arena* a, const odc_accum_item* items, uint32_t n_items, 
     L.tt.order = (uint32_t)opt.rank_major;
     L.tt.first_rank = 0;
     const auto units = [&](uint32_t i) { return items[order[i]].shard_elems; };
-    const bool short_tiles = scatter_in_short_tiles(a, n_items, next, units, opt.short_tiles_below, grad_dtype,
-                                                    acc_dtype, store);
+    const LaunchSize size = launch_size(n_items, next, kTileElems, units);
+    TileForm cut = scatter_in_short_tiles(a, size, opt.short_tiles_below, grad_dtype, acc_dtype, store) ? kShortTiles
+                                                                                                      : kWholeTiles;
+    {
+      uint64_t grad_elems = 0;
+      for (uint32_t i = next, k = 0; i < n_items && k < (uint32_t)kMaxItems; ++i) {
+        grad_elems += items[order[i]].grad_elems;
+        k += units(i) != 0;
+      }
+      L.policy = cache_policy(a, opt, grad_elems * gb, opt.cached_gradient_bytes, 0, kSymmetric);
+    }
+    const bool one_per_tile = (store ? opt.store_blocks_per_cu : opt.accum_blocks_per_cu) <= 0 &&
+                              (store || opt.accum_persistent_below_tiles == 0);
+    if (one_per_tile && !(L.policy.read && L.policy.written))
+      cut = scatter_stream_form(a, opt, size, grad_dtype, acc_dtype, store, L.policy, cut);
     const int n = fill_launch(
-        L.tt, a->world, n_items, &next, tile_units(kTileElems, short_tiles), units,
+        L.tt, a->world, n_items, &next, tile_units(kTileElems, cut), units,
         [&](uint32_t slot, uint32_t i) {
           const odc_accum_item& it = items[order[i]];
           L.item[slot] = {static_cast<const uint8_t*>(it.grad), it.grad_elems, it.acc_offset, it.shard_elems};
@@ -959,7 +1008,7 @@ int scatter_launch(odc_arena* a, const odc_accum_item* items, uint32_t n_items, 
         order);
     if (n < 0) return n;
     if (n == 0) continue;
-    L.form = tile_form(short_tiles, L.tt.n_tiles, opt.few_tiles);
+    L.form = tile_form(cut, L.tt.n_tiles, opt.few_tiles);
     // Tile order. Item-major (a rank's segment, then the next rank's, item by item) walks the
     // gradient contiguously and hops between rank regions at every segment; rank-outermost walks
     // one rank region from accumulation to accumulation (they are neighbours when registered
@@ -968,7 +1017,7 @@ int scatter_launch(odc_arena* a, const odc_accum_item* items, uint32_t n_items, 
     // rank-outermost: +1.1 % at W=4, +1.6 % at W=16 (370 tiles per segment on average), -1.9 % at
     // W=32 (185), -6 % at W=64, -10 % at W=128.
     const uint64_t segments = (uint64_t)L.tt.n_items * a->world;
-    const uint64_t whole_tiles = short_tiles ? L.tt.n_tiles / kShortTileParts : L.tt.n_tiles;
+    const uint64_t whole_tiles = L.tt.n_tiles / tile_parts(L.form);
     if (opt.accum_tile_order == 3)
       L.tt.order = whole_tiles < (uint64_t)opt.accum_short_segment_tiles * segments ? kRankOutermost : kItemMajor;
     else
@@ -987,10 +1036,7 @@ int scatter_launch(odc_arena* a, const odc_accum_item* items, uint32_t n_items, 
       ragged |= (L.item[k].acc_off & 127u) != 0 || ((L.item[k].seg_elems * ab) & 127u) != 0 ||
                 ((L.item[k].seg_elems * gb) & 127u) != 0 || ((uintptr_t)L.item[k].grad & 127u) != 0 ||
                 L.item[k].grad_elems != L.item[k].seg_elems * a->world;
-    uint64_t grad_elems = 0;
-    for (uint32_t k = 0; k < L.tt.n_items; ++k) grad_elems += L.item[k].grad_elems;
-    L.policy = cache_policy(a, opt, grad_elems * gb, opt.cached_gradient_bytes, 0, kSymmetric);
-    L.tt.resident_below = resident_below(a, opt, opt.resident_accumulation_bytes);
+    L.tt.resident_below = L.policy.read ? 0 : resident_below(a, opt, opt.resident_accumulation_bytes);
     int64_t blocks_per_cu = store ? opt.store_blocks_per_cu : opt.accum_blocks_per_cu;
     if (blocks_per_cu < 0)
       blocks_per_cu = whole_tiles < (uint64_t)opt.accum_persistent_below_tiles * segments ? 1 : 0;
@@ -1067,15 +1113,16 @@ int odc_publish(odc_arena* a, uint32_t rank, const odc_publish_item* items, uint
     L.tt.order = kItemMajor;
     L.tt.first_rank = 0;
     const auto units = [&](uint32_t i) { return items[i].elems; };
-    const bool short_tiles = publish_in_short_tiles(n_items, next, units, ab);
+    const LaunchSize size = launch_size(n_items, next, kTileElems, units);
+    const TileForm cut = publish_in_short_tiles(size, ab) ? kShortTiles : kWholeTiles;
     const int n = fill_launch(
-        L.tt, 1u, n_items, &next, tile_units(kTileElems, short_tiles), units,
+        L.tt, 1u, n_items, &next, tile_units(kTileElems, cut), units,
         [&](uint32_t slot, uint32_t i) {
           L.item[slot] = {static_cast<uint8_t*>(items[i].out), items[i].acc_offset, items[i].elems};
         });
     if (n < 0) return n;
     if (n == 0) continue;
-    L.form = tile_form(short_tiles, L.tt.n_tiles, opt.few_tiles);
+    L.form = tile_form(cut, L.tt.n_tiles, opt.few_tiles);
     // one workgroup per tile: the division sequence wants the occupancy, and the launch is short
     const uint32_t grid = grid_for(a, opt.publish_blocks_per_cu, L.tt.n_tiles, publish_threads(L.form));
     const uint32_t lds = lds_claim_for(a, opt.publish_resident_cap, grid, L.tt.n_tiles);

@@ -14,8 +14,8 @@
 // Launch model shared by the kernels: the work of one launch is cut into tiles of 1024 vectors
 // (16 KiB), done by workgroups of 256 threads or 512 (odc_launch.h says which), or into short tiles of 256
 // vectors, done by 128 threads: launches of short segments (wants_short_tiles in odc_host.cpp) and
-// every accumulate and store of 16-bit gradients into fp32 (accum_streams_short in odc_launch.h), and
-// every publish of fp32 accumulations (publish_in_short_tiles in odc_host.cpp).
+// every accumulate and store of 16-bit gradients into fp32 (accum_streams_short in odc_launch.h), every
+// publish of fp32 accumulations (publish_in_short_tiles in odc_host.cpp), and long streams (stream_form there).
 // Workgroups walk the tiles with a grid-stride loop, by default one workgroup per tile, so that,
 // at any instant, the whole chip streams one compact window of memory. Per-item
 // descriptors (<= ODC_MAX_ITEMS_PER_LAUNCH; launches of one item and of up to 16 have smaller tables) travel
@@ -247,23 +247,28 @@ struct FewTilesWalk {
 // nine items at W = 8, us, gather / accumulate / publish of bf16 into fp32 by elements per rank and item:
 // 4096 2.49 / 2.72 / 2.55 -> 2.43 / 2.70 / 2.36, 30 000 3.59 / 4.47 / 2.71 -> 3.38 / 4.42 / 2.60, 300 000
 // 13.5 / 31.9 / 5.8 -> 13.0 / 30.2 / 5.75, 3 M (HBM bound) level; converting gather 30 000 4.36 -> 4.05.
-template <class Launch>
-struct FewItemsWalk {
+// Up to kSomeItems items have four such tables behind one of their first entries: one round trip more.
+template <class Launch, uint32_t kItems>
+struct ItemsWalk {
   typedef typename Launch::Desc Desc;
   static constexpr bool kOneTile = true;
   TileHead tt;
   uint8_t* base;
   uint64_t rank_stride;
   Desc it = {};
-  u32x16 before;
+  u32x16 before;        // of the only block
+  u32x4 block_before;   // of several
 
-  __device__ __forceinline__ explicit FewItemsWalk(const Launch& launch) {
-    static_assert(kFewItems == 16, "one scalar load");
-    __builtin_memcpy(&before, launch.tt.tiles_before, sizeof(before));
+  __device__ __forceinline__ explicit ItemsWalk(const Launch& launch) {
+    static_assert(kFewItems == 16 && (kItems == kFewItems || kItems == 4 * kFewItems), "one scalar load");
+    if constexpr (kItems == kFewItems) __builtin_memcpy(&before, launch.tt.tiles_before, sizeof(before));
+    else __builtin_memcpy(&block_before, launch.tt.block_before, sizeof(block_before));
     tt = launch.tt;
     uint64_t b = (uint64_t)(uintptr_t)launch.base, stride = launch.rank_stride;
-    asm volatile("" : "+s"(tt.world), "+s"(tt.order), "+s"(tt.first_rank), "+s"(tt.tiles_per_rank), "+s"(tt.resident_below), "+s"(b), "+s"(stride),
-                      "+s"(before));
+    asm volatile("" : "+s"(tt.world), "+s"(tt.order), "+s"(tt.first_rank), "+s"(tt.tiles_per_rank), "+s"(tt.resident_below),
+                      "+s"(b), "+s"(stride));
+    if constexpr (kItems == kFewItems) asm volatile("" : "+s"(before));
+    else asm volatile("" : "+s"(block_before));
     base = as_global(reinterpret_cast<uint8_t*>((uintptr_t)b));
     rank_stride = stride;
   }
@@ -273,16 +278,22 @@ struct FewItemsWalk {
   }
   template <uint32_t kUnits>
   __device__ __forceinline__ TileCoord locate(const Launch& launch, uint32_t t) {
-    const FewItemsTile f = few_items_find(tt, before, t);
+    ItemsTile f = items_position(tt, t);
+    if constexpr (kItems != kFewItems) {
+      f.item = kFewItems * count_before<4>(block_before, f.position);
+      __builtin_memcpy(&before, launch.tt.tiles_before + f.item, sizeof(before));
+    }
+    f.item += count_before<kFewItems>(before, f.position);
     it = launch.item[f.item];
-    return few_items_coord(tt, f, launch.tt.tiles_before[f.item], (uint32_t)tiles_for(it.units(), kUnits));
+    return items_coord(tt, f, launch.tt.tiles_before[f.item], (uint32_t)tiles_for(it.units(), kUnits));
   }
 };
 
 // The walk that goes with a launch's kind of table.
 template <class Launch, bool kFew, class Table = decltype(Launch::tt)> struct WalkOf;
 template <class Launch, bool kFew> struct WalkOf<Launch, kFew, TileHead> { typedef SingleWalk<typename Launch::Desc> type; };
-template <class Launch, bool kFew> struct WalkOf<Launch, kFew, FewItemsTable> { typedef FewItemsWalk<Launch> type; };
+template <class Launch, bool kFew, uint32_t kItems>
+struct WalkOf<Launch, kFew, ItemsTable<kItems>> { typedef ItemsWalk<Launch, kItems> type; };
 template <class Launch> struct WalkOf<Launch, false, TileTable> { typedef TableWalk<Launch> type; };
 template <class Launch> struct WalkOf<Launch, true, TileTable> { typedef FewTilesWalk<Launch> type; };
 template <class Launch, bool kFew = false> using TileWalk = typename WalkOf<Launch, kFew>::type;
@@ -295,6 +306,11 @@ __device__ __forceinline__ void each_tile(const Walk& walk, const Launch& launch
   else
     for (uint32_t t = blockIdx.x; t < walk.n_tiles(launch); t += gridDim.x) body(t);
 }
+
+// Keeps a kernel at no more than so many wavefronts per SIMD: the compiler has it claim the registers of the
+// others. kStreamWaves: stream_form in odc_host.cpp.
+#define ODC_RESIDENT_WAVES(n) __attribute__((amdgpu_waves_per_eu(n, n)))
+constexpr int kMostWaves = 8, kStreamWaves = 6;
 
 // ---- gather -------------------------------------------------------------------------------
 // Everything of a tile that is not a run of T * U whole vectors: the last partial run, the
@@ -330,8 +346,8 @@ __device__ __attribute__((noinline)) void gather_edges(uint8_t* d, const uint8_t
 
 // T threads do a tile of T * U vectors in one step; the copies stream best from 512-thread
 // workgroups, of which 4 fit a CU.
-template <class Launch, bool kSrcCached, OutputForm kDst, bool kFew, int T, int U>
-__global__ __launch_bounds__(T) void gather_kernel(const Launch launch) {
+template <class Launch, bool kSrcCached, OutputForm kDst, bool kFew, int T, int U, int kWaves = kMostWaves>
+__global__ __launch_bounds__(T) ODC_RESIDENT_WAVES(kWaves) void gather_kernel(const Launch launch) {
   constexpr uint32_t kVecs = T * U;
   static_assert(kVecs == kTileVecs || kVecs == kShortTileVecs, "a whole tile or a short one");
   static_assert(T >= ODC_BODY_ALIGN - 1, "one lane per head byte");
@@ -579,8 +595,9 @@ __device__ __attribute__((noinline)) void accum_edges(uint8_t* acc, const uint8_
   if (do_tail) as[tail_at] = Codec<A>::narrow(Codec<A>::widen(tail_araw) + Codec<G>::widen(tail_graw));
 }
 
-template <class Launch, class G, class A, bool kStore, bool kGradCached, bool kAccCached, bool kFew, int T, int U>
-__global__ __launch_bounds__(T) void accum_kernel(const Launch launch) {
+template <class Launch, class G, class A, bool kStore, bool kGradCached, bool kAccCached, bool kFew, int T, int U,
+          int kWaves = kMostWaves>
+__global__ __launch_bounds__(T) ODC_RESIDENT_WAVES(kWaves) void accum_kernel(const Launch launch) {
   constexpr uint32_t kVecs = T * U;  // quads
   static_assert(kVecs == kTileVecs || kVecs == kShortTileVecs, "a whole tile or a short one");
   typedef typename Quad<G>::vec_t gvec_t;
@@ -859,6 +876,9 @@ __global__ __launch_bounds__(T) void publish_kernel(const Launch launch) {
 template <class Launch> using kernel_fn = void (*)(const Launch);
 // Launches of one item or of few have one way to find it: one kernel serves both short forms.
 template <class Launch> constexpr bool kSearches = std::is_same_v<decltype(Launch::tt), TileTable>;
+// Which launches long streams come in, and which are for nothing else.
+template <class Launch> constexpr bool kStreams = !kSearches<Launch>;
+template <class Launch> constexpr bool kStreamsOnly = std::is_same_v<decltype(Launch::tt), ItemsTable<kSomeItems>>;
 
 #define ODC_FOR_EACH_DTYPE_PAIR(X)                    \
   X(ODC_DTYPE_BF16, bf16_tag, ODC_DTYPE_BF16, bf16_tag) \
@@ -880,15 +900,35 @@ kernel_fn<L> pick_rmw(CachePolicy policy) {
                      : accum_kernel<L, G, A, false, false, false, kFew, T, U>;
 }
 
-template <class L, class G, class A, bool kFew, int T, int U>
+template <class L, class G, class A, bool kFew, int T, int U, int kWaves = kMostWaves>
 kernel_fn<L> pick_store(CachePolicy policy) {
-  return policy.read ? accum_kernel<L, G, A, true, true, false, kFew, T, U>
-                     : accum_kernel<L, G, A, true, false, false, kFew, T, U>;
+  return policy.read ? accum_kernel<L, G, A, true, true, false, kFew, T, U, kWaves>
+                     : accum_kernel<L, G, A, true, false, false, kFew, T, U, kWaves>;
 }
 
 // kShortOnly: accum_streams_short says so, there is no kernel of whole tiles.
 template <class L, class G, class A, bool kShortOnly>
+kernel_fn<L> pick_accum_tiles(bool store, CachePolicy policy, TileForm form);
+
+template <class L, class G, class A, bool kShortOnly>
 kernel_fn<L> pick_accum_form(bool store, CachePolicy policy, TileForm form) {
+  if (form == kStreamTiles) {  // into fp32: what scatter_stream_form in odc_host.cpp sends here
+    if constexpr (kStreams<L> && Codec<A>::kBytes == 4) {
+      if constexpr (Codec<G>::kBytes == 4) {
+        if (store) return pick_store<L, G, A, false, kShortThreads, kShortUnroll, kStreamWaves>(policy);
+        if (policy.read) return accum_kernel<L, G, A, false, true, false, false, kShortThreads, kShortUnroll, kStreamWaves>;
+      }
+      if (!store && !policy.read)
+        return accum_kernel<L, G, A, false, false, false, false, kShortThreads, kShortUnroll, kStreamWaves>;
+    }
+    return nullptr;
+  }
+  if constexpr (kStreamsOnly<L>) return nullptr;
+  else return pick_accum_tiles<L, G, A, kShortOnly>(store, policy, form);
+}
+
+template <class L, class G, class A, bool kShortOnly>
+kernel_fn<L> pick_accum_tiles(bool store, CachePolicy policy, TileForm form) {
   if (form == kFewShortTiles)
     return store ? pick_store<L, G, A, kSearches<L>, kShortThreads, kShortUnroll>(policy)
                  : pick_rmw<L, G, A, kSearches<L>, kShortThreads, kShortUnroll>(policy);
@@ -916,9 +956,17 @@ kernel_fn<L> pick_accum(int g, int a, bool store, CachePolicy policy, TileForm f
 
 template <class L, bool kSrcCached, OutputForm kDst>
 kernel_fn<L> pick_gather_form(TileForm form) {
+  if (form == kStreamTiles) {
+    if constexpr (kStreams<L> && kDst == kStream && !kSrcCached)
+      return gather_kernel<L, false, kStream, false, kShortThreads, kShortUnroll, kStreamWaves>;
+    else return nullptr;
+  }
+  if constexpr (kStreamsOnly<L>) return nullptr;
+  else {
   if (form == kFewShortTiles) return gather_kernel<L, kSrcCached, kDst, kSearches<L>, kShortThreads, kShortUnroll>;
   if (form == kShortTiles) return gather_kernel<L, kSrcCached, kDst, false, kShortThreads, kShortUnroll>;
   return gather_kernel<L, kSrcCached, kDst, false, kCopyThreads, kCopyUnroll>;
+  }
 }
 
 template <class L, bool kSrcCached>
@@ -974,8 +1022,8 @@ kernel_fn<L> pick_publish(int a, int o, TileForm form) {  // (accumulation dtype
 template <class Form, class Launch>
 Form short_form(const Launch& L) {
   Form s;
-  if constexpr (std::is_same_v<decltype(s.tt), FewItemsTable>) s.tt = few_items_table(L.tt);
-  else s.tt = L.tt;
+  if constexpr (std::is_same_v<decltype(s.tt), TileHead>) s.tt = L.tt;
+  else s.tt = items_table<std::size(decltype(s.tt.tiles_before){})>(L.tt);
   s.base = L.base;
   s.rank_stride = L.rank_stride;
   std::copy_n(L.item, std::min<size_t>(L.tt.n_items, std::size(s.item)), s.item);
@@ -999,15 +1047,16 @@ template <class L> struct Form { typedef L type; };
 // The short forms of a launch.
 template <class Launch> struct ShortForms {
   typedef SingleLaunch<typename Launch::Desc> Single;
-  typedef FewItemsLaunch<typename Launch::Desc> FewItems;
+  typedef ItemsLaunch<typename Launch::Desc, kFewItems> FewItems;
+  typedef ItemsLaunch<typename Launch::Desc, kSomeItems> SomeItems;
 };
 template <> struct ShortForms<PublishLaunch> {
   typedef PublishSingle Single;
   typedef PublishFewItems FewItems;
 };
 
-// pick(Form<L>) names the kernel for launches of type L.
-// by_table: several items take the full tables, however few they are.
+// pick(Form<L>) names the kernel for launches of type L. by_table: several items take the full tables,
+// however few they are.
 template <class Launch, class Pick>
 int launch_form(const Launch& L, uint32_t grid, uint32_t threads, uint32_t lds_bytes, void* stream, Pick pick,
                 bool by_table = false) {
@@ -1018,6 +1067,8 @@ int launch_form(const Launch& L, uint32_t grid, uint32_t threads, uint32_t lds_b
   if (grid != L.tt.n_tiles) return issue(L);  // workgroups of more than one tile walk the full tables
   if (L.tt.n_items == 1) return issue(short_form<typename ShortForms<Launch>::Single>(L));
   if (L.tt.n_items <= kFewItems && !by_table) return issue(short_form<typename ShortForms<Launch>::FewItems>(L));
+  if constexpr (std::is_same_v<Launch, GatherLaunch> || std::is_same_v<Launch, AccumLaunch>)
+    if (L.form == kStreamTiles) return issue(short_form<typename ShortForms<Launch>::SomeItems>(L));
   return issue(L);
 }
 

@@ -37,8 +37,10 @@ struct CachePolicy {
 enum OutputForm : uint32_t { kStream, kWriteThrough, kKeep };
 
 // How a launch is cut, and how its workgroups find their items (wants_short_tiles and tile_form in
-// odc_host.cpp).
-enum TileForm : uint32_t { kWholeTiles, kShortTiles, kFewShortTiles };
+// odc_host.cpp). kStreamTiles: short tiles of a long stream (stream_form there).
+enum TileForm : uint32_t { kWholeTiles, kShortTiles, kFewShortTiles, kStreamTiles };
+
+inline uint32_t tile_parts(TileForm form) { return form == kWholeTiles ? 1 : odc_tiles::kShortTileParts; }
 
 // 16-bit gradients into fp32 accumulations are accumulated and stored in short tiles whatever the
 // sizes. What bounds these streams is how reads and writes mix in HBM, and 16 workgroups of 128
@@ -113,16 +115,17 @@ struct SingleLaunch {
   D item[1];
 };
 
-// One of 2 to kFewItems items, as the parameters of a layer are, goes out with tables of that size: 488 to
-// 616 bytes of arguments (about 0.6 us less of host time than 4 KB), and the whole prefix table in one
-// scalar load (FewItemsWalk in odc_kernels.hip). Both short forms are for launches of one workgroup per tile.
-template <class D>
-struct FewItemsLaunch {
+// One of 2 to kFewItems items, as the parameters of a layer are, goes out with tables of that size: 496 to
+// 624 bytes of arguments (about 0.6 us less of host time than 4 KB), and the whole prefix table in one
+// scalar load (ItemsWalk in odc_kernels.hip). Both short forms are for launches of one workgroup per tile.
+// Long streams of up to kSomeItems have such tables too.
+template <class D, uint32_t kItems>
+struct ItemsLaunch {
   typedef D Desc;
-  odc_tiles::FewItemsTable tt;
+  odc_tiles::ItemsTable<kItems> tt;
   uint8_t* base;  // arena base (rank 0 region)
   uint64_t rank_stride;
-  D item[odc_tiles::kFewItems];
+  D item[kItems];
 };
 
 // One record per item, read with scalar loads by the workgroup that works on the item.
@@ -213,7 +216,7 @@ struct PublishLaunch {  // one rank's region only: tt.world == 1
 struct PublishSingle : SingleLaunch<PublishDesc> {
   PublishScale scale;
 };
-struct PublishFewItems : FewItemsLaunch<PublishDesc> {
+struct PublishFewItems : ItemsLaunch<PublishDesc, odc_tiles::kFewItems> {
   PublishScale scale;
 };
 static_assert(sizeof(SingleLaunch<ClearDesc>) == 64 && sizeof(PublishSingle) == 88, "as SingleLaunch says");

@@ -182,47 +182,59 @@ ODC_HD TileCoord single_item_coord(const TileHead& tt, uint32_t t) {
   return c;
 }
 
-// A launch of up to kFewItems items with one workgroup per tile: the table fits one scalar load, and holds
-// what the tile order needs, so that no tile divides twice: the tiles before item i in one rank segment
-// each where ranks are outermost, in the whole launch where items are. Entries past the last item hold
-// the total.
+// A launch of up to kItems items with one workgroup per tile: the table is read in blocks of kFewItems
+// entries, one scalar load each, and holds what the tile order needs, so that no tile divides twice: the tiles
+// before item i in one rank segment each where ranks are outermost, in the whole launch where items
+// are. Entries past the last item hold the total.
 constexpr uint32_t kFewItems = 16;
-struct FewItemsTable : TileHead {
-  uint32_t tiles_before[kFewItems];
+constexpr uint32_t kSomeItems = 64;
+template <uint32_t kItems>
+struct ItemsTable : TileHead {
+  uint32_t block_before[kItems / kFewItems];  // tiles_before of each block's first item
+  uint32_t tiles_before[kItems];
 };
 
-inline FewItemsTable few_items_table(const TileTable& tt) {
-  FewItemsTable few;
-  static_cast<TileHead&>(few) = tt;
-  for (uint32_t i = 0; i < kFewItems; ++i)
-    few.tiles_before[i] = tt.seg_prefix[i] * (tt.order == kRankOutermost ? 1u : tt.world);
-  return few;
+template <uint32_t kItems>
+inline ItemsTable<kItems> items_table(const TileTable& tt) {
+  static_assert(kItems % kFewItems == 0 && kItems <= (uint32_t)kMaxItems, "whole blocks of the full table");
+  ItemsTable<kItems> t;
+  static_cast<TileHead&>(t) = tt;
+  for (uint32_t i = 0; i < kItems; ++i) {
+    t.tiles_before[i] = tt.seg_prefix[i] * (tt.order == kRankOutermost ? 1u : tt.world);
+    if (i % kFewItems == 0) t.block_before[i / kFewItems] = t.tiles_before[i];
+  }
+  return t;
 }
 
 // A tile of such a launch: its item, its rank (rank outermost only) and its position, among all the launch's
 // tiles or the rank's.
-struct FewItemsTile {
+struct ItemsTile {
   uint32_t item, rank, position;
 };
 
-// before: tiles_before in any form that can be indexed (the kernels hold it in scalar registers). The item is
-// the number of later ones that do not begin behind the position, counted by sign bits: every value
-// is less than 2^31.
-template <class Before>
-ODC_HD FewItemsTile few_items_find(const TileHead& tt, const Before& before, uint32_t t) {
-  static_assert(kMaxTilesPerLaunch <= 1ull << 31, "sign bits");
-  FewItemsTile f = {kFewItems - 1, 0, t};
+// Tile t's rank and position.
+ODC_HD ItemsTile items_position(const TileHead& tt, uint32_t t) {
+  ItemsTile f = {0, 0, t};
   if (tt.order == kRankOutermost) {
     f.rank = t / tt.tiles_per_rank;
     f.position = t - f.rank * tt.tiles_per_rank;
   }
-#pragma unroll
-  for (uint32_t i = 1; i < kFewItems; ++i) f.item -= (f.position - before[i]) >> 31;
   return f;
 }
 
+// The number of before[1] .. before[n - 1] that do not lie behind the position, for ascending values less than
+// 2^31: counted by sign bits. before: in any form that can be indexed (the kernels hold it in scalar registers).
+template <uint32_t n, class Before>
+ODC_HD uint32_t count_before(const Before& before, uint32_t position) {
+  static_assert(kMaxTilesPerLaunch <= 1ull << 31, "sign bits");
+  uint32_t found = n - 1;
+#pragma unroll
+  for (uint32_t i = 1; i < n; ++i) found -= (position - before[i]) >> 31;
+  return found;
+}
+
 // first: tiles_before of the item; per_rank: the item's tiles in one rank segment
-ODC_HD TileCoord few_items_coord(const TileHead& tt, FewItemsTile f, uint32_t first, uint32_t per_rank) {
+ODC_HD TileCoord items_coord(const TileHead& tt, ItemsTile f, uint32_t first, uint32_t per_rank) {
   TileCoord c;
   c.item = f.item;
   f.position -= first;
