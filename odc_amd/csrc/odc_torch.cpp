@@ -15,6 +15,10 @@
 #include <Python.h>
 
 #include <ATen/core/Tensor.h>
+#include <ATen/ops/as_strided.h>
+#include <ATen/ops/empty.h>
+#include <torch/csrc/Dtype.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <cstddef>
@@ -580,6 +584,94 @@ PyObject* publish(PyObject*, PyObject* const* args, Py_ssize_t n) {
   });
 }
 
+// ------------------------------------------------------------------------------------------------
+// tensors that a parameter group hands out
+// ------------------------------------------------------------------------------------------------
+// The GIL is not held in its scope: the allocator may wait for a thread that wants it.
+class WithoutGil {
+ public:
+  WithoutGil() : state_(PyEval_SaveThread()) {}
+  ~WithoutGil() { PyEval_RestoreThread(state_); }
+  WithoutGil(const WithoutGil&) = delete;
+  WithoutGil& operator=(const WithoutGil&) = delete;
+
+ private:
+  PyThreadState* state_;
+};
+
+std::vector<int64_t> as_sizes(PyObject* o) {
+  const Sequence items(o, "sizes are a sequence");
+  std::vector<int64_t> sizes((size_t)items.size());
+  for (Py_ssize_t k = 0; k < items.size(); ++k) sizes[(size_t)k] = (int64_t)as_u64(items[k]);
+  return sizes;
+}
+
+PyObject* as_list(const std::vector<at::Tensor>& tensors) {
+  PyObject* list = PyList_New((Py_ssize_t)tensors.size());
+  if (!list) throw Failed();
+  for (size_t k = 0; k < tensors.size(); ++k) {
+    PyObject* t = THPVariable_Wrap(tensors[k]);
+    if (!t) {
+      Py_DECREF(list);
+      throw Failed();
+    }
+    PyList_SET_ITEM(list, (Py_ssize_t)k, t);
+  }
+  return list;
+}
+
+// Whatever `body` makes of tensors, in a list; what it throws becomes the exception that torch's own functions
+// raise (out of memory among them).
+template <class F>
+PyObject* tensor_list(F body) {
+  HANDLE_TH_ERRORS
+  try {
+    return body();
+  } catch (const Failed&) {
+    return nullptr;
+  }
+  END_HANDLE_TH_ERRORS
+}
+
+// empty_list(shapes, dtype, device index) -> a new GPU tensor of each shape, memory of its own
+PyObject* empty_list(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  return tensor_list([&] {
+    expect_args(n, 3);
+    const Sequence shapes(args[0], "shapes are a sequence");
+    if (!THPDtype_Check(args[1])) raise(PyExc_TypeError, "expected a torch.dtype, got %s", Py_TYPE(args[1])->tp_name);
+    const auto options = at::TensorOptions()
+                             .dtype(reinterpret_cast<THPDtype*>(args[1])->scalar_type)
+                             .device(at::Device(at::kCUDA, (c10::DeviceIndex)as_u64(args[2])));
+    std::vector<std::vector<int64_t>> sizes;
+    sizes.reserve((size_t)shapes.size());
+    for (Py_ssize_t k = 0; k < shapes.size(); ++k) sizes.push_back(as_sizes(shapes[k]));
+    std::vector<at::Tensor> out;
+    out.reserve(sizes.size());
+    {
+      WithoutGil nobody;
+      for (const auto& size : sizes) out.push_back(at::empty(size, options));
+    }
+    return as_list(out);
+  });
+}
+
+// strided_list(tensor, [(sizes, strides, offset), ...]) -> tensor.as_strided of each, offsets from the tensor's own
+PyObject* strided_list(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  return tensor_list([&] {
+    expect_args(n, 2);
+    const at::Tensor& t = as_tensor(args[0]);
+    const Sequence views(args[1], "views are a sequence");
+    std::vector<at::Tensor> out;
+    out.reserve((size_t)views.size());
+    for (Py_ssize_t k = 0; k < views.size(); ++k) {
+      const Sequence view(views[k], "a view is a sequence");
+      if (view.size() != 3) raise(PyExc_TypeError, "a view is sizes, strides and an offset");
+      out.push_back(at::as_strided(t, as_sizes(view[0]), as_sizes(view[1]), t.storage_offset() + (int64_t)as_u64(view[2])));
+    }
+    return as_list(out);
+  });
+}
+
 PyMethodDef module_methods[] = {
 #define ODC_METHOD(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(name)), METH_FASTCALL, nullptr}
     ODC_METHOD(bind),
@@ -588,6 +680,8 @@ PyMethodDef module_methods[] = {
     ODC_METHOD(accumulate_batch),
     ODC_METHOD(slice_layout),
     ODC_METHOD(clear),
+    ODC_METHOD(empty_list),
+    ODC_METHOD(strided_list),
     ODC_METHOD(publish),
 #undef ODC_METHOD
     {nullptr, nullptr, 0, nullptr}};
