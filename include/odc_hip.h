@@ -263,11 +263,12 @@ int odc_abi_version(void);
  *  - "short_tiles_below" (default 32): launches whose segments average fewer whole tiles are cut into
  *    short ones (0: none but those that always are). "few_tiles" (32768): up to so many short tiles
  *    a workgroup reads the whole table of the launch's items at once instead of searching it.
- *    "stream_bytes" (64 MiB): launches of up to 64 items that write more past the caches are long streams:
+ *    "stream_bytes" (8 MiB): launches of up to 64 items that write more past the caches are long streams:
  *    gathers without conversion, accumulates into fp32, stores of fp32; short tiles, fewer resident.
  *  - what a launch leaves in the caches: gathers of at most "cached_output_bytes" (64 MiB) of output
  *    leave it there, with plain stores up to "plain_output_bytes" (24 MiB) and written through the L2
- *    above; gradients of at most "cached_gradient_bytes" (128 MiB) per launch are read through the
+ *    above; converting gathers of at most "cast_output_bytes" (32 MiB) of output write it through the L2
+ *    (conversions of symmetric memory: "cached_output_bytes"); gradients of at most "cached_gradient_bytes" (128 MiB) per launch are read through the
  *    caches; so are shards and accumulations while all symmetric memory in use, over all ranks, is at most
  *    "cached_arena_bytes" (192 MiB). 0 streams past the caches. Above "resident_above" (640 MiB) in use a
  *    part of the symmetric memory is kept in the cache: of accumulations the share that

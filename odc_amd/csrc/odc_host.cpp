@@ -82,7 +82,8 @@ struct Options {
   int64_t resident_shard_bytes = 80ll << 20;
   int64_t resident_above = 640ll << 20;
   int64_t resident_clear_bytes = 48ll << 20;
-  int64_t stream_bytes = 64ll << 20;  // see stream_form
+  int64_t stream_bytes = 8ll << 20;  // see stream_form
+  int64_t cast_output_bytes = 32ll << 20;  // see cast_output_form
   int64_t short_tiles_below = 32;             // see wants_short_tiles
   int64_t few_tiles = 32768;                  // see tile_form
 };
@@ -117,6 +118,7 @@ int64_t* option_slot(const char* name) {
   if (!strcmp(name, "resident_shard_bytes")) return &g_opt.resident_shard_bytes;
   if (!strcmp(name, "resident_above")) return &g_opt.resident_above;
   if (!strcmp(name, "resident_clear_bytes")) return &g_opt.resident_clear_bytes;
+  if (!strcmp(name, "cast_output_bytes")) return &g_opt.cast_output_bytes;
   if (!strcmp(name, "stream_bytes")) return &g_opt.stream_bytes;
   if (!strcmp(name, "short_tiles_below")) return &g_opt.short_tiles_below;
   if (!strcmp(name, "few_tiles")) return &g_opt.few_tiles;
@@ -261,9 +263,8 @@ uint32_t grid_for(const odc_arena* a, int64_t blocks_per_cu, uint32_t n_tiles, u
 //     elements, 3 sets) fill + accumulate 12.7 -> 10.8 and accumulate alone 8.9 -> 7.9, with 144 MB
 //     accumulate alone 14.6 -> 12.4 and gather alone 7.0 -> 6.2; with 600 MB (24 sets) fill +
 //     accumulate 12.8 -> 13.1 and gather + read 7.4 -> 8.0. The line is 192 MiB of the 256.
-// A store does not read the accumulation and keeps it nontemporal (level at best when plain); so does
-// the converting gather with its output unless the arena fits: what the reader gains there (nine
-// items: nothing) the gather loses (17.9 -> 19.8).
+// A store does not read the accumulation and keeps it nontemporal (level at best when plain). The converting
+// gather's output: cast_output_form.
 CachePolicy cache_policy(const odc_arena* a, const Options& opt, uint64_t read_bytes, int64_t read_line,
                          uint64_t written_bytes, int64_t written_line) {
   const bool arena_fits = a->in_use.load(std::memory_order_relaxed) * a->world <= (uint64_t)opt.cached_arena_bytes;
@@ -307,6 +308,17 @@ uint32_t resident_below(const odc_arena* a, const Options& opt, int64_t most) {
 OutputForm output_form(const Options& opt, bool cached, uint64_t bytes) {
   if (!cached) return kStream;
   return bytes <= (uint64_t)opt.plain_output_bytes ? kKeep : kWriteThrough;
+}
+
+// The same for a gather that converts, and for a conversion of symmetric memory, which are ahead with the output
+// written through whoever reads it, as long as it leaves room for the gradients and accumulations of the
+// pass: up to 32 MiB, and 64 MiB of copies that the gathers behind find in the cache. Passes, fp32 into bf16 at
+// W = 8, us, nontemporal -> written through: gather + accumulate of 9 M elements 27.5 -> 26.9, 13 M 38.2 ->
+// 37.3, three microbatches of 9 M 92.7 -> 91.1, FSDP1 minibatches of 9 M 97.1 -> 95.3, 13 M 125.0 -> 122.7,
+// 18 M 162.6 -> 156; but gather + accumulate of 24 M 61.2 -> 63.0, 32 M 80.4 -> 86.5. FSDP2 minibatches
+// over converted copies of 12 to 57 MB: 185.8 -> 183.7, 245.3 -> 242.2.
+OutputForm cast_output_form(bool cached, uint64_t bytes, int64_t line) {
+  return cached ? kKeep : bytes <= (uint64_t)line ? kWriteThrough : kStream;
 }
 
 // The items that the next launch over [next, n_items) can take, and their whole tiles and units on one rank.
@@ -390,7 +402,7 @@ TileForm tile_form(TileForm cut, uint32_t n_tiles, int64_t few) {
   return cut == kShortTiles && n_tiles <= (uint64_t)few ? kFewShortTiles : cut;
 }
 
-// Whether a launch that is otherwise cut as `cut` is a long stream: more than 64 MiB written, past the caches,
+// Whether a launch that is otherwise cut as `cut` is a long stream: more than 8 MiB written, past the caches,
 // by at most 64 items. Long streams go in short tiles, of which 12 workgroups are resident per CU
 // (kStreamWaves). They are bound by how HBM mixes reads and writes, and it mixes best with some 70 KB of
 // loads in flight per CU; how many that are had been decided by the time a workgroup took to find its item,
@@ -403,7 +415,8 @@ TileForm tile_form(TileForm cut, uint32_t n_tiles, int64_t few) {
 //   gather: the layer 137.4 -> 135.0 (136.9, 136.9), at W = 64 143.5 -> 139 (143, 143), 525 M 332 -> 327 (335,
 //     333); of fp32 273 -> 268 (271, 266).
 // Passes, gather + accumulate: the layer 482 -> 473, at W = 64 496 -> 481, 40 uneven items at W = 12 728 ->
-// 704, 525 M elements 1184 -> 1157; nine items of 2 .. 2.6 M in fp32 (92 MB written) 75.5 -> 71.5. Behind:
+// 704, 525 M elements 1184 -> 1157; fp32 throughout, 20 M elements 71.0 -> 67.9, 14 M 52.9 -> 50.7, 9 M (36 MB
+// written) 35.4 -> 33.6, 3 M (12 MB) 15.9 -> 15.4. Behind:
 // converting gathers (204 -> 225), stores of 16-bit gradients into fp32 (157.6 -> 161) and accumulates
 // into 16 bits (205 -> 220), which keep their shapes. Tiles of 128 vectors with 14 workgroups: 342 for the
 // layer's accumulate, 831 for 525 M.
@@ -810,6 +823,7 @@ int odc_gather_cast(odc_arena* a, const odc_gather_cast_item* items, uint32_t n_
     const auto units = [&](uint32_t i) { return items[i].shard_elems; };
     const LaunchSize size = launch_size(n_items, next, kTileElems, units);
     L.policy = cache_policy(a, opt, 0, kSymmetric, 0, kSymmetric);
+    L.output = cast_output_form(L.policy.read, size.units * db * a->world, opt.cast_output_bytes);
     const TileForm cut = wants_short_tiles(size, opt.short_tiles_below) ? kShortTiles : kWholeTiles;
     const int n = fill_launch(
         L.tt, a->world, n_items, &next, tile_units(kTileElems, cut), units,
@@ -861,6 +875,8 @@ int odc_convert(odc_arena* a, const odc_convert_item* items, uint32_t n_items, i
     const auto units = [&](uint32_t i) { return items[i].elems; };
     const LaunchSize size = launch_size(n_items, next, kTileElems, units);
     L.policy = cache_policy(a, opt, 0, kSymmetric, 0, kSymmetric);
+    // (the copies are symmetric memory that every gather of the minibatch reads)
+    L.output = cast_output_form(L.policy.read, size.units * db * a->world, opt.cached_output_bytes);
     const TileForm cut = wants_short_tiles(size, opt.short_tiles_below) ? kShortTiles : kWholeTiles;
     const int n = fill_launch(
         L.tt, a->world, n_items, &next, tile_units(kTileElems, cut), units,

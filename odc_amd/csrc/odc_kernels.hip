@@ -112,7 +112,7 @@ __device__ __forceinline__ void store_vec(V* p, V v) {  // aligned
   if constexpr (kCached) *p = v; else __builtin_nontemporal_store(v, p);
 }
 
-// A whole tile of a gather's output: vector `i` of the kVecs that start at `tile`, an address that all
+// A whole tile of a gather's output, converted or not: vector `i` of the kVecs that start at `tile`, an address that all
 // lanes agree on. Outputs that the next kernel is to find in the last-level cache, but that are more
 // than the L2s hold, are written through the L2: left in it by plain stores they went to memory only as other
 // lines pushed them out, between the reads of whatever ran next. us, nontemporal / plain / written
@@ -121,13 +121,15 @@ __device__ __forceinline__ void store_vec(V* p, V v) {  // aligned
 //   an accumulate behind it, nothing reads the output: 32.1 / 31.9 / 29.4, 40.4 / 41.7 / 41.1;
 //   the products that read the parameters behind it (1024 tokens): 141 / 129 / 126.5, 184 / 160 / 158.5.
 constexpr int kSc1 = 16;  // of a buffer store: write through
-template <OutputForm kForm, uint32_t kVecs>
-__device__ __forceinline__ void store_output(u32x4* tile, uint32_t i, u32x4 v) {
-  if constexpr (kForm == kWriteThrough)
-    __builtin_amdgcn_raw_buffer_store_b128(v, __builtin_amdgcn_make_buffer_rsrc(tile, 0, kVecs * 16, 0x00027000),
-                                           (int)(i * 16), 0, kSc1);
-  else
+template <OutputForm kForm, uint32_t kVecs, class V>
+__device__ __forceinline__ void store_output(V* tile, uint32_t i, V v) {
+  if constexpr (kForm == kWriteThrough) {
+    const auto buffer = __builtin_amdgcn_make_buffer_rsrc(tile, 0, kVecs * sizeof(V), 0x00027000);
+    if constexpr (sizeof(V) == 16) __builtin_amdgcn_raw_buffer_store_b128(v, buffer, (int)(i * 16), 0, kSc1);
+    else __builtin_amdgcn_raw_buffer_store_b64(v, buffer, (int)(i * 8), 0, kSc1);
+  } else {
     store_vec<kForm == kKeep>(tile + i, v);
+  }
 }
 
 // ---- finding a tile's work ------------------------------------------------------------------
@@ -656,7 +658,7 @@ __global__ __launch_bounds__(T) ODC_RESIDENT_WAVES(kWaves) void accum_kernel(con
 // segment's size: the converted segments lie back to back), or, with stride = the distance
 // between rank regions and dst inside rank 0's region, the conversion of every rank's shard into
 // a second symmetric buffer.
-template <class S, class D, bool kCached, int T, int U>
+template <class S, class D, bool kSrcCached, bool kDstCached, int T, int U>
 __device__ __attribute__((noinline)) void cast_edges(uint8_t* d, const uint8_t* s, uint32_t chunk, SegShape g) {
   d = as_global(d);
   s = as_global(s);
@@ -682,7 +684,7 @@ __device__ __attribute__((noinline)) void cast_edges(uint8_t* d, const uint8_t* 
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const uint32_t q = u * T + tid;
-    if (q < left) raw[u] = load_any<kCached, svec_t>(sb + (size_t)q * sizeof(svec_t));
+    if (q < left) raw[u] = load_any<kSrcCached, svec_t>(sb + (size_t)q * sizeof(svec_t));
   }
   if (do_head) head_raw = ss[tid];
   if (do_tail) tail_raw = ss[tail_at];
@@ -692,14 +694,14 @@ __device__ __attribute__((noinline)) void cast_edges(uint8_t* d, const uint8_t* 
     if (q < left) {
       float f[4];
       Quad<S>::widen(raw[u], f);
-      store_vec<kCached>(dp + q, Quad<D>::narrow(f));
+      store_vec<kDstCached>(dp + q, Quad<D>::narrow(f));
     }
   }
   if (do_head) ds[tid] = Codec<D>::narrow(Codec<S>::widen(head_raw));
   if (do_tail) ds[tail_at] = Codec<D>::narrow(Codec<S>::widen(tail_raw));
 }
 
-template <class Launch, class S, class D, bool kCached, bool kFew, int T, int U>
+template <class Launch, class S, class D, bool kSrcCached, OutputForm kDst, bool kFew, int T, int U>
 __global__ __launch_bounds__(T) void cast_gather_kernel(const Launch launch) {
   constexpr uint32_t kVecs = T * U;  // quads
   static_assert(kVecs == kTileVecs || kVecs == kShortTileVecs, "a whole tile or a short one");
@@ -720,10 +722,10 @@ __global__ __launch_bounds__(T) void cast_gather_kernel(const Launch launch) {
     if (is_whole<kVecs>(w)) {
       const uint64_t e0 = g.head + w.v0 * 4;
       const uint8_t* sb = s + e0 * kSB + (size_t)tid * sizeof(svec_t);
-      dvec_t* dp = reinterpret_cast<dvec_t*>(d + e0 * kDB) + tid;
+      dvec_t* dp = reinterpret_cast<dvec_t*>(d + e0 * kDB);
       svec_t raw[U];
 #pragma unroll
-      for (int u = 0; u < U; ++u) raw[u] = load_any<kCached, svec_t>(sb + (size_t)u * T * sizeof(svec_t));
+      for (int u = 0; u < U; ++u) raw[u] = load_any<kSrcCached, svec_t>(sb + (size_t)u * T * sizeof(svec_t));
       // the head and the tail of the segment, when this whole tile owns them, in the same round trip
       typedef typename Codec<S>::raw_t sraw_t;
       typedef typename Codec<D>::raw_t draw_t;
@@ -739,12 +741,12 @@ __global__ __launch_bounds__(T) void cast_gather_kernel(const Launch launch) {
       for (int u = 0; u < U; ++u) {
         float f[4];
         Quad<S>::widen(raw[u], f);
-        store_vec<kCached>(dp + u * T, Quad<D>::narrow(f));
+        store_output<kDst, kVecs>(dp, u * T + tid, Quad<D>::narrow(f));
       }
       if (do_head) ds[tid] = Codec<D>::narrow(Codec<S>::widen(head_raw));
       if (do_tail) ds[tail_at] = Codec<D>::narrow(Codec<S>::widen(tail_raw));
     } else if (has_edges<kVecs>(w)) {
-      cast_edges<S, D, kCached, T, U>(d, s, c.chunk, g);
+      cast_edges<S, D, kSrcCached, kDst != kStream, T, U>(d, s, c.chunk, g);
     }
   });
 }
@@ -981,19 +983,25 @@ kernel_fn<L> pick_gather(bool shards_cached, OutputForm output, TileForm form) {
   return shards_cached ? pick_gather_output<L, true>(output, form) : pick_gather_output<L, false>(output, form);
 }
 
-// Shards and output of the converting gather are cached together or not at all.
-template <class L, class S, class D, bool kCached>
+template <class L, class S, class D, bool kSrcCached, OutputForm kDst>
 kernel_fn<L> pick_cast_gather_form(TileForm form) {
-  if (form == kFewShortTiles) return cast_gather_kernel<L, S, D, kCached, kSearches<L>, kShortThreads, kShortUnroll>;
-  if (form == kShortTiles) return cast_gather_kernel<L, S, D, kCached, false, kShortThreads, kShortUnroll>;
-  return cast_gather_kernel<L, S, D, kCached, false, kCopyThreads, kCopyUnroll>;
+  if (form == kFewShortTiles) return cast_gather_kernel<L, S, D, kSrcCached, kDst, kSearches<L>, kShortThreads, kShortUnroll>;
+  if (form == kShortTiles) return cast_gather_kernel<L, S, D, kSrcCached, kDst, false, kShortThreads, kShortUnroll>;
+  return cast_gather_kernel<L, S, D, kSrcCached, kDst, false, kCopyThreads, kCopyUnroll>;
+}
+
+// Shards are cached only together with the output, which is then kept with plain stores.
+template <class L, class S, class D>
+kernel_fn<L> pick_cast_gather_output(CachePolicy policy, OutputForm output, TileForm form) {
+  if (policy.read) return pick_cast_gather_form<L, S, D, true, kKeep>(form);
+  return output == kStream ? pick_cast_gather_form<L, S, D, false, kStream>(form)
+                           : pick_cast_gather_form<L, S, D, false, kWriteThrough>(form);
 }
 
 template <class L>
-kernel_fn<L> pick_cast_gather(int s, int d, CachePolicy policy, TileForm form) {  // (shard dtype, output dtype)
+kernel_fn<L> pick_cast_gather(int s, int d, CachePolicy policy, OutputForm output, TileForm form) {  // (shard dtype, output dtype)
 #define X(E1, T1, E2, T2) \
-  if (s == E1 && d == E2) \
-    return policy.read ? pick_cast_gather_form<L, T1, T2, true>(form) : pick_cast_gather_form<L, T1, T2, false>(form);
+  if (s == E1 && d == E2) return pick_cast_gather_output<L, T1, T2>(policy, output, form);
   ODC_FOR_EACH_DTYPE_PAIR(X)
 #undef X
   return nullptr;
@@ -1112,7 +1120,7 @@ bool is_out_of_memory(int code) { return code == (int)hipErrorOutOfMemory; }
 const char* error_string(int code) { return hipGetErrorString(static_cast<hipError_t>(code)); }
 
 bool has_accum(int g, int a) { return pick_accum<AccumLaunch>(g, a, false, {}, kShortTiles) != nullptr; }
-bool has_cast_gather(int s, int d) { return pick_cast_gather<CastGatherLaunch>(s, d, {}, kWholeTiles) != nullptr; }
+bool has_cast_gather(int s, int d) { return pick_cast_gather<CastGatherLaunch>(s, d, {}, kStream, kWholeTiles) != nullptr; }
 bool has_publish(int a, int o) { return pick_publish<PublishLaunch>(a, o, kShortTiles) != nullptr; }
 
 // Gathers of whole tiles are bound by HBM and stream better from workgroups that come to their loads one
@@ -1126,7 +1134,7 @@ int launch_gather(const GatherLaunch& L, uint32_t grid, uint32_t lds_bytes, void
 
 int launch_cast_gather(int s, int d, const CastGatherLaunch& L, uint32_t grid, uint32_t lds_bytes, void* stream) {
   return launch_form(L, grid, copy_threads(L.form), lds_bytes, stream, [&](auto form) {
-    return pick_cast_gather<typename decltype(form)::type>(s, d, L.policy, L.form);
+    return pick_cast_gather<typename decltype(form)::type>(s, d, L.policy, L.output, L.form);
   }, L.form == kWholeTiles);
 }
 

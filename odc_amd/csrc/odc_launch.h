@@ -158,7 +158,8 @@ struct CastGatherLaunch {
   TileTable tt;
   uint8_t* base;
   uint64_t rank_stride;
-  CachePolicy policy;    // these two pick the kernel
+  CachePolicy policy;    // these three pick the kernel
+  OutputForm output = kStream;
   TileForm form = kWholeTiles;
   CastGatherDesc item[kMaxItems];
 };

@@ -23,8 +23,8 @@ def _with_options(options):
 
 
 @pytest.mark.parametrize("what,elem,min_bytes", [  # bytes written per element, line of a cached input
-    (("gather",), 1, 64 * MB), (("odc_scatter_accumulate", BF16, F32), 4, 256 * MB), (("odc_scatter_accumulate", F32, F32), 4, 64 * MB),
-    (("odc_scatter_store", F32, F32), 4, 64 * MB), (("odc_scatter_store", BF16, F32), 4, None),
+    (("gather",), 1, 64 * MB), (("odc_scatter_accumulate", BF16, F32), 4, 256 * MB), (("odc_scatter_accumulate", F32, F32), 4, 8 * MB),
+    (("odc_scatter_store", F32, F32), 4, 8 * MB), (("odc_scatter_store", BF16, F32), 4, None),
     (("odc_scatter_accumulate", BF16, BF16), 2, None), (("odc_scatter_accumulate", F32, BF16), 2, None),
 ], ids=str)
 def test_which_launches_are_long_streams(what, elem, min_bytes):
