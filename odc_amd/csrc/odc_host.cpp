@@ -288,7 +288,7 @@ constexpr int64_t kSymmetric = -1;  // a line: the stream lies in symmetric memo
 // cache takes, with many the parts of all of them together still fit. us without -> with, at W = 8, three
 // units in turn: gather + accumulate of 75 M elements 165 -> 158, two microbatches of it 329 -> 313; of a
 // decoder layer 473 -> 462; a layer's store, 3 accumulates, 4 gathers and publish 1802 -> 1750; its FSDP2
-// minibatch of two microbatches, mixed 1666 -> 1656, bf16 1044 -> 1033, fp32 2063 -> 2033. (384 MiB's share:
+// minibatch of two microbatches, mixed 1666 -> 1656, bf16 1044 -> 1033, fp32 2061 -> 2039. (384 MiB's share:
 // 314, 470, 1742, 1651, 1028; 256: 460, 1751, 1658, 1031. Ten units in turn, each part small and to last for
 // 25 GB, at 384: layer 482 -> 481, minibatches 1827 -> 1803, 1685 -> 1688, 1045.5 -> 1044.6. Converting
 // gathers gain nothing.)
@@ -410,13 +410,13 @@ TileForm tile_form(TileForm cut, uint32_t n_tiles, int64_t few) {
 // data, us, as they were -> long streams (16 and 10 workgroups per CU; 2 quads per lane in each):
 //   accumulate bf16 into fp32: a decoder layer at W = 8 354 -> 338 (349, 343), at W = 64 361 -> 350 (357,
 //     356), nine items of 11 .. 27 M elements 260 -> 253 (257, 259), 525 M elements 854 -> 826 (850, 814);
-//   fp32 into fp32: the layer 438 -> 420 (423, 411), nine items of 11 .. 13 M 222 -> 207 (206, 205); store
-//     142 -> 136 (141, 137);
+//   fp32 into fp32: nine items of 11 .. 13 M 213 -> 207, their store 137 -> 135, the layer level (416 to 425);
 //   gather: the layer 137.4 -> 135.0 (136.9, 136.9), at W = 64 143.5 -> 139 (143, 143), 525 M 332 -> 327 (335,
-//     333); of fp32 273 -> 268 (271, 266).
+//     333); of fp32 273 -> 266, nine items of 11 .. 13 M 150 -> 144.
 // Passes, gather + accumulate: the layer 482 -> 473, at W = 64 496 -> 481, 40 uneven items at W = 12 728 ->
-// 704, 525 M elements 1184 -> 1157; fp32 throughout, 20 M elements 71.0 -> 67.9, 14 M 52.9 -> 50.7, 9 M (36 MB
-// written) 35.4 -> 33.6, 3 M (12 MB) 15.9 -> 15.4. Behind:
+// 704, 525 M elements 1184 -> 1157; fp32 throughout, minibatches of two microbatches, the layer 2096 -> 2067,
+// 20 M elements 132.9 -> 131.0, 14 M 97.8 -> 96.0, 9 M (36 MB written) 67.7 -> 66.6, 4.5 M 40.8 -> 39.8, 3 M
+// (12 MB) level. Behind:
 // converting gathers (204 -> 225), stores of 16-bit gradients into fp32 (157.6 -> 161) and accumulates
 // into 16 bits (205 -> 220), which keep their shapes. Tiles of 128 vectors with 14 workgroups: 342 for the
 // layer's accumulate, 831 for 525 M.

@@ -310,8 +310,9 @@ __device__ __forceinline__ void each_tile(const Walk& walk, const Launch& launch
 }
 
 // Keeps a kernel at no more than so many wavefronts per SIMD: the compiler has it claim the registers of the
-// others. kStreamWaves: stream_form in odc_host.cpp.
-#define ODC_RESIDENT_WAVES(n) __attribute__((amdgpu_waves_per_eu(n, n)))
+// others. kStreamWaves: stream_form in odc_host.cpp. kMostWaves asks for nothing: as a lower bound it would
+// have the compiler spill.
+#define ODC_RESIDENT_WAVES(n) __attribute__((amdgpu_waves_per_eu((n) < kMostWaves ? (n) : 1, n)))
 constexpr int kMostWaves = 8, kStreamWaves = 6;
 
 // ---- gather -------------------------------------------------------------------------------
