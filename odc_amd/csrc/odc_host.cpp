@@ -416,10 +416,9 @@ TileForm tile_form(TileForm cut, uint32_t n_tiles, int64_t few) {
 // Passes, gather + accumulate: the layer 482 -> 473, at W = 64 496 -> 481, 40 uneven items at W = 12 728 ->
 // 704, 525 M elements 1184 -> 1157; fp32 throughout, minibatches of two microbatches, the layer 2096 -> 2067,
 // 20 M elements 132.9 -> 131.0, 14 M 97.8 -> 96.0, 9 M (36 MB written) 67.7 -> 66.6, 4.5 M 40.8 -> 39.8, 3 M
-// (12 MB) level. Behind:
-// converting gathers (204 -> 225), stores of 16-bit gradients into fp32 (157.6 -> 161) and accumulates
-// into 16 bits (205 -> 220), which keep their shapes. Tiles of 128 vectors with 14 workgroups: 342 for the
-// layer's accumulate, 831 for 525 M.
+// (12 MB) level. Behind: converting gathers (204 -> 225), stores of 16-bit gradients into fp32 (157.6 -> 161)
+// and accumulates into 16 bits (205 -> 220), which keep their shapes. Tiles of 128 vectors with 14 workgroups:
+// 342 for the layer's accumulate, 831 for 525 M.
 TileForm stream_form(const odc_arena* a, const Options& opt, const LaunchSize& size, uint64_t written_bytes, TileForm cut) {
   const bool fits = size.items <= kSomeItems && size.tiles * a->world * tile_parts(kStreamTiles) <= kMostStreamTiles;
   return fits && written_bytes > (uint64_t)opt.stream_bytes ? kStreamTiles : cut;
