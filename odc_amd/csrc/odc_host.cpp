@@ -21,6 +21,7 @@
 #include <mutex>
 #include <new>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "odc_hip.h"
@@ -232,13 +233,17 @@ Options options_snapshot() {
 
 // blocks_per_cu > 0 asks for that many persistent workgroups per CU. Ragged launches (uneven
 // shards: unaligned reads, heads and tails) never get them: they hide their extra latency better
-// with one workgroup per tile, i.e. full occupancy (measured: +5..10 %).
-uint32_t grid_for(const odc_arena* a, int64_t blocks_per_cu, uint32_t n_tiles, uint32_t threads,
-                  bool ragged = false) {
+// with one workgroup per tile, i.e. full occupancy (measured: +5..10 %). ragged() looks at every item and
+// is asked only where persistent workgroups are.
+template <class Ragged>
+uint32_t grid_for(const odc_arena* a, int64_t blocks_per_cu, uint32_t n_tiles, uint32_t threads, Ragged ragged) {
   const uint32_t most = std::min(n_tiles, most_workgroups(threads));
-  if (blocks_per_cu <= 0 || ragged) return most;
+  if (blocks_per_cu <= 0 || ragged()) return most;
   const uint64_t cu = (uint64_t)a->n_cu, per_cu = (uint64_t)blocks_per_cu;
   return per_cu >= most ? most : (uint32_t)std::min<uint64_t>(cu * per_cu, most);
+}
+uint32_t grid_for(const odc_arena* a, int64_t blocks_per_cu, uint32_t n_tiles, uint32_t threads) {
+  return grid_for(a, blocks_per_cu, n_tiles, threads, [] { return false; });
 }
 
 // What a launch leaves in the caches. Nontemporal accesses stream fastest when nothing will be
@@ -322,22 +327,31 @@ OutputForm cast_output_form(bool cached, uint64_t bytes, int64_t line) {
 }
 
 // The items that the next launch over [next, n_items) can take, and their whole tiles and units on one rank.
+// also(i) is called for each of them: whatever else a launch's plan sums up over its items is summed on the
+// same walk. Passes of six launches, 300 small slices at W = 16, whose host time is level with their kernels',
+// took 36.7 -> 39.3 us when plans of long streams had walks of their own; with one walk, no division per
+// item and grid_for's look at the items only where it is used, 35.9 -> 36.1 and 37.5 -> 36.8 on two cards.
 struct LaunchSize {
   uint32_t items = 0;
   uint64_t tiles = 0;
   uint64_t units = 0;
 };
 constexpr uint64_t kMostStreamTiles = 1u << 24;  // well below a dispatch's most workgroups
-template <class Units>
-LaunchSize launch_size(uint32_t n_items, uint32_t next, uint64_t tile_units, Units units) {
+template <uint64_t kTileUnits, class Units, class Also>
+LaunchSize launch_size(uint32_t n_items, uint32_t next, Units units, Also also) {
   LaunchSize size;
   for (uint32_t i = next; i < n_items && size.items < (uint32_t)kMaxItems; ++i) {
     const uint64_t n = units(i);
-    size.tiles += tiles_for(n, tile_units);
+    size.tiles += tiles_for(n, kTileUnits);
     size.units += n;
     size.items += n != 0;
+    also(i);
   }
   return size;
+}
+template <uint64_t kTileUnits, class Units>
+LaunchSize launch_size(uint32_t n_items, uint32_t next, Units units) {
+  return launch_size<kTileUnits>(n_items, next, units, [](uint32_t) {});
 }
 
 // Whether the next launch over items [next, n_items) is cut into short tiles (256 vectors, done by
@@ -683,16 +697,17 @@ int dtype_bytes(int dt) {
   }
 }
 
-// Units of one tile of a launch.
-uint64_t tile_units(uint64_t whole, TileForm form) { return whole / tile_parts(form); }
-
 // odc_tiles::fill_tile_table with its failure turned into an error message.
 // `order`, when given, maps positions of the launch order to the caller's item indices (for the
-// message only: units and take already work on positions).
-template <class Units, class Take>
-int fill_launch(TileTable& tt, uint32_t world, uint32_t n_items, uint32_t* next, uint64_t tile_units,
-                Units units, Take take, const uint32_t* order = nullptr) {
-  const int n = fill_tile_table(tt, world, n_items, next, tile_units, units, take);
+// message only: units and take already work on positions). The units of a tile are constants of the code, so
+// that an item costs a shift and not a division.
+template <uint64_t kWhole, class Units, class Take>
+int fill_launch(TileTable& tt, uint32_t world, uint32_t n_items, uint32_t* next, TileForm cut, Units units, Take take,
+                const uint32_t* order = nullptr) {
+  typedef std::integral_constant<uint64_t, kWhole> Whole;
+  typedef std::integral_constant<uint64_t, kWhole / kShortTileParts> Short;
+  const int n = cut == kWholeTiles ? fill_tile_table(tt, world, n_items, next, Whole{}, units, take)
+                                   : fill_tile_table(tt, world, n_items, next, Short{}, units, take);
   if (n < 0) {
     const uint32_t at = (uint32_t)(-1 - n);
     return fail(ODC_ERR_INVALID, "item %u: %llu units per rank is too large for one launch", order ? order[at] : at,
@@ -760,27 +775,27 @@ int odc_gather(odc_arena* a, const odc_gather_item* items, uint32_t n_items, uin
     L.tt.order = (uint32_t)opt.rank_major;
     L.tt.first_rank = first_rank;
     const auto units = [&](uint32_t i) { return items[i].shard_bytes; };
-    const LaunchSize size = launch_size(n_items, next, kTileBytes, units);
+    const LaunchSize size = launch_size<kTileBytes>(n_items, next, units);
     const uint64_t out_bytes = size.units * a->world;
     L.policy = cache_policy(a, opt, 0, kSymmetric, out_bytes, opt.cached_output_bytes);
     TileForm cut = wants_short_tiles(size, opt.short_tiles_below) ? kShortTiles : kWholeTiles;
     if (cut == kWholeTiles && !L.policy.read && !L.policy.written && opt.gather_blocks_per_cu == 0)
       cut = stream_form(a, opt, size, out_bytes, cut);
-    const int n = fill_launch(
-        L.tt, a->world, n_items, &next, tile_units(kTileBytes, cut), units,
+    const int n = fill_launch<kTileBytes>(
+        L.tt, a->world, n_items, &next, cut, units,
         [&](uint32_t slot, uint32_t i) {
           L.item[slot] = {static_cast<uint8_t*>(items[i].dst), items[i].src_offset, items[i].shard_bytes};
         });
     if (n < 0) return n;
     if (n == 0) continue;
     L.form = tile_form(cut, L.tt.n_tiles, opt.few_tiles);
-    bool ragged = false;
-    uint64_t shard_bytes = 0;
-    for (uint32_t k = 0; k < L.tt.n_items; ++k) shard_bytes += L.item[k].seg_bytes;
-    L.output = output_form(opt, L.policy.written, shard_bytes * a->world);
+    L.output = output_form(opt, L.policy.written, out_bytes);
     L.tt.resident_below = resident_below(a, opt, opt.resident_shard_bytes);
-    for (uint32_t k = 0; k < L.tt.n_items; ++k)
-      ragged |= (((uintptr_t)L.item[k].dst | L.item[k].src_off | L.item[k].seg_bytes) & 15u) != 0;
+    const auto ragged = [&] {
+      uint64_t bits = 0;
+      for (uint32_t k = 0; k < L.tt.n_items; ++k) bits |= (uintptr_t)L.item[k].dst | L.item[k].src_off | L.item[k].seg_bytes;
+      return (bits & 15u) != 0;
+    };
     const uint32_t grid = grid_for(a, opt.gather_blocks_per_cu, L.tt.n_tiles, copy_threads(L.form), ragged);
     const uint32_t lds = lds_claim_for(a, opt.gather_resident_cap, grid, L.tt.n_tiles);
     if (int rc = launch_tiles(a, L, grid, [&] { return odc_device::launch_gather(L, grid, lds, stream); })) return rc;
@@ -820,12 +835,12 @@ int odc_gather_cast(odc_arena* a, const odc_gather_cast_item* items, uint32_t n_
     L.tt.order = (uint32_t)opt.rank_major;
     L.tt.first_rank = first_rank;
     const auto units = [&](uint32_t i) { return items[i].shard_elems; };
-    const LaunchSize size = launch_size(n_items, next, kTileElems, units);
+    const LaunchSize size = launch_size<kTileElems>(n_items, next, units);
     L.policy = cache_policy(a, opt, 0, kSymmetric, 0, kSymmetric);
     L.output = cast_output_form(L.policy.read, size.units * db * a->world, opt.cast_output_bytes);
     const TileForm cut = wants_short_tiles(size, opt.short_tiles_below) ? kShortTiles : kWholeTiles;
-    const int n = fill_launch(
-        L.tt, a->world, n_items, &next, tile_units(kTileElems, cut), units,
+    const int n = fill_launch<kTileElems>(
+        L.tt, a->world, n_items, &next, cut, units,
         [&](uint32_t slot, uint32_t i) {
           L.item[slot] = {static_cast<uint8_t*>(items[i].dst), items[i].shard_elems * (uint64_t)db,
                           items[i].src_offset, items[i].shard_elems};
@@ -872,13 +887,13 @@ int odc_convert(odc_arena* a, const odc_convert_item* items, uint32_t n_items, i
     L.tt.order = (uint32_t)opt.rank_major;
     L.tt.first_rank = 0;
     const auto units = [&](uint32_t i) { return items[i].elems; };
-    const LaunchSize size = launch_size(n_items, next, kTileElems, units);
+    const LaunchSize size = launch_size<kTileElems>(n_items, next, units);
     L.policy = cache_policy(a, opt, 0, kSymmetric, 0, kSymmetric);
     // (the copies are symmetric memory that every gather of the minibatch reads)
     L.output = cast_output_form(L.policy.read, size.units * db * a->world, opt.cached_output_bytes);
     const TileForm cut = wants_short_tiles(size, opt.short_tiles_below) ? kShortTiles : kWholeTiles;
-    const int n = fill_launch(
-        L.tt, a->world, n_items, &next, tile_units(kTileElems, cut), units,
+    const int n = fill_launch<kTileElems>(
+        L.tt, a->world, n_items, &next, cut, units,
         [&](uint32_t slot, uint32_t i) {
           // the gather-with-cast kernel with every rank's output in that rank's own region
           L.item[slot] = {a->origin + items[i].dst_offset, a->rank_stride, items[i].src_offset, items[i].elems};
@@ -912,8 +927,8 @@ int odc_clear(odc_arena* a, const odc_span* spans, uint32_t n_spans, void* strea
     // in a step: 117 us at W=64 against 123 item-major and 127 rank-outermost; level at W=128)
     L.tt.order = kRanksInterleaved;
     L.tt.first_rank = 0;
-    const int n = fill_launch(
-        L.tt, a->world, n_spans, &next, kTileBytes, [&](uint32_t i) { return spans[i].nbytes; },
+    const int n = fill_launch<kTileBytes>(
+        L.tt, a->world, n_spans, &next, kWholeTiles, [&](uint32_t i) { return spans[i].nbytes; },
         [&](uint32_t slot, uint32_t i) {
           L.item[slot] = {spans[i].offset, spans[i].nbytes};
         });
@@ -999,23 +1014,18 @@ int scatter_launch(odc_arena* a, const odc_accum_item* items, uint32_t n_items, 
     L.tt.order = (uint32_t)opt.rank_major;
     L.tt.first_rank = 0;
     const auto units = [&](uint32_t i) { return items[order[i]].shard_elems; };
-    const LaunchSize size = launch_size(n_items, next, kTileElems, units);
+    uint64_t grad_elems = 0;
+    const LaunchSize size = launch_size<kTileElems>(n_items, next, units,
+                                                    [&](uint32_t i) { grad_elems += items[order[i]].grad_elems; });
     TileForm cut = scatter_in_short_tiles(a, size, opt.short_tiles_below, grad_dtype, acc_dtype, store) ? kShortTiles
                                                                                                       : kWholeTiles;
-    {
-      uint64_t grad_elems = 0;
-      for (uint32_t i = next, k = 0; i < n_items && k < (uint32_t)kMaxItems; ++i) {
-        grad_elems += items[order[i]].grad_elems;
-        k += units(i) != 0;
-      }
-      L.policy = cache_policy(a, opt, grad_elems * gb, opt.cached_gradient_bytes, 0, kSymmetric);
-    }
+    L.policy = cache_policy(a, opt, grad_elems * gb, opt.cached_gradient_bytes, 0, kSymmetric);
     const bool one_per_tile = (store ? opt.store_blocks_per_cu : opt.accum_blocks_per_cu) <= 0 &&
                               (store || opt.accum_persistent_below_tiles == 0);
     if (one_per_tile && !(L.policy.read && L.policy.written))
       cut = scatter_stream_form(a, opt, size, grad_dtype, acc_dtype, store, L.policy, cut);
-    const int n = fill_launch(
-        L.tt, a->world, n_items, &next, tile_units(kTileElems, cut), units,
+    const int n = fill_launch<kTileElems>(
+        L.tt, a->world, n_items, &next, cut, units,
         [&](uint32_t slot, uint32_t i) {
           const odc_accum_item& it = items[order[i]];
           L.item[slot] = {static_cast<const uint8_t*>(it.grad), it.grad_elems, it.acc_offset, it.shard_elems};
@@ -1046,11 +1056,14 @@ int scatter_launch(odc_arena* a, const odc_accum_item* items, uint32_t n_items, 
     // without starving them. A persistent grid is never used for ragged launches (a lone
     // workgroup that straddles lines or meets heads, tails and padding falls behind: -7 % on
     // 16 B aligned uneven shards) nor for other dtype pairs than 16-bit gradients into fp32.
-    bool ragged = !(gb == 2 && ab == 4);
-    for (uint32_t k = 0; k < L.tt.n_items; ++k)
-      ragged |= (L.item[k].acc_off & 127u) != 0 || ((L.item[k].seg_elems * ab) & 127u) != 0 ||
-                ((L.item[k].seg_elems * gb) & 127u) != 0 || ((uintptr_t)L.item[k].grad & 127u) != 0 ||
-                L.item[k].grad_elems != L.item[k].seg_elems * a->world;
+    const auto ragged = [&] {
+      bool any = !(gb == 2 && ab == 4);
+      for (uint32_t k = 0; k < L.tt.n_items; ++k)
+        any |= (L.item[k].acc_off & 127u) != 0 || ((L.item[k].seg_elems * ab) & 127u) != 0 ||
+               ((L.item[k].seg_elems * gb) & 127u) != 0 || ((uintptr_t)L.item[k].grad & 127u) != 0 ||
+               L.item[k].grad_elems != L.item[k].seg_elems * a->world;
+      return any;
+    };
     L.tt.resident_below = L.policy.read ? 0 : resident_below(a, opt, opt.resident_accumulation_bytes);
     int64_t blocks_per_cu = store ? opt.store_blocks_per_cu : opt.accum_blocks_per_cu;
     if (blocks_per_cu < 0)
@@ -1128,10 +1141,10 @@ int odc_publish(odc_arena* a, uint32_t rank, const odc_publish_item* items, uint
     L.tt.order = kItemMajor;
     L.tt.first_rank = 0;
     const auto units = [&](uint32_t i) { return items[i].elems; };
-    const LaunchSize size = launch_size(n_items, next, kTileElems, units);
+    const LaunchSize size = launch_size<kTileElems>(n_items, next, units);
     const TileForm cut = publish_in_short_tiles(size, ab) ? kShortTiles : kWholeTiles;
-    const int n = fill_launch(
-        L.tt, 1u, n_items, &next, tile_units(kTileElems, cut), units,
+    const int n = fill_launch<kTileElems>(
+        L.tt, 1u, n_items, &next, cut, units,
         [&](uint32_t slot, uint32_t i) {
           L.item[slot] = {static_cast<uint8_t*>(items[i].out), items[i].acc_offset, items[i].elems};
         });

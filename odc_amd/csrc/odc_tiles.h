@@ -327,9 +327,10 @@ ODC_HD bool is_resident(uintptr_t address, uint32_t below) {
 // take(slot, i) copies item i's descriptor into slot `slot` of the launch. Returns the number of
 // items taken (0 when only empty items were left), or -1 - i when item i alone is too large for
 // one launch.
-template <class Units, class Take>
+// (tile_units: a number, or an integral constant, which makes the division a shift)
+template <class TileUnits, class Units, class Take>
 inline int fill_tile_table(TileTable& tt, uint32_t world, uint32_t n_items, uint32_t* next,
-                           uint64_t tile_units, Units units, Take take) {
+                           TileUnits tile_units, Units units, Take take) {
   uint32_t n = 0;
   uint64_t tiles = 0, per_rank = 0;
   uint32_t i = *next;
