@@ -330,7 +330,7 @@ OutputForm cast_output_form(bool cached, uint64_t bytes, int64_t line) {
 // also(i) is called for each of them: whatever else a launch's plan sums up over its items is summed on the
 // same walk. Passes of six launches, 300 small slices at W = 16, whose host time is level with their kernels',
 // took 36.7 -> 39.3 us when plans of long streams had walks of their own; with one walk, no division per
-// item and grid_for's look at the items only where it is used, 35.9 -> 36.1 and 37.5 -> 36.8 on two cards.
+// item and grid_for's look at the items only where it is used, 35.9 -> 36.1, 37.5 -> 36.8 and 36.1 -> 36.8 on three cards.
 struct LaunchSize {
   uint32_t items = 0;
   uint64_t tiles = 0;
