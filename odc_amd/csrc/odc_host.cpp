@@ -201,6 +201,7 @@ int check_compute(odc_arena* a, DeviceGuard& guard) {
 // What dry-run arenas have "launched" (process-wide, reset by odc_set_option("dry_run_reset", 0)).
 std::atomic<int64_t> g_dry_launches{0}, g_dry_tiles{0}, g_dry_workgroups{0};
 std::atomic<int64_t> g_dry_short{0}, g_dry_few{0}, g_dry_stream{0};  // of the launches: those in kShortTiles, ...
+std::atomic<int64_t> g_dry_resident{0};  // those that are told of a resident part
 
 template <class Launch> TileForm form_of(const Launch& L) { return L.form; }
 TileForm form_of(const ClearLaunch&) { return kWholeTiles; }
@@ -219,6 +220,7 @@ int launch_tiles(const odc_arena* a, const Launch& L, uint32_t grid, Issue issue
     g_dry_short += form_of(L) == kShortTiles;
     g_dry_few += form_of(L) == kFewShortTiles;
     g_dry_stream += form_of(L) == kStreamTiles;
+    g_dry_resident += L.tt.resident_below != 0;
     return ODC_OK;
   }
   const int e = issue();
@@ -466,7 +468,8 @@ int odc_abi_version(void) { return ODC_HIP_ABI_VERSION; }
 
 int odc_set_option(const char* name, int64_t value) {
   if (name && !strcmp(name, "dry_run_reset")) {
-    g_dry_launches = 0; g_dry_tiles = 0; g_dry_workgroups = 0; g_dry_short = 0; g_dry_few = 0; g_dry_stream = 0;
+    g_dry_launches = 0; g_dry_tiles = 0; g_dry_workgroups = 0;
+    g_dry_short = 0; g_dry_few = 0; g_dry_stream = 0; g_dry_resident = 0;
     return ODC_OK;
   }
   std::lock_guard<std::mutex> lk(g_opt_mu);
@@ -490,6 +493,7 @@ int odc_get_option(const char* name, int64_t* value) {
     if (!strcmp(name, "dry_run_short_launches")) { *value = g_dry_short.load(); return ODC_OK; }
     if (!strcmp(name, "dry_run_few_launches")) { *value = g_dry_few.load(); return ODC_OK; }
     if (!strcmp(name, "dry_run_stream_launches")) { *value = g_dry_stream.load(); return ODC_OK; }
+    if (!strcmp(name, "dry_run_resident_launches")) { *value = g_dry_resident.load(); return ODC_OK; }
   }
   std::lock_guard<std::mutex> lk(g_opt_mu);
   int64_t* s = option_slot(name);
