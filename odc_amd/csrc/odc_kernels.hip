@@ -884,6 +884,12 @@ template <class Launch> constexpr bool kSearches = std::is_same_v<decltype(Launc
 // Which launches long streams come in, and which are for nothing else.
 template <class Launch> constexpr bool kStreams = !kSearches<Launch>;
 template <class Launch> constexpr bool kStreamsOnly = std::is_same_v<decltype(Launch::tt), ItemsTable<kSomeItems>>;
+// Gathers of whole tiles are bound by HBM and stream better from workgroups that come to their loads one
+// after the other along the item search: a layer's 872 MB from bf16 134.1 us by the full tables, 136.4 by the
+// small ones, from fp32 196 and 199 (fewer resident workgroups: 224). The other kernels are level there. So
+// plain and converting gathers have no kernel for whole tiles by the small table.
+template <class Launch>
+constexpr bool kGathersWholeTiles = !std::is_same_v<decltype(Launch::tt), ItemsTable<kFewItems>>;
 
 #define ODC_FOR_EACH_DTYPE_PAIR(X)                    \
   X(ODC_DTYPE_BF16, bf16_tag, ODC_DTYPE_BF16, bf16_tag) \
@@ -961,17 +967,15 @@ kernel_fn<L> pick_accum(int g, int a, bool store, CachePolicy policy, TileForm f
 
 template <class L, bool kSrcCached, OutputForm kDst>
 kernel_fn<L> pick_gather_form(TileForm form) {
-  if (form == kStreamTiles) {
-    if constexpr (kStreams<L> && kDst == kStream && !kSrcCached)
-      return gather_kernel<L, false, kStream, false, kShortThreads, kShortUnroll, kStreamWaves>;
-    else return nullptr;
+  if constexpr (kStreams<L> && kDst == kStream && !kSrcCached)
+    if (form == kStreamTiles) return gather_kernel<L, false, kStream, false, kShortThreads, kShortUnroll, kStreamWaves>;
+  if constexpr (!kStreamsOnly<L>) {
+    if (form == kFewShortTiles) return gather_kernel<L, kSrcCached, kDst, kSearches<L>, kShortThreads, kShortUnroll>;
+    if (form == kShortTiles) return gather_kernel<L, kSrcCached, kDst, false, kShortThreads, kShortUnroll>;
+    if constexpr (kGathersWholeTiles<L>)
+      if (form == kWholeTiles) return gather_kernel<L, kSrcCached, kDst, false, kCopyThreads, kCopyUnroll>;
   }
-  if constexpr (kStreamsOnly<L>) return nullptr;
-  else {
-  if (form == kFewShortTiles) return gather_kernel<L, kSrcCached, kDst, kSearches<L>, kShortThreads, kShortUnroll>;
-  if (form == kShortTiles) return gather_kernel<L, kSrcCached, kDst, false, kShortThreads, kShortUnroll>;
-  return gather_kernel<L, kSrcCached, kDst, false, kCopyThreads, kCopyUnroll>;
-  }
+  return nullptr;
 }
 
 template <class L, bool kSrcCached>
@@ -990,7 +994,9 @@ template <class L, class S, class D, bool kSrcCached, OutputForm kDst>
 kernel_fn<L> pick_cast_gather_form(TileForm form) {
   if (form == kFewShortTiles) return cast_gather_kernel<L, S, D, kSrcCached, kDst, kSearches<L>, kShortThreads, kShortUnroll>;
   if (form == kShortTiles) return cast_gather_kernel<L, S, D, kSrcCached, kDst, false, kShortThreads, kShortUnroll>;
-  return cast_gather_kernel<L, S, D, kSrcCached, kDst, false, kCopyThreads, kCopyUnroll>;
+  if constexpr (kGathersWholeTiles<L>)
+    if (form == kWholeTiles) return cast_gather_kernel<L, S, D, kSrcCached, kDst, false, kCopyThreads, kCopyUnroll>;
+  return nullptr;
 }
 
 // Shards are cached only together with the output, which is then kept with plain stores.
@@ -1126,9 +1132,7 @@ bool has_accum(int g, int a) { return pick_accum<AccumLaunch>(g, a, false, {}, k
 bool has_cast_gather(int s, int d) { return pick_cast_gather<CastGatherLaunch>(s, d, {}, kStream, kWholeTiles) != nullptr; }
 bool has_publish(int a, int o) { return pick_publish<PublishLaunch>(a, o, kShortTiles) != nullptr; }
 
-// Gathers of whole tiles are bound by HBM and stream better from workgroups that come to their loads one
-// after the other along the item search: a layer's 872 MB from bf16 134.1 us by the full tables, 136.4 by the
-// small ones, from fp32 196 and 199 (fewer resident workgroups: 224). The other kernels are level there.
+// by_table for whole tiles: kGathersWholeTiles
 int launch_gather(const GatherLaunch& L, uint32_t grid, uint32_t lds_bytes, void* stream) {
   return launch_form(L, grid, copy_threads(L.form), lds_bytes, stream, [&](auto form) {
     return pick_gather<typename decltype(form)::type>(L.policy.read, L.output, L.form);
