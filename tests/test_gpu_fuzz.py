@@ -124,6 +124,16 @@ KNOBS = [
     {"short_tiles_below": 1 << 30, "few_tiles": 1 << 30, "store_blocks_per_cu": 1, "publish_blocks_per_cu": 1},
     {"cached_output_bytes": 0, "cached_gradient_bytes": 0, "cached_arena_bytes": 0},
     {"cached_output_bytes": 1 << 40, "plain_output_bytes": 0, "cached_gradient_bytes": 1 << 40, "cached_arena_bytes": 1 << 40},
+    # long streams, and the part that stays in the cache, whatever else is asked for
+    {"stream_bytes": 0, "cached_output_bytes": 0, "cached_gradient_bytes": 0, "cached_arena_bytes": 0, "short_tiles_below": 0},
+    {"stream_bytes": 0, "cached_output_bytes": 0, "cached_gradient_bytes": 0, "cached_arena_bytes": 0, "short_tiles_below": 0,
+     "gather_resident_cap": 2, "accum_resident_cap": 4, "store_resident_cap": 3},
+    {"stream_bytes": 1 << 40, "cast_output_bytes": 0, "cached_gradient_bytes": 0},
+    {"cast_output_bytes": 1 << 40, "cached_arena_bytes": 0},
+    {"resident_above": 0, "resident_accumulation_bytes": 1 << 20, "resident_shard_bytes": 1 << 20, "resident_clear_bytes": 0,
+     "cached_gradient_bytes": 0, "cached_arena_bytes": 0},
+    {"resident_above": 0, "resident_accumulation_bytes": 1 << 40, "resident_shard_bytes": 0, "resident_clear_bytes": 0,
+     "cached_gradient_bytes": 0, "cached_arena_bytes": 0, "clear_blocks_per_cu": 1},
     # arena layout (read when the world is created): packed buffers and staggered, unaligned rank
     # regions; coarse alignment
     {"alloc_align": 256, "rank_stride_align": 256, "rank_stagger_bytes": 4352},
@@ -142,7 +152,9 @@ def test_results_do_not_depend_on_launch_knobs(make_world, knobs):
              "publish_blocks_per_cu", "gather_resident_cap", "cast_resident_cap", "accum_resident_cap",
              "store_resident_cap", "rank_major", "accum_tile_order", "accum_persistent_below_tiles",
              "accum_short_segment_tiles", "accum_small_items_last", "short_tiles_below", "few_tiles",
-             "cached_output_bytes", "plain_output_bytes", "cached_gradient_bytes", "cached_arena_bytes", "alloc_align", "rank_stride_align", "rank_stagger_bytes"]
+             "cached_output_bytes", "plain_output_bytes", "cached_gradient_bytes", "cached_arena_bytes", "stream_bytes",
+             "cast_output_bytes", "resident_above", "resident_accumulation_bytes", "resident_shard_bytes",
+             "resident_clear_bytes", "alloc_align", "rank_stride_align", "rank_stagger_bytes"]
     saved = {n: _native.get_option(n) for n in names}
     try:
         for name, value in knobs.items():

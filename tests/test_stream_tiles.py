@@ -62,6 +62,85 @@ def test_which_launches_are_long_streams(what, elem, min_bytes):
             _native.set_option(name, value)
 
 
+# workgroups that walk many tiles, beside everything that would make a launch a long stream
+WALKED = [
+    {"gather_blocks_per_cu": 1, "accum_blocks_per_cu": 1, "store_blocks_per_cu": 1},
+    {"accum_persistent_below_tiles": 1 << 30},
+    {"accum_blocks_per_cu": 0, "accum_persistent_below_tiles": 1 << 30, "store_blocks_per_cu": 2},
+    {"accum_resident_cap": 2, "gather_resident_cap": 1, "store_resident_cap": 4},
+]
+FAR_STREAMS = {"stream_bytes": 0, "cached_output_bytes": 0, "cached_gradient_bytes": 0, "cached_arena_bytes": 0, "short_tiles_below": 0}
+SHARDS = {1: [96 * 4096], 3: [64 * 4096, 4096, 31 * 4096]}  # whole tiles, more of them than a GPU has CUs
+
+
+@pytest.mark.parametrize("sizes", SHARDS.values(), ids=len)
+@pytest.mark.parametrize("knobs", WALKED, ids=str)
+def test_a_long_stream_has_a_workgroup_per_tile(knobs, sizes):
+    """There are no kernels that walk a long stream's tiles: whatever asks for fewer workgroups than tiles
+    keeps a launch from being one."""
+    W, lib, handle, at = 4, _native.load(), ctypes.c_void_p(), ctypes.c_uint64()
+    saved = _with_options({**FAR_STREAMS, **knobs})
+    _native.check(lib.odc_arena_create(W, 1 << 30, _native.ODC_ARENA_DRY_RUN, ctypes.byref(handle)))
+    _native.check(lib.odc_arena_alloc(handle, 1 << 20, ctypes.byref(at)))
+    try:
+        for name, *codes in [("odc_gather", 0)] + [(call, g, a) for call in ("odc_scatter_accumulate", "odc_scatter_store")
+                                                   for g in (BF16, F16, F32) for a in (BF16, F16, F32)]:
+            is_gather = name == "odc_gather"
+            items, off = ((_native.GatherItem if is_gather else _native.AccumItem) * len(sizes))(), 0
+            for k, n in enumerate(sizes):
+                items[k] = _native.GatherItem(OUTSIDE, off, 4 * n) if is_gather else _native.AccumItem(OUTSIDE, W * n, off, n)
+                off += 4 * n
+            _native.set_option("dry_run_reset", 0)
+            _native.check(getattr(lib, name)(handle, items, len(sizes), *codes, None))
+            tiles, workgroups, streams = (_native.get_option(f"dry_run_{n}") for n in ("tiles", "workgroups", "stream_launches"))
+            assert tiles == workgroups or not streams, (name, codes)
+            if is_gather:
+                walked = "gather_blocks_per_cu" in knobs
+                assert (workgroups < tiles, streams) == (walked, not walked)
+    finally:
+        _native.check(lib.odc_arena_destroy(handle))
+        for name, value in saved.items():
+            _native.set_option(name, value)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("sizes", SHARDS.values(), ids=len)
+@pytest.mark.parametrize("knobs", WALKED, ids=str)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=str)
+def test_walked_tiles_beside_long_streams(make_world, dtype, knobs, sizes):
+    from odc_amd import GatherService, ReductionService, SymmBufferRegistry
+
+    saved = _with_options({**FAR_STREAMS, **knobs})
+    try:
+        W = 4
+        group = make_world(W, 16 * MB)
+        registry = SymmBufferRegistry.get_instance()
+        gather, red = GatherService(), ReductionService(accumulation_dtype=torch.float32, lazy_clear=True)
+        gen = torch.Generator().manual_seed(29)
+        shards = [[torch.randn(n, generator=gen).to(dtype) for _ in range(W)] for n in sizes]
+        sources = [put_shards(registry, ("p", i), s) for i, s in enumerate(shards)]
+        outs = [torch.full((W * n,), float("nan"), dtype=dtype, device="cuda") for n in sizes]
+        gather.gather_into_tensors(outs, sources, group)
+        for out, s in zip(outs, shards):
+            assert_bit_equal(out, oracle.gather(s))
+        keys = list(range(len(sizes)))
+        for key, n in zip(keys, sizes):
+            red.register(key, (n,), dtype, torch.float32, group)
+        want = [[torch.zeros(n) for _ in range(W)] for n in sizes]
+        red.clear_accumulations()
+        for _ in range(2):  # the store form, then read-modify-write
+            grads = [torch.randn(W * n, generator=gen).to(dtype) for n in sizes]
+            red.scatter_accumulate_multi(keys, [g.cuda() for g in grads], group)
+            for accs, g in zip(want, grads):
+                oracle.scatter_accumulate(accs, g)
+        for key, accs in zip(keys, want):
+            for r, got in enumerate(red.get_peer_accumulations(key)):
+                assert_bit_equal(got, accs[r], f"size {sizes[key]} rank {r}")
+    finally:
+        for name, value in saved.items():
+            _native.set_option(name, value)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("order", [0, 1, 2])  # of the tiles: interleaved ranks, item major, rank outermost
 @pytest.mark.parametrize("share", [0, 1 << 19])  # of the memory in use that stays in the cache
