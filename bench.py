@@ -16,10 +16,11 @@ scatter-accumulate, the dominant kernel) and `roofline_gather`.
 
 Prints ONE JSON line with, besides the contract's fields: `roofline.practical_ceiling` (what bare
 streaming kernels of libodc_ceiling.so reach on flat arrays of the same sizes in the same run),
-`roofline.traffic` (HBM bytes per launch from the committed rocprofv3 counter runs listed in
-profiles/traffic.json; null when a launch knob is overridden), `host_us_per_call` (host time of one
-call of each service entry point on the 9-parameter layer), the clear, the CPU oracle timed on
-the host cores (`cpu_baseline`), the parity verdict against that oracle, and `other_clear_mode`:
+`roofline.rate_of` (the GB/s and `frac` are of the algorithmic bytes; how many of them a launch finds in the
+last-level cache), `roofline.traffic` (bytes per launch between the L2s and that cache, which stands before HBM,
+from the committed rocprofv3 counter runs listed in profiles/traffic.json; null when a launch knob is
+overridden), `host_us_per_call` (host time of one call of each service entry point on the 9-parameter
+layer), the clear, the CPU oracle timed on the host cores (`cpu_baseline`), the parity verdict against that oracle, and `other_clear_mode`:
 the same minibatches with lazy clears, replayed from a graph captured inside
 `ReductionService.captured_minibatch()`: no clear kernel runs and the first scatter-accumulate of
 a minibatch stores instead (6N bytes, counted as such), checked against the oracle as well.
@@ -290,6 +291,7 @@ def model_sweep(args):
             "kernel": "accum_kernel<bf16,f32> (scatter-accumulate), all launches of the sweep",
             "bound": "hbm", "achieved": round(gbps, 1), "peak": HBM_PEAK_GBPS, "unit": "GB/s",
             "frac": round(gbps / HBM_PEAK_GBPS, 4),
+            **rate_of("resident_accumulation_bytes", round(0.4 * accum_bytes / launches)),
             "algorithmic_bytes": round(accum_bytes / launches), "avg_launch_ms": round(accum_ms / launches, 5),
             "launches_timed": launches,
             "traffic": entry[0], "traffic_source": entry[1],
@@ -305,6 +307,7 @@ def model_sweep(args):
         roofline_gather = {
             "kernel": "gather_kernel, all launches of the sweep", "bound": "hbm", "achieved": round(gbps, 1),
             "peak": HBM_PEAK_GBPS, "unit": "GB/s", "frac": round(gbps / HBM_PEAK_GBPS, 4),
+            **rate_of("resident_shard_bytes", round(0.5 * gather_bytes / launches)),
             "algorithmic_bytes": round(gather_bytes / launches), "avg_launch_ms": round(gather_ms / launches, 5),
             "launches_timed": launches, "traffic": entry[0], "traffic_source": entry[1],
             "by_unit_shape": gather_shapes,
@@ -341,8 +344,25 @@ def model_sweep(args):
         sys.exit(1)
 
 
+def rate_of(option, symmetric_bytes, streamed_bytes=None):
+    """What the GB/s of a kernel are of. Of the ``symmetric_bytes`` that one launch reads (and an accumulate writes
+    back), the part that ``option`` keeps in the last-level cache need not come from HBM; ``streamed_bytes``: of
+    gradients, which take the part's place while they are cached themselves."""
+    from odc_amd import _native
+    from odc_amd.primitives.utils import get_world
+
+    info = get_world().arena.info()
+    in_use = info.bytes_in_use * info.world_size
+    part = min(1.0, _native.get_option(option) / in_use) if in_use > _native.get_option("resident_above") else 0.0
+    if streamed_bytes is not None and streamed_bytes <= _native.get_option("cached_gradient_bytes"):
+        part = 0.0
+    return {"rate_of": "algorithmic bytes" + (", a part of them in the last-level cache" if part else ""),
+            "bytes_kept_in_last_level_cache": round(part * symmetric_bytes)}
+
+
 def load_traffic(args, W):
-    """HBM bytes per launch from the committed rocprofv3 counter runs: kernel -> (bytes, source).
+    """Bytes per launch between the L2s and the last-level cache, which stands before HBM, from the
+    committed rocprofv3 counter runs: kernel -> (bytes, source).
     Only for the configuration those runs profiled, and only with the library's default knobs."""
     if args.option or not TRAFFIC_FILE.exists():
         return {}
@@ -1169,6 +1189,7 @@ def main():
             "peak": HBM_PEAK_GBPS,
             "unit": "GB/s",
             "frac": round(accum_gbps / HBM_PEAK_GBPS, 4),
+            **rate_of("resident_accumulation_bytes", 4 * N, 2 * N),
             "traffic": traffic.get("accum", (None, None))[0],
             "traffic_source": traffic.get("accum", (None, None))[1],
             "algorithmic_bytes": 10 * N,
@@ -1187,6 +1208,7 @@ def main():
             "peak": HBM_PEAK_GBPS,
             "unit": "GB/s",
             "frac": round(gather_gbps / HBM_PEAK_GBPS, 4),
+            **rate_of("resident_shard_bytes", 2 * N),
             "traffic": traffic.get("gather", (None, None))[0],
             "traffic_source": traffic.get("gather", (None, None))[1],
             "algorithmic_bytes": 4 * N,
