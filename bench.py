@@ -672,12 +672,14 @@ def probe_launch_forms(args, tokens=1024, replays=7):
     W = args.world_size
     torch.cuda.set_device(0)
     torch.manual_seed(0)
-    far, names = 1 << 40, ("plain_output_bytes", "cached_output_bytes", "cached_gradient_bytes", "short_tiles_below")
+    far, names = 1 << 40, ("plain_output_bytes", "cached_output_bytes", "cached_gradient_bytes", "short_tiles_below",
+                           "resident_accumulation_bytes", "resident_shard_bytes")
     defaults = {name: _native.get_option(name) for name in names}
     outputs = {"streamed": {"cached_output_bytes": 0}, "written through": {"cached_output_bytes": far, "plain_output_bytes": 0},
                "plain": {"cached_output_bytes": far, "plain_output_bytes": far}, "by rule": {}}
     gradients = {"streamed": {"cached_gradient_bytes": 0}, "cached": {"cached_gradient_bytes": far}, "by rule": {}}
     tiles = {"whole tiles": {"short_tiles_below": 0}, "short tiles": {"short_tiles_below": far}, "by rule": {}}
+    residents = {"none": {"resident_accumulation_bytes": 0, "resident_shard_bytes": 0}, "by rule": {}}
 
     def timed(step, sets, options):
         for name, value in {**defaults, **options}.items():
@@ -701,7 +703,7 @@ def probe_launch_forms(args, tokens=1024, replays=7):
         return statistics.median(times)
 
     print(f"decoder layers at W={W}, microseconds per pass")
-    for hidden in (512, 1024, 1536, 2048):
+    for hidden in (512, 1024, 1536, 2048, 3072, 4096):
         ffn, kv = 2560 * hidden // 1024, hidden // 4
         shapes = [(hidden,), (hidden, hidden), (kv, hidden), (kv, hidden), (hidden, hidden), (hidden,), (ffn, hidden),
                   (ffn, hidden), (hidden, ffn)]
@@ -737,6 +739,14 @@ def probe_launch_forms(args, tokens=1024, replays=7):
                 if o.dim() == 2:
                     torch.mm(x[o.shape[0]], o, out=y[o.shape[1]])
 
+        def gradients_written(s):
+            for g, shape in zip(s["grad"], shapes):
+                if len(shape) == 2:
+                    torch.mm(x[shape[0]].t(), x[shape[1]], out=g.view(shape))
+
+        def step(s):
+            gathered(s), products(s), gathered(s), products(s), gradients_written(s), accumulated(s)
+
         print(f"hidden {hidden}: {nbytes / 2**20:.0f} MiB of parameters, {n_sets} sets of buffers")
         table = [("gather", gathered, outputs, "output"), ("gather, accumulate", lambda s: (gathered(s), accumulated(s)), outputs, "output"),
                  (f"gather, products of {tokens} tokens", lambda s: (gathered(s), products(s)), outputs, "output"),
@@ -744,8 +754,11 @@ def probe_launch_forms(args, tokens=1024, replays=7):
                  ("accumulate, bf16 into bf16", lambda s: accumulated(s, narrow, "n"), gradients, "gradient"),
                  ("gather", gathered, tiles, "tiles"),
                  ("accumulate, bf16 into bf16", lambda s: accumulated(s, narrow, "n"), tiles, "tiles")]
-        for label, step, arms, what in table:
-            figures = ", ".join(f"{name} {timed(step, sets, options):.1f}" for name, options in arms.items())
+        if hidden > 2048:  # gradients of more than 128 MiB, more than 640 MiB in use
+            table = [("gather, gather, accumulate", lambda s: (gathered(s), gathered(s), accumulated(s)), residents, "resident part"),
+                     (f"the same with a step's products, {tokens} tokens", step, residents, "resident part")]
+        for label, one_pass, arms, what in table:
+            figures = ", ".join(f"{name} {timed(one_pass, sets, options):.1f}" for name, options in arms.items())
             print(f"  {label + ' (' + what + ')':44s} {figures}", flush=True)
         for name, value in defaults.items():
             _native.set_option(name, value)
