@@ -265,18 +265,22 @@ int odc_abi_version(void);
  *  - "short_tiles_below" (default 32): launches whose segments average fewer whole tiles are cut into
  *    short ones (0: none but those that always are). "few_tiles" (32768): up to so many short tiles
  *    a workgroup reads the whole table of the launch's items at once instead of searching it.
- *    "stream_bytes" (8 MiB): launches of up to 64 items that write more past the caches are long streams:
- *    gathers without conversion, accumulates into fp32, stores of fp32; short tiles, fewer resident.
+ *    "stream_bytes" (8 MiB): launches of up to 64 items that write more past the caches are long streams, in
+ *    short tiles with fewer workgroups resident: accumulates of 16-bit gradients that are not read through the
+ *    caches into fp32; and, where they would go in whole tiles, gathers without conversion and accumulates and
+ *    stores of fp32 gradients into fp32. Launches of persistent workgroups are not.
  *  - what a launch leaves in the caches: gathers of at most "cached_output_bytes" (64 MiB) of output
  *    leave it there, with plain stores up to "plain_output_bytes" (24 MiB) and written through the L2
  *    above; converting gathers of at most "cast_output_bytes" (32 MiB) of output write it through the L2
- *    (conversions of symmetric memory: "cached_output_bytes"); gradients of at most "cached_gradient_bytes" (128 MiB) per launch are read through the
- *    caches; so are shards and accumulations while all symmetric memory in use, over all ranks, is at most
- *    "cached_arena_bytes" (192 MiB). 0 streams past the caches. Above "resident_above" (640 MiB) in use a
- *    part of the symmetric memory is kept in the cache: of accumulations the share that
- *    "resident_accumulation_bytes" (320 MiB) have of what is in use, of gathered shards the share of
- *    "resident_shard_bytes" (80 MiB); clears leave theirs there from "resident_clear_bytes" (48 MiB) per
- *    launch on. 0 keeps none.
+ *    (conversions of symmetric memory: "cached_output_bytes"); gradients of at most "cached_gradient_bytes"
+ *    (128 MiB) per launch are read through the caches; so are shards and accumulations while all symmetric
+ *    memory in use, over all ranks, is at most "cached_arena_bytes" (192 MiB). 0 streams past the caches. Above
+ *    "resident_above" (640 MiB) in use a part of the symmetric memory is kept in the last-level cache: of
+ *    accumulations the share that "resident_accumulation_bytes" (320 MiB) have of what is in use, where the
+ *    launch's gradient is not cached itself, and of shards that are gathered without conversion the share of
+ *    "resident_shard_bytes" (80 MiB); clears of more than twice "cached_gradient_bytes" leave theirs there from
+ *    "resident_clear_bytes" (48 MiB) per launch on. Whole tiles only, and not in launches of more than 16 items
+ *    in few short tiles. 0 keeps none.
  *  - "rank_stagger_bytes" (extra distance between rank regions), "rank_stride_align" (rank regions
  *    start on multiples of it, default 16384 = one tile) and "alloc_align" (allocations of at
  *    least this many bytes start on multiples of it, default 16384; smaller ones on 256): read

@@ -287,7 +287,8 @@ constexpr int64_t kSymmetric = -1;  // a line: the stream lies in symmetric memo
 // 128 MB are read through the caches takes 307 us instead of 346 with 0.9, 1.7 and 3.5 GB of nontemporal
 // copies between two of them alike), so a fixed subset of the accumulations, touched twice by every
 // accumulate, and of the shards can live there from one kernel to the next (is_resident in odc_tiles.h
-// says which bytes; only their loads, and the stores of launches that do not load, go through the caches).
+// says which bytes, and which launches leave them out: gathers read them, accumulates read and write them, and
+// stores and clears write them with plain accesses; everything else of these launches is nontemporal).
 // Up to 640 MiB in use there is none, and no accumulation's where the launch's gradient is cached: gradients
 // and gathered outputs of such sizes leave no room (bf16 into fp32, three sets of buffers in turn: gather +
 // accumulate of 17 Mi elements 41.8 us without, 48.8 with; of 40 M 85 and 99). Otherwise accumulations have
@@ -298,7 +299,10 @@ constexpr int64_t kSymmetric = -1;  // a line: the stream lies in symmetric memo
 // minibatch of two microbatches, mixed 1666 -> 1656, bf16 1044 -> 1033, fp32 2061 -> 2039. (384 MiB's share:
 // 314, 470, 1742, 1651, 1028; 256: 460, 1751, 1658, 1031. Ten units in turn, each part small and to last for
 // 25 GB, at 384: layer 482 -> 481, minibatches 1827 -> 1803, 1685 -> 1688, 1045.5 -> 1044.6. Converting
-// gathers gain nothing.)
+// gathers gain nothing.) With a layer's forward and backward products between the passes, which read through the
+// caches, a step is level: -0.4 to +0.3 % over 94 M and 218 M parameters, 1, 3 and 8 units in turn and 128 to 2048
+// tokens (218 M, 3 units, 1024 tokens 2113 -> 2105, its accumulate 339 -> 330; 128 tokens 1479 -> 1483, 344 ->
+// 338: the products give back what they no longer find).
 uint32_t resident_below(const odc_arena* a, const Options& opt, int64_t most) {
   const double in_use = (double)(a->in_use.load(std::memory_order_relaxed) * a->world);
   if (in_use <= (double)opt.resident_above) return 0;
@@ -420,9 +424,10 @@ TileForm tile_form(TileForm cut, uint32_t n_tiles, int64_t few) {
 
 // Whether a launch that is otherwise cut as `cut` is a long stream: more than 8 MiB written, past the caches,
 // by at most 64 items. Long streams go in short tiles, of which 12 workgroups are resident per CU
-// (kStreamWaves). They are bound by how HBM mixes reads and writes, and it mixes best with some 70 KB of
-// loads in flight per CU; how many that are had been decided by the time a workgroup took to find its item,
-// and by whole tiles. With the items found early (ItemsWalk) it has to be said. One kernel each on real
+// (kStreamWaves). They are bound by how HBM mixes reads and writes, which depends on how many loads are in
+// flight per CU (with 12 workgroups 72 KiB in the accumulate of 16-bit gradients, 96 KiB in that of fp32 ones, 48
+// KiB in the gather and the fp32 store); how many that are had been decided by the time a workgroup took to find
+// its item, and by whole tiles. With the items found early (ItemsWalk) it has to be said. One kernel each on real
 // data, us, as they were -> long streams (16 and 10 workgroups per CU; 2 quads per lane in each):
 //   accumulate bf16 into fp32: a decoder layer at W = 8 354 -> 338 (349, 343), at W = 64 361 -> 350 (357,
 //     356), nine items of 11 .. 27 M elements 260 -> 253 (257, 259), 525 M elements 854 -> 826 (850, 814);

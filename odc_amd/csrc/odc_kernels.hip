@@ -19,14 +19,15 @@
 // Workgroups walk the tiles with a grid-stride loop, by default one workgroup per tile, so that,
 // at any instant, the whole chip streams one compact window of memory. Per-item
 // descriptors (<= ODC_MAX_ITEMS_PER_LAUNCH; launches of one item and of up to 16 have smaller tables) travel
-// BY VALUE in the kernel argument segment and are read with scalar loads, so a call needs no device-side work list, no host->device copy and
-// no allocation; longer item lists are split over several launches.
+// BY VALUE in the kernel argument segment and are read with scalar loads, so a call needs no device-side
+// work list, no host->device copy and no allocation; longer item lists are split over several launches.
 //
 // Each wavefront issues its 2 or 4 independent 128-bit loads per stream before the first store.
 // Streams larger than the 256 MB last-level cache are nontemporal on both sides (worth ~15 % over
 // plain accesses there); what fits the cache and was just produced, or is about to be consumed, is
-// left in it (cache_policy in odc_host.cpp), and so is a part of what does not fit (resident_below there). Deeper unrolling or prefetching the next tile
-// measured slower: the memory system prefers a small window to more requests in flight.
+// left in it (cache_policy in odc_host.cpp), and so is a part of what does not fit (resident_below
+// there). Deeper unrolling or prefetching the next tile measured slower: the memory system prefers a
+// small window to more requests in flight.
 // Workgroup i runs on XCD i % 8; binding XCDs to address classes (256 B .. 64 KiB granules)
 // changed nothing measurable and giving every XCD one contiguous eighth of the tiles costs the
 // read-modify-write 3 %, so tiles are simply dealt out in address order: at any instant all

@@ -115,7 +115,7 @@ struct SingleLaunch {
   D item[1];
 };
 
-// One of 2 to kFewItems items, as the parameters of a layer are, goes out with tables of that size: 496 to
+// One of 2 to kFewItems items, as the parameters of a layer are, goes out with tables of that size: 368 to
 // 624 bytes of arguments (about 0.6 us less of host time than 4 KB), and the whole prefix table in one
 // scalar load (ItemsWalk in odc_kernels.hip). Both short forms are for launches of one workgroup per tile.
 // Long streams of up to kSomeItems have such tables too.
@@ -221,6 +221,9 @@ struct PublishFewItems : ItemsLaunch<PublishDesc, odc_tiles::kFewItems> {
   PublishScale scale;
 };
 static_assert(sizeof(SingleLaunch<ClearDesc>) == 64 && sizeof(PublishSingle) == 88, "as SingleLaunch says");
+static_assert(sizeof(ItemsLaunch<ClearDesc, odc_tiles::kFewItems>) == 368 &&
+                  sizeof(ItemsLaunch<AccumDesc, odc_tiles::kFewItems>) == 624 && sizeof(PublishFewItems) <= 624,
+              "as ItemsLaunch says");
 static_assert(sizeof(GatherLaunch) <= 4096 && sizeof(AccumLaunch) <= 4096 && sizeof(PublishLaunch) <= 4096 &&
                   sizeof(CastGatherLaunch) <= 4096 && sizeof(ClearLaunch) <= 4096,
               "launch descriptors must fit the kernel-argument segment");

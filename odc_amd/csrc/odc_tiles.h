@@ -316,8 +316,13 @@ ODC_HD bool has_edges(const TileWork& w) { return (w.nv != 0 && w.nv != kVecs) |
 
 // Whether the tile at this address of symmetric memory belongs to the part that stays in the last-level cache
 // (resident_below in odc_host.cpp): its 16 KiB granule's place in a sequence that is spread evenly over
-// [0, 2^32) lies below the line. A function of the address alone, so that launches of every kind agree,
+// [0, 2^32) lies below the line. A function of the address alone, so that launches of different kinds agree,
 // spread so that every stretch of memory has its share; a lower line keeps a part of what a higher one does.
+// The agreement is for speed only, and not complete. Asked is the address of a whole tile's first vector: where
+// tiles do not start on granules (allocations of less than one, ragged heads) a whole tile and the four short
+// ones of the same bytes can differ in the granule that they share with a neighbour. Left out are partial tiles,
+// converting gathers, publishes, accumulates and stores of cached gradients, clears below their line, and the
+// launches that read the whole table of their many items (FewTilesWalk).
 ODC_HD bool is_resident(uintptr_t address, uint32_t below) {
   return (uint32_t)(address >> 14) * 0x9E3779B1u < below;
 }
