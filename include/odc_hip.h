@@ -279,7 +279,8 @@ int odc_abi_version(void);
  *    accumulations the share that "resident_accumulation_bytes" (320 MiB) have of what is in use, where the
  *    launch's gradient is not cached itself, and of shards that are gathered without conversion the share of
  *    "resident_shard_bytes" (80 MiB); clears of more than twice "cached_gradient_bytes" leave theirs there from
- *    "resident_clear_bytes" (48 MiB) per launch on. Whole tiles only, and not in launches of more than 16 items
+ *    "resident_clear_bytes" (48 MiB) per launch on. Clears without such a part write through the L2 up to
+ *    "through_clear_bytes" (256 MiB) per launch. Resident parts: whole tiles only, and not in launches of more than 16 items
  *    in few short tiles. 0 keeps none.
  *  - "rank_stagger_bytes" (extra distance between rank regions), "rank_stride_align" (rank regions
  *    start on multiples of it, default 16384 = one tile) and "alloc_align" (allocations of at

@@ -83,6 +83,7 @@ struct Options {
   int64_t resident_shard_bytes = 80ll << 20;
   int64_t resident_above = 640ll << 20;
   int64_t resident_clear_bytes = 48ll << 20;
+  int64_t through_clear_bytes = 256ll << 20;  // see clear_form
   int64_t stream_bytes = 8ll << 20;  // see stream_form
   int64_t cast_output_bytes = 32ll << 20;  // see cast_output_form
   int64_t short_tiles_below = 32;             // see wants_short_tiles
@@ -119,6 +120,7 @@ int64_t* option_slot(const char* name) {
   if (!strcmp(name, "resident_shard_bytes")) return &g_opt.resident_shard_bytes;
   if (!strcmp(name, "resident_above")) return &g_opt.resident_above;
   if (!strcmp(name, "resident_clear_bytes")) return &g_opt.resident_clear_bytes;
+  if (!strcmp(name, "through_clear_bytes")) return &g_opt.through_clear_bytes;
   if (!strcmp(name, "cast_output_bytes")) return &g_opt.cast_output_bytes;
   if (!strcmp(name, "stream_bytes")) return &g_opt.stream_bytes;
   if (!strcmp(name, "short_tiles_below")) return &g_opt.short_tiles_below;
@@ -330,6 +332,15 @@ OutputForm output_form(const Options& opt, bool cached, uint64_t bytes) {
 // over converted copies of 12 to 57 MB: 185.8 -> 183.7, 245.3 -> 242.2.
 OutputForm cast_output_form(bool cached, uint64_t bytes, int64_t line) {
   return cached ? kKeep : bytes <= (uint64_t)line ? kWriteThrough : kStream;
+}
+
+// How a clear without a resident part writes its zeros: through the L2s while the last-level cache holds them
+// all, with plain stores beyond. Graph-replayed clears of fp32 accumulations at W = 8, us, plain -> written
+// through: one item of 0.26 M elements 1.95 -> 1.82, 1 M 2.36 -> 2.20, 2.1 M 3.06 -> 2.54, 4.2 M 4.53 -> 3.48, 8.4 M
+// 6.8 -> 5.5, 16.8 M 10.9 -> 9.7, 33 M 19.1 -> 17.8, 60 M (229 MiB) 32.8 -> 31.1; nine items, three sets in turn,
+// 33 M 23.7 -> 22.8, 60 M 41.6 -> 40.0, but 70 M 50.6 -> 53.1, 100 M 68.3 -> 72.7, a decoder layer 142 -> 148.
+OutputForm clear_form(const Options& opt, uint64_t bytes) {
+  return bytes <= (uint64_t)opt.through_clear_bytes ? kWriteThrough : kKeep;
 }
 
 // The items that the next launch over [next, n_items) can take, and their whole tiles and units on one rank.
@@ -954,6 +965,8 @@ int odc_clear(odc_arena* a, const odc_span* spans, uint32_t n_spans, void* strea
     const double resident = (double)cleared * below / 4294967296.0;
     if (cleared > 2 * (uint64_t)opt.cached_gradient_bytes && resident >= (double)opt.resident_clear_bytes)
       L.tt.resident_below = below;
+    else
+      L.output = clear_form(opt, cleared);
     const uint32_t grid = grid_for(a, opt.clear_blocks_per_cu, L.tt.n_tiles, kThreads);
     if (int rc = launch_tiles(a, L, grid, [&] { return odc_device::launch_clear(L, grid, stream); })) return rc;
   }

@@ -396,7 +396,10 @@ __global__ __launch_bounds__(T) ODC_RESIDENT_WAVES(kWaves) void gather_kernel(co
 }
 
 // ---- clear --------------------------------------------------------------------------------
-// Plain (not nontemporal) stores: for a write-only stream they measure faster here.
+// Written through the L2s into the last-level cache, which is where the next accumulate finds the zeros: with
+// plain stores the lines that the L2s hold at the end still have to leave them, which the kernel's last
+// microsecond went to. Longer clears than that cache holds (clear_form in odc_host.cpp) have plain stores,
+// which leave their end in the L2s. Nontemporal ones are behind both.
 __device__ __attribute__((noinline)) void clear_edges(uint8_t* d, uint32_t chunk, SegShape g) {
   d = as_global(d);
   const u32x4 zero = {0u, 0u, 0u, 0u};
@@ -412,7 +415,7 @@ __device__ __attribute__((noinline)) void clear_edges(uint8_t* d, uint32_t chunk
   if (w.tail && tid < g.tail) d[g.head + g.nvec * 16 + tid] = 0;
 }
 
-template <class Launch>
+template <class Launch, OutputForm kDst>
 __global__ __launch_bounds__(kThreads) void clear_kernel(const Launch launch) {
   const u32x4 zero = {0u, 0u, 0u, 0u};
   const uint32_t tid = threadIdx.x;
@@ -424,12 +427,17 @@ __global__ __launch_bounds__(kThreads) void clear_kernel(const Launch launch) {
     const SegShape g = seg_shape((uintptr_t)d, it.seg_bytes, 1, 16);
     const TileWork w = tile_work(c.chunk, g);
     if (is_whole(w)) {
-      u32x4* db = reinterpret_cast<u32x4*>(d + g.head) + w.v0 + tid;
-      const uint32_t below = walk.resident_below(launch);
-      with_policy(!below || is_resident((uintptr_t)(d + g.head + w.v0 * 16), below), [&](auto cached) {
+      u32x4* db = scalar_base(reinterpret_cast<u32x4*>(d + g.head) + w.v0);
+      if constexpr (kDst == kWriteThrough) {
 #pragma unroll
-        for (int u = 0; u < kUnroll; ++u) store_vec<cached>(db + u * kThreads, zero);
-      });
+        for (int u = 0; u < kUnroll; ++u) store_output<kWriteThrough, kTileVecs>(db, u * kThreads + tid, zero);
+      } else {
+        const uint32_t below = walk.resident_below(launch);
+        with_policy(!below || is_resident((uintptr_t)db, below), [&](auto cached) {
+#pragma unroll
+          for (int u = 0; u < kUnroll; ++u) store_vec<cached>(db + u * kThreads + tid, zero);
+        });
+      }
     }
     if (has_edges(w)) clear_edges(d, c.chunk, g);
   });
@@ -1153,8 +1161,10 @@ int launch_accum(int g, int a, bool store, const AccumLaunch& L, uint32_t grid, 
 }
 
 int launch_clear(const ClearLaunch& L, uint32_t grid, void* stream) {
-  return launch_form(L, grid, kThreads, 0u, stream,
-                     [](auto form) { return &clear_kernel<typename decltype(form)::type>; });
+  return launch_form(L, grid, kThreads, 0u, stream, [&](auto form) {
+    typedef typename decltype(form)::type F;
+    return L.output == kWriteThrough ? &clear_kernel<F, kWriteThrough> : &clear_kernel<F, kKeep>;
+  });
 }
 
 int launch_publish(int a, int o, const PublishLaunch& L, uint32_t grid, uint32_t lds_bytes, void* stream) {

@@ -32,8 +32,8 @@ struct CachePolicy {
   bool written = false;
 };
 
-// How a gather writes its output: past the caches, through the L2 into the last-level cache, or with
-// plain stores (store_output in odc_kernels.hip, output_form in odc_host.cpp).
+// How a gather writes its output, or a clear its zeros: past the caches, through the L2 into the last-level
+// cache, or with plain stores (store_output in odc_kernels.hip, output_form and clear_form in odc_host.cpp).
 enum OutputForm : uint32_t { kStream, kWriteThrough, kKeep };
 
 // How a launch is cut, and how its workgroups find their items (wants_short_tiles and tile_form in
@@ -191,6 +191,7 @@ struct ClearLaunch {
   TileTable tt;
   uint8_t* base;
   uint64_t rank_stride;
+  OutputForm output = kKeep;  // picks the kernel: kKeep or kWriteThrough
   ClearDesc item[kMaxItems];
 };
 
