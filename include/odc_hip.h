@@ -270,9 +270,10 @@ int odc_abi_version(void);
  *    caches into fp32; and, where they would go in whole tiles, gathers without conversion and accumulates and
  *    stores of fp32 gradients into fp32. Launches of persistent workgroups are not.
  *  - what a launch leaves in the caches: gathers of at most "cached_output_bytes" (64 MiB) of output
- *    leave it there, with plain stores up to "plain_output_bytes" (24 MiB) and written through the L2
- *    above; converting gathers of at most "cast_output_bytes" (32 MiB) of output write it through the L2
- *    (conversions of symmetric memory: "cached_output_bytes"); gradients of at most "cached_gradient_bytes"
+ *    leave it there, with plain stores up to "plain_output_bytes" (3 MiB) and written through the L2
+ *    above, and so do accumulates with the accumulations that they leave there; converting gathers of at most
+ *    "cast_output_bytes" (32 MiB) of output write it through the L2 (conversions of symmetric memory:
+ *    "cached_output_bytes"); gradients of at most "cached_gradient_bytes"
  *    (128 MiB) per launch are read through the caches; so are shards and accumulations while all symmetric
  *    memory in use, over all ranks, is at most "cached_arena_bytes" (192 MiB). 0 streams past the caches. Above
  *    "resident_above" (640 MiB) in use a part of the symmetric memory is kept in the last-level cache: of

@@ -77,7 +77,7 @@ struct Options {
   int64_t alloc_align = 16384;        // so do symmetric allocations at least this large
   int64_t cached_arena_bytes = 192ll << 20;   // these and the next two: see cache_policy
   int64_t cached_output_bytes = 64ll << 20;
-  int64_t plain_output_bytes = 24ll << 20;    // see output_form
+  int64_t plain_output_bytes = 3ll << 20;    // see output_form
   int64_t cached_gradient_bytes = 128ll << 20;
   int64_t resident_accumulation_bytes = 320ll << 20;  // these and the next two: see resident_below
   int64_t resident_shard_bytes = 80ll << 20;
@@ -272,8 +272,8 @@ uint32_t grid_for(const odc_arena* a, int64_t blocks_per_cu, uint32_t n_tiles, u
 //     elements, 3 sets) fill + accumulate 12.7 -> 10.8 and accumulate alone 8.9 -> 7.9, with 144 MB
 //     accumulate alone 14.6 -> 12.4 and gather alone 7.0 -> 6.2; with 600 MB (24 sets) fill +
 //     accumulate 12.8 -> 13.1 and gather + read 7.4 -> 8.0. The line is 192 MiB of the 256.
-// A store does not read the accumulation and keeps it nontemporal (level at best when plain). The converting
-// gather's output: cast_output_form.
+// A store does not read the accumulation and keeps it nontemporal (level at best when plain). How what stays is
+// written: output_form. The converting gather's output: cast_output_form.
 CachePolicy cache_policy(const odc_arena* a, const Options& opt, uint64_t read_bytes, int64_t read_line,
                          uint64_t written_bytes, int64_t written_line) {
   const bool arena_fits = a->in_use.load(std::memory_order_relaxed) * a->world <= (uint64_t)opt.cached_arena_bytes;
@@ -311,13 +311,23 @@ uint32_t resident_below(const odc_arena* a, const Options& opt, int64_t most) {
   return (uint32_t)std::min(4294967295.0, (double)most / in_use * 4294967296.0);
 }
 
-// How a gather writes an output that stays in the caches. Up to what the L2s hold (8 x 4 MB) plain
-// stores leave it there for the reader; beyond that it is written through to the last-level cache
-// (store_output in odc_kernels.hip has the figures). Below the line of 24 MiB plain stores are ahead:
-// passes of gather and accumulate over three sets of buffers in turn, us, plain -> written through: 18
-// MiB of output at W = 16 41.2 -> 42.1, 20 MiB at W = 8 41.0 -> 42.0; above it 29 MiB 61.2 -> 60.4, 34
-// MiB 98.7 -> 95.9, 42 MiB at W = 32 130.7 -> 125.0, 48 MiB 47.8 -> 45.6 (nontemporal stores: 57.9,
-// 97.0, 124.5, 43.0).
+// How a gather writes an output, and an accumulate accumulations, that stay in the caches: written through the
+// L2s to the last-level cache (store_output in odc_kernels.hip). Plain stores leave up to what the L2s hold (8 x 4
+// MB) in them as dirty lines, whose way out the kernel, or the next one, then waits for; the lines that are written
+// through stay there for the next kernel too. Below 3 MiB the two are level or plain stores ahead by up to 0.1 us.
+// Graph-replayed launches at W = 8, us, plain -> written through, one item on one set of buffers, nine items on
+// three sets in turn:
+//   gather of bf16: 1 M elements 2.25 -> 2.28, 2.55 -> 2.76; 2.1 M 2.48 -> 2.38, 3.06 -> 3.07; 4.2 M 3.27 -> 2.84, 4.24 ->
+//     3.61; 8.4 M (16 MiB of output) 4.90 -> 4.09, 6.54 -> 6.35;
+//   accumulate of bf16 into fp32: 0.26 M 2.01 -> 2.07; 1 M 2.60 -> 2.61, 3.43 -> 3.28; 2.1 M 3.37 -> 3.52, 4.80 -> 4.08;
+//     4.2 M 5.16 -> 6.49, 7.66 -> 6.96; 8.4 M 11.8 -> 9.3, 12.8 -> 12.1; 16.8 M 21.9 -> 21.1, 24.0 -> 24.0; into bf16
+//     4.2 M 4.06 -> 3.61, 6.05 -> 5.33; 8.4 M 6.21 -> 5.62, 9.28 -> 8.67;
+//   (the two that are slower repeat one accumulate and nothing else, so that accumulations of up to 16 MB never
+//   leave the L2s; with a gather in front of it the same 4.2 M elements take 9.72 -> 8.12;)
+//   a minibatch of four microbatches: 1 M 24.1 -> 22.7, 30.4 -> 27.5; 4.2 M 51.1 -> 37.7, 51.9 -> 47.8; 16.8 M 139 -> 133,
+//     162.5 -> 161.5; 33 M 279 -> 270, but its pass of one gather and one accumulate 65.1 -> 66.6.
+// With products of 128 to 1024 tokens that read the output and write the gradient behind the gather, outputs of
+// 1 to 25 MiB: level or ahead by up to 2 % (9 MiB, 512 tokens, forward 28.05 -> 27.4, with backward 57.5 -> 57.1).
 OutputForm output_form(const Options& opt, bool cached, uint64_t bytes) {
   if (!cached) return kStream;
   return bytes <= (uint64_t)opt.plain_output_bytes ? kKeep : kWriteThrough;
@@ -458,7 +468,7 @@ TileForm stream_form(const odc_arena* a, const Options& opt, const LaunchSize& s
 
 // The same for an accumulate or a store.
 TileForm scatter_stream_form(const odc_arena* a, const Options& opt, const LaunchSize& size, int grad_dtype, int acc_dtype,
-                             bool store, CachePolicy policy, TileForm cut) {
+                             bool store, AccumPolicy policy, TileForm cut) {
   if (acc_dtype != ODC_DTYPE_F32) return cut;
   if (grad_dtype == ODC_DTYPE_F32 ? cut != kWholeTiles : store || policy.read) return cut;
   return stream_form(a, opt, size, size.units * 4 * a->world, cut);
@@ -1041,10 +1051,12 @@ int scatter_launch(odc_arena* a, const odc_accum_item* items, uint32_t n_items, 
                                                     [&](uint32_t i) { grad_elems += items[order[i]].grad_elems; });
     TileForm cut = scatter_in_short_tiles(a, size, opt.short_tiles_below, grad_dtype, acc_dtype, store) ? kShortTiles
                                                                                                       : kWholeTiles;
-    L.policy = cache_policy(a, opt, grad_elems * gb, opt.cached_gradient_bytes, 0, kSymmetric);
+    const CachePolicy cached = cache_policy(a, opt, grad_elems * gb, opt.cached_gradient_bytes, 0, kSymmetric);
+    L.policy.read = cached.read;
+    L.policy.written = output_form(opt, cached.written, size.units * ab * a->world);
     const bool one_per_tile = (store ? opt.store_blocks_per_cu : opt.accum_blocks_per_cu) <= 0 &&
                               (store || opt.accum_persistent_below_tiles == 0);
-    if (one_per_tile && !(L.policy.read && L.policy.written))
+    if (one_per_tile && !(L.policy.read && L.policy.written != kStream))
       cut = scatter_stream_form(a, opt, size, grad_dtype, acc_dtype, store, L.policy, cut);
     const int n = fill_launch<kTileElems>(
         L.tt, a->world, n_items, &next, cut, units,

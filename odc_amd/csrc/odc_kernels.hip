@@ -113,11 +113,11 @@ __device__ __forceinline__ void store_vec(V* p, V v) {  // aligned
   if constexpr (kCached) *p = v; else __builtin_nontemporal_store(v, p);
 }
 
-// A whole tile of a gather's output, converted or not: vector `i` of the kVecs that start at `tile`, an address that all
-// lanes agree on. Outputs that the next kernel is to find in the last-level cache, but that are more
-// than the L2s hold, are written through the L2: left in it by plain stores they went to memory only as other
-// lines pushed them out, between the reads of whatever ran next. us, nontemporal / plain / written
-// through (a decoder layer's nine parameters, bf16, W = 8, three sets of buffers in turn):
+// A whole tile of a gather's output, converted or not, of a clear or of accumulations: vector `i` of the kVecs that
+// start at `tile`, an address that all lanes agree on. What the next kernel is to find in the last-level cache is
+// written through the L2 (output_form, cast_output_form and clear_form in odc_host.cpp say from which size on): left
+// in it by plain stores it goes to memory only at the kernel's end or as other lines push it out, between the
+// reads of whatever runs next. us, nontemporal / plain / written through (a decoder layer's nine parameters, bf16, W = 8, three sets of buffers in turn):
 //   gather alone: 35 MiB of output 14.4 / 15.7 / 13.2, 48 MiB 18.6 / 16.7 / 15.4;
 //   an accumulate behind it, nothing reads the output: 32.1 / 31.9 / 29.4, 40.4 / 41.7 / 41.1;
 //   the products that read the parameters behind it (1024 tokens): 141 / 129 / 126.5, 184 / 160 / 158.5.
@@ -533,10 +533,11 @@ template <> struct Quad<f16_tag> {
 // gradient's end may cut is read as elements by the lane that owns it. Nine items of 3 640
 // elements per rank (W = 8, one partial tile each) take 3.8 us instead of 5.4, with gradients that end inside
 // the last rank's segment 4.0 instead of 4.8 (13 889 elements per rank).
-template <class G, class A, bool kStore, bool kGradCached, bool kAccCached, int T, int U>
+template <class G, class A, bool kStore, bool kGradCached, OutputForm kAcc, int T, int U>
 __device__ __attribute__((noinline)) void accum_edges(uint8_t* acc, const uint8_t* grad, uint64_t g_seg,
                                                       uint64_t grad_elems, uint32_t chunk, SegShape g,
                                                       bool body) {
+  constexpr bool kAccCached = kAcc != kStream;
   acc = as_global(acc);
   grad = as_global(grad);
   typedef typename Quad<G>::vec_t gvec_t;
@@ -609,7 +610,8 @@ __device__ __attribute__((noinline)) void accum_edges(uint8_t* acc, const uint8_
   if (do_tail) as[tail_at] = Codec<A>::narrow(Codec<A>::widen(tail_araw) + Codec<G>::widen(tail_graw));
 }
 
-template <class Launch, class G, class A, bool kStore, bool kGradCached, bool kAccCached, bool kFew, int T, int U,
+// kAcc: how the accumulations are written; read past the caches with kStream, through them otherwise.
+template <class Launch, class G, class A, bool kStore, bool kGradCached, OutputForm kAcc, bool kFew, int T, int U,
           int kWaves = kMostWaves>
 __global__ __launch_bounds__(T) ODC_RESIDENT_WAVES(kWaves) void accum_kernel(const Launch launch) {
   constexpr uint32_t kVecs = T * U;  // quads
@@ -639,7 +641,8 @@ __global__ __launch_bounds__(T) ODC_RESIDENT_WAVES(kWaves) void accum_kernel(con
         gb[u] = scalar_base(it.grad + (g_seg + e0 + u * T * 4) * kGB);
         ap[u] = scalar_base(reinterpret_cast<avec_t*>(acc + e0 * kAB) + u * T);
       }
-      with_policy(kAccCached || is_resident((uintptr_t)(acc + e0 * kAB), walk.resident_below(launch)), [&](auto cached) {
+      with_policy(kAcc != kStream || is_resident((uintptr_t)(acc + e0 * kAB), walk.resident_below(launch)), [&](auto cached) {
+        constexpr OutputForm kWritten = kAcc == kStream && cached ? kKeep : kAcc;  // (resident parts: plain stores)
         gvec_t graw[U];
         avec_t araw[U];
 #pragma unroll
@@ -655,12 +658,12 @@ __global__ __launch_bounds__(T) ODC_RESIDENT_WAVES(kWaves) void accum_kernel(con
           if constexpr (!kStore) Quad<A>::widen(araw[u], af);
 #pragma unroll
           for (int k = 0; k < 4; ++k) af[k] = af[k] + gf[k];
-          store_vec<cached>(ap[u] + tid, Quad<A>::narrow(af));
+          store_output<kWritten, kVecs>(ap[0], u * T + tid, Quad<A>::narrow(af));
         }
       });
     }
     if (!whole ? (w.nv != 0 || w.head || w.tail) : (w.head || w.tail))
-      accum_edges<G, A, kStore, kGradCached, kAccCached, T, U>(acc, it.grad, g_seg, it.grad_elems, c.chunk, g, !whole);
+      accum_edges<G, A, kStore, kGradCached, kAcc, T, U>(acc, it.grad, g_seg, it.grad_elems, c.chunk, g, !whole);
   });
 }
 
@@ -914,32 +917,33 @@ constexpr bool kGathersWholeTiles = !std::is_same_v<decltype(Launch::tt), ItemsT
 // (gradient dtype, accumulation dtype). The store form never reads the accumulation and keeps it
 // nontemporal; the read-modify-write keeps it cached only together with the gradient.
 template <class L, class G, class A, bool kFew, int T, int U>
-kernel_fn<L> pick_rmw(CachePolicy policy) {
-  if (policy.read && policy.written) return accum_kernel<L, G, A, false, true, true, kFew, T, U>;
-  return policy.read ? accum_kernel<L, G, A, false, true, false, kFew, T, U>
-                     : accum_kernel<L, G, A, false, false, false, kFew, T, U>;
+kernel_fn<L> pick_rmw(AccumPolicy policy) {
+  if (policy.read && policy.written == kKeep) return accum_kernel<L, G, A, false, true, kKeep, kFew, T, U>;
+  if (policy.read && policy.written == kWriteThrough) return accum_kernel<L, G, A, false, true, kWriteThrough, kFew, T, U>;
+  return policy.read ? accum_kernel<L, G, A, false, true, kStream, kFew, T, U>
+                     : accum_kernel<L, G, A, false, false, kStream, kFew, T, U>;
 }
 
 template <class L, class G, class A, bool kFew, int T, int U, int kWaves = kMostWaves>
-kernel_fn<L> pick_store(CachePolicy policy) {
-  return policy.read ? accum_kernel<L, G, A, true, true, false, kFew, T, U, kWaves>
-                     : accum_kernel<L, G, A, true, false, false, kFew, T, U, kWaves>;
+kernel_fn<L> pick_store(AccumPolicy policy) {
+  return policy.read ? accum_kernel<L, G, A, true, true, kStream, kFew, T, U, kWaves>
+                     : accum_kernel<L, G, A, true, false, kStream, kFew, T, U, kWaves>;
 }
 
 // kShortOnly: accum_streams_short says so, there is no kernel of whole tiles.
 template <class L, class G, class A, bool kShortOnly>
-kernel_fn<L> pick_accum_tiles(bool store, CachePolicy policy, TileForm form);
+kernel_fn<L> pick_accum_tiles(bool store, AccumPolicy policy, TileForm form);
 
 template <class L, class G, class A, bool kShortOnly>
-kernel_fn<L> pick_accum_form(bool store, CachePolicy policy, TileForm form) {
+kernel_fn<L> pick_accum_form(bool store, AccumPolicy policy, TileForm form) {
   if (form == kStreamTiles) {  // into fp32: what scatter_stream_form in odc_host.cpp sends here
     if constexpr (kStreams<L> && Codec<A>::kBytes == 4) {
       if constexpr (Codec<G>::kBytes == 4) {
         if (store) return pick_store<L, G, A, false, kShortThreads, kShortUnroll, kStreamWaves>(policy);
-        if (policy.read) return accum_kernel<L, G, A, false, true, false, false, kShortThreads, kShortUnroll, kStreamWaves>;
+        if (policy.read) return accum_kernel<L, G, A, false, true, kStream, false, kShortThreads, kShortUnroll, kStreamWaves>;
       }
       if (!store && !policy.read)
-        return accum_kernel<L, G, A, false, false, false, false, kShortThreads, kShortUnroll, kStreamWaves>;
+        return accum_kernel<L, G, A, false, false, kStream, false, kShortThreads, kShortUnroll, kStreamWaves>;
     }
     return nullptr;
   }
@@ -948,7 +952,7 @@ kernel_fn<L> pick_accum_form(bool store, CachePolicy policy, TileForm form) {
 }
 
 template <class L, class G, class A, bool kShortOnly>
-kernel_fn<L> pick_accum_tiles(bool store, CachePolicy policy, TileForm form) {
+kernel_fn<L> pick_accum_tiles(bool store, AccumPolicy policy, TileForm form) {
   if (form == kFewShortTiles)
     return store ? pick_store<L, G, A, kSearches<L>, kShortThreads, kShortUnroll>(policy)
                  : pick_rmw<L, G, A, kSearches<L>, kShortThreads, kShortUnroll>(policy);
@@ -959,14 +963,14 @@ kernel_fn<L> pick_accum_tiles(bool store, CachePolicy policy, TileForm form) {
   else if constexpr (Codec<G>::kBytes == 2 && Codec<A>::kBytes == 2) {
     if (store) return pick_store<L, G, A, false, kThreads, kUnroll>(policy);
     return policy.read ? pick_rmw<L, G, A, false, kThreads, kUnroll>(policy)
-                       : accum_kernel<L, G, A, false, false, false, false, kNarrowRmwThreads, kNarrowRmwUnroll>;
+                       : accum_kernel<L, G, A, false, false, kStream, false, kNarrowRmwThreads, kNarrowRmwUnroll>;
   } else
     return store ? pick_store<L, G, A, false, kStoreThreads, kStoreUnroll>(policy)
                  : pick_rmw<L, G, A, false, kThreads, kUnroll>(policy);
 }
 
 template <class L>
-kernel_fn<L> pick_accum(int g, int a, bool store, CachePolicy policy, TileForm form) {
+kernel_fn<L> pick_accum(int g, int a, bool store, AccumPolicy policy, TileForm form) {
 #define X(E1, T1, E2, T2) \
   if (g == E1 && a == E2) return pick_accum_form<L, T1, T2, accum_streams_short(E1, E2)>(store, policy, form);
   ODC_FOR_EACH_DTYPE_PAIR(X)

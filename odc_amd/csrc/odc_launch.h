@@ -24,17 +24,24 @@ using odc_tiles::kTileVecs;
 using odc_tiles::TileTable;
 
 // Whether a launch leaves what it reads / what it writes in the caches (plain accesses) or streams
-// past them (nontemporal ones). For the accumulate "read" is the gradient and "written" the
-// accumulation, read and written; for the gathers they are the shards and the output (OutputForm for
+// past them (nontemporal ones). For the gathers these are the shards and the output (OutputForm for
 // the plain gather's).
 struct CachePolicy {
   bool read = false;
   bool written = false;
 };
 
-// How a gather writes its output, or a clear its zeros: past the caches, through the L2 into the last-level
-// cache, or with plain stores (store_output in odc_kernels.hip, output_form and clear_form in odc_host.cpp).
+// How a gather writes its output, an accumulate its accumulations or a clear its zeros: past the caches, through
+// the L2 into the last-level cache, or with plain stores (store_output in odc_kernels.hip, output_form and
+// clear_form in odc_host.cpp).
 enum OutputForm : uint32_t { kStream, kWriteThrough, kKeep };
+
+// The same for an accumulate: "read" is the gradient, "written" the accumulations, which are read through the
+// caches where they are written through or into them.
+struct AccumPolicy {
+  bool read = false;
+  OutputForm written = kStream;
+};
 
 // How a launch is cut, and how its workgroups find their items (wants_short_tiles and tile_form in
 // odc_host.cpp). kStreamTiles: short tiles of a long stream (stream_form there).
@@ -91,7 +98,7 @@ constexpr int kShortUnroll = (int)kShortTileVecs / kShortThreads;
 // The workgroup sizes of the launches, as the pick_* functions of odc_kernels.hip take them.
 inline uint32_t copy_threads(TileForm form) { return form != kWholeTiles ? kShortThreads : kCopyThreads; }
 inline uint32_t publish_threads(TileForm form) { return form != kWholeTiles ? kShortThreads : kThreads; }
-inline uint32_t accum_threads(int grad_dtype, int acc_dtype, bool store, CachePolicy policy, TileForm form) {
+inline uint32_t accum_threads(int grad_dtype, int acc_dtype, bool store, AccumPolicy policy, TileForm form) {
   if (form != kWholeTiles) return kShortThreads;
   if (grad_dtype != ODC_DTYPE_F32 && acc_dtype != ODC_DTYPE_F32)
     return store || policy.read ? kThreads : kNarrowRmwThreads;
@@ -176,7 +183,7 @@ struct AccumLaunch {
   TileTable tt;
   uint8_t* base;
   uint64_t rank_stride;
-  CachePolicy policy;    // these two pick the kernel
+  AccumPolicy policy;    // these two pick the kernel
   TileForm form = kWholeTiles;
   AccumDesc item[kMaxItems];
 };
