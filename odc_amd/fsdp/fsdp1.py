@@ -246,13 +246,17 @@ def unpatch_fsdp1():
 
 def pre_optimizer_step(fsdp_module):
     """fsdp1.py:317-335: wait for every add, post-divide, publish the accumulations as
-    ``flat_param.grad`` in the parameter dtype."""
+    ``flat_param.grad`` in the parameter dtype. The publish is launched behind the adds before the host
+    waits for them (``ReductionService.syncing``)."""
     shards_may_have_changed()  # the optimizer is about to change them
-    with torch.cuda.nvtx.range("scatter_accumulate_sync"):
-        get_reduction_service().sync(getattr(fsdp_module, "process_group", None))
-    if hasattr(fsdp_module, "_inter_node_pg"):
-        raise NotImplementedError("hybrid sharding needs a second node; not part of this build")
     service = get_reduction_service()
+    with torch.cuda.nvtx.range("scatter_accumulate_sync"), service.syncing(getattr(fsdp_module, "process_group", None)):
+        if hasattr(fsdp_module, "_inter_node_pg"):
+            raise NotImplementedError("hybrid sharding needs a second node; not part of this build")
+        _publish_gradients(fsdp_module, service)
+
+
+def _publish_gradients(fsdp_module, service):
     factor = getattr(fsdp_module, "_gradient_postdivide_factor", 1.0)
     divisor = factor if factor is not None and factor > 1 else 1.0  # `_div_if_needed`
     # a unit that never saw a gradient (frozen, or unused so far) has no accumulation yet

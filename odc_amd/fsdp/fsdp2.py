@@ -657,22 +657,36 @@ def pre_minibatch_start(fsdp_module):
 
 
 def pre_optimizer_step(fsdp_module):
-    """fsdp2.py:1023-1046: sync once, then publish every group's gradients."""
+    """fsdp2.py:1023-1046: sync once and publish every group's gradients. The publish is launched behind
+    the adds before the host waits for them (``ReductionService.syncing``)."""
     shards_may_have_changed()  # the optimizer is about to change the shards
     scatter = get_reduction_service()
     if _is_torch_fsdp_module(fsdp_module):
         groups = _torch_param_groups(fsdp_module)
         if groups:
-            with torch.cuda.nvtx.range("scatter_accumulate_sync"):
-                scatter.sync(groups[0].mesh_info.shard_process_group)
-            update_all_gradients(groups)
+            pg = groups[0].mesh_info.shard_process_group
+            if any(map(_has_gradient_hooks, groups)):  # theirs to run after the sync
+                with torch.cuda.nvtx.range("scatter_accumulate_sync"):
+                    scatter.sync(pg)
+                update_all_gradients(groups)
+            else:
+                with torch.cuda.nvtx.range("scatter_accumulate_sync"), scatter.syncing(pg):
+                    update_all_gradients(groups)
         return
-    for i, group in enumerate(_param_groups(fsdp_module)):
-        if i == 0:
-            with torch.cuda.nvtx.range("scatter_accumulate_sync"):
-                scatter.sync(group.pg)
-        with torch.cuda.nvtx.range(f"update_gradients:{group.name}"):
-            group.update_gradients()
+    groups = _param_groups(fsdp_module)
+    if groups:
+        with torch.cuda.nvtx.range("scatter_accumulate_sync"), scatter.syncing(groups[0].pg):
+            for group in groups:
+                with torch.cuda.nvtx.range(f"update_gradients:{group.name}"):
+                    group.update_gradients()
+
+
+def _has_gradient_hooks(fsdp_param_group) -> bool:
+    """Whether a user's code runs while the group's gradients are handed out."""
+    ctx = getattr(fsdp_param_group, "_odc_reduce_context", None)
+    return (ctx is not None and ctx["all_reduce_hook"] is not None) or any(
+        getattr(fp.sharded_param, "_post_accumulate_grad_hooks", None) for fp in fsdp_param_group.fsdp_params
+    )
 
 
 def _comm_context_lazy_init(self, device):

@@ -52,7 +52,9 @@ from odc_amd.primitives.utils import (
     StreamOrder,
     SymmBufferRegistry,
     comm_stream_section,
+    launches_in_flight,
     plain_launch_stream,
+    wait_for_events,
     wait_for_launches,
     get_world,
     group_size,
@@ -583,6 +585,24 @@ class ReductionService:
         wait_for_launches()
         with self._lock:
             self.dispatched_tasks = 0
+
+    @contextlib.contextmanager
+    def syncing(self, pg=None):
+        """``with service.syncing(pg): ...`` — ``sync`` with the block's host work and launches behind
+        the adds on the device and in front of the wait on the host: at its end every add dispatched
+        before it has landed. With the wait in front the GPU had nothing to do from the last add until
+        the host had woken up and launched the publish."""
+        if _is_capturing():  # (there is nothing the host could wait for: sync refuses)
+            self.sync(pg)
+            yield
+            return
+        events = launches_in_flight()
+        try:
+            yield
+        finally:
+            wait_for_events(events)
+            with self._lock:
+                self.dispatched_tasks = 0
 
     def stop(self):
         if torch.cuda.is_available():

@@ -711,6 +711,36 @@ def wait_for_launches() -> None:
             torch.cuda.synchronize(get_world().arena.device)
 
 
+def launches_in_flight():
+    """An event behind every launch issued so far through ``comm_stream_section``, for
+    ``wait_for_events``: ``wait_for_launches`` in two halves, so that the host can issue what comes next
+    before it waits. The current stream waits for the launches on the others, so what comes next finds
+    them done, as it would after ``wait_for_launches``."""
+    device = get_world().device
+    with _launch_lock:
+        pending = list(_launch_streams.items())
+        _launch_streams.clear()
+    current, events = torch.cuda.current_stream(device), []
+    for handle, s in pending:
+        event = torch.cuda.Event()
+        try:
+            if handle == current.cuda_stream:
+                event.record(current)
+            else:
+                event.record(s if s is not None else stream_from_handle(handle))
+                current.wait_event(event)
+        except RuntimeError:  # a stream destroyed since its launch, see wait_for_launches
+            torch.cuda.synchronize(device)
+            continue
+        events.append(event)
+    return events
+
+
+def wait_for_events(events) -> None:
+    for event in events:
+        event.synchronize()
+
+
 class BufferSplitter:
     """Sub-request sizing rule of the reference (``utils.py:212-242``), in elements.
 

@@ -1,0 +1,58 @@
+"""``ReductionService.syncing``: what its block launches comes behind the adds of every stream, and at its end the
+host has waited for them."""
+
+import types
+
+import pytest
+import torch
+
+from helpers import assert_bit_equal
+from oracle import odc_oracle as oracle
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("policy", [None, "dedicated"])
+def test_publish_behind_adds_of_a_busy_stream(make_world, policy, monkeypatch):
+    from odc_amd import ReductionService
+
+    if policy:
+        monkeypatch.setenv("ODC_COMM_STREAM", policy)
+    W, n = 4, 40_000
+    group = make_world(W, 4 << 20)
+    service = ReductionService(accumulation_dtype=torch.float32)
+    service.register("k", (n,), torch.bfloat16, torch.float32, group)
+    gen = torch.Generator().manual_seed(1)
+    grads = [torch.randn(W * n, generator=gen).bfloat16() for _ in range(3)]
+    on_device = [g.cuda() for g in grads]
+    work = [torch.randn(2048, 2048, device="cuda") for _ in grads]
+    torch.cuda.synchronize()
+    sides = [torch.cuda.Stream() for _ in range(2)]
+    for side, g, w in zip((*sides, torch.cuda.current_stream()), on_device, work):
+        with torch.cuda.stream(side):
+            for _ in range(20):
+                torch.mm(w, w).mul_(1e-4)
+            service.scatter_accumulate("k", g, group)
+    with service.syncing(group):
+        (out,) = service.publish(["k"], out_dtype=torch.bfloat16, divisor=float(W))
+    assert service.dispatched_tasks == 0
+    if not policy:  # (the adds are on the callers' streams)
+        assert all(side.query() for side in sides)
+    want = torch.zeros(n)
+    for g in grads:
+        oracle.scatter_accumulate([want] + [torch.zeros(n) for _ in range(W - 1)], g)
+    want /= W
+    assert_bit_equal(out, want.bfloat16())
+
+
+def test_users_hooks_are_seen():
+    from odc_amd.fsdp.fsdp2 import _has_gradient_hooks
+
+    def group(all_reduce_hook=None, hooks=None, reduced=True):
+        param = types.SimpleNamespace(sharded_param=types.SimpleNamespace(_post_accumulate_grad_hooks=hooks))
+        group = types.SimpleNamespace(fsdp_params=[param])
+        if reduced:
+            group._odc_reduce_context = {"all_reduce_hook": all_reduce_hook}
+        return group
+
+    assert not _has_gradient_hooks(group()) and not _has_gradient_hooks(group(hooks={}, reduced=False))
+    assert _has_gradient_hooks(group(all_reduce_hook=print)) and _has_gradient_hooks(group(hooks={0: print}))
