@@ -271,7 +271,8 @@ int odc_abi_version(void);
  *    stores of fp32 gradients into fp32. Launches of persistent workgroups are not.
  *  - what a launch leaves in the caches: gathers of at most "cached_output_bytes" (64 MiB) of output
  *    leave it there, with plain stores up to "plain_output_bytes" (3 MiB) and written through the L2
- *    above, and so do accumulates with the accumulations that they leave there; converting gathers of at most
+ *    above, and so do accumulates with the accumulations that they leave there (stores only between
+ *    "plain_output_bytes" and "cached_output_bytes"); converting gathers of at most
  *    "cast_output_bytes" (32 MiB) of output write it through the L2 (conversions of symmetric memory:
  *    "cached_output_bytes"); gradients of at most "cached_gradient_bytes"
  *    (128 MiB) per launch are read through the caches; so are shards and accumulations while all symmetric

@@ -272,8 +272,8 @@ uint32_t grid_for(const odc_arena* a, int64_t blocks_per_cu, uint32_t n_tiles, u
 //     elements, 3 sets) fill + accumulate 12.7 -> 10.8 and accumulate alone 8.9 -> 7.9, with 144 MB
 //     accumulate alone 14.6 -> 12.4 and gather alone 7.0 -> 6.2; with 600 MB (24 sets) fill +
 //     accumulate 12.8 -> 13.1 and gather + read 7.4 -> 8.0. The line is 192 MiB of the 256.
-// A store does not read the accumulation and keeps it nontemporal (level at best when plain). How what stays is
-// written: output_form. The converting gather's output: cast_output_form.
+// How what stays is written: output_form, a store's accumulations: store_output_form, the converting gather's output:
+// cast_output_form.
 CachePolicy cache_policy(const odc_arena* a, const Options& opt, uint64_t read_bytes, int64_t read_line,
                          uint64_t written_bytes, int64_t written_line) {
   const bool arena_fits = a->in_use.load(std::memory_order_relaxed) * a->world <= (uint64_t)opt.cached_arena_bytes;
@@ -331,6 +331,17 @@ uint32_t resident_below(const odc_arena* a, const Options& opt, int64_t most) {
 OutputForm output_form(const Options& opt, bool cached, uint64_t bytes) {
   if (!cached) return kStream;
   return bytes <= (uint64_t)opt.plain_output_bytes ? kKeep : kWriteThrough;
+}
+
+// A store's accumulations, which it does not read: written through from 3 to 64 MiB, nontemporal otherwise. The same
+// launches, and passes of gather, store, gather, accumulate, us, nontemporal -> written through:
+//   store of bf16 into fp32: 0.52 M elements 2.19 -> 2.24, 2.66 -> 2.60; 1 M 2.51 -> 2.41, 3.05 -> 3.00; 4.2 M 4.30 -> 4.48, 5.19
+//     -> 4.90; 16.8 M (64 MiB) 13.5 -> 12.1, 14.5 -> 14.7; into bf16 4.2 M 3.31 -> 3.02, 16.8 M 9.55 -> 7.87;
+//   passes: 1 M 9.61 -> 8.70, 11.74 -> 10.90; 4.2 M 16.06 -> 14.33, 20.02 -> 19.10; 8.4 M 28.7 -> 26.9, 34.1 -> 35.2; 33 M
+//     105 .. 107 -> 111 .. 116.
+OutputForm store_output_form(const Options& opt, bool cached, uint64_t bytes) {
+  const bool through = cached && bytes > (uint64_t)opt.plain_output_bytes && bytes <= (uint64_t)opt.cached_output_bytes;
+  return through ? kWriteThrough : kStream;
 }
 
 // The same for a gather that converts, and for a conversion of symmetric memory, which are ahead with the output
@@ -1053,10 +1064,12 @@ int scatter_launch(odc_arena* a, const odc_accum_item* items, uint32_t n_items, 
                                                                                                       : kWholeTiles;
     const CachePolicy cached = cache_policy(a, opt, grad_elems * gb, opt.cached_gradient_bytes, 0, kSymmetric);
     L.policy.read = cached.read;
-    L.policy.written = output_form(opt, cached.written, size.units * ab * a->world);
+    const uint64_t written_bytes = size.units * ab * a->world;
+    L.policy.written = store ? store_output_form(opt, cached.written, written_bytes)
+                             : output_form(opt, cached.written, written_bytes);
     const bool one_per_tile = (store ? opt.store_blocks_per_cu : opt.accum_blocks_per_cu) <= 0 &&
                               (store || opt.accum_persistent_below_tiles == 0);
-    if (one_per_tile && !(L.policy.read && L.policy.written != kStream))
+    if (one_per_tile && !(cached.read && cached.written))
       cut = scatter_stream_form(a, opt, size, grad_dtype, acc_dtype, store, L.policy, cut);
     const int n = fill_launch<kTileElems>(
         L.tt, a->world, n_items, &next, cut, units,

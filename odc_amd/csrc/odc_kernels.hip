@@ -914,8 +914,8 @@ constexpr bool kGathersWholeTiles = !std::is_same_v<decltype(Launch::tt), ItemsT
   X(ODC_DTYPE_F32, f32_tag, ODC_DTYPE_F16, f16_tag)     \
   X(ODC_DTYPE_F32, f32_tag, ODC_DTYPE_F32, f32_tag)
 
-// (gradient dtype, accumulation dtype). The store form never reads the accumulation and keeps it
-// nontemporal; the read-modify-write keeps it cached only together with the gradient.
+// (gradient dtype, accumulation dtype). Accumulations are cached only together with the gradient; by a store,
+// which does not read them, only written through (store_output_form in odc_host.cpp).
 template <class L, class G, class A, bool kFew, int T, int U>
 kernel_fn<L> pick_rmw(AccumPolicy policy) {
   if (policy.read && policy.written == kKeep) return accum_kernel<L, G, A, false, true, kKeep, kFew, T, U>;
@@ -926,6 +926,8 @@ kernel_fn<L> pick_rmw(AccumPolicy policy) {
 
 template <class L, class G, class A, bool kFew, int T, int U, int kWaves = kMostWaves>
 kernel_fn<L> pick_store(AccumPolicy policy) {
+  if (policy.read && policy.written == kWriteThrough)
+    return accum_kernel<L, G, A, true, true, kWriteThrough, kFew, T, U, kWaves>;
   return policy.read ? accum_kernel<L, G, A, true, true, kStream, kFew, T, U, kWaves>
                      : accum_kernel<L, G, A, true, false, kStream, kFew, T, U, kWaves>;
 }
