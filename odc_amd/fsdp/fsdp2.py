@@ -173,6 +173,7 @@ class ParamGroup:
         self.symm_buffer = SymmBufferRegistry.get_instance().get_or_create_symm_buffer(
             self.key, (self.total_shard_numel,), dtype
         )
+        self._gradient_layouts = {}
         self._unsharded: Optional[List[torch.Tensor]] = None
         self._reduced = False
 
@@ -281,14 +282,20 @@ class ParamGroup:
 
     # -- publish ----------------------------------------------------------------------------
     def _gradient_layout(self, rank: int):
-        """(sizes, strides, offset) of the rank's sharded gradients in the published accumulation."""
-        layout = []
-        for p, shape in enumerate(self.shapes):
-            inner, acc = [], 1  # contiguous strides of (rows, *rest), valid for rows == 0 too
-            for d in reversed(shape[1:]):
-                inner.append(acc)
-                acc *= d
-            layout.append(((self.local_shard_rows(p, rank), *shape[1:]), (acc, *reversed(inner)), self.acc_offsets[p]))
+        """(sizes, strides, offset) of the rank's sharded gradients in the published accumulation, worked out
+        once per rank: the shapes and, from the first reduce on, the offsets stay as they are."""
+        layout = self._gradient_layouts.get(rank)
+        if layout is None:
+            layout = []
+            for p, shape in enumerate(self.shapes):
+                inner, acc = [], 1  # contiguous strides of (rows, *rest), valid for rows == 0 too
+                for d in reversed(shape[1:]):
+                    inner.append(acc)
+                    acc *= d
+                layout.append(
+                    ((self.local_shard_rows(p, rank), *shape[1:]), (acc, *reversed(inner)), self.acc_offsets[p])
+                )
+            self._gradient_layouts[rank] = layout
         return layout
 
     def update_gradients(self) -> Optional[List[torch.Tensor]]:
