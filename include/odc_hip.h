@@ -62,7 +62,8 @@ enum {
                                (odc_get_option "dry_run_launches" / "dry_run_tiles" /
                                "dry_run_workgroups", and of the launches those in short tiles,
                                "dry_run_short_launches" / "dry_run_few_launches" by how a tile finds
-                               its item, long streams, "dry_run_stream_launches", and those told of a
+                               its item, of the latter those of one wavefront per tile,
+                               "dry_run_tiny_launches", long streams, "dry_run_stream_launches", and those told of a
                                resident part, "dry_run_resident_launches";
                                odc_set_option("dry_run_reset", 0) zeroes them).
                                For testing the host side of the library without a device; implies

@@ -202,7 +202,7 @@ int check_compute(odc_arena* a, DeviceGuard& guard) {
 
 // What dry-run arenas have "launched" (process-wide, reset by odc_set_option("dry_run_reset", 0)).
 std::atomic<int64_t> g_dry_launches{0}, g_dry_tiles{0}, g_dry_workgroups{0};
-std::atomic<int64_t> g_dry_short{0}, g_dry_few{0}, g_dry_stream{0};  // of the launches: those in kShortTiles, ...
+std::atomic<int64_t> g_dry_short{0}, g_dry_few{0}, g_dry_tiny{0}, g_dry_stream{0};  // of the launches: those in kShortTiles, ...
 std::atomic<int64_t> g_dry_resident{0};  // those that are told of a resident part
 
 template <class Launch> TileForm form_of(const Launch& L) { return L.form; }
@@ -220,7 +220,8 @@ int launch_tiles(const odc_arena* a, const Launch& L, uint32_t grid, Issue issue
     g_dry_tiles += L.tt.n_tiles;
     g_dry_workgroups += grid;
     g_dry_short += form_of(L) == kShortTiles;
-    g_dry_few += form_of(L) == kFewShortTiles;
+    g_dry_few += form_of(L) == kFewShortTiles || form_of(L) == kTinyTiles;
+    g_dry_tiny += form_of(L) == kTinyTiles;
     g_dry_stream += form_of(L) == kStreamTiles;
     g_dry_resident += L.tt.resident_below != 0;
     return ODC_OK;
@@ -450,8 +451,21 @@ bool publish_in_short_tiles(const LaunchSize& size, int acc_bytes) { return acc_
 //   10 of 256 .. 262 144: 6.1 -> 5.9, 6.5 -> 6.2, 7.2 -> 6.9;
 //   112 of 160 000 (17 900 tiles): 41.2 -> 39.7, 41.1 -> 40.2; 112 of 640 000 (70 000 tiles): 156 -> 159,
 //   159 -> 162; 60 of 900 000 (53 000 tiles): 115 -> 115, 116.5 -> 117.6.
-TileForm tile_form(TileForm cut, uint32_t n_tiles, int64_t few) {
-  return cut == kShortTiles && n_tiles <= (uint64_t)few ? kFewShortTiles : cut;
+//
+// What is left of their time goes with the number of wavefronts: some 0.55 us per 1000 workgroups of two. Where
+// tiles are at most half full on average the second wavefront has little to do, and from 2048 tiles on (8 per CU)
+// launches by the full tables have workgroups of one, which moves four vectors per lane in a full tile. us, 100
+// ragged items (a factor of 100 between their sizes), two wavefronts -> one, gather / accumulate of bf16 into fp32 /
+// converting gather / store:
+//   W = 64, 6400 tiles: 0.26 M elements in all 6.27 -> 4.87, 6.77 -> 5.21, 6.59 -> 4.94, 6.71 -> 5.21; 4.2 M 6.78 -> 5.49, 7.80 ->
+//     6.68, 7.28 -> 5.76, 7.29 -> 5.81; W = 32, 3200 tiles: 1 M 4.43 -> 3.99, 4.78 -> 4.25, 4.71 -> 4.24, 4.73 -> 4.20;
+//   W = 16, 2096 tiles half full: 3.97 -> 3.94, 4.21 -> 4.22, 4.12 -> 3.95, 3.96 -> 3.88; fewer tiles, gather: 784 2.98 -> 3.32,
+//     1568 3.58 -> 3.74; 2544 tiles, 94 % full, accumulate 4.61 -> 4.84; publishes of one rank never have so many.
+constexpr uint32_t kTinyFrom = 2048;
+TileForm tile_form(TileForm cut, const TileTable& tt, uint64_t units, uint64_t whole_tile_units, int64_t few) {
+  if (cut != kShortTiles || tt.n_tiles > (uint64_t)few) return cut;
+  const bool half_empty = 2 * units * tt.world <= (uint64_t)tt.n_tiles * (whole_tile_units / kShortTileParts);
+  return tt.n_items > kFewItems && tt.n_tiles >= kTinyFrom && half_empty ? kTinyTiles : kFewShortTiles;
 }
 
 // Whether a launch that is otherwise cut as `cut` is a long stream: more than 8 MiB written, past the caches,
@@ -506,7 +520,7 @@ int odc_abi_version(void) { return ODC_HIP_ABI_VERSION; }
 int odc_set_option(const char* name, int64_t value) {
   if (name && !strcmp(name, "dry_run_reset")) {
     g_dry_launches = 0; g_dry_tiles = 0; g_dry_workgroups = 0;
-    g_dry_short = 0; g_dry_few = 0; g_dry_stream = 0; g_dry_resident = 0;
+    g_dry_short = 0; g_dry_few = 0; g_dry_tiny = 0; g_dry_stream = 0; g_dry_resident = 0;
     return ODC_OK;
   }
   std::lock_guard<std::mutex> lk(g_opt_mu);
@@ -529,6 +543,7 @@ int odc_get_option(const char* name, int64_t* value) {
     if (!strcmp(name, "dry_run_workgroups")) { *value = g_dry_workgroups.load(); return ODC_OK; }
     if (!strcmp(name, "dry_run_short_launches")) { *value = g_dry_short.load(); return ODC_OK; }
     if (!strcmp(name, "dry_run_few_launches")) { *value = g_dry_few.load(); return ODC_OK; }
+    if (!strcmp(name, "dry_run_tiny_launches")) { *value = g_dry_tiny.load(); return ODC_OK; }
     if (!strcmp(name, "dry_run_stream_launches")) { *value = g_dry_stream.load(); return ODC_OK; }
     if (!strcmp(name, "dry_run_resident_launches")) { *value = g_dry_resident.load(); return ODC_OK; }
   }
@@ -829,7 +844,7 @@ int odc_gather(odc_arena* a, const odc_gather_item* items, uint32_t n_items, uin
         });
     if (n < 0) return n;
     if (n == 0) continue;
-    L.form = tile_form(cut, L.tt.n_tiles, opt.few_tiles);
+    L.form = tile_form(cut, L.tt, size.units, kTileBytes, opt.few_tiles);
     L.output = output_form(opt, L.policy.written, out_bytes);
     L.tt.resident_below = resident_below(a, opt, opt.resident_shard_bytes);
     const auto ragged = [&] {
@@ -888,7 +903,7 @@ int odc_gather_cast(odc_arena* a, const odc_gather_cast_item* items, uint32_t n_
         });
     if (n < 0) return n;
     if (n == 0) continue;
-    L.form = tile_form(cut, L.tt.n_tiles, opt.few_tiles);
+    L.form = tile_form(cut, L.tt, size.units, kTileElems, opt.few_tiles);
     const uint32_t grid = grid_for(a, opt.gather_blocks_per_cu, L.tt.n_tiles, copy_threads(L.form));
     const uint32_t lds = lds_claim_for(a, opt.cast_resident_cap, grid, L.tt.n_tiles);
     if (int rc = launch_tiles(a, L, grid, [&] {
@@ -941,7 +956,7 @@ int odc_convert(odc_arena* a, const odc_convert_item* items, uint32_t n_items, i
         });
     if (n < 0) return n;
     if (n == 0) continue;
-    L.form = tile_form(cut, L.tt.n_tiles, opt.few_tiles);
+    L.form = tile_form(cut, L.tt, size.units, kTileElems, opt.few_tiles);
     const uint32_t grid = grid_for(a, opt.gather_blocks_per_cu, L.tt.n_tiles, copy_threads(L.form));
     const uint32_t lds = lds_claim_for(a, opt.cast_resident_cap, grid, L.tt.n_tiles);
     if (int rc = launch_tiles(a, L, grid, [&] {
@@ -1080,7 +1095,7 @@ int scatter_launch(odc_arena* a, const odc_accum_item* items, uint32_t n_items, 
         order);
     if (n < 0) return n;
     if (n == 0) continue;
-    L.form = tile_form(cut, L.tt.n_tiles, opt.few_tiles);
+    L.form = tile_form(cut, L.tt, size.units, kTileElems, opt.few_tiles);
     // Tile order. Item-major (a rank's segment, then the next rank's, item by item) walks the
     // gradient contiguously and hops between rank regions at every segment; rank-outermost walks
     // one rank region from accumulation to accumulation (they are neighbours when registered
@@ -1197,7 +1212,7 @@ int odc_publish(odc_arena* a, uint32_t rank, const odc_publish_item* items, uint
         });
     if (n < 0) return n;
     if (n == 0) continue;
-    L.form = tile_form(cut, L.tt.n_tiles, opt.few_tiles);
+    L.form = tile_form(cut, L.tt, size.units, kTileElems, opt.few_tiles);
     // one workgroup per tile: the division sequence wants the occupancy, and the launch is short
     const uint32_t grid = grid_for(a, opt.publish_blocks_per_cu, L.tt.n_tiles, publish_threads(L.form));
     const uint32_t lds = lds_claim_for(a, opt.publish_resident_cap, grid, L.tt.n_tiles);

@@ -333,20 +333,25 @@ __device__ __attribute__((noinline)) void gather_edges(uint8_t* d, const uint8_t
   const uint32_t left = is_whole<T * U>(w) ? 0u : w.nv;
   const uint8_t* sb = s + g.head + w.v0 * 16;
   u32x4* db = reinterpret_cast<u32x4*>(d + g.head) + w.v0;
-  const bool do_head = w.head && tid < g.head;
   const bool do_tail = w.tail && tid < g.tail;
   const uint64_t tail_at = g.head + g.nvec * 16 + tid;
+  const uint32_t head = w.head ? g.head : 0u;
+  constexpr int kHead = (ODC_BODY_ALIGN - 2) / T + 1;  // head bytes per lane
   u32x4 v[U];
-  uint8_t head_byte = 0, tail_byte = 0;
+  uint8_t head_byte[kHead] = {}, tail_byte = 0;
 #pragma unroll
   for (int u = 0; u < U; ++u)
     if (u * T + tid < left) v[u] = load_any<kSrcCached, u32x4>(sb + (size_t)(u * T + tid) * 16);
-  if (do_head) head_byte = s[tid];
+#pragma unroll
+  for (int h = 0; h < kHead; ++h)
+    if (h * T + tid < head) head_byte[h] = s[h * T + tid];
   if (do_tail) tail_byte = s[tail_at];
 #pragma unroll
   for (int u = 0; u < U; ++u)
     if (u * T + tid < left) store_vec<kDstCached>(db + u * T + tid, v[u]);
-  if (do_head) d[tid] = head_byte;
+#pragma unroll
+  for (int h = 0; h < kHead; ++h)
+    if (h * T + tid < head) d[h * T + tid] = head_byte[h];
   if (do_tail) d[tail_at] = tail_byte;
 }
 
@@ -356,7 +361,6 @@ template <class Launch, bool kSrcCached, OutputForm kDst, bool kFew, int T, int 
 __global__ __launch_bounds__(T) ODC_RESIDENT_WAVES(kWaves) void gather_kernel(const Launch launch) {
   constexpr uint32_t kVecs = T * U;
   static_assert(kVecs == kTileVecs || kVecs == kShortTileVecs, "a whole tile or a short one");
-  static_assert(T >= ODC_BODY_ALIGN - 1, "one lane per head byte");
   const uint32_t tid = threadIdx.x;
   TileWalk<Launch, kFew> walk(launch);
   each_tile(walk, launch, [&](uint32_t t) {
@@ -378,15 +382,20 @@ __global__ __launch_bounds__(T) ODC_RESIDENT_WAVES(kWaves) void gather_kernel(co
         for (int u = 0; u < U; ++u) v[u] = load_any<cached, u32x4>(sb[u] + tid * 16);
         // a whole tile that also owns its segment's head or tail (the first and last tile of a
         // ragged segment) reads those bytes with the same round trip as its vectors
-        const bool do_head = w.head && tid < g.head;
         const bool do_tail = w.tail && tid < g.tail;
         const uint64_t tail_at = g.head + g.nvec * 16 + tid;
-        uint8_t head_byte = 0, tail_byte = 0;
-        if (do_head) head_byte = s[tid];
+        const uint32_t head = w.head ? g.head : 0u;
+        constexpr int kHead = (ODC_BODY_ALIGN - 2) / T + 1;  // head bytes per lane
+        uint8_t head_byte[kHead] = {}, tail_byte = 0;
+#pragma unroll
+        for (int h = 0; h < kHead; ++h)
+          if (h * T + tid < head) head_byte[h] = s[h * T + tid];
         if (do_tail) tail_byte = s[tail_at];
 #pragma unroll
         for (int u = 0; u < U; ++u) store_output<kDst, kVecs>(db, u * T + tid, v[u]);
-        if (do_head) d[tid] = head_byte;
+#pragma unroll
+        for (int h = 0; h < kHead; ++h)
+          if (h * T + tid < head) d[h * T + tid] = head_byte[h];
         if (do_tail) d[tail_at] = tail_byte;
       });
     } else if (has_edges<kVecs>(w)) {
@@ -955,6 +964,10 @@ kernel_fn<L> pick_accum_form(bool store, AccumPolicy policy, TileForm form) {
 
 template <class L, class G, class A, bool kShortOnly>
 kernel_fn<L> pick_accum_tiles(bool store, AccumPolicy policy, TileForm form) {
+  if constexpr (kSearches<L>)
+    if (form == kTinyTiles)
+      return store ? pick_store<L, G, A, true, kTinyThreads, kTinyUnroll>(policy)
+                   : pick_rmw<L, G, A, true, kTinyThreads, kTinyUnroll>(policy);
   if (form == kFewShortTiles)
     return store ? pick_store<L, G, A, kSearches<L>, kShortThreads, kShortUnroll>(policy)
                  : pick_rmw<L, G, A, kSearches<L>, kShortThreads, kShortUnroll>(policy);
@@ -985,6 +998,8 @@ kernel_fn<L> pick_gather_form(TileForm form) {
   if constexpr (kStreams<L> && kDst == kStream && !kSrcCached)
     if (form == kStreamTiles) return gather_kernel<L, false, kStream, false, kShortThreads, kShortUnroll, kStreamWaves>;
   if constexpr (!kStreamsOnly<L>) {
+    if constexpr (kSearches<L>)
+      if (form == kTinyTiles) return gather_kernel<L, kSrcCached, kDst, true, kTinyThreads, kTinyUnroll>;
     if (form == kFewShortTiles) return gather_kernel<L, kSrcCached, kDst, kSearches<L>, kShortThreads, kShortUnroll>;
     if (form == kShortTiles) return gather_kernel<L, kSrcCached, kDst, false, kShortThreads, kShortUnroll>;
     if constexpr (kGathersWholeTiles<L>)
@@ -1007,6 +1022,8 @@ kernel_fn<L> pick_gather(bool shards_cached, OutputForm output, TileForm form) {
 
 template <class L, class S, class D, bool kSrcCached, OutputForm kDst>
 kernel_fn<L> pick_cast_gather_form(TileForm form) {
+  if constexpr (kSearches<L>)
+    if (form == kTinyTiles) return cast_gather_kernel<L, S, D, kSrcCached, kDst, true, kTinyThreads, kTinyUnroll>;
   if (form == kFewShortTiles) return cast_gather_kernel<L, S, D, kSrcCached, kDst, kSearches<L>, kShortThreads, kShortUnroll>;
   if (form == kShortTiles) return cast_gather_kernel<L, S, D, kSrcCached, kDst, false, kShortThreads, kShortUnroll>;
   if constexpr (kGathersWholeTiles<L>)

@@ -44,8 +44,9 @@ struct AccumPolicy {
 };
 
 // How a launch is cut, and how its workgroups find their items (wants_short_tiles and tile_form in
-// odc_host.cpp). kStreamTiles: short tiles of a long stream (stream_form there).
-enum TileForm : uint32_t { kWholeTiles, kShortTiles, kFewShortTiles, kStreamTiles };
+// odc_host.cpp). kTinyTiles: kFewShortTiles by workgroups of one wavefront; kStreamTiles: short tiles of a long
+// stream (stream_form there).
+enum TileForm : uint32_t { kWholeTiles, kShortTiles, kFewShortTiles, kTinyTiles, kStreamTiles };
 
 inline uint32_t tile_parts(TileForm form) { return form == kWholeTiles ? 1 : odc_tiles::kShortTileParts; }
 
@@ -95,10 +96,17 @@ constexpr int kNarrowRmwUnroll = (int)kTileVecs / kNarrowRmwThreads;
 constexpr int kShortThreads = 128;
 constexpr int kShortUnroll = (int)kShortTileVecs / kShortThreads;
 
+// The same tiles where most of them are not full: one wavefront each (tile_form in odc_host.cpp).
+constexpr int kTinyThreads = 64;
+constexpr int kTinyUnroll = (int)kShortTileVecs / kTinyThreads;
+
 // The workgroup sizes of the launches, as the pick_* functions of odc_kernels.hip take them.
-inline uint32_t copy_threads(TileForm form) { return form != kWholeTiles ? kShortThreads : kCopyThreads; }
+inline uint32_t copy_threads(TileForm form) {
+  return form == kWholeTiles ? kCopyThreads : form == kTinyTiles ? kTinyThreads : kShortThreads;
+}
 inline uint32_t publish_threads(TileForm form) { return form != kWholeTiles ? kShortThreads : kThreads; }
 inline uint32_t accum_threads(int grad_dtype, int acc_dtype, bool store, AccumPolicy policy, TileForm form) {
+  if (form == kTinyTiles) return kTinyThreads;
   if (form != kWholeTiles) return kShortThreads;
   if (grad_dtype != ODC_DTYPE_F32 && acc_dtype != ODC_DTYPE_F32)
     return store || policy.read ? kThreads : kNarrowRmwThreads;
