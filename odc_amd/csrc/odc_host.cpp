@@ -352,8 +352,11 @@ OutputForm store_output_form(const Options& opt, bool cached, uint64_t bytes) {
 // 37.3, three microbatches of 9 M 92.7 -> 91.1, FSDP1 minibatches of 9 M 97.1 -> 95.3, 13 M 125.0 -> 122.7,
 // 18 M 162.6 -> 156; but gather + accumulate of 24 M 61.2 -> 63.0, 32 M 80.4 -> 86.5. FSDP2 minibatches
 // over converted copies of 12 to 57 MB: 185.8 -> 183.7, 245.3 -> 242.2.
-OutputForm cast_output_form(bool cached, uint64_t bytes, int64_t line) {
-  return cached ? kKeep : bytes <= (uint64_t)line ? kWriteThrough : kStream;
+// Where all symmetric memory fits they are written through as plain gathers are, us, plain -> written through, one
+// item on one set of buffers, nine items on three sets: 1 M elements 2.27 -> 2.13, 2.94 -> 3.00; 2.1 M 2.92 -> 2.66, 3.87 ->
+// 3.61; 4.2 M 3.95 -> 3.43, 5.70 -> 5.41; 8.4 M 8.09 -> 5.83, 8.74 -> 8.69; 16.8 M and more level.
+OutputForm cast_output_form(const Options& opt, bool cached, uint64_t bytes, int64_t line) {
+  return cached ? output_form(opt, true, bytes) : bytes <= (uint64_t)line ? kWriteThrough : kStream;
 }
 
 // How a clear without a resident part writes its zeros: through the L2s while the last-level cache holds them
@@ -893,7 +896,7 @@ int odc_gather_cast(odc_arena* a, const odc_gather_cast_item* items, uint32_t n_
     const auto units = [&](uint32_t i) { return items[i].shard_elems; };
     const LaunchSize size = launch_size<kTileElems>(n_items, next, units);
     L.policy = cache_policy(a, opt, 0, kSymmetric, 0, kSymmetric);
-    L.output = cast_output_form(L.policy.read, size.units * db * a->world, opt.cast_output_bytes);
+    L.output = cast_output_form(opt, L.policy.read, size.units * db * a->world, opt.cast_output_bytes);
     const TileForm cut = wants_short_tiles(size, opt.short_tiles_below) ? kShortTiles : kWholeTiles;
     const int n = fill_launch<kTileElems>(
         L.tt, a->world, n_items, &next, cut, units,
@@ -946,7 +949,7 @@ int odc_convert(odc_arena* a, const odc_convert_item* items, uint32_t n_items, i
     const LaunchSize size = launch_size<kTileElems>(n_items, next, units);
     L.policy = cache_policy(a, opt, 0, kSymmetric, 0, kSymmetric);
     // (the copies are symmetric memory that every gather of the minibatch reads)
-    L.output = cast_output_form(L.policy.read, size.units * db * a->world, opt.cached_output_bytes);
+    L.output = cast_output_form(opt, L.policy.read, size.units * db * a->world, opt.cached_output_bytes);
     const TileForm cut = wants_short_tiles(size, opt.short_tiles_below) ? kShortTiles : kWholeTiles;
     const int n = fill_launch<kTileElems>(
         L.tt, a->world, n_items, &next, cut, units,

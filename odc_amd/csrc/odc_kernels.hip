@@ -1031,10 +1031,12 @@ kernel_fn<L> pick_cast_gather_form(TileForm form) {
   return nullptr;
 }
 
-// Shards are cached only together with the output, which is then kept with plain stores.
+// Shards are cached only together with the output.
 template <class L, class S, class D>
 kernel_fn<L> pick_cast_gather_output(CachePolicy policy, OutputForm output, TileForm form) {
-  if (policy.read) return pick_cast_gather_form<L, S, D, true, kKeep>(form);
+  if (policy.read)
+    return output == kKeep ? pick_cast_gather_form<L, S, D, true, kKeep>(form)
+                           : pick_cast_gather_form<L, S, D, true, kWriteThrough>(form);
   return output == kStream ? pick_cast_gather_form<L, S, D, false, kStream>(form)
                            : pick_cast_gather_form<L, S, D, false, kWriteThrough>(form);
 }

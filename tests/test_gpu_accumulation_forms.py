@@ -1,10 +1,10 @@
-"""Accumulations that stay in the caches, written with plain stores and through the L2s: accumulates and stores
-at the edges of their tiles give the oracle's bits, and nothing beside the accumulations is written."""
+"""Accumulations and converted outputs that stay in the caches, written with plain stores and through the L2s:
+launches at the edges of their tiles give the oracle's bits, and nothing beside what they write is written."""
 
 import pytest
 import torch
 
-from helpers import assert_bit_equal
+from helpers import assert_bit_equal, put_shards
 from odc_amd import _native
 from oracle import odc_oracle as oracle
 
@@ -54,6 +54,34 @@ def test_bits_and_bounds(make_world, sizes, grad_dtype, acc_dtype, plain):
             reduction.sync(group)
             for r, peer in enumerate(peers):
                 assert_bit_equal(peer, want[r], f"rank {r} store {store}")
+    finally:
+        for name, value in saved.items():
+            _native.set_option(name, value)
+
+
+@pytest.mark.parametrize("plain", [0, 1 << 40], ids=["written through", "plain"])
+@pytest.mark.parametrize("src,dst", [(F32, BF16), (BF16, F32), (F16, BF16)])
+@pytest.mark.parametrize("sizes", [[8 * 4096], [1023, 1024, 1025, 4096 + 3], [640] * 17, [40 * 4096 + 5] * 2],
+                         ids=lambda sizes: f"{len(sizes)}x{max(sizes)}")
+def test_converted_outputs(make_world, sizes, src, dst, plain):
+    from odc_amd import GatherService, SymmBufferRegistry
+
+    options = {"plain_output_bytes": plain, "cached_arena_bytes": 1 << 40}
+    saved = {name: _native.get_option(name) for name in options}
+    try:
+        for name, value in options.items():
+            _native.set_option(name, value)
+        W, pad = 3, 67
+        group = make_world(W, sum(sizes) * 4 + (2 << 20))
+        gen = torch.Generator().manual_seed(4)
+        shards = [[torch.randn(n, generator=gen).to(src) for _ in range(W)] for n in sizes]
+        sources = [put_shards(SymmBufferRegistry.get_instance(), ("p", i), s) for i, s in enumerate(shards)]
+        around = [torch.full((W * n + 2 * pad,), 7.0, dtype=dst, device="cuda") for n in sizes]
+        GatherService().gather_into_tensors([t[pad : pad + W * n] for t, n in zip(around, sizes)], sources, group)
+        for t, s, n in zip(around, shards, sizes):
+            want = torch.full((W * n + 2 * pad,), 7.0, dtype=dst)
+            want[pad : pad + W * n] = oracle.gather_cast(s, dst)
+            assert_bit_equal(t, want, f"size {n}")
     finally:
         for name, value in saved.items():
             _native.set_option(name, value)
