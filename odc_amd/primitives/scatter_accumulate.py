@@ -126,14 +126,17 @@ _MIXED = "mixed"
 class _Syncing:
     """``ReductionService.syncing`` (a class: a generator costs the host 1 us more)."""
 
-    __slots__ = ("_service", "_events")
+    __slots__ = ("_service", "_pg", "_events")
 
-    def __init__(self, service):
-        self._service = service
+    def __init__(self, service, pg):
+        self._service, self._pg = service, pg
 
     def __enter__(self):
-        if _is_capturing():  # (there is nothing the host could wait for: sync refuses)
-            self._service.sync()
+        service = self._service
+        # Under capture there is nothing that the host could wait for: sync refuses. A sync of the caller's
+        # own stays in front of the block.
+        if _is_capturing() or type(service).sync is not ReductionService.sync or "sync" in service.__dict__:
+            service.sync(self._pg)
         self._events = launches_in_flight()
 
     def __exit__(self, exc_type, exc, tb):
@@ -610,7 +613,7 @@ class ReductionService:
         the adds on the device and in front of the wait on the host: at its end every add dispatched
         before it has landed. With the wait in front the GPU had nothing to do from the last add until
         the host had woken up and launched the publish."""
-        return _Syncing(self)
+        return _Syncing(self, pg)
 
     def stop(self):
         if torch.cuda.is_available():

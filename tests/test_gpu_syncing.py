@@ -44,6 +44,23 @@ def test_publish_behind_adds_of_a_busy_stream(make_world, policy, monkeypatch):
     assert_bit_equal(out, want.bfloat16())
 
 
+@pytest.mark.gpu
+def test_a_sync_of_the_callers_own_is_called_first(make_world):
+    from odc_amd import ReductionService
+
+    calls = []
+
+    class Service(ReductionService):
+        def sync(self, pg=None):
+            calls.append(("sync", pg))
+            super().sync(pg)
+
+    group = make_world(2, 1 << 20)
+    with Service().syncing(group):
+        calls.append("block")
+    assert calls == [("sync", group), "block"]
+
+
 def test_users_hooks_are_seen():
     from odc_amd.fsdp.fsdp2 import _has_gradient_hooks
 
