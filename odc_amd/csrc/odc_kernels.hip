@@ -13,7 +13,7 @@
 //
 // Launch model shared by the kernels: the work of one launch is cut into tiles of 1024 vectors
 // (16 KiB), done by workgroups of 256 threads or 512 (odc_launch.h says which), or into short tiles of 256
-// vectors, done by 128 threads: launches of short segments (wants_short_tiles in odc_host.cpp) and
+// vectors, done by 128 threads (64 where most are part-empty, kTinyTiles): launches of short segments (wants_short_tiles in odc_host.cpp) and
 // every accumulate and store of 16-bit gradients into fp32 (accum_streams_short in odc_launch.h), every
 // publish of fp32 accumulations (publish_in_short_tiles in odc_host.cpp), and long streams (stream_form there).
 // Workgroups walk the tiles with a grid-stride loop, by default one workgroup per tile, so that,
@@ -25,8 +25,8 @@
 // Each wavefront issues its 2 or 4 independent 128-bit loads per stream before the first store.
 // Streams larger than the 256 MB last-level cache are nontemporal on both sides (worth ~15 % over
 // plain accesses there); what fits the cache and was just produced, or is about to be consumed, is
-// left in it (cache_policy in odc_host.cpp), and so is a part of what does not fit (resident_below
-// there). Deeper unrolling or prefetching the next tile measured slower: the memory system prefers a
+// left in it (cache_policy in odc_host.cpp), written through the L2s from 3 MiB on (output_form there), and so
+// is a part of what does not fit (resident_below there). Deeper unrolling or prefetching the next tile measured slower: the memory system prefers a
 // small window to more requests in flight.
 // Workgroup i runs on XCD i % 8; binding XCDs to address classes (256 B .. 64 KiB granules)
 // changed nothing measurable and giving every XCD one contiguous eighth of the tiles costs the

@@ -7,7 +7,7 @@
 // Vocabulary. A launch carries up to kMaxItems ITEMS (one shard of one tensor). An item has one
 // SEGMENT per rank: `n` units (bytes or elements) at the same symmetric offset of every rank
 // region. A segment is cut into TILES of kTileVecs vectors (or of kShortTileVecs, a launch of short
-// ones); a workgroup of 128, 256 or 512 threads does one tile at a time.
+// ones); a workgroup of 64, 128, 256 or 512 threads does one tile at a time.
 #ifndef ODC_TILES_H_
 #define ODC_TILES_H_
 
