@@ -337,7 +337,8 @@ OutputForm output_form(const Options& opt, bool cached, uint64_t bytes) {
 // A store's accumulations, which it does not read: written through from 3 to 64 MiB, nontemporal otherwise. The same
 // launches, and passes of gather, store, gather, accumulate, us, nontemporal -> written through:
 //   store of bf16 into fp32: 0.52 M elements 2.19 -> 2.24, 2.66 -> 2.60; 1 M 2.51 -> 2.41, 3.05 -> 3.00; 4.2 M 4.30 -> 4.48, 5.19
-//     -> 4.90; 16.8 M (64 MiB) 13.5 -> 12.1, 14.5 -> 14.7 (one item over three sets 13.4 -> 15.9, level in passes); into bf16 4.2 M 3.31 -> 3.02, 16.8 M 9.55 -> 7.87;
+//     -> 4.90; 16.8 M (64 MiB) 13.5 -> 12.1, 14.5 -> 14.7 (one item over three sets 13.4 -> 15.9, level in
+//     passes); into bf16 4.2 M 3.31 -> 3.02, 16.8 M 9.55 -> 7.87;
 //   passes: 1 M 9.61 -> 8.70, 11.74 -> 10.90; 4.2 M 16.06 -> 14.33, 20.02 -> 19.10; 8.4 M 28.7 -> 26.9, 34.1 -> 35.2; 33 M
 //     105 .. 107 -> 111 .. 116.
 OutputForm store_output_form(const Options& opt, bool cached, uint64_t bytes) {
