@@ -58,6 +58,7 @@ from odc_amd.primitives.utils import (
     wait_for_launches,
     get_world,
     group_size,
+    has_launches,
     native_dtype,
 )
 
@@ -133,9 +134,10 @@ class _Syncing:
 
     def __enter__(self):
         service = self._service
-        # Under capture there is nothing that the host could wait for: sync refuses. A sync of the caller's
+        # Under capture there is no launch that the host could wait for: sync refuses. A sync of the caller's
         # own stays in front of the block.
-        if _is_capturing() or type(service).sync is not ReductionService.sync or "sync" in service.__dict__:
+        own = type(service).sync is not ReductionService.sync or "sync" in service.__dict__
+        if own or (has_launches() and _is_capturing()):
             service.sync(self._pg)
         self._events = launches_in_flight()
 

@@ -711,15 +711,23 @@ def wait_for_launches() -> None:
             torch.cuda.synchronize(get_world().arena.device)
 
 
+def has_launches() -> bool:
+    """Whether anything was launched through ``comm_stream_section`` since the last wait."""
+    return bool(_launch_streams)
+
+
 def launches_in_flight():
     """An event behind every launch issued so far through ``comm_stream_section``, for
     ``wait_for_events``: ``wait_for_launches`` in two halves, so that the host can issue what comes next
     before it waits. The current stream waits for the launches on the others, so what comes next finds
-    them done, as it would after ``wait_for_launches``."""
-    device = get_world().device
+    them done, as it would after ``wait_for_launches``. With no launches there is nothing to ask of arena or
+    device."""
     with _launch_lock:
         pending = list(_launch_streams.items())
         _launch_streams.clear()
+    if not pending:
+        return []
+    device = get_world().device
     current, events = torch.cuda.current_stream(device), []
     for handle, s in pending:
         event = torch.cuda.Event()
