@@ -26,6 +26,7 @@ import torch.nn.functional as F
 
 import odc_amd
 from odc_amd.fsdp.shard_copies import compute_dtype_shards_of, shards_may_have_changed
+from odc_amd.primitives.scatter_accumulate import syncing
 from odc_amd.primitives.utils import group_size
 
 logger = logging.getLogger(__name__)
@@ -247,10 +248,10 @@ def unpatch_fsdp1():
 def pre_optimizer_step(fsdp_module):
     """fsdp1.py:317-335: wait for every add, post-divide, publish the accumulations as
     ``flat_param.grad`` in the parameter dtype. The publish is launched behind the adds before the host
-    waits for them (``ReductionService.syncing``)."""
+    waits for them (``syncing``)."""
     shards_may_have_changed()  # the optimizer is about to change them
     service = get_reduction_service()
-    with torch.cuda.nvtx.range("scatter_accumulate_sync"), service.syncing(getattr(fsdp_module, "process_group", None)):
+    with torch.cuda.nvtx.range("scatter_accumulate_sync"), syncing(service, getattr(fsdp_module, "process_group", None)):
         if hasattr(fsdp_module, "_inter_node_pg"):
             raise NotImplementedError("hybrid sharding needs a second node; not part of this build")
         _publish_gradients(fsdp_module, service)

@@ -43,7 +43,7 @@ import torch
 from odc_amd import _native
 from odc_amd.fsdp.shard_copies import compute_dtype_shards_of, shards_may_have_changed
 from odc_amd.primitives.gather import GatherService
-from odc_amd.primitives.scatter_accumulate import ReductionService
+from odc_amd.primitives.scatter_accumulate import ReductionService, syncing
 from odc_amd.primitives.utils import (
     SymmBufferRegistry,
     finalize_distributed,
@@ -665,7 +665,7 @@ def pre_minibatch_start(fsdp_module):
 
 def pre_optimizer_step(fsdp_module):
     """fsdp2.py:1023-1046: sync once and publish every group's gradients. The publish is launched behind
-    the adds before the host waits for them (``ReductionService.syncing``)."""
+    the adds before the host waits for them (``syncing``)."""
     shards_may_have_changed()  # the optimizer is about to change the shards
     scatter = get_reduction_service()
     if _is_torch_fsdp_module(fsdp_module):
@@ -677,12 +677,12 @@ def pre_optimizer_step(fsdp_module):
                     scatter.sync(pg)
                 update_all_gradients(groups)
             else:
-                with torch.cuda.nvtx.range("scatter_accumulate_sync"), scatter.syncing(pg):
+                with torch.cuda.nvtx.range("scatter_accumulate_sync"), syncing(scatter, pg):
                     update_all_gradients(groups)
         return
     groups = _param_groups(fsdp_module)
     if groups:
-        with torch.cuda.nvtx.range("scatter_accumulate_sync"), scatter.syncing(groups[0].pg):
+        with torch.cuda.nvtx.range("scatter_accumulate_sync"), syncing(scatter, groups[0].pg):
             for group in groups:
                 with torch.cuda.nvtx.range(f"update_gradients:{group.name}"):
                     group.update_gradients()

@@ -124,24 +124,33 @@ _MAX_SLICE_PLANS = 16  # per key: one, unless the caller changes which parameter
 _MIXED = "mixed"
 
 
-class _Syncing:
-    """``ReductionService.syncing`` (a class: a generator costs the host 1 us more)."""
+class syncing:
+    """``with syncing(service, pg): ...`` — ``service.sync(pg)`` with the block's host work and launches behind
+    the adds on the device and in front of the wait on the host: at its end every add dispatched before it
+    has landed. With the wait in front the GPU had nothing to do from the last add until the host had woken up
+    and launched the publish. (A class: a generator costs the host 1 us more.)
+
+    A ``sync`` that is not the one of this package stays in front of the block: a subclass's, one that was put on
+    the service or on ``ReductionService``, or that of any other object with a ``sync``."""
 
     __slots__ = ("_service", "_pg", "_events")
 
-    def __init__(self, service, pg):
+    def __init__(self, service, pg=None):
         self._service, self._pg = service, pg
 
     def __enter__(self):
         service = self._service
-        # Under capture there is no launch that the host could wait for: sync refuses. A sync of the caller's
-        # own stays in front of the block.
-        own = type(service).sync is not ReductionService.sync or "sync" in service.__dict__
+        own = getattr(type(service), "sync", None) is not _sync or "sync" in getattr(service, "__dict__", ())
+        # (under capture there is no launch that the host could wait for: sync refuses)
         if own or (has_launches() and _is_capturing()):
             service.sync(self._pg)
-        self._events = launches_in_flight()
+            self._events = None
+        else:
+            self._events = launches_in_flight()
 
     def __exit__(self, exc_type, exc, tb):
+        if self._events is None:
+            return
         wait_for_events(self._events)
         with self._service._lock:
             self._service.dispatched_tasks = 0
@@ -611,12 +620,12 @@ class ReductionService:
             self.dispatched_tasks = 0
 
     def syncing(self, pg=None):
-        """``with service.syncing(pg): ...`` — ``sync`` with the block's host work and launches behind
-        the adds on the device and in front of the wait on the host: at its end every add dispatched
-        before it has landed. With the wait in front the GPU had nothing to do from the last add until
-        the host had woken up and launched the publish."""
-        return _Syncing(self, pg)
+        """``sync`` behind the launches of a ``with`` block: see ``syncing``."""
+        return syncing(self, pg)
 
     def stop(self):
         if torch.cuda.is_available():
             wait_for_launches()
+
+
+_sync = ReductionService.sync  # as it is here, whatever is put in its place later: see syncing
