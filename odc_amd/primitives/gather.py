@@ -20,10 +20,12 @@ from odc_amd import _native
 from odc_amd.primitives.utils import (
     BufferSplitter,
     SymmBufferRegistry,
+    _launch_streams,
     comm_stream_section,
     get_world,
     group_size,
     native_dtype,
+    note_launch,
     plain_launch_stream,
     stream_from_handle,
 )
@@ -69,6 +71,8 @@ class GatherService:
             if self._conversion is not None:
                 self._order_after_conversion(stream)
             status = entry(world.arena.raw_handle, W, world.rank, stream, *call)
+            if stream not in _launch_streams:
+                note_launch(stream)
         else:
             with comm_stream_section("odc.gather") as comm:
                 if self._conversion is not None:

@@ -49,17 +49,18 @@ import torch
 from odc_amd import _native
 from odc_amd.primitives.utils import (
     BufferSplitter,
+    LaunchesInFlight,
     StreamOrder,
     SymmBufferRegistry,
+    _launch_streams,
     comm_stream_section,
-    launches_in_flight,
-    plain_launch_stream,
-    wait_for_events,
-    wait_for_launches,
     get_world,
     group_size,
     has_launches,
     native_dtype,
+    note_launch,
+    plain_launch_stream,
+    wait_for_launches,
 )
 
 logger = logging.getLogger(__name__)
@@ -133,27 +134,31 @@ class syncing:
     A ``sync`` that is not the one of this package stays in front of the block: a subclass's, one that was put on
     the service or on ``ReductionService``, or that of any other object with a ``sync``."""
 
-    __slots__ = ("_service", "_pg", "_events")
+    __slots__ = ("_service", "_pg", "_dispatched", "_launches")
 
     def __init__(self, service, pg=None):
         self._service, self._pg = service, pg
 
     def __enter__(self):
-        service = self._service
-        own = getattr(type(service), "sync", None) is not _sync or "sync" in getattr(service, "__dict__", ())
-        # (under capture there is no launch that the host could wait for: sync refuses)
-        if own or (has_launches() and _is_capturing()):
+        service, self._dispatched, self._launches = self._service, None, None
+        if getattr(type(service), "sync", None) is not _sync or "sync" in getattr(service, "__dict__", ()):
             service.sync(self._pg)
-            self._events = None
+            return
+        self._dispatched = service._tasks
+        if not has_launches():
+            return
+        if _is_capturing():
+            # an event of the captured stream is nothing that the host could wait for: as sync does, which is
+            # refused unless everything was launched on other streams and the capture allows waits for those
+            service.sync(self._pg)
         else:
-            self._events = launches_in_flight()
+            self._launches = LaunchesInFlight(torch.cuda.current_stream(get_world().device))
 
     def __exit__(self, exc_type, exc, tb):
-        if self._events is None:
-            return
-        wait_for_events(self._events)
-        with self._service._lock:
-            self._service.dispatched_tasks = 0
+        if self._launches is not None:
+            self._launches.wait()
+        if self._dispatched is not None:
+            self._service._landed(self._dispatched)
 
 
 class ReductionService:
@@ -162,7 +167,7 @@ class ReductionService:
         self.accumulations = _LiveAccumulations(self)  # index -> the calling rank's live tensor
         self.accumulation_indices = {}
         self.accumulation_dtype = accumulation_dtype
-        self.dispatched_tasks = 0
+        self._tasks = self._landed_tasks = 0  # adds ever dispatched, and how many of them are known to have landed
         self.buffer_splitter = BufferSplitter()
         if lazy_clear is None:
             lazy_clear = os.environ.get("ODC_LAZY_CLEAR", "0") == "1"
@@ -242,6 +247,8 @@ class ReductionService:
         if stream is not None:
             self._order_after_writers(keys, stream)
             status = _host_path.clear(world.arena.raw_handle, stream, table, keys)
+            if stream not in _launch_streams:
+                note_launch(stream)
         else:
             with comm_stream_section("odc.clear") as comm:
                 self._order_after_writers(keys, comm.cuda_stream)
@@ -362,6 +369,8 @@ class ReductionService:
         if stream is not None:
             self._order_after_writers(keys, stream)
             status = items.launch(world.arena.raw_handle, stream, store)
+            if stream not in _launch_streams:
+                note_launch(stream)
         else:
             with comm_stream_section("odc.scatter_store" if store else "odc.scatter_accumulate") as comm:
                 self._order_after_writers(keys, comm.cuda_stream)
@@ -446,7 +455,7 @@ class ReductionService:
                                      store)
                 if zero:
                     zero.difference_update(keys)
-            self.dispatched_tasks += n
+            self._tasks += n
 
     def scatter_accumulate_slices(
         self,
@@ -507,7 +516,7 @@ class ReductionService:
                     written = None
             self._written[key] = plan.disjoint if plan.disjoint is not None and written in (None, plan.disjoint) else _MIXED
             self._launch((key,), items, n, items.grad_code, items.acc_code, store)
-            self.dispatched_tasks += 1
+            self._tasks += 1
 
     def _plan_slices(self, key, slice_offsets, slice_numels, grad_dtype, pg, accumulation_numel, accumulation_dtype):
         """First call with these slices of ``key``: registers the key when it is new."""
@@ -589,6 +598,8 @@ class ReductionService:
             if stream is not None:
                 self._order_after_writers(keys, stream)
                 status = _host_path.publish(world.arena.raw_handle, world.rank, stream, *call)
+                if stream not in _launch_streams:
+                    note_launch(stream)
             else:
                 with comm_stream_section("odc.publish") as comm:
                     self._order_after_writers(keys, comm.cuda_stream)
@@ -615,9 +626,26 @@ class ReductionService:
     def sync(self, pg=None):
         """Block until every dispatched add has landed (:734-743: the reference counts tasks
         across ranks and waits for its watcher; here it waits for the streams launched on)."""
+        dispatched = self._tasks
         wait_for_launches()
+        self._landed(dispatched)
+
+    @property
+    def dispatched_tasks(self) -> int:
+        """Adds dispatched and not yet known to have landed."""
         with self._lock:
-            self.dispatched_tasks = 0
+            return self._tasks - self._landed_tasks
+
+    @dispatched_tasks.setter
+    def dispatched_tasks(self, tasks: int) -> None:
+        with self._lock:
+            self._tasks = self._landed_tasks + tasks
+
+    def _landed(self, tasks: int) -> None:
+        """The first ``tasks`` adds ever dispatched have landed; later ones, of other threads, stay counted."""
+        with self._lock:
+            if tasks > self._landed_tasks:
+                self._landed_tasks = tasks
 
     def syncing(self, pg=None):
         """``sync`` behind the launches of a ``with`` block: see ``syncing``."""

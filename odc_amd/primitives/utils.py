@@ -260,6 +260,7 @@ def finalize_distributed():
     _bare_allocations.clear()
     with _launch_lock:
         _launch_streams.clear()  # handles of a world that is gone are not waited for
+        _waits.clear()
     stream = None
 
 
@@ -488,7 +489,15 @@ def get_comm_stream():
 
 
 _launch_streams = {}  # stream handle -> torch stream with launches since the last wait (None: not wrapped yet)
+_waits = {}  # LaunchesInFlight that are being waited for -> what it took from _launch_streams
 _launch_lock = threading.Lock()  # launches come from several host threads (autograd's device thread)
+
+
+def note_launch(handle: int, stream=None) -> None:
+    """What was launched on the stream ``handle`` is to be waited for. Called behind the launch: listed in front of
+    it, the stream would be taken off the list by a wait of another thread in between."""
+    with _launch_lock:
+        _launch_streams.setdefault(handle, stream)
 
 
 def stream_from_handle(handle: int):
@@ -655,7 +664,7 @@ class comm_stream_section:
     This sits on the host path of every launch, so the default policy asks torch for the raw
     handle of the current stream only (a stream object is built when ``sync`` needs one)."""
 
-    __slots__ = ("label", "cuda_stream", "_traced", "_current", "_comm")
+    __slots__ = ("label", "cuda_stream", "_traced", "_current", "_comm", "_stream")
 
     def __init__(self, label: str = "odc"):
         self.label = label
@@ -666,17 +675,12 @@ class comm_stream_section:
         if self._traced:
             torch.cuda.nvtx.range_push(self.label)
         try:
+            self._stream = None
             if launch_stream_policy() == "caller":
-                handle = _current_raw_stream(get_world().arena.device)
-                if handle not in _launch_streams:
-                    with _launch_lock:
-                        _launch_streams.setdefault(handle, None)
-                self.cuda_stream = handle
+                self.cuda_stream = _current_raw_stream(get_world().arena.device)
                 return self
             current = torch.cuda.current_stream()
-            comm = get_comm_stream()
-            with _launch_lock:
-                _launch_streams[comm.cuda_stream] = comm
+            self._stream = comm = get_comm_stream()
             self.cuda_stream = comm.cuda_stream
             if current == comm:
                 return self
@@ -690,6 +694,7 @@ class comm_stream_section:
 
     def __exit__(self, exc_type, exc, tb):
         try:
+            note_launch(self.cuda_stream, self._stream)
             if self._comm is not None:
                 self._current.wait_stream(self._comm)
         finally:
@@ -698,55 +703,83 @@ class comm_stream_section:
         return False
 
 
-def wait_for_launches() -> None:
-    """Block the host until every launch issued through ``comm_stream_section`` has finished."""
-    with _launch_lock:
-        pending = list(_launch_streams.items())
-        _launch_streams.clear()
-    for handle, s in pending:
+class LaunchesInFlight:
+    """Everything launched so far through ``comm_stream_section`` and not yet waited for, to be waited for by the
+    host. Until that wait is over, other waits find it too, in ``_waits``: what a thread has taken off the list is
+    not done because it is no longer listed. If the wait fails all of it is listed again.
+
+    ``current``: the torch stream that the host goes on issuing work on before it waits. It is made to wait for the
+    launches on the others, so what comes next finds them done, and ``wait`` is for what was launched up to here. It
+    stays listed itself, for what comes next (a minibatch's launches are all there as a rule, and this costs it
+    nothing)."""
+
+    __slots__ = ("_streams", "_events")
+
+    def __init__(self, current=None):
+        current_handle = None if current is None else current.cuda_stream
+        with _launch_lock:
+            self._streams = streams = _launch_streams.copy()
+            if len(streams) > (current_handle in streams):
+                _waits[self] = taken = {handle: s for handle, s in streams.items() if handle != current_handle}
+                for handle in taken:
+                    del _launch_streams[handle]
+            if _waits:
+                for others in _waits.values():
+                    streams.update(others)
+        self._events = None
+        if current is None:
+            return
+        self._events = events = []
         try:
-            (s if s is not None else stream_from_handle(handle)).synchronize()
-        except RuntimeError:
-            # a stream destroyed since its launch cannot be waited for by name
-            torch.cuda.synchronize(get_world().arena.device)
+            for handle, s in streams.items():
+                event = torch.cuda.Event()
+                try:
+                    if handle == current_handle:
+                        event.record(current)
+                    else:
+                        event.record(s if s is not None else stream_from_handle(handle))
+                        current.wait_event(event)
+                except RuntimeError:  # a stream destroyed since its launch, see wait
+                    torch.cuda.synchronize(get_world().arena.device)
+                    continue
+                events.append(event)
+        except BaseException:
+            self._give_back()
+            raise
+
+    def wait(self) -> None:
+        try:
+            if self._events is not None:
+                for event in self._events:
+                    event.synchronize()
+            else:
+                for handle, s in self._streams.items():
+                    try:
+                        (s if s is not None else stream_from_handle(handle)).synchronize()
+                    except RuntimeError:
+                        # a stream destroyed since its launch cannot be waited for by name
+                        torch.cuda.synchronize(get_world().arena.device)
+        except BaseException:
+            self._give_back()
+            raise
+        if self in _waits:
+            with _launch_lock:
+                _waits.pop(self, None)
+
+    def _give_back(self) -> None:
+        with _launch_lock:
+            for handle, s in _waits.pop(self, {}).items():
+                _launch_streams.setdefault(handle, s)
 
 
 def has_launches() -> bool:
-    """Whether anything was launched through ``comm_stream_section`` since the last wait."""
-    return bool(_launch_streams)
+    """Whether there is anything to wait for: without it neither arena nor device need be asked."""
+    return bool(_launch_streams or _waits)
 
 
-def launches_in_flight():
-    """An event behind every launch issued so far through ``comm_stream_section``, for
-    ``wait_for_events``: ``wait_for_launches`` in two halves, so that the host can issue what comes next
-    before it waits. The current stream waits for the launches on the others, so what comes next finds
-    them done, as it would after ``wait_for_launches``. With no launches there is nothing to ask of arena or
-    device."""
-    with _launch_lock:
-        pending = list(_launch_streams.items())
-        _launch_streams.clear()
-    if not pending:
-        return []
-    device = get_world().device
-    current, events = torch.cuda.current_stream(device), []
-    for handle, s in pending:
-        event = torch.cuda.Event()
-        try:
-            if handle == current.cuda_stream:
-                event.record(current)
-            else:
-                event.record(s if s is not None else stream_from_handle(handle))
-                current.wait_event(event)
-        except RuntimeError:  # a stream destroyed since its launch, see wait_for_launches
-            torch.cuda.synchronize(device)
-            continue
-        events.append(event)
-    return events
-
-
-def wait_for_events(events) -> None:
-    for event in events:
-        event.synchronize()
+def wait_for_launches() -> None:
+    """Block the host until every launch issued through ``comm_stream_section`` has finished."""
+    LaunchesInFlight().wait()
 
 
 class BufferSplitter:

@@ -20,7 +20,7 @@ def no_device(monkeypatch):
         raise RuntimeError("asked the device")
 
     monkeypatch.setattr(utils, "_world", None)
-    monkeypatch.setattr(utils, "_launch_streams", {})
+    assert not utils._launch_streams
     monkeypatch.setattr(scatter_accumulate, "_is_capturing", refuse)
     monkeypatch.setattr(torch.cuda, "current_stream", refuse)
 
