@@ -13,6 +13,19 @@ def pytest_configure(config):
 
 
 @pytest.fixture
+def launch_list():
+    """The list of streams with launches, empty for the test (a test with a stand-in for the stream may have left
+    one there) and as it was behind it."""
+    from odc_amd.primitives import utils
+
+    saved = dict(utils._launch_streams)
+    utils._launch_streams.clear()
+    yield utils._launch_streams
+    utils._launch_streams.clear()
+    utils._launch_streams.update(saved)
+
+
+@pytest.fixture
 def make_world():
     """Factory: make_world(W, bytes_per_rank) -> VirtualGroup; everything is torn down after
     the test (registry, arena, comm stream)."""

@@ -8,6 +8,8 @@ import pytest
 from odc_amd import ReductionService
 from odc_amd.fsdp import fsdp1, fsdp2
 
+pytestmark = pytest.mark.usefixtures("launch_list")
+
 
 def _minibatch_ends(module, monkeypatch, service, calls):
     monkeypatch.setattr(module, "reduction_service", service)

@@ -34,21 +34,17 @@ class Event:
 
 
 @pytest.fixture
-def streams(monkeypatch):
+def streams(monkeypatch, launch_list):
     """Two streams with launches, 1 (the current one) and 2; wrapped as the services leave them."""
     made = {1: Stream(1), 2: Stream(2)}
-    saved = dict(utils._launch_streams)
-    utils._launch_streams.clear()
-    utils._launch_streams.update({1: None, 2: made[2]})
+    launch_list.update({1: None, 2: made[2]})
     monkeypatch.setattr(utils, "stream_from_handle", made.__getitem__)
     for module in (utils, scatter_accumulate):
         monkeypatch.setattr(module, "get_world", lambda: type("World", (), {"device": 0}))
     monkeypatch.setattr(scatter_accumulate, "_is_capturing", lambda: False)
     monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: made[1])
     monkeypatch.setattr(torch.cuda, "Event", Event)
-    yield made
-    utils._launch_streams.clear()
-    utils._launch_streams.update(saved)
+    return made
 
 
 def _in_thread(call):
