@@ -63,8 +63,9 @@ enum {
                                "dry_run_workgroups", and of the launches those in short tiles,
                                "dry_run_short_launches" / "dry_run_few_launches" by how a tile finds
                                its item, of the latter those of one wavefront per tile,
-                               "dry_run_tiny_launches", long streams, "dry_run_stream_launches", and those told of a
-                               resident part, "dry_run_resident_launches";
+                               "dry_run_tiny_launches", long streams, "dry_run_stream_launches", those told of a
+                               resident part, "dry_run_resident_launches", and those that write
+                               through the L2s, "dry_run_through_launches";
                                odc_set_option("dry_run_reset", 0) zeroes them).
                                For testing the host side of the library without a device; implies
                                ODC_ARENA_NO_BACKING for odc_arena_ptr / odc_arena_locate. */
@@ -272,8 +273,9 @@ int odc_abi_version(void);
  *    stores of fp32 gradients into fp32. Launches of persistent workgroups are not.
  *  - what a launch leaves in the caches: gathers of at most "cached_output_bytes" (64 MiB) of output
  *    leave it there, with plain stores up to "plain_output_bytes" (3 MiB) and written through the L2
- *    above, and so do accumulates with the accumulations that they leave there (stores only between
- *    "plain_output_bytes" and "cached_output_bytes"); converting gathers of at most
+ *    above, and so do accumulates with the accumulations that they leave there, from
+ *    "plain_accumulation_bytes" (3 MiB) on; scatter-stores write theirs through the L2 from there to
+ *    "through_store_bytes" (44 MiB) and past the caches otherwise; converting gathers of at most
  *    "cast_output_bytes" (32 MiB) of output write it through the L2 (conversions of symmetric memory:
  *    "cached_output_bytes"); gradients of at most "cached_gradient_bytes"
  *    (128 MiB) per launch are read through the caches; so are shards and accumulations while all symmetric

@@ -83,6 +83,8 @@ struct Options {
   int64_t resident_shard_bytes = 80ll << 20;
   int64_t resident_above = 640ll << 20;
   int64_t resident_clear_bytes = 48ll << 20;
+  int64_t plain_accumulation_bytes = 3ll << 20;  // see accumulation_form
+  int64_t through_store_bytes = 44ll << 20;  // see store_output_form
   int64_t through_clear_bytes = 256ll << 20;  // see clear_form
   int64_t stream_bytes = 8ll << 20;  // see stream_form
   int64_t cast_output_bytes = 32ll << 20;  // see cast_output_form
@@ -120,6 +122,8 @@ int64_t* option_slot(const char* name) {
   if (!strcmp(name, "resident_shard_bytes")) return &g_opt.resident_shard_bytes;
   if (!strcmp(name, "resident_above")) return &g_opt.resident_above;
   if (!strcmp(name, "resident_clear_bytes")) return &g_opt.resident_clear_bytes;
+  if (!strcmp(name, "plain_accumulation_bytes")) return &g_opt.plain_accumulation_bytes;
+  if (!strcmp(name, "through_store_bytes")) return &g_opt.through_store_bytes;
   if (!strcmp(name, "through_clear_bytes")) return &g_opt.through_clear_bytes;
   if (!strcmp(name, "cast_output_bytes")) return &g_opt.cast_output_bytes;
   if (!strcmp(name, "stream_bytes")) return &g_opt.stream_bytes;
@@ -204,9 +208,13 @@ int check_compute(odc_arena* a, DeviceGuard& guard) {
 std::atomic<int64_t> g_dry_launches{0}, g_dry_tiles{0}, g_dry_workgroups{0};
 std::atomic<int64_t> g_dry_short{0}, g_dry_few{0}, g_dry_tiny{0}, g_dry_stream{0};  // of the launches: those in kShortTiles, ...
 std::atomic<int64_t> g_dry_resident{0};  // those that are told of a resident part
+std::atomic<int64_t> g_dry_through{0};   // those that write through the L2s
 
 template <class Launch> TileForm form_of(const Launch& L) { return L.form; }
 TileForm form_of(const ClearLaunch&) { return kWholeTiles; }
+template <class Launch> bool writes_through(const Launch& L) { return L.output == kWriteThrough; }
+bool writes_through(const AccumLaunch& L) { return L.policy.read && L.policy.written == kWriteThrough; }
+bool writes_through(const PublishLaunch&) { return false; }
 
 // The one place kernels are launched from: `issue` is the odc_device launch of the entry point.
 // On a dry-run arena the launch is only counted: the host-side validation, work-list splitting
@@ -224,6 +232,7 @@ int launch_tiles(const odc_arena* a, const Launch& L, uint32_t grid, Issue issue
     g_dry_tiny += form_of(L) == kTinyTiles;
     g_dry_stream += form_of(L) == kStreamTiles;
     g_dry_resident += L.tt.resident_below != 0;
+    g_dry_through += writes_through(L);
     return ODC_OK;
   }
   const int e = issue();
@@ -273,8 +282,8 @@ uint32_t grid_for(const odc_arena* a, int64_t blocks_per_cu, uint32_t n_tiles, u
 //     elements, 3 sets) fill + accumulate 12.7 -> 10.8 and accumulate alone 8.9 -> 7.9, with 144 MB
 //     accumulate alone 14.6 -> 12.4 and gather alone 7.0 -> 6.2; with 600 MB (24 sets) fill +
 //     accumulate 12.8 -> 13.1 and gather + read 7.4 -> 8.0. The line is 192 MiB of the 256.
-// How what stays is written: output_form, a store's accumulations: store_output_form, the converting gather's output:
-// cast_output_form.
+// How what stays is written: output_form, accumulation_form, a store's accumulations: store_output_form, the converting
+// gather's output: cast_output_form.
 CachePolicy cache_policy(const odc_arena* a, const Options& opt, uint64_t read_bytes, int64_t read_line,
                          uint64_t written_bytes, int64_t written_line) {
   const bool arena_fits = a->in_use.load(std::memory_order_relaxed) * a->world <= (uint64_t)opt.cached_arena_bytes;
@@ -312,21 +321,13 @@ uint32_t resident_below(const odc_arena* a, const Options& opt, int64_t most) {
   return (uint32_t)std::min(4294967295.0, (double)most / in_use * 4294967296.0);
 }
 
-// How a gather writes an output, and an accumulate accumulations, that stay in the caches: written through the
-// L2s to the last-level cache (store_output in odc_kernels.hip). Plain stores leave up to what the L2s hold (8 x 4
-// MB) in them as dirty lines, whose way out the kernel, or the next one, then waits for; the lines that are written
-// through stay there for the next kernel too. Below 3 MiB the two are level or plain stores ahead by up to 0.1 us.
-// Graph-replayed launches at W = 8, us, plain -> written through, one item on one set of buffers, nine items on
-// three sets in turn:
-//   gather of bf16: 1 M elements 2.25 -> 2.28, 2.55 -> 2.76; 2.1 M 2.48 -> 2.38, 3.06 -> 3.07; 4.2 M 3.27 -> 2.84, 4.24 ->
-//     3.61; 8.4 M (16 MiB of output) 4.90 -> 4.09, 6.54 -> 6.35;
-//   accumulate of bf16 into fp32: 0.26 M 2.01 -> 2.07; 1 M 2.60 -> 2.61, 3.43 -> 3.28; 2.1 M 3.37 -> 3.52, 4.80 -> 4.08;
-//     4.2 M 5.16 -> 6.49, 7.66 -> 6.96; 8.4 M 11.8 -> 9.3, 12.8 -> 12.1; 16.8 M 21.9 -> 21.1, 24.0 -> 24.0; into bf16
-//     4.2 M 4.06 -> 3.61, 6.05 -> 5.33; 8.4 M 6.21 -> 5.62, 9.28 -> 8.67;
-//   (the two that are slower repeat one accumulate and nothing else, so that accumulations of up to 16 MB never
-//   leave the L2s; with a gather in front of it the same 4.2 M elements take 9.72 -> 8.12;)
-//   a minibatch of four microbatches: 1 M 24.1 -> 22.7, 30.4 -> 27.5; 4.2 M 51.1 -> 37.7, 51.9 -> 47.8; 16.8 M 139 -> 133,
-//     162.5 -> 161.5; 33 M 279 -> 270, but its pass of one gather and one accumulate 65.1 -> 66.6.
+// How a gather writes an output that stays in the caches: written through the L2s to the last-level cache
+// (store_output in odc_kernels.hip). Plain stores leave up to what the L2s hold (8 x 4 MB) in them as dirty lines,
+// whose way out the kernel, or the next one, then waits for; the lines that are written through stay there for the
+// next kernel too. Below 3 MiB the two are level or plain stores ahead by up to 0.2 us. Graph-replayed gathers of
+// bf16 at W = 8, us, plain -> written through, one item on one set of buffers, nine items on three sets in turn:
+//   1 M elements 2.25 -> 2.28, 2.55 -> 2.76; 2.1 M (4 MiB) 2.48 -> 2.38, 3.06 -> 3.07; 4.2 M 3.27 -> 2.84, 4.24 -> 3.61; 8.4 M
+//   4.90 -> 4.09, 6.54 -> 6.35; 16.8 M and more level.
 // With products of 128 to 1024 tokens that read the output and write the gradient behind the gather, outputs of
 // 1 to 25 MiB: level or ahead by up to 2 % (9 MiB, 512 tokens, forward 28.05 -> 27.4, with backward 57.5 -> 57.1).
 OutputForm output_form(const Options& opt, bool cached, uint64_t bytes) {
@@ -334,19 +335,39 @@ OutputForm output_form(const Options& opt, bool cached, uint64_t bytes) {
   return bytes <= (uint64_t)opt.plain_output_bytes ? kKeep : kWriteThrough;
 }
 
-// A store's accumulations, which it does not read: written through from 3 to 64 MiB, nontemporal otherwise. The same
-// launches, and passes of gather, store, gather, accumulate, us, nontemporal -> written through:
-//   store of bf16 into fp32: 0.52 M elements 2.19 -> 2.24, 2.66 -> 2.60; 1 M 2.51 -> 2.41, 3.05 -> 3.00; 4.2 M 4.30 -> 4.48, 5.19
-//     -> 4.90; 16.8 M (64 MiB) 13.5 -> 12.1, 14.5 -> 14.7 (one item over three sets 13.4 -> 15.9, level in
-//     passes); into bf16 4.2 M 3.31 -> 3.02, 16.8 M 9.55 -> 7.87;
-//   passes: 1 M 9.61 -> 8.70, 11.74 -> 10.90; 4.2 M 16.06 -> 14.33, 20.02 -> 19.10; 8.4 M 28.7 -> 26.9, 34.1 -> 35.2; 33 M
-//     105 .. 107 -> 111 .. 116.
+// How an accumulate writes accumulations that stay in the caches: likewise from 3 MiB of them on. Where one
+// accumulate is repeated over one set of buffers with at most a gather between, accumulations of 8 to 16 MiB never
+// leave the L2s and plain stores are ahead; with a clear, other buffers, more items or larger ones between it is the
+// other way round, and a minibatch has those. us as above, bf16 into fp32, plain -> written through:
+//   accumulate: 1 M elements (4 MiB) 2.86 -> 2.85, 3.35 -> 3.27; 2.1 M 3.45 -> 3.61, 4.60 -> 4.09; 3 M 4.12 -> 4.48, 6.28 -> 5.11;
+//     4.2 M (16 MiB) 4.87 -> 5.59, 7.52 -> 6.84; 8.4 M 12.05 -> 9.31, 12.8 -> 12.4; 12.6 M 17.1 -> 15.0, 18.3 -> 18.0; 16.8 M
+//     21.9 -> 21.2, 24.0 -> 23.9; into bf16 4.2 M 4.09 -> 3.61, 6.06 -> 5.33, 8.4 M 6.20 -> 5.61, 9.75 -> 8.91;
+//   gather, accumulate: 1 M 5.03 -> 4.97, 6.10 -> 5.75; 2.1 M 5.88 -> 6.05, 8.27 -> 7.57; 3 M 6.81 -> 7.11, 9.95 -> 9.40; 4.2 M
+//     9.05 -> 8.58, 11.9 -> 11.7; 8.4 M 17.6 -> 16.8, 22.2 -> 22.0; 33.5 M 65.4 -> 66.6, 81.7 -> 81.4;
+//   minibatches (clear, four times that, publish): 1 M 24.8 -> 23.4, 29.6 -> 27.2; 2.1 M 30.3 -> 28.2, 36.3 -> 34.9; 4.2 M 47.5 ->
+//     39.8, 48.5 -> 48.2 (one item, three sets 43.0 -> 44.2); 8.4 M 84.9 -> 73.1, 89.1 -> 86.7; 12.6 M 113.5 -> 107.8,
+//     121.7 -> 121.2; 33.5 M 279 -> 270, 302 -> 302.
+OutputForm accumulation_form(const Options& opt, bool cached, uint64_t bytes) {
+  if (!cached) return kStream;
+  return bytes <= (uint64_t)opt.plain_accumulation_bytes ? kKeep : kWriteThrough;
+}
+
+// A store's accumulations, which it does not read: written through from 3 to 44 MiB, nontemporal otherwise. us as
+// above, nontemporal -> written through:
+//   store of bf16 into fp32: 0.52 M elements 2.19 -> 2.24, 2.66 -> 2.60; 1 M 2.51 -> 2.41, 3.05 -> 3.00; 4.2 M 4.19 -> 4.16, 5.38 ->
+//     4.99; 8.4 M 6.46 -> 6.47, 8.40 -> 8.50; 10.5 M (40 MiB) 7.66 -> 7.31, 9.95 -> 9.97; 12.6 M (48 MiB) 9.15 -> 8.44, 11.7 ->
+//     13.0; 14.7 M 11.4 -> 9.92, 13.1 -> 16.1; 16.8 M 13.4 -> 12.0, 14.4 -> 14.3, one item over three sets 13.5 -> 16.0;
+//   gather, store, gather, accumulate: 4.2 M 17.4 -> 16.0, 20.0 -> 19.2; 8.4 M 29.4 -> 27.8, 35.5 -> 35.9; 10.5 M 35.5 -> 34.5,
+//     45.7 -> 43.6; 12.6 M 42.7 -> 42.3, 48.2 -> 48.3; 14.7 M 48.2 -> 47.8, 54.6 -> 54.6; 16.8 M 52.1 -> 51.8, 60.3 -> 60.0;
+//   lazy minibatches: 4.2 M 37.0 -> 35.5, 43.3 -> 42.4; 10.5 M 80.5 -> 79.5, 96.5 -> 94.4; 12.6 M 94.7 -> 94.0, 108.4 -> 108.2; 16.8 M
+//     115.8 -> 115.3, 134.2 -> 134.0.
+// From 48 MiB on what one set gains in passes, 1 %, is less than what the store itself loses over several.
 OutputForm store_output_form(const Options& opt, bool cached, uint64_t bytes) {
-  const bool through = cached && bytes > (uint64_t)opt.plain_output_bytes && bytes <= (uint64_t)opt.cached_output_bytes;
+  const bool through = cached && bytes > (uint64_t)opt.plain_accumulation_bytes && bytes <= (uint64_t)opt.through_store_bytes;
   return through ? kWriteThrough : kStream;
 }
 
-// The same for a gather that converts, and for a conversion of symmetric memory, which are ahead with the output
+// output_form for a gather that converts, and for a conversion of symmetric memory, which are ahead with the output
 // written through whoever reads it, as long as it leaves room for the gradients and accumulations of the
 // pass: up to 32 MiB, and 64 MiB of copies that the gathers behind find in the cache. Passes, fp32 into bf16 at
 // W = 8, us, nontemporal -> written through: gather + accumulate of 9 M elements 27.5 -> 26.9, 13 M 38.2 ->
@@ -524,7 +545,7 @@ int odc_abi_version(void) { return ODC_HIP_ABI_VERSION; }
 int odc_set_option(const char* name, int64_t value) {
   if (name && !strcmp(name, "dry_run_reset")) {
     g_dry_launches = 0; g_dry_tiles = 0; g_dry_workgroups = 0;
-    g_dry_short = 0; g_dry_few = 0; g_dry_tiny = 0; g_dry_stream = 0; g_dry_resident = 0;
+    g_dry_short = 0; g_dry_few = 0; g_dry_tiny = 0; g_dry_stream = 0; g_dry_resident = 0; g_dry_through = 0;
     return ODC_OK;
   }
   std::lock_guard<std::mutex> lk(g_opt_mu);
@@ -550,6 +571,7 @@ int odc_get_option(const char* name, int64_t* value) {
     if (!strcmp(name, "dry_run_tiny_launches")) { *value = g_dry_tiny.load(); return ODC_OK; }
     if (!strcmp(name, "dry_run_stream_launches")) { *value = g_dry_stream.load(); return ODC_OK; }
     if (!strcmp(name, "dry_run_resident_launches")) { *value = g_dry_resident.load(); return ODC_OK; }
+    if (!strcmp(name, "dry_run_through_launches")) { *value = g_dry_through.load(); return ODC_OK; }
   }
   std::lock_guard<std::mutex> lk(g_opt_mu);
   int64_t* s = option_slot(name);
@@ -1085,7 +1107,7 @@ int scatter_launch(odc_arena* a, const odc_accum_item* items, uint32_t n_items, 
     L.policy.read = cached.read;
     const uint64_t written_bytes = size.units * ab * a->world;
     L.policy.written = store ? store_output_form(opt, cached.written, written_bytes)
-                             : output_form(opt, cached.written, written_bytes);
+                             : accumulation_form(opt, cached.written, written_bytes);
     const bool one_per_tile = (store ? opt.store_blocks_per_cu : opt.accum_blocks_per_cu) <= 0 &&
                               (store || opt.accum_persistent_below_tiles == 0);
     if (one_per_tile && !(cached.read && cached.written))

@@ -20,8 +20,8 @@ BF16, F16, F32 = torch.bfloat16, torch.float16, torch.float32
 def test_bits_and_bounds(make_world, sizes, grad_dtype, acc_dtype, plain):
     from odc_amd import ReductionService, SymmBufferRegistry
 
-    options = {"plain_output_bytes": plain, "cached_arena_bytes": 1 << 40, "cached_gradient_bytes": 1 << 40,
-               "cached_output_bytes": 1 << 40}
+    options = {"plain_accumulation_bytes": plain, "through_store_bytes": 1 << 40, "cached_arena_bytes": 1 << 40,
+               "cached_gradient_bytes": 1 << 40}
     saved = {name: _native.get_option(name) for name in options}
     try:
         for name, value in options.items():
