@@ -266,7 +266,9 @@ int odc_abi_version(void);
  *    of less than one tile per rank after the others; 0 keeps the caller's order.
  *  - "short_tiles_below" (default 32): launches whose segments average fewer whole tiles are cut into
  *    short ones (0: none but those that always are). "few_tiles" (32768): up to so many short tiles
- *    a workgroup reads the whole table of the launch's items at once instead of searching it.
+ *    a workgroup reads the whole table of the launch's items at once instead of searching it, and of those from
+ *    "tiny_tiles_from" (2048) tiles on that are at most half full on average, of more than 16 items, each has one
+ *    wavefront.
  *    "stream_bytes" (8 MiB): launches of up to 64 items that write more past the caches are long streams, in
  *    short tiles with fewer workgroups resident: accumulates of 16-bit gradients that are not read through the
  *    caches into fp32; and, where they would go in whole tiles, gathers without conversion and accumulates and

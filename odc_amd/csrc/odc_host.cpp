@@ -89,7 +89,8 @@ struct Options {
   int64_t stream_bytes = 8ll << 20;  // see stream_form
   int64_t cast_output_bytes = 32ll << 20;  // see cast_output_form
   int64_t short_tiles_below = 32;             // see wants_short_tiles
-  int64_t few_tiles = 32768;                  // see tile_form
+  int64_t few_tiles = 32768;                  // see table_form
+  int64_t tiny_tiles_from = 2048;             // see tile_form
 };
 Options g_opt;
 std::mutex g_opt_mu;
@@ -128,6 +129,7 @@ int64_t* option_slot(const char* name) {
   if (!strcmp(name, "cast_output_bytes")) return &g_opt.cast_output_bytes;
   if (!strcmp(name, "stream_bytes")) return &g_opt.stream_bytes;
   if (!strcmp(name, "short_tiles_below")) return &g_opt.short_tiles_below;
+  if (!strcmp(name, "tiny_tiles_from")) return &g_opt.tiny_tiles_from;
   if (!strcmp(name, "few_tiles")) return &g_opt.few_tiles;
   return nullptr;
 }
@@ -476,7 +478,10 @@ bool publish_in_short_tiles(const LaunchSize& size, int acc_bytes) { return acc_
 //   10 of 256 .. 262 144: 6.1 -> 5.9, 6.5 -> 6.2, 7.2 -> 6.9;
 //   112 of 160 000 (17 900 tiles): 41.2 -> 39.7, 41.1 -> 40.2; 112 of 640 000 (70 000 tiles): 156 -> 159,
 //   159 -> 162; 60 of 900 000 (53 000 tiles): 115 -> 115, 116.5 -> 117.6.
-//
+TileForm table_form(TileForm cut, uint32_t n_tiles, int64_t few) {
+  return cut == kShortTiles && n_tiles <= (uint64_t)few ? kFewShortTiles : cut;
+}
+
 // What is left of their time goes with the number of wavefronts: some 0.55 us per 1000 workgroups of two. Where
 // tiles are at most half full on average the second wavefront has little to do, and from 2048 tiles on (8 per CU)
 // launches by the full tables have workgroups of one, which moves four vectors per lane in a full tile. us, 100
@@ -485,12 +490,13 @@ bool publish_in_short_tiles(const LaunchSize& size, int acc_bytes) { return acc_
 //   W = 64, 6400 tiles: 0.26 M elements in all 6.27 -> 4.87, 6.77 -> 5.21, 6.59 -> 4.94, 6.71 -> 5.21; 4.2 M 6.78 -> 5.49, 7.80 ->
 //     6.68, 7.28 -> 5.76, 7.29 -> 5.81; W = 32, 3200 tiles: 1 M 4.43 -> 3.99, 4.78 -> 4.25, 4.71 -> 4.24, 4.73 -> 4.20;
 //   W = 16, 2096 tiles half full: 3.97 -> 3.94, 4.21 -> 4.22, 4.12 -> 3.95, 3.96 -> 3.88; fewer tiles, gather: 784 2.98 -> 3.32,
-//     1568 3.58 -> 3.74; 2544 tiles, 94 % full, accumulate 4.61 -> 4.84; publishes of one rank never have so many.
-constexpr uint32_t kTinyFrom = 2048;
-TileForm tile_form(TileForm cut, const TileTable& tt, uint64_t units, uint64_t whole_tile_units, int64_t few) {
-  if (cut != kShortTiles || tt.n_tiles > (uint64_t)few) return cut;
+//     1568 3.58 -> 3.74; 2544 tiles, 94 % full, accumulate 4.61 -> 4.84.
+// (Publishes, of one rank, never have so many half-empty tiles, and no kernels for them.)
+TileForm tile_form(TileForm cut, const TileTable& tt, uint64_t units, uint64_t whole_tile_units, const Options& opt) {
+  const TileForm form = table_form(cut, tt.n_tiles, opt.few_tiles);
+  if (form != kFewShortTiles || tt.n_items <= kFewItems || tt.n_tiles < (uint64_t)opt.tiny_tiles_from) return form;
   const bool half_empty = 2 * units * tt.world <= (uint64_t)tt.n_tiles * (whole_tile_units / kShortTileParts);
-  return tt.n_items > kFewItems && tt.n_tiles >= kTinyFrom && half_empty ? kTinyTiles : kFewShortTiles;
+  return half_empty ? kTinyTiles : form;
 }
 
 // Whether a launch that is otherwise cut as `cut` is a long stream: more than 8 MiB written, past the caches,
@@ -870,7 +876,7 @@ int odc_gather(odc_arena* a, const odc_gather_item* items, uint32_t n_items, uin
         });
     if (n < 0) return n;
     if (n == 0) continue;
-    L.form = tile_form(cut, L.tt, size.units, kTileBytes, opt.few_tiles);
+    L.form = tile_form(cut, L.tt, size.units, kTileBytes, opt);
     L.output = output_form(opt, L.policy.written, out_bytes);
     L.tt.resident_below = resident_below(a, opt, opt.resident_shard_bytes);
     const auto ragged = [&] {
@@ -929,7 +935,7 @@ int odc_gather_cast(odc_arena* a, const odc_gather_cast_item* items, uint32_t n_
         });
     if (n < 0) return n;
     if (n == 0) continue;
-    L.form = tile_form(cut, L.tt, size.units, kTileElems, opt.few_tiles);
+    L.form = tile_form(cut, L.tt, size.units, kTileElems, opt);
     const uint32_t grid = grid_for(a, opt.gather_blocks_per_cu, L.tt.n_tiles, copy_threads(L.form));
     const uint32_t lds = lds_claim_for(a, opt.cast_resident_cap, grid, L.tt.n_tiles);
     if (int rc = launch_tiles(a, L, grid, [&] {
@@ -982,7 +988,7 @@ int odc_convert(odc_arena* a, const odc_convert_item* items, uint32_t n_items, i
         });
     if (n < 0) return n;
     if (n == 0) continue;
-    L.form = tile_form(cut, L.tt, size.units, kTileElems, opt.few_tiles);
+    L.form = tile_form(cut, L.tt, size.units, kTileElems, opt);
     const uint32_t grid = grid_for(a, opt.gather_blocks_per_cu, L.tt.n_tiles, copy_threads(L.form));
     const uint32_t lds = lds_claim_for(a, opt.cast_resident_cap, grid, L.tt.n_tiles);
     if (int rc = launch_tiles(a, L, grid, [&] {
@@ -1121,7 +1127,7 @@ int scatter_launch(odc_arena* a, const odc_accum_item* items, uint32_t n_items, 
         order);
     if (n < 0) return n;
     if (n == 0) continue;
-    L.form = tile_form(cut, L.tt, size.units, kTileElems, opt.few_tiles);
+    L.form = tile_form(cut, L.tt, size.units, kTileElems, opt);
     // Tile order. Item-major (a rank's segment, then the next rank's, item by item) walks the
     // gradient contiguously and hops between rank regions at every segment; rank-outermost walks
     // one rank region from accumulation to accumulation (they are neighbours when registered
@@ -1238,7 +1244,7 @@ int odc_publish(odc_arena* a, uint32_t rank, const odc_publish_item* items, uint
         });
     if (n < 0) return n;
     if (n == 0) continue;
-    L.form = tile_form(cut, L.tt, size.units, kTileElems, opt.few_tiles);
+    L.form = table_form(cut, L.tt.n_tiles, opt.few_tiles);
     // one workgroup per tile: the division sequence wants the occupancy, and the launch is short
     const uint32_t grid = grid_for(a, opt.publish_blocks_per_cu, L.tt.n_tiles, publish_threads(L.form));
     const uint32_t lds = lds_claim_for(a, opt.publish_resident_cap, grid, L.tt.n_tiles);

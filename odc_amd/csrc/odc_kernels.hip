@@ -196,7 +196,7 @@ struct SingleWalk {
   template <uint32_t>
   __device__ __forceinline__ TileCoord locate(const SingleLaunch<D>&, uint32_t t) const { return single_item_coord(tt, t); }
 };
-// Few short tiles of several items (tile_form in odc_host.cpp): again a chain of latencies, the binary
+// Few short tiles of several items (table_form in odc_host.cpp): again a chain of latencies, the binary
 // search being most of it. The whole prefix table is read together with the header instead, one entry
 // per lane (two for its second half), and the item found by counting the entries that are not greater
 // than the tile's position:
@@ -320,6 +320,12 @@ __device__ __forceinline__ void each_tile(const Walk& walk, const Launch& launch
 constexpr int kMostWaves = 8, kStreamWaves = 6;
 
 // ---- gather -------------------------------------------------------------------------------
+// The bytes of a segment's head that one of T lanes moves.
+template <int T> constexpr int kHeadBytes = (ODC_BODY_ALIGN - 2) / T + 1;
+static_assert(kHeadBytes<kTinyThreads> * kTinyThreads >= ODC_BODY_ALIGN - 1 &&
+                  kHeadBytes<kShortThreads> * kShortThreads >= ODC_BODY_ALIGN - 1,
+              "every byte of a head has a lane");
+
 // Everything of a tile that is not a run of T * U whole vectors: the last partial run, the
 // head and the tail. Kept out of line so that the streaming loop stays tight (inline, the
 // short-segment kernels, which come here for most of their tiles, were 5 % slower too).
@@ -337,7 +343,7 @@ __device__ __attribute__((noinline)) void gather_edges(uint8_t* d, const uint8_t
   const bool do_tail = w.tail && tid < g.tail;
   const uint64_t tail_at = g.head + g.nvec * 16 + tid;
   const uint32_t head = w.head ? g.head : 0u;
-  constexpr int kHead = (ODC_BODY_ALIGN - 2) / T + 1;  // head bytes per lane
+  constexpr int kHead = kHeadBytes<T>;
   u32x4 v[U];
   uint8_t head_byte[kHead] = {}, tail_byte = 0;
 #pragma unroll
@@ -386,7 +392,7 @@ __global__ __launch_bounds__(T) ODC_RESIDENT_WAVES(kWaves) void gather_kernel(co
         const bool do_tail = w.tail && tid < g.tail;
         const uint64_t tail_at = g.head + g.nvec * 16 + tid;
         const uint32_t head = w.head ? g.head : 0u;
-        constexpr int kHead = (ODC_BODY_ALIGN - 2) / T + 1;  // head bytes per lane
+        constexpr int kHead = kHeadBytes<T>;
         uint8_t head_byte[kHead] = {}, tail_byte = 0;
 #pragma unroll
         for (int h = 0; h < kHead; ++h)
@@ -411,6 +417,7 @@ __global__ __launch_bounds__(T) ODC_RESIDENT_WAVES(kWaves) void gather_kernel(co
 // microsecond went to. Longer clears than that cache holds (clear_form in odc_host.cpp) have plain stores,
 // which leave their end in the L2s. Nontemporal ones are behind both.
 __device__ __attribute__((noinline)) void clear_edges(uint8_t* d, uint32_t chunk, SegShape g) {
+  static_assert(kThreads >= ODC_BODY_ALIGN - 1, "one lane per head byte");
   d = as_global(d);
   const u32x4 zero = {0u, 0u, 0u, 0u};
   const uint32_t tid = threadIdx.x;
@@ -1051,7 +1058,8 @@ kernel_fn<L> pick_cast_gather(int s, int d, CachePolicy policy, OutputForm outpu
   return nullptr;
 }
 
-// publish_in_short_tiles: fp32 accumulations have no kernel of whole tiles.
+// publish_in_short_tiles: fp32 accumulations have no kernel of whole tiles. (table_form: nor are there any of one
+// wavefront.)
 template <class L, class A, class O>
 kernel_fn<L> pick_publish_form(TileForm form) {
   if (form == kFewShortTiles) return publish_kernel<L, A, O, kSearches<L>, kShortThreads, kShortUnroll>;

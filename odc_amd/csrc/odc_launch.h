@@ -43,7 +43,7 @@ struct AccumPolicy {
   OutputForm written = kStream;
 };
 
-// How a launch is cut, and how its workgroups find their items (wants_short_tiles and tile_form in
+// How a launch is cut, and how its workgroups find their items (wants_short_tiles, table_form and tile_form in
 // odc_host.cpp). kTinyTiles: kFewShortTiles by workgroups of one wavefront; kStreamTiles: short tiles of a long
 // stream (stream_form there).
 enum TileForm : uint32_t { kWholeTiles, kShortTiles, kFewShortTiles, kTinyTiles, kStreamTiles };

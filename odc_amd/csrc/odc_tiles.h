@@ -273,9 +273,10 @@ template <uint32_t kVecs = kTileVecs>
 ODC_HD SegShape seg_shape(uintptr_t written_addr, uint64_t n, uint32_t unit_bytes, uint32_t vec_units) {
   // The body starts on a 128 B line of the written side, not merely on a vector boundary: a
   // wavefront's 64 vector stores then cover whole lines, none shared with the next wavefront.
-  // (The head is at most 127 bytes, i.e. fewer units than a workgroup has lanes.)
+  // (The head is at most kLine - 1 bytes. In bytes that can be more units than a workgroup of one wavefront has
+  // lanes; each kernel asserts what it takes.)
   constexpr uint32_t kLine = ODC_BODY_ALIGN;
-  static_assert(kLine >= 16 && kLine - 1 <= kThreads, "one lane per head unit");
+  static_assert(kLine >= 16, "whole vectors");
   SegShape g;
   uint64_t head = ((kLine - (uint32_t)(written_addr & (kLine - 1))) & (kLine - 1)) / unit_bytes;
   if (head > n) head = n;
