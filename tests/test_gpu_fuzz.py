@@ -123,7 +123,10 @@ KNOBS = [
     {"short_tiles_below": 1 << 30, "few_tiles": 0, "gather_blocks_per_cu": 1, "accum_blocks_per_cu": 1},
     {"short_tiles_below": 1 << 30, "few_tiles": 1 << 30, "store_blocks_per_cu": 1, "publish_blocks_per_cu": 1},
     {"cached_output_bytes": 0, "cached_gradient_bytes": 0, "cached_arena_bytes": 0},
-    {"cached_output_bytes": 1 << 40, "plain_output_bytes": 0, "cached_gradient_bytes": 1 << 40, "cached_arena_bytes": 1 << 40},
+    {"cached_output_bytes": 1 << 40, "plain_output_bytes": 0, "cached_gradient_bytes": 1 << 40, "cached_arena_bytes": 1 << 40,
+     "plain_accumulation_bytes": 0, "through_store_bytes": 1 << 40, "through_clear_bytes": 1 << 40, "tiny_tiles_from": 0},
+    {"cached_output_bytes": 1 << 40, "plain_output_bytes": 1 << 40, "cached_gradient_bytes": 1 << 40, "cached_arena_bytes": 1 << 40,
+     "plain_accumulation_bytes": 1 << 40, "through_store_bytes": 0, "through_clear_bytes": 0, "tiny_tiles_from": 1 << 40},
     # long streams, and the part that stays in the cache, whatever else is asked for
     {"stream_bytes": 0, "cached_output_bytes": 0, "cached_gradient_bytes": 0, "cached_arena_bytes": 0, "short_tiles_below": 0},
     {"stream_bytes": 0, "cached_output_bytes": 0, "cached_gradient_bytes": 0, "cached_arena_bytes": 0, "short_tiles_below": 0,
@@ -152,6 +155,7 @@ def test_results_do_not_depend_on_launch_knobs(make_world, knobs):
              "publish_blocks_per_cu", "gather_resident_cap", "cast_resident_cap", "accum_resident_cap",
              "store_resident_cap", "rank_major", "accum_tile_order", "accum_persistent_below_tiles",
              "accum_short_segment_tiles", "accum_small_items_last", "short_tiles_below", "few_tiles",
+             "plain_accumulation_bytes", "through_store_bytes", "through_clear_bytes", "tiny_tiles_from",
              "cached_output_bytes", "plain_output_bytes", "cached_gradient_bytes", "cached_arena_bytes", "stream_bytes",
              "cast_output_bytes", "resident_above", "resident_accumulation_bytes", "resident_shard_bytes",
              "resident_clear_bytes", "alloc_align", "rank_stride_align", "rank_stagger_bytes"]

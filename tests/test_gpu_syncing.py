@@ -45,6 +45,34 @@ def test_publish_behind_adds_of_a_busy_stream(make_world, policy, monkeypatch):
 
 
 @pytest.mark.gpu
+def test_a_sync_of_another_thread_during_the_block(make_world):
+    """It waits for the adds that the block has yet to wait for, and they are counted until then."""
+    import threading
+
+    from odc_amd import ReductionService
+    from odc_amd.primitives import utils
+
+    W, n = 4, 40_000
+    group = make_world(W, 4 << 20)
+    service = ReductionService(accumulation_dtype=torch.float32)
+    service.register("k", (n,), torch.bfloat16, torch.float32, group)
+    grad = torch.ones(W * n, dtype=torch.bfloat16, device="cuda")
+    work, side, seen = torch.randn(2048, 2048, device="cuda"), torch.cuda.Stream(), []
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        for _ in range(40):
+            torch.mm(work, work).mul_(1e-4)
+        service.scatter_accumulate("k", grad, group)
+    with service.syncing(group):
+        seen.append(service.dispatched_tasks)
+        other = threading.Thread(target=lambda: (service.sync(group), seen.append(side.query())))
+        other.start()
+        other.join()
+    assert seen == [1, True] and service.dispatched_tasks == 0 and not utils._waits
+    assert torch.equal(service.get_accumulation("k"), torch.ones(n, device="cuda"))
+
+
+@pytest.mark.gpu
 def test_a_sync_of_the_callers_own_is_called_first(make_world):
     from odc_amd import ReductionService
 
