@@ -53,10 +53,10 @@ from odc_amd.primitives.utils import (
     StreamOrder,
     SymmBufferRegistry,
     _launch_streams,
+    _waits,
     comm_stream_section,
     get_world,
     group_size,
-    has_launches,
     native_dtype,
     note_launch,
     plain_launch_stream,
@@ -145,7 +145,7 @@ class syncing:
             service.sync(self._pg)
             return
         self._dispatched = service._tasks
-        if not has_launches():
+        if not _launch_streams and not _waits:  # nothing to wait for: neither arena nor device is asked
             return
         if _is_capturing():
             # an event of the captured stream is nothing that the host could wait for: as sync does, which is
@@ -155,10 +155,11 @@ class syncing:
             self._launches = LaunchesInFlight(torch.cuda.current_stream(get_world().device))
 
     def __exit__(self, exc_type, exc, tb):
-        if self._launches is not None:
-            self._launches.wait()
-        if self._dispatched is not None:
-            self._service._landed(self._dispatched)
+        launches, dispatched = self._launches, self._dispatched
+        if launches is not None:
+            launches.wait()
+        if dispatched is not None:
+            self._service._landed(dispatched)
 
 
 class ReductionService:

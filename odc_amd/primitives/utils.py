@@ -772,11 +772,6 @@ class LaunchesInFlight:
                 _launch_streams.setdefault(handle, s)
 
 
-def has_launches() -> bool:
-    """Whether there is anything to wait for: without it neither arena nor device need be asked."""
-    return bool(_launch_streams or _waits)
-
-
 def wait_for_launches() -> None:
     """Block the host until every launch issued through ``comm_stream_section`` has finished."""
     LaunchesInFlight().wait()
