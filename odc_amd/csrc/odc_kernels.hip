@@ -15,7 +15,8 @@
 // (16 KiB), done by workgroups of 256 threads or 512 (odc_launch.h says which), or into short tiles of 256
 // vectors, done by 128 threads (64 where most are part-empty, kTinyTiles): launches of short segments
 // (wants_short_tiles in odc_host.cpp) and every accumulate and store of 16-bit gradients into fp32
-// (accum_streams_short in odc_launch.h), every publish of fp32 accumulations (publish_in_short_tiles in odc_host.cpp), and long streams (stream_form there).
+// (accum_streams_short in odc_launch.h), every publish of fp32 accumulations (publish_in_short_tiles in
+// odc_host.cpp), and long streams (stream_form there).
 // Workgroups walk the tiles with a grid-stride loop, by default one workgroup per tile, so that,
 // at any instant, the whole chip streams one compact window of memory. Per-item
 // descriptors (<= ODC_MAX_ITEMS_PER_LAUNCH; launches of one item and of up to 16 have smaller tables) travel
@@ -25,9 +26,9 @@
 // Each wavefront issues its 2 or 4 independent 128-bit loads per stream before the first store.
 // Streams larger than the 256 MB last-level cache are nontemporal on both sides (worth ~15 % over
 // plain accesses there); what fits the cache and was just produced, or is about to be consumed, is
-// left in it (cache_policy in odc_host.cpp), written through the L2s from 3 MiB on (output_form there), and so
-// is a part of what does not fit (resident_below there). Deeper unrolling or prefetching the next tile measured
-// slower: the memory system prefers a small window to more requests in flight.
+// left in it (cache_policy in odc_host.cpp), written through the L2s from 3 MiB on (output_form and those after it
+// there), and so is a part of what does not fit (resident_below there). Deeper unrolling or prefetching the next
+// tile measured slower: the memory system prefers a small window to more requests in flight.
 // Workgroup i runs on XCD i % 8; binding XCDs to address classes (256 B .. 64 KiB granules)
 // changed nothing measurable and giving every XCD one contiguous eighth of the tiles costs the
 // read-modify-write 3 %, so tiles are simply dealt out in address order: at any instant all
@@ -115,10 +116,10 @@ __device__ __forceinline__ void store_vec(V* p, V v) {  // aligned
 
 // A whole tile of a gather's output, converted or not, of a clear or of accumulations: vector `i` of the kVecs that
 // start at `tile`, an address that all lanes agree on. What the next kernel is to find in the last-level cache is
-// written through the L2 (output_form, cast_output_form and clear_form in odc_host.cpp say from which size on): left
-// in it by plain stores it goes to memory only at the kernel's end or as other lines push it out, between the
-// reads of whatever runs next. us, nontemporal / plain / written through (a decoder layer's nine parameters,
-// bf16, W = 8, three sets of buffers in turn):
+// written through the L2 (output_form, accumulation_form, store_output_form, cast_output_form and clear_form in
+// odc_host.cpp say from which size on): left in it by plain stores it goes to memory only at the kernel's end or as
+// other lines push it out, between the reads of whatever runs next. us, nontemporal / plain / written through (a
+// decoder layer's nine parameters, bf16, W = 8, three sets of buffers in turn):
 //   gather alone: 35 MiB of output 14.4 / 15.7 / 13.2, 48 MiB 18.6 / 16.7 / 15.4;
 //   an accumulate behind it, nothing reads the output: 32.1 / 31.9 / 29.4, 40.4 / 41.7 / 41.1;
 //   the products that read the parameters behind it (1024 tokens): 141 / 129 / 126.5, 184 / 160 / 158.5.

@@ -33,7 +33,7 @@ struct CachePolicy {
 
 // How a gather writes its output, an accumulate its accumulations or a clear its zeros: past the caches, through
 // the L2 into the last-level cache, or with plain stores (store_output in odc_kernels.hip, output_form and
-// clear_form in odc_host.cpp).
+// those after it in odc_host.cpp).
 enum OutputForm : uint32_t { kStream, kWriteThrough, kKeep };
 
 // The same for an accumulate: "read" is the gradient, "written" the accumulations, which are read through the
