@@ -640,7 +640,10 @@ class ReductionService:
     @dispatched_tasks.setter
     def dispatched_tasks(self, tasks: int) -> None:
         with self._lock:
-            self._tasks = self._landed_tasks + tasks
+            if tasks >= self._tasks - self._landed_tasks:
+                self._tasks = self._landed_tasks + tasks
+            else:  # (a wait in progress has noted _tasks, which therefore only grows)
+                self._landed_tasks = self._tasks - tasks
 
     def _landed(self, tasks: int) -> None:
         """The first ``tasks`` adds ever dispatched have landed; later ones, of other threads, stay counted."""

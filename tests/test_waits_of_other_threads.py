@@ -216,3 +216,16 @@ def test_tasks_dispatched_during_a_wait_stay_counted(streams):
         assert service.dispatched_tasks == 2
         service.sync()
         assert service.dispatched_tasks == 0
+
+
+def test_a_count_that_is_set_during_a_wait(streams):
+    service = ReductionService()
+    service.dispatched_tasks = 5
+    _release(streams)
+    with service.syncing():
+        service.dispatched_tasks = 0
+        assert service.dispatched_tasks == 0
+        service.dispatched_tasks += 2
+    assert service.dispatched_tasks == 2
+    service.sync()
+    assert service.dispatched_tasks == 0
